@@ -2,7 +2,8 @@
 //
 // For every spin s and particle type t with backflow between them,
 //   h_t += sum_{ip in t, idim} sum_{j,k} Re[(qa F)(qa F)]   (reptation.f:10241-10259)
-// which is the symmetric contraction sum_{r,q} M[r][q] S_t[r][q] over rows
+//   h_t -= sum_{ip in t, idim} sum_j qa qa (F_a F_b)_jj     (reptation.f:10195-10240)
+// of which the first is the symmetric contraction sum_{r,q} M[r][q] S_t[r][q] over rows
 // r = (j, a) of the spin's particles (R = 2m <= 128 rows) with
 //   M[(j,a),(k,b)] = Re(F_a(k,j) F_b(j,k))            (symmetric),
 //   S_t = V_t V_t^T,  V_t[(j,a),(ip,idim)] = qa(a,idim,j,ip),
@@ -36,21 +37,52 @@ __host__ __device__ constexpr bool xc_needs(int g, int h, int b) {
 
 #define XC_TPW 5  // most tiles per wavefront
 
+// real part of the product of two elements of F (complex, or real orbitals')
+__device__ __forceinline__ double xc_re(zd a, zd b) { return a.x * b.x - a.y * b.y; }
+__device__ __forceinline__ double xc_re(double a, double b) { return a * b; }
+
 // Empty statement that takes the accumulator in registers: the MFMAs that
 // produce it are issued before this point.
 __device__ __forceinline__ void xc_pin(xc_d4& a) { __asm__ volatile("" : "+v"(a)); }
 
-// Sums over the wavefront's tiles of M o S_0 and M o S_1, M formed from F
-// here once for both particle types (weight 2 off the diagonal).  The
-// accumulator of v_mfma_f64_16x16x4f64 holds, in lane l and register v,
-// element (row l/16 + 4v, column l%16) of the 16 x 16 tile.
+// The 2 x 2 diagonal blocks of S_t (rows and columns (j, a), (j, b); the
+// three distinct entries at index a + b), from the wavefronts that hold the
+// diagonal tiles: sd[(t * 64 + j) * 3 + a + b].
 template <int G, int H>
-__device__ __forceinline__ void xc_contract(const xc_d4 (&acc)[2][XC_TPW], const zd* __restrict__ Fg, int m,
-                                            int lane_in, int nT, double& t0, double& t1) {
+__device__ __forceinline__ void xc_diag_blocks(const xc_d4 (&acc)[2][XC_TPW], double* __restrict__ sd, int lane) {
+#pragma unroll
+  for (int q = 0; q < xc_nt(H); q++) {
+    const int TJ = xc_tj(G, xc_i0(H) + q), TK = xc_tk(G, xc_i0(H) + q);
+    if (TJ != TK) continue;
+    const int c = lane & 15;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int r = (lane >> 4) + 4 * v;
+      if ((r >> 1) == (c >> 1) && r <= c) {
+        const int e = (8 * TJ + (r >> 1)) * 3 + (r & 1) + (c & 1);
+        sd[e] = acc[0][q][v];
+        sd[192 + e] = acc[1][q][v];
+      }
+    }
+  }
+}
+
+// Sums over the wavefront's tiles of M o (S_t - S_t's diagonal blocks), M
+// formed from F here once for both particle types.  The diagonal blocks are
+// the second-derivative terms sum_ab (F_a F_b)_jj S_t[(j,a),(j,b)]
+// (reptation.f:10195-10240): (F_a F_b)_jj is the sum over k of M[(j,a),(k,b)],
+// so each element of M takes both S_t[(j,a),(k,b)] and the block of its row.
+// An element above the diagonal stands for its mirror image too, whose row is
+// its column.  The accumulator of v_mfma_f64_16x16x4f64 holds, in lane l and
+// register v, element (row l/16 + 4v, column l%16) of the 16 x 16 tile.
+template <int G, int H, typename Z>
+__device__ __forceinline__ void xc_contract(const xc_d4 (&acc)[2][XC_TPW], const double* __restrict__ sd,
+                                            const Z* __restrict__ Fg, int m, int lane_in, int nT, double& t0,
+                                            double& t1) {
   const int R = 2 * m;
   // the addresses of F are formed here, not hoisted out of the chunk loops
   // (where they would have to be spilled)
-  const zd* Fq = Fg;
+  const Z* Fq = Fg;
   int lane = lane_in;
   __asm__ volatile("" : "+s"(Fq), "+v"(lane));
   t0 = t1 = 0.0;
@@ -66,15 +98,20 @@ __device__ __forceinline__ void xc_contract(const xc_d4 (&acc)[2][XC_TPW], const
         const int r = 16 * TJ + (lane >> 4) + 4 * v;
         if (r < R && sc < R) {
           const int jr = r >> 1, ar = r & 1;
-          const zd f1 = Fq[(ar * m + ks) * m + jr];
-          const zd f2 = Fq[(bs * m + jr) * m + ks];
-          const double mv = f1.x * f2.x - f1.y * f2.y;
-          u0 = fma(mv, acc[0][q][v], u0);
-          u1 = fma(mv, acc[1][q][v], u1);
+          const double mv = xc_re(Fq[(ar * m + ks) * m + jr], Fq[(bs * m + jr) * m + ks]);
+          const double* dj = sd + 3 * jr + ar + bs;
+          if (TJ == TK) {
+            u0 = fma(mv, acc[0][q][v] - dj[0], u0);
+            u1 = fma(mv, acc[1][q][v] - dj[192], u1);
+          } else {
+            const double* dk = sd + 3 * ks + ar + bs;
+            u0 = fma(mv, 2.0 * acc[0][q][v] - (dj[0] + dk[0]), u0);
+            u1 = fma(mv, 2.0 * acc[1][q][v] - (dj[192] + dk[192]), u1);
+          }
         }
       }
-      t0 += TJ == TK ? u0 : 2.0 * u0;
-      t1 += TJ == TK ? u1 : 2.0 * u1;
+      t0 += u0;
+      t1 += u1;
     }
     // one tile's F values in flight at a time
     __asm__ volatile("" ::: "memory");
@@ -122,9 +159,9 @@ __shared__ __attribute__((aligned(16))) unsigned xc_sink[256];
 // double-buffered: while the matrix cores take this chunk's products the
 // vector units build the next chunk into the other buffer (two entries per
 // thread, placed between the MFMA steps), so a chunk costs one barrier.
-template <int G, int H>
+template <int G, int H, typename Z>
 __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ dsc, const double* __restrict__ Qd,
-                                        const zd* __restrict__ Fg, const double* __restrict__ xs,
+                                        const Z* __restrict__ Fg, const double* __restrict__ xs,
                                         double* __restrict__ Vt, double* red, int sp, int m, int p0, int tid) {
   const int lane = tid & 63;
   const int nT = (2 * m + 15) >> 4;
@@ -189,9 +226,9 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
         // quarter at every other step, so the contraction below reads it
         // from there instead of waiting on HBM tile by tile
         if (nt < 0 && (ks & 1)) {
-          const int nz = 2 * m * m;
+          const int nz = 2 * m * m * (int)sizeof(Z) / 16;
           for (int i = tid + (ks >> 1) * XC_THREADS; i < nz; i += 4 * XC_THREADS)
-            __builtin_amdgcn_global_load_lds((const void*)(Fg + i), (void __attribute__((address_space(3)))*)xc_sink,
+            __builtin_amdgcn_global_load_lds((const void*)((const double2*)Fg + i), (void __attribute__((address_space(3)))*)xc_sink,
                                              16, 0, 0);
         }
         // the next step's operands are read after this step's MFMAs issue
@@ -201,8 +238,11 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
       cur ^= 1;
     }
   }
+  // the chunk buffers are free: the diagonal blocks go there
+  xc_diag_blocks<G, H>(acc, Vt, lane);
+  __syncthreads();
   double u0, u1;
-  xc_contract<G, H>(acc, Fg, m, lane, nT, u0, u1);
+  xc_contract<G, H>(acc, Vt, Fg, m, lane, nT, u0, u1);
   u0 = block_sum<XC_THREADS>(u0, red);
   u1 = block_sum<XC_THREADS>(u1, red);
   if (tid == 0) {
@@ -213,9 +253,9 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
 
 // LDS: xs[2N], then two Vt[XC_KC][XC_RS] chunk buffers (column = (particle,
 // idim) of the chunk, row = (j, a)).
-__global__ __launch_bounds__(XC_THREADS, 4) void k_cross(DevSys s, WsLayout L, const double* __restrict__ x,
-                                                         double* __restrict__ ws,
-                                                         const double* __restrict__ Fbuf) {
+template <typename Z>
+__device__ __forceinline__ void k_cross_body(const DevSys& s, const WsLayout& L, const double* __restrict__ x,
+                                             double* __restrict__ ws, const double* __restrict__ Fbuf) {
   extern __shared__ __attribute__((aligned(16))) double sm[];
   __shared__ double red[XC_THREADS / 64];
   // walkers and spins in the reverse of the order in which k_gjm wrote their
@@ -231,7 +271,7 @@ __global__ __launch_bounds__(XC_THREADS, 4) void k_cross(DevSys s, WsLayout L, c
   double* dsc = wsw + pick2(L.off_det, sp);
   if (dsc[DS_SING] != 0.0) return;
   const double* Qd = dsc + DS_N + 2 * N;
-  const zd* Fg = (const zd*)(Fbuf + (int64_t)w * L.f_per_walker + pick2(L.f_off, sp));
+  const Z* Fg = (const Z*)(Fbuf + (int64_t)w * L.f_per_walker + pick2(L.f_off, sp));
   double* xs = sm;
   double* Vt = sm + 2 * N;
   const double* xw = x + (int64_t)w * 2 * N;
@@ -247,4 +287,18 @@ __global__ __launch_bounds__(XC_THREADS, 4) void k_cross(DevSys s, WsLayout L, c
     case 6: xc_body<2, 1>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
     default: xc_body<3, 1>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
   }
+}
+
+// F complex (k_gjm, k_det)
+__global__ __launch_bounds__(XC_THREADS, 4) void k_cross(DevSys s, WsLayout L, const double* __restrict__ x,
+                                                         double* __restrict__ ws,
+                                                         const double* __restrict__ Fbuf) {
+  k_cross_body<zd>(s, L, x, ws, Fbuf);
+}
+
+// F real (k_gjr)
+__global__ __launch_bounds__(XC_THREADS, 4) void k_cross_real(DevSys s, WsLayout L, const double* __restrict__ x,
+                                                              double* __restrict__ ws,
+                                                              const double* __restrict__ Fbuf) {
+  k_cross_body<double>(s, L, x, ws, Fbuf);
 }

@@ -75,6 +75,11 @@ struct DevSys {
   // orbitals
   const double* gvec;      // [ng][2]
   int ng, has_det;
+  // real orbitals: every spin's plane waves come with their opposites.  Per
+  // spin the pairs' g vectors [nslot][2], the zero vector (zslot = 1) first as
+  // a pair of its own
+  int real_orb, nslot[2], zslot[2];
+  const double* gpair[2];
   // walkers evaluated: the first *nact of the batch when not null (the
   // reptation sweep evaluates only the reptiles that still move a bead)
   const int* nact;
@@ -304,11 +309,11 @@ __device__ __forceinline__ int ptype(const DevSys& s, int i) { return i >= s.ipf
 // (weight 3: both ends take drift terms) then nB = 64 steps across to the
 // other type (weight 2), split into four runs of equal weight, one per
 // wavefront.  A wavefront's LDS partial sums hold the backflow sums qb[5][64]
-// of the spin's particles, then zs[6][64] (drift and Laplacian terms of the
-// spin's particles) when its run has own-block steps and zo[6][64] (those of
+// of the spin's particles, then zs[5][64] (drift and Laplacian terms of the
+// spin's particles) when its run has own-block steps and zo[5][64] (those of
 // the other type) when it has steps across.  Scalar functions of (nA, nB, w)
 // rather than a table, which a varying w would index in scratch memory.
-#define FG_NZ 6
+#define FG_NZ 5
 #define FG_NQ 5
 // first step of wavefront w's run (w = 4: the end)
 __host__ __device__ inline int fg_u(int nA, int nB, int w) {
@@ -356,10 +361,24 @@ __device__ __forceinline__ double gj_readlane(double v, int l) {
 
 // Block-wide sum of a double over QMC_BLOCK threads; red must hold
 // QMC_BLOCK/64 doubles.  All threads get the result.
+// v of the lane a DPP control names (every lane of the row active).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+}
+// Sum over the wavefront in every lane (all lanes active): quads by DPP
+// swaps, rows of 16 by DPP rotations, then the four row sums from the scalar
+// side.  Register moves throughout: a shuffle goes through the LDS unit, six
+// of which in a chain take several times as long.
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v += dpp_f64<0xB1>(v);
+  v += dpp_f64<0x4E>(v);
+  v += dpp_f64<0x124>(v);
+  v += dpp_f64<0x128>(v);
+  return (gj_readlane(v, 0) + gj_readlane(v, 16)) + (gj_readlane(v, 32) + gj_readlane(v, 48));
 }
 // Sum over a workgroup of NT threads (red holds NT / 64 doubles).
 template <int NT = QMC_BLOCK>

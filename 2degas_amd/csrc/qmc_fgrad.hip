@@ -1,11 +1,10 @@
-// qmc_fgrad.hip -- drift and diagonal Laplacian terms of the backflow
-// determinants for up to 64 particles per spin (reptation.f:10195-10240).
+// qmc_fgrad.hip -- drift and first-derivative Laplacian terms of the backflow
+// determinants for up to 64 particles per spin (reptation.f:10195-10240; the
+// second-derivative terms are k_cross's).
 //
-// The per-orbital factors d_j = F_b(j,j) and diag(A^-1 G_a G_b A)_j =
-// sum_k F_a(j,k) F_b(k,j) (A^-1 G_a G_b A = F_a F_b) come from the
-// determinant kernel (k_gjm stores them beside the determinant scalars);
-// this kernel adds the backflow Jacobian, regenerated from the eta table,
-// over the pairs.
+// The per-orbital factors d_j = F_b(j,j) come from the determinant kernel
+// (stored beside the determinant scalars); this kernel adds the backflow
+// Jacobian, regenerated from the eta table, over the pairs.
 //
 // One workgroup per (walker, spin sp); every pair with a particle of sp is
 // evaluated once, on the round-robin schedule of k_pairs: steps d = 1..32 of
@@ -18,11 +17,11 @@
 // in LDS, which are added in a fixed order at the end.
 #include "qmc_dev.h"
 
-// LDS: xs[2N], dl[4][64] (F_x(j,j), F_y(j,j) as re, im), dd[3][64] (diag of
-// F_x F_x, F_x F_y, F_y F_y), component-major so that lanes reading the
-// factors of consecutive particles touch consecutive banks, then the
-// wavefronts' partial sums where fg_off puts them (drift and Laplacian terms
-// zxr, zxi, zyr, zyi, hq, hd; backflow block Q11, Q12, Q22, bx, by).
+// LDS: xs[2N], dl[4][64] (F_x(j,j), F_y(j,j) as re, im), component-major so
+// that lanes reading the factors of consecutive particles touch consecutive
+// banks, then the wavefronts' partial sums where fg_off puts them (drift and
+// Laplacian terms zxr, zxi, zyr, zyi, hq; backflow block Q11, Q12, Q22, bx,
+// by).
 __global__ __launch_bounds__(QMC_BLOCK) void k_fgrad(DevSys s, WsLayout L,
                                                      const double* __restrict__ x,
                                                      double* __restrict__ ws) {
@@ -40,16 +39,13 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_fgrad(DevSys s, WsLayout L,
   if (dsc[DS_SING] != 0.0) return;
   double* xs = sm;
   double* dl = sm + 2 * N;
-  double* dd = dl + 4 * 64;
-  double* parts = dd + 3 * 64;
+  double* parts = dl + 4 * 64;
   const double* xw = x + (int64_t)w * 2 * N;
   for (int k = tid; k < 2 * N; k += QMC_BLOCK) xs[k] = xw[k];
   const double* Fd = dsc + DS_N + 2 * N + 3 * m;
   for (int e = tid; e < m; e += QMC_BLOCK) {
 #pragma unroll
-    for (int c = 0; c < 4; c++) dl[c * 64 + e] = Fd[7 * e + c];
-#pragma unroll
-    for (int c = 0; c < 3; c++) dd[c * 64 + e] = Fd[7 * e + 4 + c];
+    for (int c = 0; c < 4; c++) dl[c * 64 + e] = Fd[4 * e + c];
   }
   const int ot = 1 - sp;
   const int mo = s.ntypes > 1 ? pick2(s.np, ot) : 0;
@@ -72,14 +68,12 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_fgrad(DevSys s, WsLayout L,
   const bool li = l < m;
   const int ip = p0 + l;
   const double xi = li ? xs[2 * ip] : 0.0, yi = li ? xs[2 * ip + 1] : 0.0;
-  double dlr[4] = {0, 0, 0, 0}, ddr[3] = {0, 0, 0};
+  double dlr[4] = {0, 0, 0, 0};
   if (li) {
 #pragma unroll
     for (int c = 0; c < 4; c++) dlr[c] = dl[c * 64 + l];
-#pragma unroll
-    for (int c = 0; c < 3; c++) ddr[c] = dd[c * 64 + l];
   }
-  double iz[FG_NZ] = {0, 0, 0, 0, 0, 0}, iq[FG_NQ] = {0, 0, 0, 0, 0};
+  double iz[FG_NZ] = {0, 0, 0, 0, 0}, iq[FG_NQ] = {0, 0, 0, 0, 0};
   for (int u = u0; u < u1; u++) {
     const bool blkA = u < nA;
     const int d = blkA ? u + 1 : u - nA;
@@ -96,7 +90,6 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_fgrad(DevSys s, WsLayout L,
     const double cb = deta * p.byr;
     const double mb11 = eta + cb * p.ux * p.ux, mb12 = cb * p.ux * p.uy, mb22 = eta + cb * p.uy * p.uy;
     const double cc = ddeta + 3.0 * cb;
-    const double a11 = mb11 * mb11 + mb12 * mb12, a12 = mb12 * (mb11 + mb22), a22 = mb12 * mb12 + mb22 * mb22;
     // i's backflow block
     iq[0] += mb11;
     iq[1] += mb12;
@@ -109,7 +102,6 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_fgrad(DevSys s, WsLayout L,
     pz[2 * 64] -= dlr[0] * mb12 + dlr[2] * mb22;
     pz[3 * 64] -= dlr[1] * mb12 + dlr[3] * mb22;
     pz[4 * 64] += cc * (dlr[0] * p.ux + dlr[2] * p.uy);
-    pz[5 * 64] += ddr[0] * a11 + 2.0 * ddr[1] * a12 + ddr[2] * a22;
     if (blkA) {
       // j is a particle of the spin too: its backflow block, and i's terms
       // against j's orbital factors
@@ -125,7 +117,6 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_fgrad(DevSys s, WsLayout L,
       iz[2] -= dxr * mb12 + dyr * mb22;
       iz[3] -= dxi * mb12 + dyi * mb22;
       iz[4] -= cc * (dxr * p.ux + dyr * p.uy);
-      iz[5] += dd[jl] * a11 + 2.0 * dd[64 + jl] * a12 + dd[128 + jl] * a22;
     }
   }
   if (li && u1 > u0) {
@@ -153,7 +144,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_fgrad(DevSys s, WsLayout L,
     }
     // the wavefronts' partial sums, added in wavefront order
     const int jx = insp ? pp - p0 : pp - pick2(s.ipf, ot);
-    double z[FG_NZ] = {0, 0, 0, 0, 0, 0}, q[FG_NQ] = {0, 0, 0, 0, 0};
+    double z[FG_NZ] = {0, 0, 0, 0, 0}, q[FG_NQ] = {0, 0, 0, 0, 0};
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       if (fg_u(nA, nB, v + 1) == fg_u(nA, nB, v)) continue;
@@ -178,8 +169,6 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_fgrad(DevSys s, WsLayout L,
       z[2] += dxr * a12 + dyr * a22;
       z[3] += dxi * a12 + dyi * a22;
       z[4] += dxr * q[3] + dyr * q[4];
-      const double b11 = a11 * a11 + a12 * a12, b12 = a12 * (a11 + a22), b22 = a12 * a12 + a22 * a22;
-      z[5] += dd[jf] * b11 + 2.0 * dd[64 + jf] * b12 + dd[128 + jf] * b22;
       Qd[3 * jf] = q[0];
       Qd[3 * jf + 1] = q[1];
       Qd[3 * jf + 2] = q[2];
@@ -187,8 +176,8 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_fgrad(DevSys s, WsLayout L,
     gdet[2 * pp] = -z[0];
     gdet[2 * pp + 1] = -z[2];
     acc_g2 += pick2(s.hbs2m, ti) * (z[1] * z[1] + z[3] * z[3]);
-    if (ti == 0) acc_h0 -= z[4] + z[5];
-    else acc_h1 -= z[4] + z[5];
+    if (ti == 0) acc_h0 -= z[4];
+    else acc_h1 -= z[4];
   }
   acc_g2 = block_sum(acc_g2, red);
   acc_h0 = block_sum(acc_h0, red);

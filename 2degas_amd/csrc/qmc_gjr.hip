@@ -1,0 +1,305 @@
+// qmc_gjr.hip -- determinant path for real orbitals: spins whose plane waves
+// come with their opposites (every untwisted closed shell), up to 64
+// particles per spin.
+//
+// With g and -g both occupied the two rows e^{+-i g.q} of A are a constant
+// combination of cos(g.q) and sin(g.q) (a 2 x 2 block of determinant -2i), so
+// with R the real matrix of those rows F_b = A^-1 (i g^b A) equals
+// R^-1 D_b R, D_b R being the derivative rows (-g^b sin, g^b cos), and
+// log|det A| = log|det R| + (pairs) log 2.  Everything is real: a quarter of
+// the arithmetic of the complex matrices of qmc_gjm.hip and half of their
+// registers.
+//
+// One workgroup of NT wavefronts per (walker, spin), NT the 16-row tiles of R.
+// The augmented matrix [R | D_x R | D_y R] is held in v_mfma_f64_16x16x4f64
+// accumulators, wavefront c holding column tile c of each of the three parts
+// (3 NT tiles), and R is eliminated by Gauss-Jordan steps with partial
+// pivoting, so that row p_k of the two right parts ends as piv_k F_b(k, .):
+// there is no inverse and no second product.  Columns are eliminated in
+// blocks of 4.  The wavefront that holds the block's columns passes them
+// through LDS (lane = row), takes the 4 pivot steps and posts the block's row
+// operations as a rank-4 update M += F' U, U the block's 4 pivot rows as they
+// were before it.  Every wavefront takes U for its own columns from its own
+// accumulators, so one barrier per block suffices, the posted operands being
+// double buffered.  Column tiles of R whose columns are all eliminated are
+// left out.
+//
+// Rows: the two rows of plane-wave pair n sit in one lane of a tile (rows
+// r and r + 4), so that one sin/cos gives R and both derivatives of both
+// rows.  A zero plane wave is the cos row of a pair of its own, whose sin row
+// does not take part.
+#include <type_traits>
+
+#include "qmc_dev.h"
+
+typedef double gr_d4 __attribute__((ext_vector_type(4)));
+
+template <int NT>
+struct GrShared {
+  double q[2 * 64], g[2 * 32];
+  double panel[16 * NT * 4];      // the block's columns, row r at 4 r
+  double Fl[2][16 * NT * 4];      // F' of the block, row r at 4 r
+  double u[NT][3][4 * 16];        // per wavefront: the block's pivot rows in its column tiles
+  double pinv[16 * NT], pabs[16 * NT];  // by pivot row
+  int prow[2][4];
+  int rank[16 * NT];              // step of pivot row r, -1: none
+  int used[16 * NT];
+  int sing;
+};
+
+__device__ __forceinline__ gr_d4 gr_mfma(double a, double b, gr_d4 c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// 1/d: hardware reciprocal and two Newton steps.
+__device__ __forceinline__ double gr_rcp(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  double e = fma(-d, y, 1.0);
+  y = fma(y, e, y);
+  e = fma(-d, y, 1.0);
+  return fma(y, e, y);
+}
+
+// LDS traffic between lanes of one wavefront.
+__device__ __forceinline__ void gr_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// f(integral_constant<i>) for the uniform run-time i in [0, 4 NT): a jump,
+// since registers cannot be indexed by a run-time value.
+template <int NT, class F>
+__device__ __forceinline__ void gr_switch(int i, F&& f) {
+#define GR_CASE(k)                                                     \
+  case k:                                                              \
+    if constexpr (k < 4 * NT) f(std::integral_constant<int, k>{});     \
+    break;
+  switch (i) {
+    GR_CASE(0) GR_CASE(1) GR_CASE(2) GR_CASE(3) GR_CASE(4) GR_CASE(5) GR_CASE(6) GR_CASE(7)
+    GR_CASE(8) GR_CASE(9) GR_CASE(10) GR_CASE(11) GR_CASE(12) GR_CASE(13) GR_CASE(14) GR_CASE(15)
+  }
+#undef GR_CASE
+}
+
+// The pivot steps of columns k0..k0+nb-1 (panel in LDS) by one wavefront,
+// lane = row.  Pivot: the largest magnitude among the unused rows, rows whose
+// top 14 bits agree in the order of their index.  Every lane forms the
+// reciprocal of its own entry while the maximum is searched, so that the
+// chain waits for the longer of the two only.
+template <int NT>
+__device__ __forceinline__ void gr_pivots(GrShared<NT>& sh, int buf, int k0, int nb, int lane) {
+  const bool in = NT == 4 || lane < 16 * NT;
+  double P[4] = {0, 0, 0, 0}, Fp[4] = {0, 0, 0, 0};
+  bool used = true;
+  if (in) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) P[j] = sh.panel[4 * lane + j];
+    used = sh.used[lane] != 0;
+  }
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    if (j < nb) {
+      const unsigned top = (unsigned)(__double_as_longlong(P[j]) >> 32) & 0x7fffffffu;
+      const unsigned key = used ? 0u : ((((top >> 6) + 1u) << 6) | (unsigned)(63 - lane));
+      const double ri = gr_rcp(P[j]);
+      const int p = 63 - (int)(gj_wave_max(key) & 63u);
+      const double pi = gj_readlane(ri, p);
+      const bool me = lane == p;
+      const double nf = me ? 0.0 : -(P[j] * pi);
+#pragma unroll
+      for (int jj = j + 1; jj < 4; jj++) P[jj] = fma(nf, gj_readlane(P[jj], p), P[jj]);
+#pragma unroll
+      for (int i = 0; i < j; i++) Fp[i] = fma(nf, gj_readlane(Fp[i], p), Fp[i]);
+      Fp[j] = nf;
+      if (me) {
+        used = true;
+        const double a = fabs(P[j]);
+        sh.prow[buf][j] = p;
+        sh.rank[p] = k0 + j;
+        sh.pinv[p] = pi;
+        sh.pabs[p] = a;
+        sh.used[p] = 1;
+        if (!(a > 0.0)) sh.sing = 1;
+      }
+    }
+  }
+  if (in) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) sh.Fl[buf][4 * lane + j] = Fp[j];
+  }
+}
+
+template <int NT, bool VAL>
+__global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLayout L, double* __restrict__ ws,
+                                                                  double* __restrict__ Fbuf, int sp0) {
+  constexpr int NP = VAL ? 1 : 3;  // parts of the augmented matrix
+  __shared__ __attribute__((aligned(16))) GrShared<NT> sh;
+  const int w = blockIdx.x, sp = sp0 + blockIdx.y;
+  if (s.nact && w >= *s.nact) return;
+  const int m = pick2(s.np, sp);
+  if (m == 0) return;
+  const int p0 = pick2(s.ipf, sp), nslot = pick2(s.nslot, sp), zero = pick2(s.zslot, sp);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // MFMA lane roles: accumulator rows lr + 4v, column lc; operand k index lr
+  const int lr = lane >> 4, lc = lane & 15;
+  const int ct = wave, col = 16 * ct + lc;
+  const double* qw = ws + (int64_t)w * L.per_walker + L.off_q + 2 * p0;
+  const double* gp = sp ? s.gpair[1] : s.gpair[0];
+  for (int e = tid; e < 2 * m; e += 64 * NT) sh.q[e] = qw[e];
+  for (int e = tid; e < 2 * nslot; e += 64 * NT) sh.g[e] = gp[e];
+  for (int r = tid; r < 16 * NT; r += 64 * NT) {
+    // row r = 16 T + lr + 4 v: pair T * 8 + (v >> 1) * 4 + lr, cos (v even) or sin
+    const int v = (r >> 2) & 3, sl = (r >> 4) * 8 + (v >> 1) * 4 + (r & 3);
+    sh.used[r] = sl >= nslot || (zero && sl == 0 && (v & 1));
+    sh.rank[r] = -1;
+  }
+  if (tid == 0) sh.sing = 0;
+  __syncthreads();
+
+  gr_d4 acc[NP][NT];
+  {
+    const bool jn = col < m;
+    const double qx = jn ? sh.q[2 * col] : 0.0, qy = jn ? sh.q[2 * col + 1] : 0.0;
+#pragma unroll
+    for (int T = 0; T < NT; T++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int sl = T * 8 + h * 4 + lr;
+        double sv = 0.0, cv = 0.0, gx = 0.0, gy = 0.0;
+        if (jn && sl < nslot) {
+          gx = sh.g[2 * sl];
+          gy = sh.g[2 * sl + 1];
+          qsincos_sreg(gx * qx + gy * qy, &sv, &cv);
+        }
+        acc[0][T][2 * h] = cv;
+        acc[0][T][2 * h + 1] = sv;
+        if constexpr (!VAL) {
+          acc[1][T][2 * h] = -gx * sv;
+          acc[1][T][2 * h + 1] = gx * cv;
+          acc[2][T][2 * h] = -gy * sv;
+          acc[2][T][2 * h + 1] = gy * cv;
+        }
+      }
+  }
+  // the block's columns from the accumulators of the wavefront that holds
+  // them to LDS, and its pivot steps
+  auto panel = [&](int k0, int buf) {
+    const int j = lc - (k0 & 15);
+    if (j >= 0 && j < 4) {
+#pragma unroll
+      for (int T = 0; T < NT; T++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) sh.panel[4 * (16 * T + lr + 4 * v) + j] = acc[0][T][v];
+    }
+    gr_wave_sync();
+    // every other wavefront waits for these steps: they issue first
+    __builtin_amdgcn_s_setprio(1);
+    gr_pivots<NT>(sh, buf, k0, min(4, m - k0), lane);
+    __builtin_amdgcn_s_setprio(0);
+  };
+  if (ct == 0) panel(0, 0);
+  for (int k0 = 0; k0 < m; k0 += 4) {
+    const int buf = (k0 >> 2) & 1, nb = min(4, m - k0);
+    __syncthreads();
+    const bool left = (k0 >> 4) <= ct;  // R's columns here are not all eliminated
+    double* ub = &sh.u[wave][0][0];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      if (k < nb) {
+        const int p = __builtin_amdgcn_readfirstlane(sh.prow[buf][k]);
+        const bool me = lr == (p & 3);
+        gr_switch<NT>(p >> 2, [&](auto ic) {
+          constexpr int I = decltype(ic)::value;
+          if (me) {
+#pragma unroll
+            for (int t = 0; t < NP; t++) ub[t * 64 + k * 16 + lc] = acc[t][I >> 2][I & 3];
+          }
+        });
+      }
+    }
+    gr_wave_sync();
+    double fo[NT], uo[NP];
+#pragma unroll
+    for (int T = 0; T < NT; T++) fo[T] = sh.Fl[buf][4 * (16 * T + lc) + lr];
+#pragma unroll
+    for (int t = 0; t < NP; t++) uo[t] = lr < nb ? ub[t * 64 + lane] : 0.0;
+    if (left) {
+#pragma unroll
+      for (int T = 0; T < NT; T++) acc[0][T] = gr_mfma(fo[T], uo[0], acc[0][T]);
+    }
+    if constexpr (!VAL) {
+#pragma unroll
+      for (int t = 1; t < 3; t++)
+#pragma unroll
+        for (int T = 0; T < NT; T++) acc[t][T] = gr_mfma(fo[T], uo[t], acc[t][T]);
+    }
+    if (k0 + 4 < m && ((k0 + 4) >> 4) == ct) panel(k0 + 4, buf ^ 1);
+  }
+  __syncthreads();
+  double* dsc = ws + (int64_t)w * L.per_walker + pick2(L.off_det, sp);
+  if constexpr (!VAL) {
+    // F_b(k, j): row p_k of part b over piv_k; the diagonal also goes to the
+    // per-orbital terms (real and imaginary parts)
+    double* Fd = dsc + DS_N + 2 * s.nptot + 3 * m;
+    double* Fg = Fbuf + (int64_t)w * L.f_per_walker + pick2(L.f_off, sp);
+    const int j = col;
+    if (j < m) {
+#pragma unroll
+      for (int T = 0; T < NT; T++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const int r = 16 * T + lr + 4 * v;
+          const int k = sh.rank[r];
+          if (k >= 0) {
+            const double pi = sh.pinv[r];
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+              const double f = acc[1 + b][T][v] * pi;
+              Fg[(b * m + k) * m + j] = f;
+              if (k == j) {
+                Fd[4 * j + 2 * b] = f;
+                Fd[4 * j + 2 * b + 1] = 0.0;
+              }
+            }
+          }
+        }
+    }
+  }
+  if (wave == 0) {
+    const bool piv = lane < 16 * NT && sh.rank[lane < 16 * NT ? lane : 0] >= 0;
+    const double t = wave_sum(piv ? log(sh.pabs[lane]) : 0.0);
+    if (lane == 0) {
+      dsc[DS_LOGDET] = t + (nslot - zero) * 0.6931471805599453;
+      dsc[DS_SING] = sh.sing ? 1.0 : 0.0;
+    }
+  }
+}
+
+template <bool VAL>
+static void gjr_spins(const DevSys& s, const WsLayout& L, int nw, int sp0, int nsp, int nt, double* ws, double* F,
+                      hipStream_t st) {
+  const dim3 grid(nw, nsp);
+  switch (nt) {
+    case 1: hipLaunchKernelGGL((k_gjr<1, VAL>), grid, dim3(64), 0, st, s, L, ws, F, sp0); break;
+    case 2: hipLaunchKernelGGL((k_gjr<2, VAL>), grid, dim3(128), 0, st, s, L, ws, F, sp0); break;
+    case 3: hipLaunchKernelGGL((k_gjr<3, VAL>), grid, dim3(192), 0, st, s, L, ws, F, sp0); break;
+    default: hipLaunchKernelGGL((k_gjr<4, VAL>), grid, dim3(256), 0, st, s, L, ws, F, sp0); break;
+  }
+}
+
+// Queue the real determinant path of every spin on st: one launch when the
+// spins have the same tile count, else one per spin.  A spin of m particles
+// has m or, with the zero plane wave (m odd), m + 1 rows.
+void launch_gjr(const DevSys& s, const WsLayout& L, int nw, bool value, double* ws, double* F, hipStream_t st) {
+  int nt[2] = {0, 0};
+  for (int sp = 0; sp < s.ntypes; sp++) nt[sp] = s.np[sp] ? (2 * s.nslot[sp] + 15) / 16 : 0;
+  auto go = [&](int sp0, int nsp, int n) {
+    if (n == 0) return;
+    if (value) gjr_spins<true>(s, L, nw, sp0, nsp, n, ws, F, st);
+    else gjr_spins<false>(s, L, nw, sp0, nsp, n, ws, F, st);
+  };
+  if (s.ntypes == 2 && nt[0] == nt[1]) return go(0, 2, nt[0]);
+  for (int sp = 0; sp < s.ntypes; sp++) go(sp, 1, nt[sp]);
+}

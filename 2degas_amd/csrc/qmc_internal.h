@@ -110,6 +110,9 @@ int launch_eval(qmc_ctx* c, int nw, const double* d_x, double* d_props, double* 
 // nothing used; the matrix-core determinant path only.
 int launch_value(qmc_ctx* c, int nw, const double* d_x, double* d_ltf, int32_t* d_status, double* d_props,
                  hipStream_t st, int precision);
+// The real-orbital determinant kernels of every spin (s.real_orb); value:
+// log|det A| alone.
+void launch_gjr(const DevSys& s, const WsLayout& L, int nw, bool value, double* ws, double* F, hipStream_t st);
 void free_vmc(qmc_ctx* c);
 void free_vmc_graph(qmc_ctx* c);
 // Workspace of the evaluation kernels for nw walkers (allocates when it grows).

@@ -697,28 +697,13 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
         }
     }
   }
-  // diag(A^-1 d2A) real parts: dd[j] = (xx, xy, yy)
-  double* dd = U + 4 * m;
-  double* xs = dd + 3 * m;
-  for (int j = tid; j < m; j += QMC_BLOCK) {
-    double sxx = 0, sxy = 0, syy = 0;
-    for (int k = 0; k < m; k++) {
-      const zd P = zmul(A[k * m + j], Ag[k * m + j]);
-      const double gx = s.gvec[2 * k], gy = s.gvec[2 * k + 1];
-      sxx -= gx * gx * P.x;
-      sxy -= gx * gy * P.x;
-      syy -= gy * gy * P.x;
-    }
-    dd[3 * j] = sxx;
-    dd[3 * j + 1] = sxy;
-    dd[3 * j + 2] = syy;
-  }
+  double* xs = U + 4 * m;
   const double* xw = x + (int64_t)w * 2 * N;
   for (int k = tid; k < 2 * N; k += QMC_BLOCK) xs[k] = xw[k];
   __syncthreads();
 
-  // 5. drift and the diagonal Laplacian terms for every particle
-  // (reptation.f:10195-10240), with the backflow Jacobian qa and the
+  // 5. drift and the first-derivative Laplacian terms for every particle
+  // (reptation.f:10195-10240; the second-derivative ones are k_cross's), with the backflow Jacobian qa and the
   // quasi-coordinate Laplacian qb regenerated from the pair table.
   const double* dl = U;
   const int tpp = 1 << tpp_log2;
@@ -732,7 +717,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
     const int ti = act ? ptype(s, ip) : 0;
     const bool on = act && (sp ? pick2(s.iub_flag[1], ti) : pick2(s.iub_flag[0], ti));
     const bool insp = ip >= p0 && ip < p0 + m;
-    double zxr = 0, zxi = 0, zyr = 0, zyi = 0, hq = 0, hd = 0;
+    double zxr = 0, zxi = 0, zyr = 0, zyi = 0, hq = 0;
     double q11 = 0, q12 = 0, q22 = 0, bx = 0, by = 0;
     if (on) {
       const double xi = xs[2 * ip], yi = xs[2 * ip + 1];
@@ -762,9 +747,6 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
           zyi -= dxi * mb12 + dyi * mb22;
           // qb(.,ip,c) = -cc u
           hq -= cc * (dxr * p.ux + dyr * p.uy);
-          const double a11 = mb11 * mb11 + mb12 * mb12, a12 = mb12 * (mb11 + mb22),
-                       a22 = mb12 * mb12 + mb22 * mb22;
-          hd += dd[3 * jf] * a11 + 2.0 * dd[3 * jf + 1] * a12 + dd[3 * jf + 2] * a22;
         }
       }
     }
@@ -774,7 +756,6 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
       zyr += __shfl_xor(zyr, o, 64);
       zyi += __shfl_xor(zyi, o, 64);
       hq += __shfl_xor(hq, o, 64);
-      hd += __shfl_xor(hd, o, 64);
       q11 += __shfl_xor(q11, o, 64);
       q12 += __shfl_xor(q12, o, 64);
       q22 += __shfl_xor(q22, o, 64);
@@ -793,9 +774,6 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
           zyr += dxr * a12 + dyr * a22;
           zyi += dxi * a12 + dyi * a22;
           hq += dxr * bx + dyr * by;
-          const double b11 = a11 * a11 + a12 * a12, b12 = a12 * (a11 + a22),
-                       b22 = a12 * a12 + a22 * a22;
-          hd += dd[3 * jf] * b11 + 2.0 * dd[3 * jf + 1] * b12 + dd[3 * jf + 2] * b22;
           Qd[3 * jf] = q11;
           Qd[3 * jf + 1] = q12;
           Qd[3 * jf + 2] = q22;
@@ -803,8 +781,8 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
         gdet[2 * ip] = -zxr;
         gdet[2 * ip + 1] = -zyr;
         acc_g2 += pick2(s.hbs2m, ti) * (zxi * zxi + zyi * zyi);
-        if (ti == 0) acc_h0 -= hq + hd;
-        else acc_h1 -= hq + hd;
+        if (ti == 0) acc_h0 -= hq;
+        else acc_h1 -= hq;
       } else {
         gdet[2 * ip] = 0.0;
         gdet[2 * ip + 1] = 0.0;
