@@ -64,6 +64,15 @@ struct DevSys {
   double dkx, dky;
   const int* kxy;          // [nkslot] factorized rho_k slots: kxi | kyi << 8 | (k + 1) << 16
   int nkslot;
+  // FP64 rho_k: k = (+-kax_a, +-kby_b) over few distinct magnitudes (nkax = 0:
+  // direct sin/cos per k-vector); kaprog: both are arithmetic progressions
+  // with steps dkax, dkby.  kcell[a * 16 ceil(nkby / 16) + b] lists the cell's
+  // k-vectors, k * 4 + (kx < 0) * 2 + (ky < 0), -1 for none
+  int nkax, nkby, kaprog;
+  double dkax, dkby;
+  const double* kax;
+  const double* kby;
+  const int4* kcell;
   int nke[3];              // nk_ewald of the v2 table of each type pair
   const double* vk[3];     // [nke]
   double vk0[3];

@@ -41,6 +41,8 @@ struct qmc_ctx {
   double* d_gvec = nullptr;
   double* d_kxyv = nullptr;  // distinct kx then ky components
   int* d_kxy = nullptr;
+  double* d_kab = nullptr;   // distinct |kx| then |ky|
+  int4* d_kcell = nullptr;
   TpInfo* d_tpi = nullptr;
   // workspace sized for ws_nw walkers
   int ws_nw = 0;
@@ -110,6 +112,12 @@ int launch_eval(qmc_ctx* c, int nw, const double* d_x, double* d_props, double* 
 // nothing used; the matrix-core determinant path only.
 int launch_value(qmc_ctx* c, int nw, const double* d_x, double* d_ltf, int32_t* d_status, double* d_props,
                  hipStream_t st, int precision);
+// The pair kernel (qmc_kernels.hip): its LDS for kc particles per phase chunk,
+// the doubles of its FP64 phase rows, and its launch.
+size_t pairs_lds(const DevSys& s, int kc, bool mix);
+size_t rho_doubles(const DevSys& s, int kc);
+void launch_pairs(const DevSys& s, const WsLayout& L, int nw, bool mix, size_t lds, const double* x, double* ws,
+                  double* props, hipStream_t st);
 // The real-orbital determinant kernels of every spin (s.real_orb); value:
 // log|det A| alone.
 void launch_gjr(const DevSys& s, const WsLayout& L, int nw, bool value, double* ws, double* F, hipStream_t st);

@@ -18,9 +18,11 @@
 //             as a symmetric contraction of S = V V^T against M = Re(F o F^T).
 //   k_final   kinetic and potential energies and the property slots
 //             (kinetic, reptation.f:2729-2775; potential tail, 4088-4096).
+#include <algorithm>
 #include <type_traits>
+#include <utility>
 
-#include "qmc_dev.h"
+#include "qmc_internal.h"
 
 // k-vectors per thread and pass in k_pairs
 #define KMAXPT 4
@@ -28,36 +30,235 @@
 
 // ---------------------------------------------------------------------------
 // k_pairs
-// LDS: xs[2N], Gs[2N], red[8], then a region shared by the per-wavefront
-// partial sums of the pair passes (4 x 6 x N doubles) and, afterwards, the
-// kchunk x (nkxv + nkyv) phases of rho_k.
+// LDS: xs[2N], Gs[2N], ks[2N], red[8 NW], then a region shared by the partial
+// sums of the pair passes (NA x 6 x N doubles) and, afterwards, the phases of
+// rho_k.
 //
 // The pair passes visit every unordered pair once, on a round-robin
-// schedule: the particles of type t sit in lanes 0..np_t-1 of a block of 64
-// (np_t <= 64), and step d of block pair (I, J) pairs lane l of I with lane
-// (l + d) mod 64 of J, so within a step every lane has a distinct partner.
-// Within one type d runs over 1..32 (d = 32 on lanes 0..31 only), across the
-// two types over 0..63; the steps are split into four contiguous runs, one
-// per wavefront.  A pair's contribution to i stays in registers until the
-// wavefront's run leaves block I; its contribution to j is added to the
-// wavefront's own partial sums in LDS (distinct j within a step, so no two
-// lanes touch one address), and the four partial sums are added in a fixed
-// order afterwards: the result does not depend on scheduling.
+// schedule over blocks of P lanes, P = 16, 32 or 64 the power of two that
+// holds the larger type: the particles of type t sit in lanes 0..np_t-1 of a
+// block, and step d of block pair (I, J) pairs lane l of I with lane
+// (l + d) mod P of J, so within a step every lane has a distinct partner.
+// Within one type d runs over 1..P/2 (d = P/2 on the lower half of the lanes
+// only), across the two types over 0..P-1.  A wavefront takes 64 / P steps of
+// one block pair at a time, one per group of P lanes (P^2 / 32 wavefront
+// steps in all: with one group of 64 lanes for every size, N = 26 would take
+// 128 steps of 13 live lanes instead of 8), and the wavefront steps are split
+// into NW contiguous runs.  A pair's contribution to i stays in registers
+// until the wavefront's run leaves block I; its contribution to j is added to
+// the lane group's own partial sums in LDS (distinct j within a step, so no
+// two lanes touch one address), and the NA = NW 64 / P partial sums are added
+// in a fixed order afterwards: the result does not depend on scheduling.
+//
+// What bounds it: a step is a chain of some 1500 cycles (geometry, table
+// loads, spline, LDS sums), so short runs count where few walkers are in
+// flight, and occupancy where many are.  Measured, 8 wavefronts against 4:
+// N=74, 256 walkers 42 us (75 before the blocks of P lanes, with 4); N=58, 256
+// walkers 26 against 31 us, 8192 walkers 326 against 260; N=122, 4096 walkers
+// 500 against 528.  16 wavefronts: 701 us there.  The mixed kernel's FP32
+// phases need more registers, and 4 wavefronts are the better count at both
+// ends (N=122 413 against 554 us, N=58 at 8192 walkers 276 against 445).  The
+// count depends on the deck alone, not on the batch, so that a walker's result
+// does not depend on the batch it is in.
 #define PP_NQ 6  // per-particle sums of a pass
+template <bool MIX, int P>
+struct PairShape {
+  static constexpr int NW = P == 16 || MIX ? 4 : 8;  // wavefronts
+  static constexpr int T = 64 * NW, SUB = 64 / P, NA = NW * SUB;
+  static constexpr int OWN = P / 2 / SUB, ACROSS = P / SUB;  // wavefront steps of a block pair
+};
 
-// Step u of the schedule: block (particle type) pair and lane offset.
-__device__ __forceinline__ void rr_unit(int u, bool two, int t1, int& ti, int& tj, int& d) {
-  if (!two) { ti = tj = t1; d = u + 1; }
-  else if (u < 32) { ti = tj = 0; d = u + 1; }
-  else if (u < 64) { ti = tj = 1; d = u - 31; }
-  else { ti = 0; tj = 1; d = u - 64; }
-}
-
-// part[q * N + p] += v for the wavefront's partial sums
+// part[q * N + p] += v for the lane group's partial sums
 __device__ __forceinline__ void pp_add(double* part, int N, int p, const double (&v)[PP_NQ], int nq) {
 #pragma unroll
   for (int q = 0; q < PP_NQ; q++)
     if (q < nq) part[q * N + p] += v[q];
+}
+
+// The wavefront's run of pair steps: pair(ti, tj, T, i, j) for each of its
+// lanes' pairs, end(ti) when the run leaves block ti.
+template <bool MIX, int P, class Pair, class End>
+__device__ __forceinline__ void pair_run(const DevSys& s, int wv, int l, Pair&& pair, End&& end) {
+  using S = PairShape<MIX, P>;
+  const int lp = l & (P - 1), sub = l / P;
+  // schedule: both types present, or the one type t1
+  const bool two = s.ntypes > 1 && s.np[0] > 0 && s.np[1] > 0;
+  const int t1 = (s.ntypes > 1 && s.np[0] == 0) ? 1 : 0;
+  const int nU = two ? 2 * S::OWN + S::ACROSS : S::OWN;
+  const int u0 = wv * nU / S::NW, u1 = (wv + 1) * nU / S::NW;
+  // blocks (0, 0), (0, 1), (1, 1): type 0's own and across are one stretch of i
+  for (int blk = 0; blk < 3; blk++) {
+    if (!two && blk > 0) break;
+    const int ti = two ? (blk == 2 ? 1 : 0) : t1, tj = two ? (blk == 0 ? 0 : 1) : t1;
+    const int b0 = blk == 0 ? 0 : (blk == 1 ? S::OWN : S::OWN + S::ACROSS);
+    const int b1 = blk == 0 ? S::OWN : (blk == 1 ? S::OWN + S::ACROSS : 2 * S::OWN + S::ACROSS);
+    const int a = max(u0, b0), b = min(u1, b1);
+    if (a < b) {
+      const TpInfo* T = s.tpi + tpair(ti, tj);
+      const int ni = pick2(s.np, ti), nj = pick2(s.np, tj), i = pick2(s.ipf, ti) + lp;
+      for (int u = a; u < b; u++) {
+        const int d = (u - b0) * S::SUB + sub + (ti == tj ? 1 : 0);
+        const int jl = (lp + d) & (P - 1);
+        if (lp < ni && jl < nj && (ti != tj || d < P / 2 || lp < P / 2)) pair(ti, tj, T, i, pick2(s.ipf, tj) + jl);
+      }
+    }
+    if (u0 < u1 && (blk == 2 || !two || (blk == 1 && u0 < b1))) end(ti);
+  }
+}
+
+// The NA partial sums of each of the nq N per-particle sums, added in order
+// into the first one.
+template <bool MIX, int P>
+__device__ __forceinline__ void pp_reduce(double* parts, int N, int nq, int tid) {
+  using S = PairShape<MIX, P>;
+  __syncthreads();
+  for (int e = tid; e < nq * N; e += S::T) {
+    double v = parts[e];
+#pragma unroll
+    for (int a = 1; a < S::NA; a++) v += parts[a * PP_NQ * N + e];
+    parts[e] = v;
+  }
+  __syncthreads();
+}
+
+// Ewald sums over the k-vectors that carry coefficients, from the rho_k of a
+// k-vector: ordered type pairs (0,0), (0,1), (1,0), (1,1) (reptation.f:4034-4052).
+__device__ __forceinline__ void kspace_terms(const DevSys& s, int k, double c0, double s0, double c1, double s1,
+                                             double& pk0, double& pk1, double& pkt) {
+  if (k < s.nke[0]) {
+    const double aux = s.vk[0][k] * (c0 * c0 + s0 * s0);
+    pk0 += aux;
+    pkt += aux;
+  }
+  if (s.ntypes > 1) {
+    if (k < s.nke[1]) {
+      const double aux = s.vk[1][k] * (c0 * c1 + s0 * s1);
+      pk0 += aux;
+      pk1 += aux;
+      pkt += 2.0 * aux;
+    }
+    if (k < s.nke[2]) {
+      const double aux = s.vk[2][k] * (c1 * c1 + s1 * s1);
+      pk1 += aux;
+      pkt += aux;
+    }
+  }
+}
+
+// rho_k in FP64 on the matrix cores, for k-vectors over few distinct |kx| and
+// |ky|: with C_a, S_a = cos, sin(|kx|_a x_i) and likewise in y, the four
+// products CC, CS, SC, SS over a type's particles hold every sign combination
+// of (kx, ky) at once:
+//   rho = sum_i e^{i k.r_i} = (CC - sx sy SS) + i (sx SC + sy CS).
+// A task is one 16 x 16 tile of (a, b) of one type, 4 accumulators on one
+// wavefront; the phases of kchunk particles of each type at a time go to LDS
+// (row = particle: C_a, S_a, C_b, S_b), an operand being one 8-byte read a
+// lane.  On vector units, one product per k-vector, the same sums read three
+// 16-byte phases from LDS for each pair of k-vectors and particle and took
+// twice as many operations (both signs of ky separately).
+#define KRUN2 5  // phases of one particle from one sin/cos and the step's products
+typedef double pk_d4 __attribute__((ext_vector_type(4)));
+
+template <int P>
+__device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restrict__ xs, double* __restrict__ ks,
+                                          double* __restrict__ ph, double* __restrict__ pw, int tid) {
+  using S = PairShape<false, P>;
+  const int N = s.nptot, lane = tid & 63, lr = lane >> 4, lc = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int na = s.nkax, nb = s.nkby, ta = (na + 15) >> 4, tb = (nb + 15) >> 4;
+  const int ox = 16 * ta, oy = 32 * ta, ld = 32 * (ta + tb) + 16;
+  const int nt = s.ntypes > 1 ? 2 : 1, ntask = ta * tb * nt;
+  const int kc = (s.kchunk + 3) & ~3;  // rows per type and chunk
+  const int nmax = max(s.np[0], nt > 1 ? s.np[1] : 0);
+  // e^{i dk x}, e^{i dk y} of every particle
+  if (s.kaprog)
+    for (int e = tid; e < 2 * N; e += S::T) {
+      double sv, cv;
+      qsincos_sreg(((e & 1) ? s.dkby : s.dkax) * xs[e], &sv, &cv);
+      ks[2 * e] = cv;
+      ks[2 * e + 1] = sv;
+    }
+  for (int t0 = 0; t0 < ntask; t0 += S::NW) {
+    const int task = t0 + wv;
+    const bool on = task < ntask;
+    const int type = on ? task / (ta * tb) : 0, tile = on ? task % (ta * tb) : 0;
+    const int ra = 16 * (tile / tb), rb = 16 * (tile % tb);
+    pk_d4 cc{0, 0, 0, 0}, cs{0, 0, 0, 0}, sc{0, 0, 0, 0}, ss{0, 0, 0, 0};
+    for (int c0 = 0; c0 < nmax; c0 += kc) {
+      __syncthreads();
+      // rows: type t's particles c0..c0+kc-1 (zero beyond its count, up to a
+      // multiple of 4); items of a row: runs of KRUN2 phases
+      const int gx = (na + KRUN2 - 1) / KRUN2, ng = gx + (nb + KRUN2 - 1) / KRUN2;
+      for (int e = tid; e < nt * kc * ng; e += S::T) {
+        const int row = e / ng, g = e - row * ng;
+        const int t = row >= kc ? 1 : 0, c = c0 + row - t * kc;
+        const int np_t = pick2(s.np, t);
+        if (c >= ((np_t + 3) & ~3)) continue;
+        const bool isx = g < gx, live = c < np_t;
+        const int v0 = (isx ? g : g - gx) * KRUN2, n = isx ? na : nb, nrun = min(KRUN2, n - v0);
+        double* dst = ph + row * ld + (isx ? 0 : oy) + v0;
+        const int od = isx ? ox : 16 * tb;  // from the cosines to the sines
+        const int i = pick2(s.ipf, t) + c;
+        const double* kv = isx ? s.kax : s.kby;
+        const double u = live ? xs[2 * i + (isx ? 0 : 1)] : 0.0;
+        double sa = 0.0, ca = 0.0, sd = 0.0, cd = 0.0;
+        if (live) {
+          qsincos_sreg(kv[v0] * u, &sa, &ca);
+          if (s.kaprog) {
+            cd = ks[4 * i + (isx ? 0 : 2)];
+            sd = ks[4 * i + (isx ? 1 : 3)];
+          }
+        }
+        dst[0] = ca;
+        dst[od] = sa;
+#pragma unroll
+        for (int r = 1; r < KRUN2; r++) {
+          if (r < nrun) {
+            if (s.kaprog) {
+              const double c2 = fma(ca, cd, -sa * sd);
+              sa = fma(ca, sd, sa * cd);
+              ca = c2;
+            } else if (live) {
+              qsincos_sreg(kv[v0 + r] * u, &sa, &ca);
+            }
+            dst[r] = ca;
+            dst[od + r] = sa;
+          }
+        }
+      }
+      __syncthreads();
+      if (on) {
+        const int cn = min(kc, pick2(s.np, type) - c0);
+        const double* base = ph + (type * kc + lr) * ld + lc;
+        for (int k = 0; k < cn; k += 4) {
+          const double* row = base + k * ld;
+          const double ca = row[ra], sa = row[ox + ra], cb = row[oy + rb], sb = row[oy + 16 * tb + rb];
+          cc = __builtin_amdgcn_mfma_f64_16x16x4f64(ca, cb, cc, 0, 0, 0);
+          cs = __builtin_amdgcn_mfma_f64_16x16x4f64(ca, sb, cs, 0, 0, 0);
+          sc = __builtin_amdgcn_mfma_f64_16x16x4f64(sa, cb, sc, 0, 0, 0);
+          ss = __builtin_amdgcn_mfma_f64_16x16x4f64(sa, sb, ss, 0, 0, 0);
+        }
+      }
+    }
+    // each (a, b) cell's k-vectors: k * 4 + (kx < 0) * 2 + (ky < 0), -1 none
+    const int irk = on ? pick2(s.irhok, type) : 0;
+    if (irk) {
+      double* out = pw + s.jrhok + (irk - 1) * 2 * s.nk;
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int4 cell = s.kcell[(ra + lr + 4 * v) * 16 * tb + rb + lc];
+        const int ent[4] = {cell.x, cell.y, cell.z, cell.w};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          if (ent[q] < 0) continue;
+          const bool nx = ent[q] & 2, ny = ent[q] & 1;
+          const int k = ent[q] >> 2;
+          out[2 * k] = nx != ny ? cc[v] + ss[v] : cc[v] - ss[v];
+          out[2 * k + 1] = (nx ? -sc[v] : sc[v]) + (ny ? -cs[v] : cs[v]);
+        }
+      }
+    }
+  }
 }
 
 // MIX (the mixed-precision evaluation): the u2, u3 and pair-potential
@@ -66,109 +267,97 @@ __device__ __forceinline__ void pp_add(double* part, int N, int p, const double 
 // over each chunk of particles in FP32, the chunk sums added in FP64; the
 // pair geometry, the backflow coordinates, every accumulator and the k-space
 // sum stay FP64.
-template <bool MIX>
+template <bool MIX, int P>
 __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
                                              const double* __restrict__ x,
                                              double* __restrict__ ws,
                                              double* __restrict__ props) {
+  using S = PairShape<MIX, P>;
   extern __shared__ __attribute__((aligned(16))) double sm[];
   const int w = blockIdx.x;
   if (s.nact && w >= *s.nact) return;
   const int N = s.nptot;
   double* xs = sm;
-  double* Gs = sm + 2 * N;
-  double* red = sm + 4 * N;
-  double* parts = sm + 4 * N + 8;
+  double* Gs = sm + 2 * N;  // with ks: the phase steps of rho_k
+  double* red = sm + 6 * N;
+  double* parts = sm + 6 * N + 8 * S::NW;
   const double* xw = x + (int64_t)w * 2 * N;
   const int tid = threadIdx.x, l = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  double* part = parts + wv * PP_NQ * N;
-  for (int k = tid; k < 2 * N; k += QMC_BLOCK) xs[k] = xw[k];
-  for (int k = tid; k < 4 * PP_NQ * N; k += QMC_BLOCK) parts[k] = 0.0;
+  double* part = parts + (wv * S::SUB + l / P) * PP_NQ * N;
+  const int lp = l & (P - 1);
+  for (int k = tid; k < 2 * N; k += S::T) xs[k] = xw[k];
+  for (int k = tid; k < S::NA * PP_NQ * N; k += S::T) parts[k] = 0.0;
   __syncthreads();
   double* wsw = ws + (int64_t)w * L.per_walker;
   double acc_ltf = 0.0, acc_h0 = 0.0, acc_h1 = 0.0, acc_v0 = 0.0, acc_v1 = 0.0;
-  // schedule: both types present, or the one type t1
-  const bool two = s.ntypes > 1 && s.np[0] > 0 && s.np[1] > 0;
-  const int t1 = (s.ntypes > 1 && s.np[0] == 0) ? 1 : 0;
-  const int nU = two ? 128 : 32;
-  const int u0 = wv * nU / 4, u1 = (wv + 1) * nU / 4;
 
   // pass 1: u2, the pair term and G of u3, backflow q, pair potential
   {
     double ia[PP_NQ] = {0, 0, 0, 0, 0, 0};  // gx, gy, Gx, Gy, qx, qy of particle i
-    int icur = -1;
-    for (int u = u0; u < u1; u++) {
-      int ti, tj, d;
-      rr_unit(u, two, t1, ti, tj, d);
-      if (ti != icur) {
-        if (icur >= 0 && l < pick2(s.np, icur)) pp_add(part, N, pick2(s.ipf, icur) + l, ia, PP_NQ);
+    pair_run<MIX, P>(
+        s, wv, l,
+        [&](int ti, int tj, const TpInfo* T, int i, int j) {
+          const TabRef tu2{T->row[TK_U2], T->ng[TK_U2]}, tu3{T->row[TK_U3], T->ng[TK_U3]},
+              tb{T->row[TK_B], T->ng[TK_B]}, tv{T->row[TK_V], T->ng[TK_V]};
+          const double2 xi2 = ld2(xs, i), xj2 = ld2(xs, j);
+          PairGeo p = pair_geo(s, xi2.x, xi2.y, xj2.x, xj2.y);
+          double ja[PP_NQ] = {0, 0, 0, 0, 0, 0};
+          double hh = 0.0;
+          double f, df, ddf;
+          if (tu2.row0 >= 0) {
+            spline3m<MIX>(s, tu2, p.ind, p.rem, f, df, ddf);
+            acc_ltf += f;
+            const double dtr = df * p.byr;
+            ja[0] -= dtr * p.ux;
+            ja[1] -= dtr * p.uy;
+            hh += ddf + dtr;
+          }
+          if (tu3.row0 >= 0) {
+            spline3m<MIX>(s, tu3, p.ind, p.rem, f, df, ddf);
+            ja[2] += f * p.ux;
+            ja[3] += f * p.uy;
+            // (xi r)^2 pair term of the three-body factor (reptation.f:2822-2832)
+            const double r = p.r;
+            const double tr = f * r;
+            const double d3 = 2.0 * f * (f + r * df);
+            const double dd3 = 2.0 * (f * f + 4.0 * r * f * df + r * r * (df * df + ddf * f));
+            acc_ltf += tr * tr;
+            ja[0] -= d3 * p.ux;
+            ja[1] -= d3 * p.uy;
+            hh += dd3 + d3;
+          }
+          if (tb.row0 >= 0) {
+            spline3(s, tb, p.ind, p.rem, f, df, ddf);
+            ja[4] -= f * p.ux;
+            ja[5] -= f * p.uy;
+          }
+          // the pair gives i the opposite of j's vector terms (u -> -u)
 #pragma unroll
-        for (int q = 0; q < PP_NQ; q++) ia[q] = 0.0;
-        icur = ti;
-      }
-      const int jl = (l + d) & 63;
-      if (l < pick2(s.np, ti) && jl < pick2(s.np, tj) && (ti != tj || d < 32 || l < 32)) {
-        const int i = pick2(s.ipf, ti) + l, j = pick2(s.ipf, tj) + jl;
-        const TpInfo* T = s.tpi + tpair(ti, tj);
-        const TabRef tu2{T->row[TK_U2], T->ng[TK_U2]}, tu3{T->row[TK_U3], T->ng[TK_U3]},
-                     tb{T->row[TK_B], T->ng[TK_B]}, tv{T->row[TK_V], T->ng[TK_V]};
-        const double2 xi2 = ld2(xs, i), xj2 = ld2(xs, j);
-        PairGeo p = pair_geo(s, xi2.x, xi2.y, xj2.x, xj2.y);
-        double ja[PP_NQ] = {0, 0, 0, 0, 0, 0};
-        double hh = 0.0;
-        double f, df, ddf;
-        if (tu2.row0 >= 0) {
-          spline3m<MIX>(s, tu2, p.ind, p.rem, f, df, ddf);
-          acc_ltf += f;
-          const double dtr = df * p.byr;
-          ja[0] -= dtr * p.ux;
-          ja[1] -= dtr * p.uy;
-          hh += ddf + dtr;
-        }
-        if (tu3.row0 >= 0) {
-          spline3m<MIX>(s, tu3, p.ind, p.rem, f, df, ddf);
-          ja[2] += f * p.ux;
-          ja[3] += f * p.uy;
-          // (xi r)^2 pair term of the three-body factor (reptation.f:2822-2832)
-          const double r = p.r;
-          const double tr = f * r;
-          const double d3 = 2.0 * f * (f + r * df);
-          const double dd3 = 2.0 * (f * f + 4.0 * r * f * df + r * r * (df * df + ddf * f));
-          acc_ltf += tr * tr;
-          ja[0] -= d3 * p.ux;
-          ja[1] -= d3 * p.uy;
-          hh += dd3 + d3;
-        }
-        if (tb.row0 >= 0) {
-          spline3(s, tb, p.ind, p.rem, f, df, ddf);
-          ja[4] -= f * p.ux;
-          ja[5] -= f * p.uy;
-        }
-        // the pair gives i the opposite of j's vector terms (u -> -u)
+          for (int q = 0; q < PP_NQ; q++) ia[q] -= ja[q];
+          if (ti == 0) acc_h0 += hh; else acc_h1 += hh;
+          if (tj == 0) acc_h0 += hh; else acc_h1 += hh;
+          if (tv.row0 >= 0) {
+            const double vv = 0.5 * spline0<MIX>(s, tv, T->vexp, p.ind, p.rem, p.byr) * T->v2value;
+            if (ti == 0) acc_v0 += vv; else acc_v1 += vv;
+            if (tj == 0) acc_v0 += vv; else acc_v1 += vv;
+          }
+          pp_add(part, N, j, ja, PP_NQ);
+        },
+        [&](int ti) {
+          if (lp < pick2(s.np, ti)) pp_add(part, N, pick2(s.ipf, ti) + lp, ia, PP_NQ);
 #pragma unroll
-        for (int q = 0; q < PP_NQ; q++) ia[q] -= ja[q];
-        if (ti == 0) acc_h0 += hh; else acc_h1 += hh;
-        if (tj == 0) acc_h0 += hh; else acc_h1 += hh;
-        if (tv.row0 >= 0) {
-          const double vv = 0.5 * spline0<MIX>(s, tv, T->vexp, p.ind, p.rem, p.byr) * T->v2value;
-          if (ti == 0) acc_v0 += vv; else acc_v1 += vv;
-          if (tj == 0) acc_v0 += vv; else acc_v1 += vv;
-        }
-        pp_add(part, N, j, ja, PP_NQ);
-      }
-    }
-    if (icur >= 0 && l < pick2(s.np, icur)) pp_add(part, N, pick2(s.ipf, icur) + l, ia, PP_NQ);
+          for (int q = 0; q < PP_NQ; q++) ia[q] = 0.0;
+        });
   }
-  __syncthreads();
-  // per-particle sums in a fixed order; Gs for pass 2, q out, g kept
+  pp_reduce<MIX, P>(parts, N, PP_NQ, tid);
+  // Gs for pass 2, q out, g kept
   double gpx = 0.0, gpy = 0.0;  // gradient of particle tid (N <= 128)
-  for (int p = tid; p < N; p += QMC_BLOCK) {
+  if (tid < N) {
+    const int p = tid;
     double v[PP_NQ];
 #pragma unroll
-    for (int q = 0; q < PP_NQ; q++)
-      v[q] = ((parts[(0 * PP_NQ + q) * N + p] + parts[(1 * PP_NQ + q) * N + p]) +
-              parts[(2 * PP_NQ + q) * N + p]) + parts[(3 * PP_NQ + q) * N + p];
+    for (int q = 0; q < PP_NQ; q++) v[q] = parts[q * N + p];
     gpx = v[0];
     gpy = v[1];
     Gs[2 * p] = v[2];
@@ -185,89 +374,90 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   // with M = xi I + (xi'/r) u u^T and a = xi'' + 3 xi'/r; M and a.(u dG) are
   // even in the pair, M dG is odd
   if (s.has_u3) {
-    for (int k = tid; k < 4 * PP_NQ * N; k += QMC_BLOCK) parts[k] = 0.0;
+    for (int k = tid; k < S::NA * PP_NQ * N; k += S::T) parts[k] = 0.0;
     __syncthreads();
     double ia[PP_NQ] = {0, 0, 0, 0, 0, 0};  // g3x, g3y, e11, e12, e22 of particle i
-    int icur = -1;
-    for (int u = u0; u < u1; u++) {
-      int ti, tj, d;
-      rr_unit(u, two, t1, ti, tj, d);
-      if (ti != icur) {
-        if (icur >= 0 && l < pick2(s.np, icur)) pp_add(part, N, pick2(s.ipf, icur) + l, ia, 5);
+    pair_run<MIX, P>(
+        s, wv, l,
+        [&](int ti, int tj, const TpInfo* T, int i, int j) {
+          const TabRef tu3{T->row[TK_U3], T->ng[TK_U3]};
+          if (tu3.row0 < 0) return;
+          const double2 xi2 = ld2(xs, i), xj2 = ld2(xs, j);
+          PairGeo p = pair_geo(s, xi2.x, xi2.y, xj2.x, xj2.y);
+          double t, dt, ddt;
+          spline3m<MIX>(s, tu3, p.ind, p.rem, t, dt, ddt);
+          const double c = dt * p.byr;
+          const double m11 = t + c * p.ux * p.ux, m12 = c * p.ux * p.uy, m22 = t + c * p.uy * p.uy;
+          const double2 Gi = ld2(Gs, i), Gj = ld2(Gs, j);
+          const double dGx = Gi.x - Gj.x, dGy = Gi.y - Gj.y;
+          const double g3x = m11 * dGx + m12 * dGy, g3y = m12 * dGx + m22 * dGy;
+          const double nm2 = m11 * m11 + 2.0 * m12 * m12 + m22 * m22;
+          const double h3 = (ddt + 3.0 * c) * (p.ux * dGx + p.uy * dGy) - nm2;
+          ia[0] += g3x;
+          ia[1] += g3y;
+          ia[2] += m11;
+          ia[3] += m12;
+          ia[4] += m22;
+          const double ja[PP_NQ] = {-g3x, -g3y, m11, m12, m22, 0.0};
+          pp_add(part, N, j, ja, 5);
+          if (ti == 0) acc_h0 += h3; else acc_h1 += h3;
+          if (tj == 0) acc_h0 += h3; else acc_h1 += h3;
+        },
+        [&](int ti) {
+          if (lp < pick2(s.np, ti)) pp_add(part, N, pick2(s.ipf, ti) + lp, ia, 5);
 #pragma unroll
-        for (int q = 0; q < PP_NQ; q++) ia[q] = 0.0;
-        icur = ti;
-      }
-      const TpInfo* T = s.tpi + tpair(ti, tj);
-      const TabRef tu3{T->row[TK_U3], T->ng[TK_U3]};
-      const int jl = (l + d) & 63;
-      if (tu3.row0 >= 0 && l < pick2(s.np, ti) && jl < pick2(s.np, tj) && (ti != tj || d < 32 || l < 32)) {
-        const int i = pick2(s.ipf, ti) + l, j = pick2(s.ipf, tj) + jl;
-        const double2 xi2 = ld2(xs, i), xj2 = ld2(xs, j);
-        PairGeo p = pair_geo(s, xi2.x, xi2.y, xj2.x, xj2.y);
-        double t, dt, ddt;
-        spline3m<MIX>(s, tu3, p.ind, p.rem, t, dt, ddt);
-        const double c = dt * p.byr;
-        const double m11 = t + c * p.ux * p.ux, m12 = c * p.ux * p.uy, m22 = t + c * p.uy * p.uy;
-        const double2 Gi = ld2(Gs, i), Gj = ld2(Gs, j);
-        const double dGx = Gi.x - Gj.x, dGy = Gi.y - Gj.y;
-        const double g3x = m11 * dGx + m12 * dGy, g3y = m12 * dGx + m22 * dGy;
-        const double nm2 = m11 * m11 + 2.0 * m12 * m12 + m22 * m22;
-        const double h3 = (ddt + 3.0 * c) * (p.ux * dGx + p.uy * dGy) - nm2;
-        ia[0] += g3x;
-        ia[1] += g3y;
-        ia[2] += m11;
-        ia[3] += m12;
-        ia[4] += m22;
-        const double ja[PP_NQ] = {-g3x, -g3y, m11, m12, m22, 0.0};
-        pp_add(part, N, j, ja, 5);
-        if (ti == 0) acc_h0 += h3; else acc_h1 += h3;
-        if (tj == 0) acc_h0 += h3; else acc_h1 += h3;
-      }
-    }
-    if (icur >= 0 && l < pick2(s.np, icur)) pp_add(part, N, pick2(s.ipf, icur) + l, ia, 5);
-    __syncthreads();
-    for (int p = tid; p < N; p += QMC_BLOCK) {
+          for (int q = 0; q < PP_NQ; q++) ia[q] = 0.0;
+        });
+    pp_reduce<MIX, P>(parts, N, 5, tid);
+    if (tid < N) {
       double v[5];
 #pragma unroll
-      for (int q = 0; q < 5; q++)
-        v[q] = ((parts[(0 * PP_NQ + q) * N + p] + parts[(1 * PP_NQ + q) * N + p]) +
-                parts[(2 * PP_NQ + q) * N + p]) + parts[(3 * PP_NQ + q) * N + p];
+      for (int q = 0; q < 5; q++) v[q] = parts[q * N + tid];
       gpx += v[0];
       gpy += v[1];
       const double e2 = v[2] * v[2] + 2.0 * v[3] * v[3] + v[4] * v[4];
-      if (ptype(s, p) == 0) acc_h0 -= e2; else acc_h1 -= e2;
+      if (ptype(s, tid) == 0) acc_h0 -= e2; else acc_h1 -= e2;
     }
   }
-  for (int p = tid; p < N; p += QMC_BLOCK) {
-    wsw[L.off_gj + 2 * p] = gpx;
-    wsw[L.off_gj + 2 * p + 1] = gpy;
+  if (tid < N) {
+    wsw[L.off_gj + 2 * tid] = gpx;
+    wsw[L.off_gj + 2 * tid + 1] = gpy;
   }
 
   // rho_k per type and the k-space Ewald sum
   double pk0 = 0.0, pk1 = 0.0, pkt = 0.0;
-  if (s.nrhok) {
-    double* pw = props + (int64_t)w * s.n_props;
+  double* pw = props + (int64_t)w * s.n_props;
+  if (!MIX && s.nrhok && s.nkax > 0) {
+    __syncthreads();  // Gs and the partial sums have been read
+    rho_tiles<P>(s, xs, Gs, parts, pw, tid);
+    __syncthreads();  // rho_k of this walker is in memory
+    const double* r0 = s.irhok[0] ? pw + s.jrhok + (s.irhok[0] - 1) * 2 * s.nk : nullptr;
+    const double* r1 = s.ntypes > 1 && s.irhok[1] ? pw + s.jrhok + (s.irhok[1] - 1) * 2 * s.nk : nullptr;
+    for (int k = tid; k < s.nk; k += S::T)
+      kspace_terms(s, k, r0 ? r0[2 * k] : 0.0, r0 ? r0[2 * k + 1] : 0.0, r1 ? r1[2 * k] : 0.0,
+                   r1 ? r1[2 * k + 1] : 0.0, pk0, pk1, pkt);
+  } else if (s.nrhok) {
     // passes of KMAXPT slots per thread: slots q = 2h, 2h+1 of a thread are
     // the two k-vectors of one item, which share their ky component
-    for (int kb = 0; kb < s.nkslot; kb += KMAXPT * QMC_BLOCK) {
+    const bool items = MIX && s.nkxv > 0;  // else one slot per k-vector
+    const int nslot = items ? s.nkslot : s.nk;
+    for (int kb = 0; kb < nslot; kb += KMAXPT * S::T) {
       double rc0[KMAXPT], rc1[KMAXPT], rs0[KMAXPT], rs1[KMAXPT];
       int kq[KMAXPT];              // k-vector of slot q (-1: none)
       int ox[KMAXPT], oy[KMAXPT];  // kx and ky phase slots of slot q (0 when none)
 #pragma unroll
       for (int q = 0; q < KMAXPT; q++) {
         rc0[q] = rc1[q] = rs0[q] = rs1[q] = 0.0;
-        const int n = kb + 2 * (threadIdx.x + (q >> 1) * QMC_BLOCK) + (q & 1);
-        const int code = (n < s.nkslot && s.nkxv > 0) ? s.kxy[n] : 0;
-        kq[q] = n >= s.nkslot ? -1 : (s.nkxv > 0 ? (code >> 16) - 1 : n);
+        const int n = kb + 2 * (threadIdx.x + (q >> 1) * S::T) + (q & 1);
+        const int code = items && n < nslot ? s.kxy[n] : 0;
+        kq[q] = n >= nslot ? -1 : (items ? (code >> 16) - 1 : n);
         ox[q] = code & 0xff;
         oy[q] = ((code >> 8) & 0xff) + s.nkxv;
       }
-      if (s.nkxv > 0) {
+      if (items) {
         // e^{i k.x} = e^{i kx x} e^{i ky y}: per particle chunk, the distinct
         // x and y phases go to LDS, then each thread multiplies its k's pairs
-        using ph_t = typename std::conditional<MIX, float2, double2>::type;
-        ph_t* ph = (ph_t*)(sm + 4 * N + 8);
+        float2* ph = (float2*)parts;
         const int nv = s.nkxv + s.nkyv;
         for (int c0 = 0; c0 < N; c0 += s.kchunk) {
           const int cn = min(s.kchunk, N - c0);
@@ -276,7 +466,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
             // runs of KRUN phases: the first directly, the rest by products
             // with e^{i dk x} (at most KRUN - 1 roundings from a direct value)
             const int gx = (s.nkxv + KRUN - 1) / KRUN, ng = gx + (s.nkyv + KRUN - 1) / KRUN;
-            for (int e = threadIdx.x; e < cn * ng; e += QMC_BLOCK) {
+            for (int e = threadIdx.x; e < cn * ng; e += S::T) {
               const int pc = e / ng, g = e - pc * ng;
               const int i = c0 + pc;
               const bool isx = g < gx;
@@ -285,26 +475,26 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
               double sa, ca, sd, cd;
               qsincos_sreg((isx ? s.kxv[v0] : s.kyv[v0]) * u, &sa, &ca);
               qsincos_sreg((isx ? s.dkx : s.dky) * u, &sd, &cd);
-              ph_t* dst = ph + pc * nv + (isx ? 0 : s.nkxv) + v0;
-              dst[0] = ph_t{(decltype(ph_t::x))ca, (decltype(ph_t::x))sa};
+              float2* dst = ph + pc * nv + (isx ? 0 : s.nkxv) + v0;
+              dst[0] = float2{(float)ca, (float)sa};
 #pragma unroll
               for (int r = 1; r < KRUN; r++) {
                 if (r < nrun) {
                   const double c2 = fma(ca, cd, -sa * sd);
                   sa = fma(ca, sd, sa * cd);
                   ca = c2;
-                  dst[r] = ph_t{(decltype(ph_t::x))ca, (decltype(ph_t::x))sa};
+                  dst[r] = float2{(float)ca, (float)sa};
                 }
               }
             }
           } else {
-            for (int e = threadIdx.x; e < cn * nv; e += QMC_BLOCK) {
+            for (int e = threadIdx.x; e < cn * nv; e += S::T) {
               const int pc = e / nv, v = e - pc * nv;
               const int i = c0 + pc;
               const double arg = v < s.nkxv ? s.kxv[v] * xs[2 * i] : s.kyv[v - s.nkxv] * xs[2 * i + 1];
               double sv, cv;
               qsincos_sreg(arg, &sv, &cv);
-              ph[e] = ph_t{(decltype(ph_t::x))cv, (decltype(ph_t::x))sv};
+              ph[e] = float2{(float)cv, (float)sv};
             }
           }
           __syncthreads();
@@ -312,41 +502,27 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
           // type a loop of its own
           const int split = s.ntypes > 1 ? min(max(s.ipf[1] - c0, 0), cn) : cn;
           auto accum = [&](int pa, int pb, double (&rc)[KMAXPT], double (&rs)[KMAXPT]) {
-            if constexpr (!MIX) {
-              for (int pc = pa; pc < pb; pc++) {
-                const ph_t* row = ph + pc * nv;
+            // the chunk's products summed in FP32, the chunk sum added to
+            // the FP64 accumulators
+            float qc[KMAXPT], qs[KMAXPT];
 #pragma unroll
-                for (int h = 0; h < KMAXPT; h += 2) {
-                  // one ky phase for the item's two kx phases
-                  const ph_t b = row[oy[h]], a0 = row[ox[h]], a1 = row[ox[h + 1]];
-                  rc[h] = fma(a0.x, b.x, fma(-a0.y, b.y, rc[h]));
-                  rs[h] = fma(a0.x, b.y, fma(a0.y, b.x, rs[h]));
-                  rc[h + 1] = fma(a1.x, b.x, fma(-a1.y, b.y, rc[h + 1]));
-                  rs[h + 1] = fma(a1.x, b.y, fma(a1.y, b.x, rs[h + 1]));
-                }
+            for (int h = 0; h < KMAXPT; h++) qc[h] = qs[h] = 0.0f;
+            for (int pc = pa; pc < pb; pc++) {
+              const float2* row = ph + pc * nv;
+#pragma unroll
+              for (int h = 0; h < KMAXPT; h += 2) {
+                // one ky phase for the item's two kx phases
+                const float2 b = row[oy[h]], a0 = row[ox[h]], a1 = row[ox[h + 1]];
+                qc[h] = fmaf(a0.x, b.x, fmaf(-a0.y, b.y, qc[h]));
+                qs[h] = fmaf(a0.x, b.y, fmaf(a0.y, b.x, qs[h]));
+                qc[h + 1] = fmaf(a1.x, b.x, fmaf(-a1.y, b.y, qc[h + 1]));
+                qs[h + 1] = fmaf(a1.x, b.y, fmaf(a1.y, b.x, qs[h + 1]));
               }
-            } else {
-              // the chunk's products summed in FP32, the chunk sum added to
-              // the FP64 accumulators
-              float qc[KMAXPT], qs[KMAXPT];
+            }
 #pragma unroll
-              for (int h = 0; h < KMAXPT; h++) qc[h] = qs[h] = 0.0f;
-              for (int pc = pa; pc < pb; pc++) {
-                const ph_t* row = ph + pc * nv;
-#pragma unroll
-                for (int h = 0; h < KMAXPT; h += 2) {
-                  const ph_t b = row[oy[h]], a0 = row[ox[h]], a1 = row[ox[h + 1]];
-                  qc[h] = fmaf(a0.x, b.x, fmaf(-a0.y, b.y, qc[h]));
-                  qs[h] = fmaf(a0.x, b.y, fmaf(a0.y, b.x, qs[h]));
-                  qc[h + 1] = fmaf(a1.x, b.x, fmaf(-a1.y, b.y, qc[h + 1]));
-                  qs[h + 1] = fmaf(a1.x, b.y, fmaf(a1.y, b.x, qs[h + 1]));
-                }
-              }
-#pragma unroll
-              for (int h = 0; h < KMAXPT; h++) {
-                rc[h] += (double)qc[h];
-                rs[h] += (double)qs[h];
-              }
+            for (int h = 0; h < KMAXPT; h++) {
+              rc[h] += (double)qc[h];
+              rs[h] += (double)qs[h];
             }
           };
           accum(0, split, rc0, rs0);
@@ -389,38 +565,30 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
           pw[slot] = rc1[q];
           pw[slot + 1] = rs1[q];
         }
-        // ordered type pairs (0,0), (0,1), (1,0), (1,1) (reptation.f:4034-4052)
-        if (k < s.nke[0]) {
-          const double aux = s.vk[0][k] * (rc0[q] * rc0[q] + rs0[q] * rs0[q]);
-          pk0 += aux;
-          pkt += aux;
-        }
-        if (s.ntypes > 1) {
-          if (k < s.nke[1]) {
-            const double aux = s.vk[1][k] * (rc0[q] * rc1[q] + rs0[q] * rs1[q]);
-            pk0 += aux;
-            pk1 += aux;
-            pkt += 2.0 * aux;
-          }
-          if (k < s.nke[2]) {
-            const double aux = s.vk[2][k] * (rc1[q] * rc1[q] + rs1[q] * rs1[q]);
-            pk1 += aux;
-            pkt += aux;
-          }
-        }
+        kspace_terms(s, k, rc0[q], rs0[q], rc1[q], rs1[q], pk0, pk1, pkt);
       }
     }
   }
 
-  acc_ltf = block_sum(acc_ltf, red);
-  acc_h0 = block_sum(acc_h0, red);
-  acc_h1 = block_sum(acc_h1, red);
-  acc_v0 = block_sum(acc_v0, red);
-  acc_v1 = block_sum(acc_v1, red);
-  pk0 = block_sum(pk0, red);
-  pk1 = block_sum(pk1, red);
-  pkt = block_sum(pkt, red);
-  if (threadIdx.x == 0) {
+  // the walker's eight sums: over each wavefront, then over the wavefronts
+  {
+    const double v[8] = {wave_sum(acc_ltf), wave_sum(acc_h0), wave_sum(acc_h1), wave_sum(acc_v0),
+                         wave_sum(acc_v1),  wave_sum(pk0),    wave_sum(pk1),    wave_sum(pkt)};
+    if (l == 0) {
+#pragma unroll
+      for (int q = 0; q < 8; q++) red[8 * wv + q] = v[q];
+    }
+  }
+  __syncthreads();
+  if (wv != 0) return;
+  // lane q adds sum q of the wavefronts
+  double mine = 0.0;
+#pragma unroll
+  for (int a = 0; a < S::NW; a++) mine += red[8 * a + (l & 7)];
+  double v[8];
+#pragma unroll
+  for (int q = 0; q < 8; q++) v[q] = gj_readlane(mine, q);
+  if (l == 0) {
     double c0 = 0.0, c1 = 0.0, ct = 0.0;
     for (int it = 0; it < s.ntypes; it++)
       for (int jt = 0; jt < s.ntypes; jt++) {
@@ -433,29 +601,76 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
         }
       }
     double* sc = wsw + L.off_sc;
-    sc[SC_LTF] = acc_ltf;
-    sc[SC_H0] = acc_h0;
-    sc[SC_H1] = acc_h1;
+    sc[SC_LTF] = v[0];
+    sc[SC_H0] = v[1];
+    sc[SC_H1] = v[2];
     // the pair-potential tail constants are added in k_final (held here
     // through the pair loops, they had taken scalar registers the loops need)
-    sc[SC_P0] = acc_v0 + pk0 + c0;
-    sc[SC_P1] = acc_v1 + pk1 + c1;
-    sc[SC_PT] = acc_v0 + acc_v1 + pkt + ct;
+    sc[SC_P0] = v[3] + v[5] + c0;
+    sc[SC_P1] = v[4] + v[6] + c1;
+    sc[SC_PT] = v[3] + v[4] + v[7] + ct;
   }
 }
 
-__global__ __launch_bounds__(QMC_BLOCK, 5) void k_pairs(DevSys s, WsLayout L,
-                                                     const double* __restrict__ x,
-                                                     double* __restrict__ ws,
-                                                     double* __restrict__ props) {
-  k_pairs_body<false>(s, L, x, ws, props);
+template <bool MIX, int P>
+__global__ __launch_bounds__((PairShape<MIX, P>::T), MIX ? 5 : 6) void k_pairs(DevSys s, WsLayout L, const double* __restrict__ x,
+                                                              double* __restrict__ ws,
+                                                              double* __restrict__ props) {
+  k_pairs_body<MIX, P>(s, L, x, ws, props);
 }
 
-__global__ __launch_bounds__(QMC_BLOCK, 5) void k_pairs_mix(DevSys s, WsLayout L,
-                                                         const double* __restrict__ x,
-                                                         double* __restrict__ ws,
-                                                         double* __restrict__ props) {
-  k_pairs_body<true>(s, L, x, ws, props);
+// Lanes per block of the pair schedule for a system.
+static int pair_lanes(const DevSys& s) {
+  const int m = s.np[0] > s.np[1] ? s.np[0] : s.np[1];
+  return m <= 16 ? 16 : m <= 32 ? 32 : 64;
+}
+
+// f(integral_constant P) for the system's lanes per block.
+template <class F>
+static auto with_lanes(const DevSys& s, F&& f) {
+  switch (pair_lanes(s)) {
+    case 16: return f(std::integral_constant<int, 16>{});
+    case 32: return f(std::integral_constant<int, 32>{});
+    default: return f(std::integral_constant<int, 64>{});
+  }
+}
+
+// LDS bytes of the pair kernels with kc particles per phase chunk (0: no
+// phases).
+size_t pairs_lds(const DevSys& s, int kc, bool mix) {
+  const size_t N = s.nptot;
+  auto sums = [&](auto m) {
+    return with_lanes(s, [&](auto p) {
+      using S = PairShape<decltype(m)::value, decltype(p)::value>;
+      return std::pair<size_t, size_t>(8 * S::NW, (size_t)S::NA * PP_NQ * N);
+    });
+  };
+  const auto [red, parts] = mix ? sums(std::true_type{}) : sums(std::false_type{});
+  size_t region = sizeof(double) * parts;
+  if (mix) {
+    if (s.nkxv) region = std::max(region, sizeof(float) * 2 * (size_t)kc * (s.nkxv + s.nkyv));
+  } else if (s.nkax) {
+    region = std::max(region, sizeof(double) * rho_doubles(s, kc));
+  }
+  return sizeof(double) * (6 * N + red) + region;
+}
+
+// Doubles of the FP64 phase rows of kc particles of each type.
+size_t rho_doubles(const DevSys& s, int kc) {
+  const size_t ld = 32 * (size_t)((s.nkax + 15) / 16 + (s.nkby + 15) / 16) + 16;
+  return (s.ntypes > 1 ? 2 : 1) * (size_t)((kc + 3) & ~3) * ld;
+}
+
+// Queue the pair kernel of nw walkers on st.
+void launch_pairs(const DevSys& s, const WsLayout& L, int nw, bool mix, size_t lds, const double* x, double* ws,
+                  double* props, hipStream_t st) {
+  with_lanes(s, [&](auto p) {
+    constexpr int P = decltype(p)::value;
+    if (mix)
+      hipLaunchKernelGGL((k_pairs<true, P>), dim3(nw), dim3(PairShape<true, P>::T), lds, st, s, L, x, ws, props);
+    else
+      hipLaunchKernelGGL((k_pairs<false, P>), dim3(nw), dim3(PairShape<false, P>::T), lds, st, s, L, x, ws, props);
+  });
 }
 
 // ---------------------------------------------------------------------------
