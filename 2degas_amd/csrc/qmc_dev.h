@@ -89,6 +89,10 @@ struct DevSys {
   // a pair of its own
   int real_orb, nslot[2], zslot[2];
   const double* gpair[2];
+  // no backflow (every table zero, q = r): the determinants need F's diagonal
+  // alone, k_final takes their terms; g2sum: sum of |g|^2 over a spin's orbitals
+  int plain;
+  double g2sum[2];
   // walkers evaluated: the first *nact of the batch when not null (the
   // reptation sweep evaluates only the reptiles that still move a bead)
   const int* nact;

@@ -329,7 +329,7 @@ __device__ __forceinline__ void gjm_run(DevSys s, WsLayout L, double* __restrict
   #pragma unroll
             for (int b = 0; b < 2; b++) {
               const zd f = zmul(zmk(h[t][b][0][v], h[t][b][1][v]), pi);
-              Fg[(b * m + k) * m + j] = f;
+              if (!s.plain) Fg[(b * m + k) * m + j] = f;
               // the diagonal F_b(j, j) also goes to the per-orbital terms
               if (k == j) {
                 Fd[4 * j + 2 * b] = f.x;

@@ -257,7 +257,7 @@ __global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLa
 #pragma unroll
             for (int b = 0; b < 2; b++) {
               const double f = acc[1 + b][T][v] * pi;
-              Fg[(b * m + k) * m + j] = f;
+              if (!s.plain) Fg[(b * m + k) * m + j] = f;
               if (k == j) {
                 Fd[4 * j + 2 * b] = f;
                 Fd[4 * j + 2 * b + 1] = 0.0;

@@ -1017,6 +1017,13 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
 // ---------------------------------------------------------------------------
 // k_final: one wavefront per walker.  delta is the current time step (the
 // COMMON delta that kinetic's drift cutoff reads, reptation.f:2755).
+//
+// Without backflow (s.plain) the Jacobian is the identity, and what k_fgrad
+// and k_cross compute reduces to F's diagonal d_j: the drift is -Re d_j, the
+// cross term sum_j Re(d_j . d_j), and the second-derivative term, a trace,
+// sum_j (A^-1 G^2 A)_jj = -sum_k |g_k|^2.  Those two kernels are not launched
+// (at N=26, 256 walkers 31 of an 82 us VMC step, at N=122 1.05 of a 1.9 ms
+// evaluation).
 __global__ __launch_bounds__(QMC_BLOCK) void k_final(DevSys s, WsLayout L, double* __restrict__ ws,
                                                      double* __restrict__ props,
                                                      double* __restrict__ gout,
@@ -1049,6 +1056,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_final(DevSys s, WsLayout L, doubl
     for (int sp = 0; sp < s.ntypes; sp++) {
       if (pick2(s.np, sp) == 0) continue;
       const double* dsc = wsw + pick2(L.off_det, sp);
+      if (s.plain) continue;
       h[0] += dsc[DS_H0] + dsc[DS_X0];
       h[1] += dsc[DS_H1] + dsc[DS_X1];
       g2ph += dsc[DS_G2];
@@ -1056,9 +1064,24 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_final(DevSys s, WsLayout L, doubl
   }
   double* gw = gout + (int64_t)w * 2 * N;
   double g2t[2] = {0.0, 0.0}, ggs = 0.0;
+  double dd[2] = {0.0, 0.0}, im2 = 0.0;  // s.plain: Re sum d.d per type, fixed-phase term
   for (int i = lane; i < N; i += 64) {
     double gx = wsw[L.off_gj + 2 * i], gy = wsw[L.off_gj + 2 * i + 1];
-    if (use_det) {
+    if (use_det && s.plain) {
+      // particles of a type couple to their own spin's orbitals alone
+      const int t = ptype(s, i);
+      if (t ? s.iub_flag[1][1] : s.iub_flag[0][0]) {
+        const double* Fd =
+            wsw + pick2(L.off_det, t) + DS_N + 2 * N + 3 * pick2(s.np, t) + 4 * (i - pick2(s.ipf, t));
+        const double xr = Fd[0], xi = Fd[1], yr = Fd[2], yi = Fd[3];
+        gx -= xr;
+        gy -= yr;
+        const double v = (xr * xr - xi * xi) + (yr * yr - yi * yi);
+        if (t == 0) dd[0] += v;
+        else dd[1] += v;
+        im2 += pick2(s.hbs2m, t) * (xi * xi + yi * yi);
+      }
+    } else if (use_det) {
       for (int sp = 0; sp < s.ntypes; sp++) {
         if (pick2(s.np, sp) == 0) continue;
         const double* gd = wsw + pick2(L.off_det, sp) + DS_N;
@@ -1086,6 +1109,12 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_final(DevSys s, WsLayout L, doubl
   g2t[0] = wave_sum(g2t[0]);
   g2t[1] = wave_sum(g2t[1]);
   ggs = wave_sum(ggs);
+  if (use_det && s.plain) {
+    g2ph = wave_sum(im2);
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+      if (t < s.ntypes && s.np[t] > 0 && s.iub_flag[t][t]) h[t] += s.g2sum[t] + wave_sum(dd[t]);
+  }
   if (lane == 0) {
     double* p = props + (int64_t)w * s.n_props;
     double kin0 = 0.0;
