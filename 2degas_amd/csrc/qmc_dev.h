@@ -89,6 +89,7 @@ struct DevSys {
   // a pair of its own
   int real_orb, nslot[2], zslot[2];
   const double* gpair[2];
+  const int2* kpm[2];      // [nslot] places of g and -g in gvec
   // no backflow (every table zero, q = r): the determinants need F's diagonal
   // alone, k_final takes their terms; g2sum: sum of |g|^2 over a spin's orbitals
   int plain;

@@ -130,24 +130,12 @@ __device__ __forceinline__ void gr_pivots(GrShared<NT>& sh, int buf, int k0, int
   }
 }
 
-template <int NT, bool VAL>
-__global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLayout L, double* __restrict__ ws,
-                                                                  double* __restrict__ Fbuf, int sp0) {
-  constexpr int NP = VAL ? 1 : 3;  // parts of the augmented matrix
-  __shared__ __attribute__((aligned(16))) GrShared<NT> sh;
-  const int w = blockIdx.x, sp = sp0 + blockIdx.y;
-  if (s.nact && w >= *s.nact) return;
-  const int m = pick2(s.np, sp);
-  if (m == 0) return;
-  const int p0 = pick2(s.ipf, sp), nslot = pick2(s.nslot, sp), zero = pick2(s.zslot, sp);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // MFMA lane roles: accumulator rows lr + 4v, column lc; operand k index lr
-  const int lr = lane >> 4, lc = lane & 15;
-  const int ct = wave, col = 16 * ct + lc;
-  const double* qw = ws + (int64_t)w * L.per_walker + L.off_q + 2 * p0;
-  const double* gp = sp ? s.gpair[1] : s.gpair[0];
-  for (int e = tid; e < 2 * m; e += 64 * NT) sh.q[e] = qw[e];
+// Tables of the spin into LDS: quasi-coordinates (or positions) and pairs;
+// rows without an orbital are marked used.
+template <int NT>
+__device__ __forceinline__ void gr_setup(GrShared<NT>& sh, const double* __restrict__ q, const double* __restrict__ gp,
+                                         int m, int nslot, int zero, int tid) {
+  for (int e = tid; e < 2 * m; e += 64 * NT) sh.q[e] = q[e];
   for (int e = tid; e < 2 * nslot; e += 64 * NT) sh.g[e] = gp[e];
   for (int r = tid; r < 16 * NT; r += 64 * NT) {
     // row r = 16 T + lr + 4 v: pair T * 8 + (v >> 1) * 4 + lr, cos (v even) or sin
@@ -157,32 +145,45 @@ __global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLa
   }
   if (tid == 0) sh.sing = 0;
   __syncthreads();
+}
 
-  gr_d4 acc[NP][NT];
-  {
-    const bool jn = col < m;
-    const double qx = jn ? sh.q[2 * col] : 0.0, qy = jn ? sh.q[2 * col + 1] : 0.0;
+// The wavefront's column tile of R and, with NP = 3, of its two derivatives.
+template <int NT, int NP>
+__device__ __forceinline__ void gr_build(const GrShared<NT>& sh, gr_d4 (&acc)[NP][NT], int m, int nslot, int col,
+                                         int lr) {
+  const bool jn = col < m;
+  const double qx = jn ? sh.q[2 * col] : 0.0, qy = jn ? sh.q[2 * col + 1] : 0.0;
 #pragma unroll
-    for (int T = 0; T < NT; T++)
+  for (int T = 0; T < NT; T++)
 #pragma unroll
-      for (int h = 0; h < 2; h++) {
-        const int sl = T * 8 + h * 4 + lr;
-        double sv = 0.0, cv = 0.0, gx = 0.0, gy = 0.0;
-        if (jn && sl < nslot) {
-          gx = sh.g[2 * sl];
-          gy = sh.g[2 * sl + 1];
-          qsincos_sreg(gx * qx + gy * qy, &sv, &cv);
-        }
-        acc[0][T][2 * h] = cv;
-        acc[0][T][2 * h + 1] = sv;
-        if constexpr (!VAL) {
-          acc[1][T][2 * h] = -gx * sv;
-          acc[1][T][2 * h + 1] = gx * cv;
-          acc[2][T][2 * h] = -gy * sv;
-          acc[2][T][2 * h + 1] = gy * cv;
-        }
+    for (int h = 0; h < 2; h++) {
+      const int sl = T * 8 + h * 4 + lr;
+      double sv = 0.0, cv = 0.0, gx = 0.0, gy = 0.0;
+      if (jn && sl < nslot) {
+        gx = sh.g[2 * sl];
+        gy = sh.g[2 * sl + 1];
+        qsincos_sreg(gx * qx + gy * qy, &sv, &cv);
       }
-  }
+      acc[0][T][2 * h] = cv;
+      acc[0][T][2 * h + 1] = sv;
+      if constexpr (NP == 3) {
+        acc[1][T][2 * h] = -gx * sv;
+        acc[1][T][2 * h + 1] = gx * cv;
+        acc[2][T][2 * h] = -gy * sv;
+        acc[2][T][2 * h + 1] = gy * cv;
+      }
+    }
+}
+
+// The elimination, in blocks of 4 columns.  INPLACE (NP = 1): the columns of
+// an eliminated block take the columns e_{p_j} of the identity, so that after
+// the last block column k holds column p_k of the accumulated transform S,
+// S R having row p_k equal to piv_k e_k; else R's eliminated column tiles are
+// left out.  Ends with a barrier.
+template <int NT, int NP, bool INPLACE>
+__device__ __forceinline__ void gr_eliminate(GrShared<NT>& sh, gr_d4 (&acc)[NP][NT], int m, int wave, int lane) {
+  // MFMA lane roles: accumulator rows lr + 4v, column lc; operand k index lr
+  const int lr = lane >> 4, lc = lane & 15, ct = wave;
   // the block's columns from the accumulators of the wavefront that holds
   // them to LDS, and its pivot steps
   auto panel = [&](int k0, int buf) {
@@ -203,12 +204,13 @@ __global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLa
   for (int k0 = 0; k0 < m; k0 += 4) {
     const int buf = (k0 >> 2) & 1, nb = min(4, m - k0);
     __syncthreads();
-    const bool left = (k0 >> 4) <= ct;  // R's columns here are not all eliminated
+    const bool left = INPLACE || (k0 >> 4) <= ct;  // R's columns here are not all eliminated
     double* ub = &sh.u[wave][0][0];
+    int pb[4] = {-1, -1, -1, -1};
 #pragma unroll
     for (int k = 0; k < 4; k++) {
       if (k < nb) {
-        const int p = __builtin_amdgcn_readfirstlane(sh.prow[buf][k]);
+        const int p = pb[k] = __builtin_amdgcn_readfirstlane(sh.prow[buf][k]);
         const bool me = lr == (p & 3);
         gr_switch<NT>(p >> 2, [&](auto ic) {
           constexpr int I = decltype(ic)::value;
@@ -225,19 +227,48 @@ __global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLa
     for (int T = 0; T < NT; T++) fo[T] = sh.Fl[buf][4 * (16 * T + lc) + lr];
 #pragma unroll
     for (int t = 0; t < NP; t++) uo[t] = lr < nb ? ub[t * 64 + lane] : 0.0;
+    if constexpr (INPLACE) {
+      const int jj = lc - (k0 & 15);
+      if ((k0 >> 4) == ct && jj >= 0 && jj < nb) {
+        const int pr = jj == 0 ? pb[0] : (jj == 1 ? pb[1] : (jj == 2 ? pb[2] : pb[3]));
+#pragma unroll
+        for (int T = 0; T < NT; T++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) acc[0][T][v] = 16 * T + lr + 4 * v == pr ? 1.0 : 0.0;
+        uo[0] = lr == jj ? 1.0 : 0.0;
+      }
+    }
     if (left) {
 #pragma unroll
       for (int T = 0; T < NT; T++) acc[0][T] = gr_mfma(fo[T], uo[0], acc[0][T]);
     }
-    if constexpr (!VAL) {
 #pragma unroll
-      for (int t = 1; t < 3; t++)
+    for (int t = 1; t < NP; t++)
 #pragma unroll
-        for (int T = 0; T < NT; T++) acc[t][T] = gr_mfma(fo[T], uo[t], acc[t][T]);
-    }
+      for (int T = 0; T < NT; T++) acc[t][T] = gr_mfma(fo[T], uo[t], acc[t][T]);
     if (k0 + 4 < m && ((k0 + 4) >> 4) == ct) panel(k0 + 4, buf ^ 1);
   }
   __syncthreads();
+}
+
+template <int NT, bool VAL>
+__global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLayout L, double* __restrict__ ws,
+                                                                  double* __restrict__ Fbuf, int sp0) {
+  constexpr int NP = VAL ? 1 : 3;  // parts of the augmented matrix
+  __shared__ __attribute__((aligned(16))) GrShared<NT> sh;
+  const int w = blockIdx.x, sp = sp0 + blockIdx.y;
+  if (s.nact && w >= *s.nact) return;
+  const int m = pick2(s.np, sp);
+  if (m == 0) return;
+  const int nslot = pick2(s.nslot, sp), zero = pick2(s.zslot, sp);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane >> 4, col = 16 * wave + (lane & 15);
+  gr_setup(sh, ws + (int64_t)w * L.per_walker + L.off_q + 2 * pick2(s.ipf, sp), sp ? s.gpair[1] : s.gpair[0], m,
+           nslot, zero, tid);
+  gr_d4 acc[NP][NT];
+  gr_build<NT, NP>(sh, acc, m, nslot, col, lr);
+  gr_eliminate<NT, NP, false>(sh, acc, m, wave, lane);
   double* dsc = ws + (int64_t)w * L.per_walker + pick2(L.off_det, sp);
   if constexpr (!VAL) {
     // F_b(k, j): row p_k of part b over piv_k; the diagonal also goes to the
@@ -277,6 +308,68 @@ __global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLa
   }
 }
 
+// A^-1 of single-electron moves (row = particle, column = orbital, complex)
+// for real orbitals: R^-1 by the in-place elimination, R^-1(k, p_c) = M(p_k, c)
+// / piv_k, brought into row order in LDS, where the two rows of a pair meet:
+// A^-1(k, +-g) = (X_cos -+ i X_sin) / 2.  Bound by the pivot chains and the
+// complex store (0.98 GB for 4096 walkers of N=122).
+template <int NT>
+struct GrInverse {
+  static constexpr int LD = 16 * NT + 1;
+  GrShared<NT> sh;
+  double X[16 * NT * LD];  // X(k, r) at k LD + r
+  int pcol[16 * NT];       // pivot row of column c
+};
+
+template <int NT>
+__global__ __launch_bounds__(64 * NT, 4) void k_gjr_inverse(DevSys s, int sp0, const double* __restrict__ x,
+                                                            double2* __restrict__ ainv, int mm) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char gi_lds[];
+  GrInverse<NT>& gi = *reinterpret_cast<GrInverse<NT>*>(gi_lds);
+  GrShared<NT>& sh = gi.sh;
+  const int w = blockIdx.x, sp = sp0 + blockIdx.y;
+  const int m = pick2(s.np, sp);
+  if (m == 0) return;
+  const int nslot = pick2(s.nslot, sp), zero = pick2(s.zslot, sp);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane >> 4, col = 16 * wave + (lane & 15);
+  gr_setup(sh, x + ((int64_t)w * s.nptot + pick2(s.ipf, sp)) * 2, sp ? s.gpair[1] : s.gpair[0], m, nslot, zero, tid);
+  gr_d4 acc[1][NT];
+  gr_build<NT, 1>(sh, acc, m, nslot, col, lr);
+  gr_eliminate<NT, 1, true>(sh, acc, m, wave, lane);
+  for (int r = tid; r < 16 * NT; r += 64 * NT)
+    if (sh.rank[r] >= 0) gi.pcol[sh.rank[r]] = r;
+  __syncthreads();
+  if (col < m) {
+    const int pc = gi.pcol[col];
+#pragma unroll
+    for (int T = 0; T < NT; T++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int r = 16 * T + lr + 4 * v;
+        const int k = sh.rank[r];
+        if (k >= 0) gi.X[k * GrInverse<NT>::LD + pc] = acc[0][T][v] * sh.pinv[r];
+      }
+  }
+  __syncthreads();
+  double2* out = ainv + ((int64_t)w * 2 + sp) * mm * mm;
+  const int2* kpm = sp ? s.kpm[1] : s.kpm[0];
+  for (int e = tid; e < m * nslot; e += 64 * NT) {
+    const int k = e / nslot, sl = e - k * nslot;
+    const int r = (sl >> 3) * 16 + ((sl >> 2) & 1) * 8 + (sl & 3);
+    const double xc = gi.X[k * GrInverse<NT>::LD + r];
+    const int2 o = kpm[sl];
+    if (zero && sl == 0) {
+      out[k * mm + o.x] = make_double2(xc, 0.0);
+    } else {
+      const double hc = 0.5 * xc, hs = 0.5 * gi.X[k * GrInverse<NT>::LD + r + 4];
+      out[k * mm + o.x] = make_double2(hc, -hs);
+      out[k * mm + o.y] = make_double2(hc, hs);
+    }
+  }
+}
+
 template <bool VAL>
 static void gjr_spins(const DevSys& s, const WsLayout& L, int nw, int sp0, int nsp, int nt, double* ws, double* F,
                       hipStream_t st) {
@@ -289,17 +382,37 @@ static void gjr_spins(const DevSys& s, const WsLayout& L, int nw, int sp0, int n
   }
 }
 
-// Queue the real determinant path of every spin on st: one launch when the
-// spins have the same tile count, else one per spin.  A spin of m particles
-// has m or, with the zero plane wave (m odd), m + 1 rows.
-void launch_gjr(const DevSys& s, const WsLayout& L, int nw, bool value, double* ws, double* F, hipStream_t st) {
+// go(first spin, spins, tile count) for every launch of a real-orbital kernel:
+// one when the spins have the same tile count, else one per spin.  A spin of m
+// particles has m or, with the zero plane wave (m odd), m + 1 rows.
+template <class G>
+static void gjr_launches(const DevSys& s, G&& go) {
   int nt[2] = {0, 0};
   for (int sp = 0; sp < s.ntypes; sp++) nt[sp] = s.np[sp] ? (2 * s.nslot[sp] + 15) / 16 : 0;
-  auto go = [&](int sp0, int nsp, int n) {
-    if (n == 0) return;
-    if (value) gjr_spins<true>(s, L, nw, sp0, nsp, n, ws, F, st);
-    else gjr_spins<false>(s, L, nw, sp0, nsp, n, ws, F, st);
-  };
-  if (s.ntypes == 2 && nt[0] == nt[1]) return go(0, 2, nt[0]);
-  for (int sp = 0; sp < s.ntypes; sp++) go(sp, 1, nt[sp]);
+  if (s.ntypes == 2 && nt[0] == nt[1]) {
+    if (nt[0]) go(0, 2, nt[0]);
+    return;
+  }
+  for (int sp = 0; sp < s.ntypes; sp++)
+    if (nt[sp]) go(sp, 1, nt[sp]);
+}
+
+void launch_gjr(const DevSys& s, const WsLayout& L, int nw, bool value, double* ws, double* F, hipStream_t st) {
+  gjr_launches(s, [&](int sp0, int nsp, int nt) {
+    if (value) gjr_spins<true>(s, L, nw, sp0, nsp, nt, ws, F, st);
+    else gjr_spins<false>(s, L, nw, sp0, nsp, nt, ws, F, st);
+  });
+}
+
+void launch_gjr_inverse(const DevSys& s, int nw, const double* x, void* ainv, int mm, hipStream_t st) {
+  double2* a = (double2*)ainv;
+  gjr_launches(s, [&](int sp0, int nsp, int nt) {
+    const dim3 grid(nw, nsp);
+    switch (nt) {
+      case 1: hipLaunchKernelGGL(k_gjr_inverse<1>, grid, dim3(64), sizeof(GrInverse<1>), st, s, sp0, x, a, mm); break;
+      case 2: hipLaunchKernelGGL(k_gjr_inverse<2>, grid, dim3(128), sizeof(GrInverse<2>), st, s, sp0, x, a, mm); break;
+      case 3: hipLaunchKernelGGL(k_gjr_inverse<3>, grid, dim3(192), sizeof(GrInverse<3>), st, s, sp0, x, a, mm); break;
+      default: hipLaunchKernelGGL(k_gjr_inverse<4>, grid, dim3(256), sizeof(GrInverse<4>), st, s, sp0, x, a, mm); break;
+    }
+  });
 }

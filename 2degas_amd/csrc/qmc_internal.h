@@ -121,6 +121,8 @@ void launch_pairs(const DevSys& s, const WsLayout& L, int nw, bool mix, size_t l
 // The real-orbital determinant kernels of every spin (s.real_orb); value:
 // log|det A| alone.
 void launch_gjr(const DevSys& s, const WsLayout& L, int nw, bool value, double* ws, double* F, hipStream_t st);
+// The FP64 inverses of single-electron moves at positions x (s.real_orb).
+void launch_gjr_inverse(const DevSys& s, int nw, const double* x, void* ainv, int mm, hipStream_t st);
 void free_vmc(qmc_ctx* c);
 void free_vmc_graph(qmc_ctx* c);
 // Workspace of the evaluation kernels for nw walkers (allocates when it grows).

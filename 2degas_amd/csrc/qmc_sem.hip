@@ -22,63 +22,10 @@
 // particle, column = orbital), in FP64 or, with QMC_PREC_MIXED, in FP32 (the
 // ratio and the update in FP32, the Jastrow and positions in FP64), and are
 // recomputed in FP64 by qmc_sem_refresh (Gauss-Jordan with partial pivoting).
+#include <algorithm>
 #include <cstring>
 
-#include "qmc_internal.h"
-
-// exp and log for the move loop, their constants kept in scalar registers
-// (qk<true>) so that the loop does not hold them in vector registers next to
-// the inverse.  exp: Cody-Waite reduction x = n ln2 + r (ln2 over two
-// doubles), |r| <= ln2 / 2, the Taylor series of e^r through r^13
-// (truncation below 5e-18), scaled by 2^n; arguments are clamped to
-// [-746, 710], beyond which the result is 0 or +inf.  log: x = m 2^e with
-// m in [sqrt(1/2), sqrt(2)), log m = 2 atanh(s), s = (m - 1) / (m + 1),
-// |s| <= 0.1716, the series through s^21 (truncation below 1e-18), plus
-// e ln2; x > 0.
-__device__ __forceinline__ double sem_exp(double x) {
-  x = fmin(fmax(x, -746.0), 710.0);
-  const double n = rint(x * qk<true>(0x1.71547652b82fep+0));
-  double r = fma(-n, qk<true>(0x1.62e42fefa39efp-1), x);
-  r = fma(-n, qk<true>(0x1.abc9e3b39803fp-56), r);
-  double p = qk<true>(1.0 / 6227020800.0);
-  p = fma(p, r, qk<true>(1.0 / 479001600.0));
-  p = fma(p, r, qk<true>(1.0 / 39916800.0));
-  p = fma(p, r, qk<true>(1.0 / 3628800.0));
-  p = fma(p, r, qk<true>(1.0 / 362880.0));
-  p = fma(p, r, qk<true>(1.0 / 40320.0));
-  p = fma(p, r, qk<true>(1.0 / 5040.0));
-  p = fma(p, r, qk<true>(1.0 / 720.0));
-  p = fma(p, r, qk<true>(1.0 / 120.0));
-  p = fma(p, r, qk<true>(1.0 / 24.0));
-  p = fma(p, r, qk<true>(1.0 / 6.0));
-  p = fma(p, r, 0.5);
-  p = fma(p, r, 1.0);
-  p = fma(p, r, 1.0);
-  return ldexp(p, (int)n);
-}
-
-__device__ __forceinline__ double sem_log(double x) {
-  int e;
-  double m = frexp(x, &e);
-  if (m < qk<true>(0x1.6a09e667f3bcdp-1)) {
-    m *= 2.0;
-    e -= 1;
-  }
-  const double sv = (m - 1.0) / (m + 1.0), s2 = sv * sv;
-  double p = qk<true>(1.0 / 21.0);
-  p = fma(p, s2, qk<true>(1.0 / 19.0));
-  p = fma(p, s2, qk<true>(1.0 / 17.0));
-  p = fma(p, s2, qk<true>(1.0 / 15.0));
-  p = fma(p, s2, qk<true>(1.0 / 13.0));
-  p = fma(p, s2, qk<true>(1.0 / 11.0));
-  p = fma(p, s2, qk<true>(1.0 / 9.0));
-  p = fma(p, s2, qk<true>(1.0 / 7.0));
-  p = fma(p, s2, qk<true>(1.0 / 5.0));
-  p = fma(p, s2, qk<true>(1.0 / 3.0));
-  const double lm = 2.0 * fma(sv * s2, p, sv);
-  const double de = (double)e;
-  return fma(de, qk<true>(0x1.62e42fefa39efp-1), fma(de, qk<true>(0x1.abc9e3b39803fp-56), lm));
-}
+#include "qmc_sem.h"
 
 template <typename Z>
 struct SemZ;
@@ -488,22 +435,6 @@ __global__ __launch_bounds__(MR* CG, (SemWaves<Z, MR, CG>::value)) void k_sem_mo
 // block reads its job's system description from device memory (uniform
 // loads) and runs the same per-walker body.  MR is the launch's row class
 // (16, 32 or 64); a job with fewer particles leaves the extra rows idle.
-struct SemJob {
-  const DevSys* sys;
-  double* x;
-  int64_t* rng;
-  void* ainv;
-  double* dlogpsi;
-  double* nacc;
-  double sigma;
-  int w0, nw, j0, j1, sp, mm;
-};
-#define SEM_MAX_PACK 16
-struct SemJobs {
-  SemJob job[SEM_MAX_PACK];
-  int njobs;
-};
-
 template <typename Z, int MR, int CG, bool U3>
 __global__ __launch_bounds__(MR* CG, (SemWaves<Z, MR, CG>::value)) void k_sem_moves_packed(const SemJobs jobs) {
   int k = 0;
@@ -512,6 +443,8 @@ __global__ __launch_bounds__(MR* CG, (SemWaves<Z, MR, CG>::value)) void k_sem_mo
   sem_moves_walker<Z, MR, CG, U3>(*jb.sys, blockIdx.x - jb.w0, jb.j0, jb.j1, jb.sp, jb.sigma, jb.x, jb.rng,
                                   (Z*)jb.ainv, jb.mm, jb.dlogpsi, jb.nacc);
 }
+
+static int sem_mm(const qmc_ctx* c) { return std::max(c->s.np[0], c->s.ntypes > 1 ? c->s.np[1] : 0); }
 
 // The context's system description in device memory, sent again before a
 // launch that reads it only when it has changed since it was last sent (new
@@ -657,7 +590,52 @@ static int sem_moves_full(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_state*
   return QMC_OK;
 }
 
-static int sem_mm(const qmc_ctx* c) { return std::max(c->s.np[0], c->s.ntypes > 1 ? c->s.np[1] : 0); }
+
+// FP64 moves of jobs with real orbitals, which take the spins of their ranges
+// in order: one launch of the jobs with a spin of more than 32 rows (two
+// wavefronts per walker), one of the others (one wavefront).  Jobs with the
+// most electrons come first, so that the longest walkers start first.
+static int sem_moves_real(const qmc_sem_job* jobs, int njobs, hipStream_t st) {
+  std::vector<const qmc_sem_job*> order;
+  for (int k = 0; k < njobs; k++)
+    if (jobs[k].w->nw > 0 && jobs[k].j0 < jobs[k].j1) order.push_back(jobs + k);
+  std::stable_sort(order.begin(), order.end(), [](const qmc_sem_job* a, const qmc_sem_job* b) {
+    return a->ctx->s.nptot > b->ctx->s.nptot;
+  });
+  for (int wide = 1; wide >= 0; wide--) {
+    SemJobs jb{};
+    int nblocks = 0, nmax = 0;
+    bool u3 = false;
+    for (const qmc_sem_job* j : order) {
+      qmc_ctx* c = j->ctx;
+      int rows = 0;
+      for (int sp = 0; sp < c->s.ntypes; sp++) rows = std::max({rows, c->s.np[sp], 2 * c->s.nslot[sp]});
+      if ((rows > 32) != (wide != 0)) continue;
+      const int rc = upload_sys(c, st);
+      if (rc) return rc;
+      SemJob& e = jb.job[jb.njobs++];
+      e.sys = c->d_sys;
+      e.x = j->w->x;
+      e.rng = j->w->rng;
+      e.ainv = j->d->ainv;
+      e.dlogpsi = j->d->dlogpsi;
+      e.nacc = j->d->nacc;
+      e.sigma = j->sigma;
+      e.w0 = nblocks;
+      e.nw = j->w->nw;
+      e.j0 = j->j0;
+      e.j1 = j->j1;
+      e.mm = sem_mm(c);
+      nblocks += e.nw;
+      u3 = u3 || c->s.has_u3;
+      nmax = std::max(nmax, c->s.nptot);
+    }
+    if (jb.njobs == 0) continue;
+    const int rc = launch_sem_real(jb, nblocks, u3, wide != 0, nmax, st);
+    if (rc) return rc;
+  }
+  return QMC_OK;
+}
 
 extern "C" int qmc_sem_refresh(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_state* d, int precision,
                                void* stream) {
@@ -666,6 +644,11 @@ extern "C" int qmc_sem_refresh(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_s
   if (w->nw == 0 || !c->b_zero) return QMC_OK;  // backflow: no inverse is carried
   HIPCHK(hipSetDevice(c->device));
   const int mm = sem_mm(c);
+  if (c->s.real_orb && precision == QMC_PREC_FP64) {
+    launch_gjr_inverse(c->s, w->nw, w->x, d->ainv, mm, (hipStream_t)stream);
+    HIPCHK(hipGetLastError());
+    return QMC_OK;
+  }
   for (int sp = 0; sp < c->s.ntypes; sp++) {
     if (c->s.np[sp] == 0) continue;
     rc = precision == QMC_PREC_MIXED ? sem_inverse_spin<float2>(c, w, d, sp, mm, (hipStream_t)stream)
@@ -684,6 +667,10 @@ extern "C" int qmc_sem_moves(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_sta
   if (w->nw == 0 || j0 == j1) return QMC_OK;
   HIPCHK(hipSetDevice(c->device));
   if (!c->b_zero) return sem_moves_full(c, w, d, j0, j1, sigma, precision, (hipStream_t)stream);
+  if (c->s.real_orb && precision == QMC_PREC_FP64) {
+    const qmc_sem_job one = {c, w, d, j0, j1, sigma};
+    return sem_moves_real(&one, 1, (hipStream_t)stream);
+  }
   rc = upload_sys(c, (hipStream_t)stream);
   if (rc) return rc;
   const int mm = sem_mm(c);
@@ -733,6 +720,16 @@ extern "C" int qmc_sem_moves_packed(const qmc_sem_job* jobs, int njobs, int prec
     if (!(jb.sigma > 0.0)) return arg_fail("sigma must be positive");
   }
   HIPCHK(hipSetDevice(jobs[0].ctx->device));
+  // FP64 jobs with real orbitals go together; the others below
+  std::vector<qmc_sem_job> real, rest;
+  for (int k = 0; k < njobs; k++)
+    (jobs[k].ctx->s.real_orb && precision == QMC_PREC_FP64 ? real : rest).push_back(jobs[k]);
+  if (!real.empty()) {
+    const int rc = sem_moves_real(real.data(), (int)real.size(), st);
+    if (rc) return rc;
+  }
+  jobs = rest.data();
+  njobs = (int)rest.size();
   for (int k = 0; k < njobs; k++) {
     int rc = upload_sys(jobs[k].ctx, st);
     if (rc) return rc;
