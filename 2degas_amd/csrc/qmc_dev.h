@@ -220,13 +220,21 @@ __device__ __forceinline__ TabRef tabref(const DevSys& s, int tp) {
   return TabRef{pick3(s.trow[KIND], tp), pick3(s.tng[KIND], tp)};
 }
 
+// Row of a table at grid index ind >= 0 (rows beyond the last one: the last).
+// The byte offset is 32 bits from a uniform base, so that a lane's address is
+// two integer instructions (and the load's own base), not a 64-bit sum.
+template <typename V>
+__device__ __forceinline__ V tab_row(const V* tab, TabRef t, int ind) {
+  const unsigned i = (unsigned)(ind < t.ng ? ind : t.ng) * (unsigned)sizeof(V);
+  return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(tab + t.row0) + i);
+}
+
 // Cubic spline on the uniform grid, value and two derivatives
 // (getf, reptation.f:4114-4125).
 __device__ __forceinline__ void spline3(const DevSys& s, TabRef t, int ind, double rem, double& f,
                                         double& df, double& ddf) {
-  int i = ind < t.ng ? (ind > 0 ? ind : 0) : t.ng;
-  double4 c = s.tab[t.row0 + i];
-  double rm = rem * s.drti;
+  const double4 c = tab_row(s.tab, t, ind);
+  const double rm = rem * s.drti;
   f = c.x + rm * (c.y + rm * (c.z + rm * c.w));
   df = (c.y + rm * (2.0 * c.z + rm * (3.0 * c.w))) * s.drti;
   ddf = (c.z + rm * (3.0 * c.w)) * s.drti2;
@@ -241,8 +249,7 @@ __device__ __forceinline__ void spline3m(const DevSys& s, TabRef t, int ind, dou
     spline3(s, t, ind, rem, f, df, ddf);
     return;
   }
-  int i = ind < t.ng ? (ind > 0 ? ind : 0) : t.ng;
-  const float4 c = s.tab32[t.row0 + i];
+  const float4 c = tab_row(s.tab32, t, ind);
   const float rm = (float)(rem * s.drti);
   const float di = (float)s.drti;
   f = (double)(c.x + rm * (c.y + rm * (c.z + rm * c.w)));
@@ -254,14 +261,13 @@ __device__ __forceinline__ void spline3m(const DevSys& s, TabRef t, int ind, dou
 template <bool MIX = false>
 __device__ __forceinline__ double spline0(const DevSys& s, TabRef t, int e, int ind, double rem,
                                          double byr) {
-  int i = ind < t.ng ? (ind > 0 ? ind : 0) : t.ng;
   double f;
   if (MIX) {
-    const float4 c = s.tab32[t.row0 + i];
+    const float4 c = tab_row(s.tab32, t, ind);
     const float rm = (float)(rem * s.drti);
     f = (double)(c.x + rm * (c.y + rm * (c.z + rm * c.w)));
   } else {
-    const double4 c = s.tab[t.row0 + i];
+    const double4 c = tab_row(s.tab, t, ind);
     const double rm = rem * s.drti;
     f = c.x + rm * (c.y + rm * (c.z + rm * c.w));
   }

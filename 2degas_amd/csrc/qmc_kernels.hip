@@ -30,9 +30,9 @@
 
 // ---------------------------------------------------------------------------
 // k_pairs
-// LDS: xs[2N], Gs[2N], ks[2N], red[8 NW], then a region shared by the partial
-// sums of the pair passes (NA x 6 x N doubles) and, afterwards, the phases of
-// rho_k.
+// LDS: xs[2N], Gs[2N], red[8 NW], then a region shared by the partial sums of
+// the pair passes (NA x 6 x 2P doubles) and, afterwards, the phase steps (4N) and
+// phases of rho_k.
 //
 // The pair passes visit every unordered pair once, on a round-robin
 // schedule over blocks of P lanes, P = 16, 32 or 64 the power of two that
@@ -66,19 +66,23 @@ struct PairShape {
   static constexpr int NW = P == 16 || MIX ? 4 : 8;  // wavefronts
   static constexpr int T = 64 * NW, SUB = 64 / P, NA = NW * SUB;
   static constexpr int OWN = P / 2 / SUB, ACROSS = P / SUB;  // wavefront steps of a block pair
+  static constexpr int NS = 2 * P;  // particles a sum's row holds
+  static constexpr int PART = 6 * NS;  // doubles of one group's partial sums
 };
 
-// part[q * N + p] += v for the lane group's partial sums
-__device__ __forceinline__ void pp_add(double* part, int N, int p, const double (&v)[PP_NQ], int nq) {
+// part[q * NS + p] += v for the lane group's partial sums
+template <int NS>
+__device__ __forceinline__ void pp_add(double* part, int p, const double (&v)[PP_NQ], int nq) {
 #pragma unroll
   for (int q = 0; q < PP_NQ; q++)
-    if (q < nq) part[q * N + p] += v[q];
+    if (q < nq) part[q * NS + p] += v[q];
 }
 
-// The wavefront's run of pair steps: pair(ti, tj, T, i, j) for each of its
-// lanes' pairs, end(ti) when the run leaves block ti.
-template <bool MIX, int P, class Pair, class End>
-__device__ __forceinline__ void pair_run(const DevSys& s, int wv, int l, Pair&& pair, End&& end) {
+// The wavefront's run of pair steps: pair(T, i, j) for each of its lanes'
+// pairs, block(ti, tj) after each block pair's, end(ti) when the run leaves
+// block ti.
+template <bool MIX, int P, class Pair, class Block, class End>
+__device__ __forceinline__ void pair_run(const DevSys& s, int wv, int l, Pair&& pair, Block&& block, End&& end) {
   using S = PairShape<MIX, P>;
   const int lp = l & (P - 1), sub = l / P;
   // schedule: both types present, or the one type t1
@@ -99,23 +103,24 @@ __device__ __forceinline__ void pair_run(const DevSys& s, int wv, int l, Pair&& 
       for (int u = a; u < b; u++) {
         const int d = (u - b0) * S::SUB + sub + (ti == tj ? 1 : 0);
         const int jl = (lp + d) & (P - 1);
-        if (lp < ni && jl < nj && (ti != tj || d < P / 2 || lp < P / 2)) pair(ti, tj, T, i, pick2(s.ipf, tj) + jl);
+        if (lp < ni && jl < nj && (ti != tj || d < P / 2 || lp < P / 2)) pair(T, i, pick2(s.ipf, tj) + jl);
       }
+      block(ti, tj);
     }
     if (u0 < u1 && (blk == 2 || !two || (blk == 1 && u0 < b1))) end(ti);
   }
 }
 
-// The NA partial sums of each of the nq N per-particle sums, added in order
+// The NA partial sums of each of the nq per-particle sums, added in order
 // into the first one.
 template <bool MIX, int P>
-__device__ __forceinline__ void pp_reduce(double* parts, int N, int nq, int tid) {
+__device__ __forceinline__ void pp_reduce(double* parts, int nq, int tid) {
   using S = PairShape<MIX, P>;
   __syncthreads();
-  for (int e = tid; e < nq * N; e += S::T) {
+  for (int e = tid; e < nq * S::NS; e += S::T) {
     double v = parts[e];
 #pragma unroll
-    for (int a = 1; a < S::NA; a++) v += parts[a * PP_NQ * N + e];
+    for (int a = 1; a < S::NA; a++) v += parts[a * S::PART + e];
     parts[e] = v;
   }
   __syncthreads();
@@ -170,6 +175,9 @@ __device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restr
   const int nt = s.ntypes > 1 ? 2 : 1, ntask = ta * tb * nt;
   const int kc = (s.kchunk + 3) & ~3;  // rows per type and chunk
   const int nmax = max(s.np[0], nt > 1 ? s.np[1] : 0);
+  // items of a phase row: runs of KRUN2 phases; the thread's first item
+  const int gx = (na + KRUN2 - 1) / KRUN2, ng = gx + (nb + KRUN2 - 1) / KRUN2;
+  const int row_0 = tid / ng, g_0 = tid - row_0 * ng, row_d = S::T / ng, g_d = S::T - row_d * ng;
   // e^{i dk x}, e^{i dk y} of every particle
   if (s.kaprog)
     for (int e = tid; e < 2 * N; e += S::T) {
@@ -187,10 +195,13 @@ __device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restr
     for (int c0 = 0; c0 < nmax; c0 += kc) {
       __syncthreads();
       // rows: type t's particles c0..c0+kc-1 (zero beyond its count, up to a
-      // multiple of 4); items of a row: runs of KRUN2 phases
-      const int gx = (na + KRUN2 - 1) / KRUN2, ng = gx + (nb + KRUN2 - 1) / KRUN2;
-      for (int e = tid; e < nt * kc * ng; e += S::T) {
-        const int row = e / ng, g = e - row * ng;
+      // multiple of 4)
+      for (int row = row_0, g = g_0; row < nt * kc; row += row_d, g += g_d) {
+        if (g >= ng) {
+          g -= ng;
+          row++;
+          if (row >= nt * kc) break;
+        }
         const int t = row >= kc ? 1 : 0, c = c0 + row - t * kc;
         const int np_t = pick2(s.np, t);
         if (c >= ((np_t + 3) & ~3)) continue;
@@ -278,16 +289,16 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   if (s.nact && w >= *s.nact) return;
   const int N = s.nptot;
   double* xs = sm;
-  double* Gs = sm + 2 * N;  // with ks: the phase steps of rho_k
-  double* red = sm + 6 * N;
-  double* parts = sm + 6 * N + 8 * S::NW;
+  double* Gs = sm + 2 * N;
+  double* red = sm + 4 * N;
+  double* parts = sm + 4 * N + 8 * S::NW;
   const double* xw = x + (int64_t)w * 2 * N;
   const int tid = threadIdx.x, l = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  double* part = parts + (wv * S::SUB + l / P) * PP_NQ * N;
+  double* part = parts + (wv * S::SUB + l / P) * S::PART;
   const int lp = l & (P - 1);
   for (int k = tid; k < 2 * N; k += S::T) xs[k] = xw[k];
-  for (int k = tid; k < S::NA * PP_NQ * N; k += S::T) parts[k] = 0.0;
+  for (int k = tid; k < S::NA * S::PART; k += S::T) parts[k] = 0.0;
   __syncthreads();
   double* wsw = ws + (int64_t)w * L.per_walker;
   double acc_ltf = 0.0, acc_h0 = 0.0, acc_h1 = 0.0, acc_v0 = 0.0, acc_v1 = 0.0;
@@ -295,9 +306,10 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   // pass 1: u2, the pair term and G of u3, backflow q, pair potential
   {
     double ia[PP_NQ] = {0, 0, 0, 0, 0, 0};  // gx, gy, Gx, Gy, qx, qy of particle i
+    double hb = 0.0, vb = 0.0;              // the block pair's Laplacian and potential
     pair_run<MIX, P>(
         s, wv, l,
-        [&](int ti, int tj, const TpInfo* T, int i, int j) {
+        [&](const TpInfo* T, int i, int j) {
           const TabRef tu2{T->row[TK_U2], T->ng[TK_U2]}, tu3{T->row[TK_U3], T->ng[TK_U3]},
               tb{T->row[TK_B], T->ng[TK_B]}, tv{T->row[TK_V], T->ng[TK_V]};
           const double2 xi2 = ld2(xs, i), xj2 = ld2(xs, j);
@@ -335,29 +347,33 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
           // the pair gives i the opposite of j's vector terms (u -> -u)
 #pragma unroll
           for (int q = 0; q < PP_NQ; q++) ia[q] -= ja[q];
-          if (ti == 0) acc_h0 += hh; else acc_h1 += hh;
-          if (tj == 0) acc_h0 += hh; else acc_h1 += hh;
-          if (tv.row0 >= 0) {
-            const double vv = 0.5 * spline0<MIX>(s, tv, T->vexp, p.ind, p.rem, p.byr) * T->v2value;
-            if (ti == 0) acc_v0 += vv; else acc_v1 += vv;
-            if (tj == 0) acc_v0 += vv; else acc_v1 += vv;
-          }
-          pp_add(part, N, j, ja, PP_NQ);
+          hb += hh;
+          if (tv.row0 >= 0) vb += 0.5 * spline0<MIX>(s, tv, T->vexp, p.ind, p.rem, p.byr) * T->v2value;
+          pp_add<S::NS>(part, j, ja, PP_NQ);
+        },
+        [&](int ti, int tj) {
+          const double h0 = (ti == 0 ? hb : 0.0) + (tj == 0 ? hb : 0.0);
+          acc_h0 += h0;
+          acc_h1 += 2.0 * hb - h0;
+          const double v0 = (ti == 0 ? vb : 0.0) + (tj == 0 ? vb : 0.0);
+          acc_v0 += v0;
+          acc_v1 += 2.0 * vb - v0;
+          hb = vb = 0.0;
         },
         [&](int ti) {
-          if (lp < pick2(s.np, ti)) pp_add(part, N, pick2(s.ipf, ti) + lp, ia, PP_NQ);
+          if (lp < pick2(s.np, ti)) pp_add<S::NS>(part, pick2(s.ipf, ti) + lp, ia, PP_NQ);
 #pragma unroll
           for (int q = 0; q < PP_NQ; q++) ia[q] = 0.0;
         });
   }
-  pp_reduce<MIX, P>(parts, N, PP_NQ, tid);
+  pp_reduce<MIX, P>(parts, PP_NQ, tid);
   // Gs for pass 2, q out, g kept
   double gpx = 0.0, gpy = 0.0;  // gradient of particle tid (N <= 128)
   if (tid < N) {
     const int p = tid;
     double v[PP_NQ];
 #pragma unroll
-    for (int q = 0; q < PP_NQ; q++) v[q] = parts[q * N + p];
+    for (int q = 0; q < PP_NQ; q++) v[q] = parts[q * S::NS + p];
     gpx = v[0];
     gpy = v[1];
     Gs[2 * p] = v[2];
@@ -374,12 +390,13 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   // with M = xi I + (xi'/r) u u^T and a = xi'' + 3 xi'/r; M and a.(u dG) are
   // even in the pair, M dG is odd
   if (s.has_u3) {
-    for (int k = tid; k < S::NA * PP_NQ * N; k += S::T) parts[k] = 0.0;
+    for (int k = tid; k < S::NA * S::PART; k += S::T) parts[k] = 0.0;
     __syncthreads();
     double ia[PP_NQ] = {0, 0, 0, 0, 0, 0};  // g3x, g3y, e11, e12, e22 of particle i
+    double hb = 0.0;
     pair_run<MIX, P>(
         s, wv, l,
-        [&](int ti, int tj, const TpInfo* T, int i, int j) {
+        [&](const TpInfo* T, int i, int j) {
           const TabRef tu3{T->row[TK_U3], T->ng[TK_U3]};
           if (tu3.row0 < 0) return;
           const double2 xi2 = ld2(xs, i), xj2 = ld2(xs, j);
@@ -399,20 +416,25 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
           ia[3] += m12;
           ia[4] += m22;
           const double ja[PP_NQ] = {-g3x, -g3y, m11, m12, m22, 0.0};
-          pp_add(part, N, j, ja, 5);
-          if (ti == 0) acc_h0 += h3; else acc_h1 += h3;
-          if (tj == 0) acc_h0 += h3; else acc_h1 += h3;
+          pp_add<S::NS>(part, j, ja, 5);
+          hb += h3;
+        },
+        [&](int ti, int tj) {
+          const double h0 = (ti == 0 ? hb : 0.0) + (tj == 0 ? hb : 0.0);
+          acc_h0 += h0;
+          acc_h1 += 2.0 * hb - h0;
+          hb = 0.0;
         },
         [&](int ti) {
-          if (lp < pick2(s.np, ti)) pp_add(part, N, pick2(s.ipf, ti) + lp, ia, 5);
+          if (lp < pick2(s.np, ti)) pp_add<S::NS>(part, pick2(s.ipf, ti) + lp, ia, 5);
 #pragma unroll
           for (int q = 0; q < PP_NQ; q++) ia[q] = 0.0;
         });
-    pp_reduce<MIX, P>(parts, N, 5, tid);
+    pp_reduce<MIX, P>(parts, 5, tid);
     if (tid < N) {
       double v[5];
 #pragma unroll
-      for (int q = 0; q < 5; q++) v[q] = parts[q * N + tid];
+      for (int q = 0; q < 5; q++) v[q] = parts[q * S::NS + tid];
       gpx += v[0];
       gpy += v[1];
       const double e2 = v[2] * v[2] + 2.0 * v[3] * v[3] + v[4] * v[4];
@@ -429,7 +451,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   double* pw = props + (int64_t)w * s.n_props;
   if (!MIX && s.nrhok && s.nkax > 0) {
     __syncthreads();  // Gs and the partial sums have been read
-    rho_tiles<P>(s, xs, Gs, parts, pw, tid);
+    rho_tiles<P>(s, xs, parts, parts + 4 * N, pw, tid);
     __syncthreads();  // rho_k of this walker is in memory
     const double* r0 = s.irhok[0] ? pw + s.jrhok + (s.irhok[0] - 1) * 2 * s.nk : nullptr;
     const double* r1 = s.ntypes > 1 && s.irhok[1] ? pw + s.jrhok + (s.irhok[1] - 1) * 2 * s.nk : nullptr;
@@ -642,7 +664,7 @@ size_t pairs_lds(const DevSys& s, int kc, bool mix) {
   auto sums = [&](auto m) {
     return with_lanes(s, [&](auto p) {
       using S = PairShape<decltype(m)::value, decltype(p)::value>;
-      return std::pair<size_t, size_t>(8 * S::NW, (size_t)S::NA * PP_NQ * N);
+      return std::pair<size_t, size_t>(8 * S::NW, (size_t)S::NA * S::PART);
     });
   };
   const auto [red, parts] = mix ? sums(std::true_type{}) : sums(std::false_type{});
@@ -650,9 +672,9 @@ size_t pairs_lds(const DevSys& s, int kc, bool mix) {
   if (mix) {
     if (s.nkxv) region = std::max(region, sizeof(float) * 2 * (size_t)kc * (s.nkxv + s.nkyv));
   } else if (s.nkax) {
-    region = std::max(region, sizeof(double) * rho_doubles(s, kc));
+    region = std::max(region, sizeof(double) * (4 * N + rho_doubles(s, kc)));
   }
-  return sizeof(double) * (6 * N + red) + region;
+  return sizeof(double) * (4 * N + red) + region;
 }
 
 // Doubles of the FP64 phase rows of kc particles of each type.
