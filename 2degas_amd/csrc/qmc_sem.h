@@ -58,7 +58,7 @@ __device__ __forceinline__ double sem_log(double x) {
 }
 
 // One job of a launch: blocks w0 .. w0 + nw - 1 move electrons j0..j1-1 of its
-// walkers, one block per walker.
+// walkers, one block per walker (per two, narrow).
 struct SemJob {
   const DevSys* sys;
   double* x;
@@ -67,7 +67,9 @@ struct SemJob {
   double* dlogpsi;
   double* nacc;
   double sigma;
-  int w0, nw, j0, j1, sp, mm;
+  int w0, nw, j0, j1, mm;
+  int tile[3];  // threads per row of spins of up to 16, 32, 64 rows
+  int narrow;   // two walkers per block of two wavefronts, one each
 };
 #define SEM_MAX_PACK 16
 struct SemJobs {
@@ -75,7 +77,6 @@ struct SemJobs {
   int njobs;
 };
 
-// FP64 moves of real-orbital jobs (qmc_sem_real.hip), both spins of each, in
-// one launch; wide: jobs with a spin of more than 32 rows (else none has one);
-// nmax: electrons of the largest job.
-int launch_sem_real(const SemJobs& jobs, int nblocks, bool u3, bool wide, int nmax, hipStream_t st);
+// Moves of jobs of one kind of row (0 real, 1 complex FP64, 2 complex FP32) and
+// wavefronts per walker (qmc_sem_moves.hip); nmax: electrons of the largest.
+int launch_sem_moves(const SemJobs& jobs, int nblocks, int kind, int waves, bool u3, int nmax, hipStream_t st);

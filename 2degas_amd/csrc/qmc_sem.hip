@@ -163,287 +163,6 @@ static int sem_inverse_spin(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_stat
   return launch_sem_inverse<Z, 64>(c, w, d, sp, mm, st);
 }
 
-// Moves of electrons j0..j1-1 of spin sp, in order: one workgroup of
-// MR x CG threads per walker, the walker's m x m inverse (m <= MR) held in
-// registers: thread (l, c) = (tid / CG, tid % CG) keeps row l at columns
-// c, c + CG, ..., MR / CG complex entries.  The proposals come first: lane i
-// of the first wavefront jumps the walker's stream 3i draws ahead and forms
-// move i's Gaussian step (Box-Muller) and acceptance uniform, kept in LDS.
-// Per move, threads 0..m-1 put the new orbital column a' in LDS; each thread
-// forms its part of t_l = (A^-1 a')_l and the CG threads of a row sum them
-// by lane shuffles; the threads of row j' put that row and R = t_j' in LDS
-// while every thread sums its share of the Jastrow change; after the
-// barrier every thread takes the same decision, and an accepted move
-// updates each thread's entries from its own t_l and the shared row.
-// Entries beyond m are zero and stay zero.  Two barriers per move, reached
-// by every thread.  The log|R| of the accepted moves are summed as a
-// product kept as mantissa and exponent (frexp), one log at the end.
-// The FP64 inverse of a 64-row spin takes 64 registers per thread; left to
-// itself the compiler spends some 110 more and fits 2 waves per SIMD.  A
-// bound of 3 costs a few spilled registers and is 17% faster at N=122
-// (measured, 4096 walkers).  Other shapes fit 4 or more waves unbounded (a
-// bound of 5 on the FP32 64-row shape spills and is 8% slower).
-template <typename Z, int MR, int CG>
-struct SemWaves {
-  static constexpr int value = (sizeof(Z) == 16 && MR == 64 && CG == 4) ? 3 : 1;
-};
-
-template <typename Z, int MR, int CG, bool U3>
-__device__ __forceinline__ void sem_moves_walker(const DevSys& s, int w, int j0, int j1, int sp, double sigma,
-                                                 double* __restrict__ x, int64_t* __restrict__ rng,
-                                                 Z* __restrict__ ainv, int mm, double* __restrict__ dlogpsi,
-                                                 double* __restrict__ nacc) {
-  typedef typename SemZ<Z>::R R;
-  constexpr int T = MR * CG, EPT = MR / CG, NWV = T / 64 > 0 ? T / 64 : 1;
-  constexpr int PMAX = (128 + T - 1) / T;  // partners per thread (N <= 128)
-  __shared__ Z ap[2][MR];  // new orbital column a' (two buffers: moves alternate)
-  __shared__ Z rowj[MR];  // row j' of the inverse before the update
-  __shared__ Z rz_sh;     // R
-  __shared__ double red[3 * NWV];
-  __shared__ double2 step[64];  // move i's displacement
-  __shared__ double uacc[64];   // move i's acceptance uniform
-  extern __shared__ __attribute__((aligned(16))) unsigned char sem_lds[];
-  double* xs = reinterpret_cast<double*>(sem_lds);  // positions [N][2]
-  double* Gs = xs + 2 * s.nptot;                     // U3: G_p [N][2]
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int N = s.nptot, nmv = j1 - j0;
-  const int m = pick2(s.np, sp), p0 = pick2(s.ipf, sp);
-  const int l = tid / CG, cg = tid % CG;
-  const Z* gin = ainv + ((int64_t)w * 2 + sp) * mm * mm;
-  Z b[EPT];
-#pragma unroll
-  for (int i = 0; i < EPT; i++) {
-    const int k = cg + CG * i;
-    b[i] = (l < m && k < m) ? gin[l * mm + k] : Z{(R)0, (R)0};
-  }
-  if (tid < MR) ap[0][tid] = ap[1][tid] = Z{(R)0, (R)0};
-  for (int e = tid; e < 2 * N; e += T) xs[e] = x[(int64_t)w * 2 * N + e];
-  const uint64_t st0 = (uint64_t)rng[w];
-  if (tid < nmv) {
-    // the proposal of move tid: a Gaussian step of width sigma per dimension
-    uint64_t st = (st0 * lcg_pow(3 * (uint64_t)tid)) & ((1ULL << 48) - 1ULL);
-    const double u1 = rannyu(st), u2 = rannyu(st), ua = rannyu(st);
-    double sv, cv;
-    qsincos(6.283185307179586 * u2, &sv, &cv);
-    const double rad = sigma * sqrt(-2.0 * sem_log(u1));
-    step[tid] = make_double2(rad * cv, rad * sv);
-    uacc[tid] = ua;
-  }
-  double du_acc = 0.0, na = 0.0, pm = 1.0;
-  int pe = 0;
-  if (U3) {
-    // G_p = sum_b xi(r_pb) (x_b - x_p), minimum image: the per-particle
-    // vector of the three-body factor
-    __syncthreads();
-    for (int p = tid; p < N; p += T) {
-      double gx = 0.0, gy = 0.0;
-      const int tp = ptype(s, p);
-      for (int q = 0; q < N; q++) {
-        if (q == p) continue;
-        const TabRef tu3 = tabref<TK_U3>(s, tpair(tp, ptype(s, q)));
-        if (tu3.row0 < 0) continue;
-        const PairGeo g = pair_geo(s, xs[2 * q], xs[2 * q + 1], xs[2 * p], xs[2 * p + 1]);
-        double f, d1, d2;
-        spline3(s, tu3, g.ind, g.rem, f, d1, d2);
-        gx += f * g.ux;
-        gy += f * g.uy;
-      }
-      Gs[2 * p] = gx;
-      Gs[2 * p + 1] = gy;
-    }
-  }
-  __syncthreads();
-  // a'(k) = exp(i g_k . r') of a move into buffer ab, entry k by this thread
-  auto put_col = [&](Z* ab, int k, double px, double py) {
-    double so, co;
-    qsincos_sreg(s.gvec[2 * k] * px + s.gvec[2 * k + 1] * py, &so, &co);
-    ab[k] = Z{(R)co, (R)so};
-  };
-  // With a wavefront's worth of threads beyond the Jastrow sum's partners
-  // (the last m threads, all >= N), those threads form the next move's a'
-  // while the others sum, so that a move starts from a' already in LDS;
-  // otherwise threads 0..m-1 form it at the start of the move.  Either way
-  // from the same inputs (electron j+1 has not moved before its own move).
-  // FP32 inverses only: with FP64 ones the extra live values spill inside the
-  // loop, and the move measured 1% slower instead of 3% faster.
-  constexpr bool PRE = sizeof(typename SemZ<Z>::R) == 4 && PMAX == 1;
-  const bool pre = PRE && T - m >= N;
-  for (int j = j0; j < j1; j++) {
-    const int jj = j - p0, c = (j - j0) & 1;
-    const double2 dx = step[j - j0];
-    const double xo = xs[2 * j], yo = xs[2 * j + 1];
-    const double xn = xo + dx.x, yn = yo + dx.y;
-    if ((!pre || j == j0) && tid < m) put_col(ap[c], tid, xn, yn);
-    __syncthreads();
-    // t as explicit FMAs into two accumulator pairs (even and odd entries)
-    R tr = 0, ti = 0, tr2 = 0, ti2 = 0;
-#pragma unroll
-    for (int i = 0; i < EPT; i += 2) {
-      const Z a = ap[c][cg + CG * i];
-      tr = fma(b[i].x, a.x, tr);
-      tr = fma(-b[i].y, a.y, tr);
-      ti = fma(b[i].x, a.y, ti);
-      ti = fma(b[i].y, a.x, ti);
-      if (i + 1 < EPT) {
-        const Z a2 = ap[c][cg + CG * (i + 1)];
-        tr2 = fma(b[i + 1].x, a2.x, tr2);
-        tr2 = fma(-b[i + 1].y, a2.y, tr2);
-        ti2 = fma(b[i + 1].x, a2.y, ti2);
-        ti2 = fma(b[i + 1].y, a2.x, ti2);
-      }
-    }
-    tr += tr2;
-    ti += ti2;
-#pragma unroll
-    for (int o = 1; o < CG; o <<= 1) {
-      tr += __shfl_xor(tr, o, 64);
-      ti += __shfl_xor(ti, o, 64);
-    }
-    if (l == jj) {
-#pragma unroll
-      for (int i = 0; i < EPT; i++) rowj[cg + CG * i] = b[i];
-      if (cg == 0) rz_sh = Z{tr, ti};
-    }
-    // the Jastrow change over the partners of j: the u2 terms and, with U3,
-    // the three-body factor's pair terms (xi r)^2 and its -1/2 sum_p |G_p|^2
-    // (G_p of each partner changes by dG_p = xi' u' - xi u, u = x_j - x_p
-    // folded; G_j becomes -sum_p xi' u')
-    double du = 0.0, gjx = 0.0, gjy = 0.0;
-    double dgx[PMAX], dgy[PMAX];
-    const double2 Gj = U3 ? ld2(Gs, j) : make_double2(0.0, 0.0);
-#pragma unroll
-    for (int k = 0; k < PMAX; k++) {
-      const int p = tid + k * T;
-      dgx[k] = dgy[k] = 0.0;
-      if (p >= N || p == j) continue;
-      const int tp = tpair(sp, ptype(s, p));
-      const TabRef tu2 = tabref<TK_U2>(s, tp);
-      const double xp = xs[2 * p], yp = xs[2 * p + 1];
-      const PairGeo pn = pair_geo(s, xn, yn, xp, yp), po = pair_geo(s, xo, yo, xp, yp);
-      double fn, fo, d1, d2;
-      if (tu2.row0 >= 0) {
-        spline3(s, tu2, pn.ind, pn.rem, fn, d1, d2);
-        spline3(s, tu2, po.ind, po.rem, fo, d1, d2);
-        du += fn - fo;
-      }
-      if (U3) {
-        const TabRef tu3 = tabref<TK_U3>(s, tp);
-        if (tu3.row0 >= 0) {
-          spline3(s, tu3, pn.ind, pn.rem, fn, d1, d2);
-          spline3(s, tu3, po.ind, po.rem, fo, d1, d2);
-          const double an = fn * pn.r, ao = fo * po.r;
-          dgx[k] = fn * pn.ux - fo * po.ux;
-          dgy[k] = fn * pn.uy - fo * po.uy;
-          const double2 G = ld2(Gs, p);
-          du += (an * an - ao * ao) - (G.x * dgx[k] + G.y * dgy[k]) - 0.5 * (dgx[k] * dgx[k] + dgy[k] * dgy[k]);
-          gjx -= fn * pn.ux;
-          gjy -= fn * pn.uy;
-        }
-      }
-    }
-    if (pre && j + 1 < j1 && tid >= T - m) {
-      const double2 d = step[j + 1 - j0];
-      put_col(ap[c ^ 1], tid - (T - m), xs[2 * (j + 1)] + d.x, xs[2 * (j + 1) + 1] + d.y);
-    }
-    du = wave_sum(du);
-    if (U3) {
-      gjx = wave_sum(gjx);
-      gjy = wave_sum(gjy);
-    }
-    if (lane == 0) {
-      red[wv] = du;
-      red[NWV + wv] = gjx;
-      red[2 * NWV + wv] = gjy;
-    }
-    __syncthreads();
-    du = 0.0;
-    gjx = 0.0;
-    gjy = 0.0;
-#pragma unroll
-    for (int k = 0; k < NWV; k++) {
-      du += red[k];
-      gjx += red[NWV + k];
-      gjy += red[2 * NWV + k];
-    }
-    if (U3) du -= 0.5 * ((gjx * gjx + gjy * gjy) - (Gj.x * Gj.x + Gj.y * Gj.y));
-    const Z rz = rz_sh;
-    const double mod2 = (double)rz.x * (double)rz.x + (double)rz.y * (double)rz.y;
-    if (uacc[j - j0] < mod2 * sem_exp(-2.0 * du)) {
-      // A^-1 -= (t - e_j') (row j' of A^-1) / R, 1/R as conj(R) / |R|^2
-      const R inv2 = (R)(1.0 / mod2);
-      const R vr = l == jj ? tr - (R)1 : tr;
-      const R fr = -(vr * rz.x + ti * rz.y) * inv2, fi = -(ti * rz.x - vr * rz.y) * inv2;
-#pragma unroll
-      for (int i = 0; i < EPT; i++) {
-        const Z q = rowj[cg + CG * i];
-        b[i].x = fma(fr, q.x, b[i].x);
-        b[i].x = fma(-fi, q.y, b[i].x);
-        b[i].y = fma(fr, q.y, b[i].y);
-        b[i].y = fma(fi, q.x, b[i].y);
-      }
-      if (tid == 0) {
-        xs[2 * j] = xn;
-        xs[2 * j + 1] = yn;
-      }
-      if (U3) {
-#pragma unroll
-        for (int k = 0; k < PMAX; k++) {
-          const int p = tid + k * T;
-          if (p < N && p != j) {
-            Gs[2 * p] += dgx[k];
-            Gs[2 * p + 1] += dgy[k];
-          }
-        }
-        if (tid == 0) {
-          Gs[2 * j] = gjx;
-          Gs[2 * j + 1] = gjy;
-        }
-      }
-      int e;
-      pm = frexp(pm * mod2, &e);
-      pe += e;
-      du_acc += du;
-      na += 1.0;
-    }
-  }
-  __syncthreads();
-  Z* gout = ainv + ((int64_t)w * 2 + sp) * mm * mm;
-#pragma unroll
-  for (int i = 0; i < EPT; i++) {
-    const int k = cg + CG * i;
-    if (l < m && k < m) gout[l * mm + k] = b[i];
-  }
-  for (int e = tid; e < 2 * N; e += T) x[(int64_t)w * 2 * N + e] = xs[e];
-  if (tid == 0) {
-    rng[w] = (int64_t)((st0 * lcg_pow(3 * (uint64_t)nmv)) & ((1ULL << 48) - 1ULL));
-    dlogpsi[w] += 0.5 * (sem_log(pm) + pe * 0.6931471805599453) - du_acc;
-    nacc[w] += na;
-  }
-}
-
-template <typename Z, int MR, int CG, bool U3>
-__global__ __launch_bounds__(MR* CG, (SemWaves<Z, MR, CG>::value)) void k_sem_moves(const DevSys* __restrict__ sys,
-                                                                                 int j0, int j1, int sp,
-                                                                                 double sigma, double* x, int64_t* rng,
-                                                                                 Z* ainv, int mm, double* dlogpsi,
-                                                                                 double* nacc) {
-  sem_moves_walker<Z, MR, CG, U3>(*sys, blockIdx.x, j0, j1, sp, sigma, x, rng, ainv, mm, dlogpsi, nacc);
-}
-
-// Several jobs (contexts of different N, decks and walker sets) in one
-// launch: job k owns blocks w0[k] .. w0[k] + nw[k] - 1, one per walker; each
-// block reads its job's system description from device memory (uniform
-// loads) and runs the same per-walker body.  MR is the launch's row class
-// (16, 32 or 64); a job with fewer particles leaves the extra rows idle.
-template <typename Z, int MR, int CG, bool U3>
-__global__ __launch_bounds__(MR* CG, (SemWaves<Z, MR, CG>::value)) void k_sem_moves_packed(const SemJobs jobs) {
-  int k = 0;
-  while (k + 1 < jobs.njobs && (int)blockIdx.x >= jobs.job[k + 1].w0) k++;
-  const SemJob& jb = jobs.job[k];
-  sem_moves_walker<Z, MR, CG, U3>(*jb.sys, blockIdx.x - jb.w0, jb.j0, jb.j1, jb.sp, jb.sigma, jb.x, jb.rng,
-                                  (Z*)jb.ainv, jb.mm, jb.dlogpsi, jb.nacc);
-}
-
 static int sem_mm(const qmc_ctx* c) { return std::max(c->s.np[0], c->s.ntypes > 1 ? c->s.np[1] : 0); }
 
 // The context's system description in device memory, sent again before a
@@ -459,37 +178,7 @@ static int upload_sys(qmc_ctx* c, hipStream_t st) {
   return QMC_OK;
 }
 
-template <typename Z, int MR, int CG>
-static int launch_sem_moves(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_state* d, int j0, int j1, int sp,
-                            double sigma, int mm, hipStream_t st) {
-  const bool u3 = c->s.has_u3 != 0;
-  const size_t lds = (u3 ? 4 : 2) * (size_t)c->s.nptot * sizeof(double);
-  if (u3)
-    hipLaunchKernelGGL((k_sem_moves<Z, MR, CG, true>), dim3(w->nw), dim3(MR * CG), lds, st, c->d_sys, j0, j1, sp,
-                       sigma, w->x, w->rng, (Z*)d->ainv, mm, d->dlogpsi, d->nacc);
-  else
-    hipLaunchKernelGGL((k_sem_moves<Z, MR, CG, false>), dim3(w->nw), dim3(MR * CG), lds, st, c->d_sys, j0, j1, sp,
-                       sigma, w->x, w->rng, (Z*)d->ainv, mm, d->dlogpsi, d->nacc);
-  HIPCHK(hipGetLastError());
-  return QMC_OK;
-}
-
 static int sem_class(int m) { return m <= 16 ? 0 : m <= 32 ? 1 : 2; }
-
-// The row class of the spin and the context's threads per row for it (16
-// rows: 4 threads, one wavefront; 32 and 64 rows: 2 or 4).
-template <typename Z>
-static int sem_moves_spin(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_state* d, int j0, int j1, int sp,
-                          double sigma, int mm, hipStream_t st) {
-  const int cls = sem_class(c->s.np[sp]);
-  const int cg = c->sem_cg[sizeof(Z) == 16 ? 0 : 1][cls];
-  if (cls == 0) return launch_sem_moves<Z, 16, 4>(c, w, d, j0, j1, sp, sigma, mm, st);
-  if (cls == 1)
-    return cg == 2 ? launch_sem_moves<Z, 32, 2>(c, w, d, j0, j1, sp, sigma, mm, st)
-                   : launch_sem_moves<Z, 32, 4>(c, w, d, j0, j1, sp, sigma, mm, st);
-  return cg == 2 ? launch_sem_moves<Z, 64, 2>(c, w, d, j0, j1, sp, sigma, mm, st)
-                 : launch_sem_moves<Z, 64, 4>(c, w, d, j0, j1, sp, sigma, mm, st);
-}
 
 extern "C" int qmc_sem_set_tile(qmc_ctx* c, int precision, int rows, int threads_per_row) {
   if (!c) return arg_fail("null context");
@@ -591,49 +280,83 @@ static int sem_moves_full(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_state*
 }
 
 
-// FP64 moves of jobs with real orbitals, which take the spins of their ranges
-// in order: one launch of the jobs with a spin of more than 32 rows (two
-// wavefronts per walker), one of the others (one wavefront).  Jobs with the
-// most electrons come first, so that the longest walkers start first.
-static int sem_moves_real(const qmc_sem_job* jobs, int njobs, hipStream_t st) {
+// Kind of row and wavefronts per walker of a job's moves: real rows in FP64
+// where the orbitals are real (one wavefront up to 32 rows per spin, two above),
+// else complex ones with the context's threads per row for each class (16 rows:
+// 4 threads; 32 and 64 rows: 2 or 4), as many wavefronts as the larger spin
+// needs.
+static void sem_shape(const qmc_ctx* c, int precision, int& kind, int& waves) {
+  kind = precision == QMC_PREC_MIXED ? 2 : c->s.real_orb ? 0 : 1;
+  waves = 1;
+  for (int sp = 0; sp < c->s.ntypes; sp++) {
+    const int m = c->s.np[sp];
+    if (m == 0) continue;
+    if (kind == 0) {
+      waves = std::max(waves, std::max(m, 2 * c->s.nslot[sp]) <= 32 ? 1 : 2);
+    } else {
+      const int cls = sem_class(m);
+      waves = std::max(waves, (16 << cls) * (cls == 0 ? 4 : c->sem_cg[precision == QMC_PREC_MIXED ? 1 : 0][cls]) / 64);
+    }
+  }
+}
+
+// Moves of jobs, each taking the spins of its range in order: one launch per
+// kind of row and wavefronts per walker.  Jobs with the most electrons come
+// first, so that the longest walkers start first.  A job's results do not
+// depend on the others: its kind, wavefronts and tiles are its context's (the
+// three-body variant also serves jobs without u3, whose u3 terms are skipped
+// and add nothing).
+static int sem_moves_jobs(const qmc_sem_job* jobs, int njobs, int precision, hipStream_t st) {
   std::vector<const qmc_sem_job*> order;
   for (int k = 0; k < njobs; k++)
     if (jobs[k].w->nw > 0 && jobs[k].j0 < jobs[k].j1) order.push_back(jobs + k);
   std::stable_sort(order.begin(), order.end(), [](const qmc_sem_job* a, const qmc_sem_job* b) {
     return a->ctx->s.nptot > b->ctx->s.nptot;
   });
-  for (int wide = 1; wide >= 0; wide--) {
-    SemJobs jb{};
-    int nblocks = 0, nmax = 0;
-    bool u3 = false;
-    for (const qmc_sem_job* j : order) {
-      qmc_ctx* c = j->ctx;
-      int rows = 0;
-      for (int sp = 0; sp < c->s.ntypes; sp++) rows = std::max({rows, c->s.np[sp], 2 * c->s.nslot[sp]});
-      if ((rows > 32) != (wide != 0)) continue;
-      const int rc = upload_sys(c, st);
-      if (rc) return rc;
-      SemJob& e = jb.job[jb.njobs++];
-      e.sys = c->d_sys;
-      e.x = j->w->x;
-      e.rng = j->w->rng;
-      e.ainv = j->d->ainv;
-      e.dlogpsi = j->d->dlogpsi;
-      e.nacc = j->d->nacc;
-      e.sigma = j->sigma;
-      e.w0 = nblocks;
-      e.nw = j->w->nw;
-      e.j0 = j->j0;
-      e.j1 = j->j1;
-      e.mm = sem_mm(c);
-      nblocks += e.nw;
-      u3 = u3 || c->s.has_u3;
-      nmax = std::max(nmax, c->s.nptot);
-    }
-    if (jb.njobs == 0) continue;
-    const int rc = launch_sem_real(jb, nblocks, u3, wide != 0, nmax, st);
-    if (rc) return rc;
+  // real-row jobs of one wavefront per walker join a launch of two
+  bool wide = false;
+  for (const qmc_sem_job* j : order) {
+    int k, w;
+    sem_shape(j->ctx, precision, k, w);
+    wide = wide || (k == 0 && w == 2);
   }
+  for (int kind = 0; kind < 3; kind++)
+    for (int waves = 4; waves >= 1; waves >>= 1) {
+      SemJobs jb{};
+      int nblocks = 0, nmax = 0;
+      bool u3 = false;
+      for (const qmc_sem_job* j : order) {
+        qmc_ctx* c = j->ctx;
+        int k, w;
+        sem_shape(c, precision, k, w);
+        const bool narrow = k == 0 && w == 1 && wide;
+        if (narrow) w = 2;
+        if (k != kind || w != waves) continue;
+        const int rc = upload_sys(c, st);
+        if (rc) return rc;
+        SemJob& e = jb.job[jb.njobs++];
+        e.sys = c->d_sys;
+        e.x = j->w->x;
+        e.rng = j->w->rng;
+        e.ainv = j->d->ainv;
+        e.dlogpsi = j->d->dlogpsi;
+        e.nacc = j->d->nacc;
+        e.sigma = j->sigma;
+        e.w0 = nblocks;
+        e.nw = j->w->nw;
+        e.j0 = j->j0;
+        e.j1 = j->j1;
+        e.mm = sem_mm(c);
+        for (int t = 0; t < 3; t++) e.tile[t] = c->sem_cg[precision == QMC_PREC_MIXED ? 1 : 0][t];
+        e.narrow = narrow;
+        nblocks += narrow ? (e.nw + 1) / 2 : e.nw;
+        u3 = u3 || c->s.has_u3;
+        nmax = std::max(nmax, narrow ? 2 * c->s.nptot : c->s.nptot);
+      }
+      if (jb.njobs == 0) continue;
+      const int rc = launch_sem_moves(jb, nblocks, kind, waves, u3, nmax, st);
+      if (rc) return rc;
+    }
   return QMC_OK;
 }
 
@@ -667,43 +390,8 @@ extern "C" int qmc_sem_moves(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_sta
   if (w->nw == 0 || j0 == j1) return QMC_OK;
   HIPCHK(hipSetDevice(c->device));
   if (!c->b_zero) return sem_moves_full(c, w, d, j0, j1, sigma, precision, (hipStream_t)stream);
-  if (c->s.real_orb && precision == QMC_PREC_FP64) {
-    const qmc_sem_job one = {c, w, d, j0, j1, sigma};
-    return sem_moves_real(&one, 1, (hipStream_t)stream);
-  }
-  rc = upload_sys(c, (hipStream_t)stream);
-  if (rc) return rc;
-  const int mm = sem_mm(c);
-  // one launch per spin the range touches, in order
-  for (int sp = 0; sp < c->s.ntypes; sp++) {
-    const int a = std::max(j0, c->s.ipf[sp]), b = std::min(j1, c->s.ipf[sp] + c->s.np[sp]);
-    if (a >= b) continue;
-    rc = precision == QMC_PREC_MIXED ? sem_moves_spin<float2>(c, w, d, a, b, sp, sigma, mm, (hipStream_t)stream)
-                                     : sem_moves_spin<double2>(c, w, d, a, b, sp, sigma, mm, (hipStream_t)stream);
-    if (rc) return rc;
-  }
-  return QMC_OK;
-}
-
-template <typename Z, int MR, int CG, bool U3>
-static int launch_sem_packed(const SemJobs& jb, int nblocks, size_t lds, hipStream_t st) {
-  hipLaunchKernelGGL((k_sem_moves_packed<Z, MR, CG, U3>), dim3(nblocks), dim3(MR * CG), lds, st, jb);
-  HIPCHK(hipGetLastError());
-  return QMC_OK;
-}
-
-template <typename Z, int MR, int CG>
-static int sem_packed_u3(const SemJobs& jb, int nblocks, bool u3, size_t lds, hipStream_t st) {
-  return u3 ? launch_sem_packed<Z, MR, CG, true>(jb, nblocks, lds, st)
-            : launch_sem_packed<Z, MR, CG, false>(jb, nblocks, lds, st);
-}
-
-template <typename Z>
-static int sem_packed_phase(const SemJobs& jb, int nblocks, int cls, int cg, bool u3, size_t lds, hipStream_t st) {
-  if (cls == 0) return sem_packed_u3<Z, 16, 4>(jb, nblocks, u3, lds, st);
-  if (cls == 1)
-    return cg == 2 ? sem_packed_u3<Z, 32, 2>(jb, nblocks, u3, lds, st) : sem_packed_u3<Z, 32, 4>(jb, nblocks, u3, lds, st);
-  return cg == 2 ? sem_packed_u3<Z, 64, 2>(jb, nblocks, u3, lds, st) : sem_packed_u3<Z, 64, 4>(jb, nblocks, u3, lds, st);
+  const qmc_sem_job one = {c, w, d, j0, j1, sigma};
+  return sem_moves_jobs(&one, 1, precision, (hipStream_t)stream);
 }
 
 extern "C" int qmc_sem_moves_packed(const qmc_sem_job* jobs, int njobs, int precision, void* stream) {
@@ -720,65 +408,5 @@ extern "C" int qmc_sem_moves_packed(const qmc_sem_job* jobs, int njobs, int prec
     if (!(jb.sigma > 0.0)) return arg_fail("sigma must be positive");
   }
   HIPCHK(hipSetDevice(jobs[0].ctx->device));
-  // FP64 jobs with real orbitals go together; the others below
-  std::vector<qmc_sem_job> real, rest;
-  for (int k = 0; k < njobs; k++)
-    (jobs[k].ctx->s.real_orb && precision == QMC_PREC_FP64 ? real : rest).push_back(jobs[k]);
-  if (!real.empty()) {
-    const int rc = sem_moves_real(real.data(), (int)real.size(), st);
-    if (rc) return rc;
-  }
-  jobs = rest.data();
-  njobs = (int)rest.size();
-  for (int k = 0; k < njobs; k++) {
-    int rc = upload_sys(jobs[k].ctx, st);
-    if (rc) return rc;
-  }
-  // spin 0 of every job, then spin 1: each job sees its moves in the order
-  // qmc_sem_moves makes them.  Within a spin, one launch per row class and
-  // threads per row (as qmc_sem_moves picks for each job's context), so
-  // that each job runs with the thread layout of its own call and its sums
-  // are added in the same order; the three-body variant also serves jobs
-  // without u3 (their u3 terms are skipped and add nothing).
-  const int pi = precision == QMC_PREC_MIXED ? 1 : 0;
-  for (int sp = 0; sp < 2; sp++)
-  for (int cls = 0; cls < 3; cls++)
-  for (int cg = 2; cg <= 4; cg += 2) {
-    SemJobs jb{};
-    int nblocks = 0, mr = 0;
-    bool u3 = false;
-    size_t lds = 0;
-    for (int k = 0; k < njobs; k++) {
-      qmc_ctx* c = jobs[k].ctx;
-      if (sp >= c->s.ntypes || jobs[k].w->nw == 0) continue;
-      const int m = c->s.np[sp];
-      if (sem_class(m) != cls || (cls == 0 ? 4 : c->sem_cg[pi][cls]) != cg) continue;
-      const int a = std::max(jobs[k].j0, c->s.ipf[sp]), b = std::min(jobs[k].j1, c->s.ipf[sp] + c->s.np[sp]);
-      if (a >= b) continue;
-      SemJob& e = jb.job[jb.njobs++];
-      e.sys = c->d_sys;
-      e.x = jobs[k].w->x;
-      e.rng = jobs[k].w->rng;
-      e.ainv = jobs[k].d->ainv;
-      e.dlogpsi = jobs[k].d->dlogpsi;
-      e.nacc = jobs[k].d->nacc;
-      e.sigma = jobs[k].sigma;
-      e.w0 = nblocks;
-      e.nw = jobs[k].w->nw;
-      e.j0 = a;
-      e.j1 = b;
-      e.sp = sp;
-      e.mm = sem_mm(c);
-      nblocks += e.nw;
-      mr = std::max(mr, c->s.np[sp]);
-      u3 = u3 || c->s.has_u3;
-      lds = std::max(lds, (c->s.has_u3 ? 4 : 2) * (size_t)c->s.nptot * sizeof(double));
-    }
-    if (jb.njobs == 0) continue;
-    (void)mr;
-    const int rc = precision == QMC_PREC_MIXED ? sem_packed_phase<float2>(jb, nblocks, cls, cg, u3, lds, st)
-                                               : sem_packed_phase<double2>(jb, nblocks, cls, cg, u3, lds, st);
-    if (rc) return rc;
-  }
-  return QMC_OK;
+  return sem_moves_jobs(jobs, njobs, precision, st);
 }
