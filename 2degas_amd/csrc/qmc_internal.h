@@ -56,6 +56,7 @@ struct qmc_ctx {
   int st_nw = 0;
   double *d_x = nullptr, *d_props = nullptr, *d_g = nullptr, *d_h = nullptr, *d_g2 = nullptr;
   int32_t* d_status = nullptr;
+  double* h_stage = nullptr;  // pinned: what goes in, then what comes out
   hipStream_t stream = nullptr;
   double delta = 0.0;  // current time step (COMMON delta) for the drift cutoff
   int kc = 16;
