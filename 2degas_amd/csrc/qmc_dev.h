@@ -194,11 +194,23 @@ __device__ __forceinline__ double rannyu(uint64_t& x) {
 }
 
 // a^n mod 2^48 for rannyu's multiplier: the stream n draws ahead is a^n x.
-__device__ __forceinline__ uint64_t lcg_pow(uint64_t n) {
+__device__ __forceinline__ uint64_t lcg_pow(uint32_t n) {
   uint64_t p = 1, q = 34522712143931ULL;
   for (; n; n >>= 1) {
     if (n & 1) p = (p * q) & ((1ULL << 48) - 1ULL);
     q = (q * q) & ((1ULL << 48) - 1ULL);
+  }
+  return p;
+}
+
+// The same for n < 1024 without the loop: the squares are constants.
+__device__ __forceinline__ uint64_t lcg_pow10(uint32_t n) {
+  const uint64_t msk = (1ULL << 48) - 1ULL;
+  uint64_t p = 1, q = 34522712143931ULL;
+#pragma unroll
+  for (int i = 0; i < 10; i++) {
+    p = (p * ((n >> i) & 1 ? q : 1)) & msk;
+    q = (q * q) & msk;
   }
   return p;
 }
@@ -313,13 +325,16 @@ __device__ __forceinline__ PairGeo pair_geo(const DevSys& s, double xi, double y
                                             double yj) {
   PairGeo p;
   double dx = xi - xj, dy = yi - yj;
-  dx = dx - s.el[0] * qround(s.eli[0] * dx);
-  dy = dy - s.el[1] * qround(s.eli[1] * dy);
+  // explicit FMAs: which product of a sum the compiler would fuse depends on
+  // the code around it, and with it the last bit, from one kernel variant to
+  // another
+  dx = fma(-s.el[0], qround(s.eli[0] * dx), dx);
+  dy = fma(-s.el[1], qround(s.eli[1] * dy), dy);
   p.ux = dx;
   p.uy = dy;
-  qrsqrt(dx * dx + dy * dy, p.r, p.byr);
+  qrsqrt(fma(dx, dx, dy * dy), p.r, p.byr);
   p.ind = (int)(p.r * s.drti);
-  p.rem = p.r - p.ind * s.drt;
+  p.rem = fma(-(double)p.ind, s.drt, p.r);
   return p;
 }
 

@@ -446,6 +446,15 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
     wsw[L.off_gj + 2 * tid + 1] = gpy;
   }
 
+  // the pair sums over each wavefront (lane 0 of each has a row of red)
+  {
+    const double v[5] = {wave_sum(acc_ltf), wave_sum(acc_h0), wave_sum(acc_h1), wave_sum(acc_v0), wave_sum(acc_v1)};
+    if (l == 0) {
+#pragma unroll
+      for (int q = 0; q < 5; q++) red[8 * wv + q] = v[q];
+    }
+  }
+
   // rho_k per type and the k-space Ewald sum
   double pk0 = 0.0, pk1 = 0.0, pkt = 0.0;
   double* pw = props + (int64_t)w * s.n_props;
@@ -458,6 +467,26 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
     for (int k = tid; k < s.nk; k += S::T)
       kspace_terms(s, k, r0 ? r0[2 * k] : 0.0, r0 ? r0[2 * k + 1] : 0.0, r1 ? r1[2 * k] : 0.0,
                    r1 ? r1[2 * k + 1] : 0.0, pk0, pk1, pkt);
+  } else if (!MIX && s.nrhok) {
+    // k-vectors off the grid: each thread sums its own directly
+    for (int k = tid; k < s.nk; k += S::T) {
+      const double kx = s.kvec[2 * k], ky = s.kvec[2 * k + 1];
+      double rc[2] = {0.0, 0.0}, rs[2] = {0.0, 0.0};
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        if (t >= s.ntypes || !s.irhok[t]) continue;
+        for (int i = s.ipf[t]; i < s.ipf[t] + s.np[t]; i++) {
+          double sv, cv;
+          qsincos_sreg(kx * xs[2 * i] + ky * xs[2 * i + 1], &sv, &cv);
+          rc[t] += cv;
+          rs[t] += sv;
+        }
+        const int slot = s.jrhok + (s.irhok[t] - 1) * 2 * s.nk + 2 * k;
+        pw[slot] = rc[t];
+        pw[slot + 1] = rs[t];
+      }
+      kspace_terms(s, k, rc[0], rs[0], rc[1], rs[1], pk0, pk1, pkt);
+    }
   } else if (s.nrhok) {
     // passes of KMAXPT slots per thread: slots q = 2h, 2h+1 of a thread are
     // the two k-vectors of one item, which share their ky component
@@ -594,11 +623,10 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
 
   // the walker's eight sums: over each wavefront, then over the wavefronts
   {
-    const double v[8] = {wave_sum(acc_ltf), wave_sum(acc_h0), wave_sum(acc_h1), wave_sum(acc_v0),
-                         wave_sum(acc_v1),  wave_sum(pk0),    wave_sum(pk1),    wave_sum(pkt)};
+    const double v[3] = {wave_sum(pk0), wave_sum(pk1), wave_sum(pkt)};
     if (l == 0) {
 #pragma unroll
-      for (int q = 0; q < 8; q++) red[8 * wv + q] = v[q];
+      for (int q = 0; q < 3; q++) red[8 * wv + 5 + q] = v[q];
     }
   }
   __syncthreads();
@@ -634,6 +662,8 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   }
 }
 
+// (6 and 5 wavefronts per SIMD fit without spilling vector registers: the pair
+// sums leave for LDS before the phases, whose loops need the registers)
 template <bool MIX, int P>
 __global__ __launch_bounds__((PairShape<MIX, P>::T), MIX ? 5 : 6) void k_pairs(DevSys s, WsLayout L, const double* __restrict__ x,
                                                               double* __restrict__ ws,

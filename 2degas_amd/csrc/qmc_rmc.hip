@@ -133,7 +133,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_rmc_propose(
     if (!(t ? k.mov[1] : k.mov[0])) continue;
     const int o = t ? m0 + e - 2 * k.ipf[1] : e - 2 * k.ipf[0];
     const double var = t ? k.var[1] : k.var[0];
-    const uint64_t x1 = (lcg_pow(2 * (uint64_t)o + 1) * st0) & msk, x2 = (a * x1) & msk;
+    const uint64_t x1 = (lcg_pow(2 * o + 1) * st0) & msk, x2 = (a * x1) & msk;
     const double u1 = (double)x1 * 0x1p-48, u2 = (double)x2 * 0x1p-48;
     const double ua = k.bm_order == 0 ? u1 : u2, ub = k.bm_order == 0 ? u2 : u1;
     const double drift = -var * gj[e];
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_rmc_propose(
       acc = acc + v * (t ? k.vari[1] : k.vari[0]);
     }
     sc[3 * sl + (lane == 0 ? 0 : (lane == 1 ? 1 : 2))] = acc;
-    if (lane == 0) rng[r] = (int64_t)((lcg_pow(2 * (uint64_t)nmov) * st0) & msk);
+    if (lane == 0) rng[r] = (int64_t)((lcg_pow(2 * nmov) * st0) & msk);
   }
 }
 

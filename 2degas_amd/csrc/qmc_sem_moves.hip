@@ -31,11 +31,14 @@
 
 #include "qmc_sem.h"
 
-// Value of a table's cubic at the pair's grid index and remainder.
+// Value of a table's cubic at the pair's grid index and remainder.  (FMAs are
+// written out in this file where a sum has two products to choose from or a
+// block boundary may part them: the kernels' variants must agree to the bit, as
+// a job's results do not depend on the variant its launch takes.)
 __device__ __forceinline__ double sem_spline(const DevSys& s, TabRef t, const PairGeo& p) {
   const double4 c = tab_row(s.tab, t, p.ind);
   const double rm = p.rem * s.drti;
-  return c.x + rm * (c.y + rm * (c.z + rm * c.w));
+  return fma(rm, fma(rm, fma(rm, c.w, c.z), c.y), c.x);
 }
 
 __device__ __forceinline__ void sem_wave_sync() {
@@ -201,13 +204,13 @@ struct CplxRow {
     for (int i = 0; i < EPT; i++) row[cg + CG * i] = b[i];
   }
   static __device__ __forceinline__ double mod2(Ratio r) {
-    return (double)r.x * (double)r.x + (double)r.y * (double)r.y;
+    return fma((double)r.x, (double)r.x, (double)r.y * (double)r.y);
   }
   // A^-1 -= (t - e_j') (row j' of A^-1) / R, 1/R as conj(R) / |R|^2
   __device__ __forceinline__ void update(const Col* row, Ratio rz, double m2, bool mine, int cg) {
     const R inv2 = (R)(1.0 / m2);
     const R vr = mine ? tr - (R)1 : tr;
-    const R fr = -(vr * rz.x + ti * rz.y) * inv2, fi = -(ti * rz.x - vr * rz.y) * inv2;
+    const R fr = -fma(vr, rz.x, ti * rz.y) * inv2, fi = -fma(ti, rz.x, -(vr * rz.y)) * inv2;
 #pragma unroll
     for (int i = 0; i < EPT; i++) {
       const Z q = row[cg + CG * i];
@@ -227,20 +230,29 @@ struct SemShared {
   typename Row::Ratio ratio[2];        // R
   double2 gj[2];                       // three-body vector of electron j
   double red[2][W][3];                 // the wavefronts' Jastrow sums
+  double2 g[Row::NCOL];                // the columns' plane waves
   double2 step[64];                    // move i's displacement
   double uacc[64];                     // move i's acceptance uniform
+  uint64_t rng;                        // the walker's stream
 };
 
 // The thread's partner electron (N <= 64 W): position, three-body vector.
 struct SemWalk {
   double px, py, gx, gy;
-  double dlog, nacc;
 };
 
 template <int W>
 __device__ __forceinline__ void sem_sync() {
   if (W > 1) __syncthreads();
   else sem_wave_sync();
+}
+
+// The index of wavefront wv's thread, formed anew at each call: kept from one
+// phase to the next, it and what follows from it took the registers of the row.
+__device__ __forceinline__ int sem_tid(int wv) {
+  int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  __asm__ volatile("" : "+v"(l));
+  return 64 * wv + l;
 }
 
 // Moves of electrons j0..j1-1 of spin sp, in order.  The proposals come first:
@@ -250,38 +262,35 @@ __device__ __forceinline__ void sem_sync() {
 // end.
 template <class Row, int W, bool U3, class Sh>
 __device__ __forceinline__ void sem_spin(const DevSys& s, Sh& sh, const double* __restrict__ xs, SemWalk& wk, int w,
-                                         int tid, int sp, int j0, int j1, double sigma, uint64_t& st0,
-                                         typename Row::Z* __restrict__ ainv, int mm) {
+                                         int wv, int sp, int j0, int j1, const SemJob& jb) {
   typedef typename Row::Col Col;
-  // (what follows from the thread's index is formed anew for each spin and
-  // phase: kept from one to the next, it took the registers of the row)
-  __asm__ volatile("" : "+v"(tid));
-  const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), N = s.nptot;
+  int tid = sem_tid(wv);
+  const int lane = tid & 63, N = __builtin_amdgcn_readfirstlane(s.nptot);
   const SemSpin q = Row::spin(s, sp);
   const int p0 = pick2(s.ipf, sp), nc = Row::ncol(q);
   const int l = tid / Row::CG, cg = tid % Row::CG;
-  const double gx = lane < nc ? q.g[2 * lane] : 0.0, gy = lane < nc ? q.g[2 * lane + 1] : 0.0;
   const int nmv = j1 - j0;
   sem_sync<W>();
+  const uint64_t st0 = sh.rng;
+  if (tid < Row::NCOL) sh.g[tid] = tid < nc ? make_double2(q.g[2 * tid], q.g[2 * tid + 1]) : make_double2(0.0, 0.0);
   if (tid < nmv) {
-    uint64_t st = (st0 * lcg_pow(3 * (uint64_t)tid)) & ((1ULL << 48) - 1ULL);
+    uint64_t st = (st0 * lcg_pow(3 * tid)) & ((1ULL << 48) - 1ULL);
     const double u1 = rannyu(st), u2 = rannyu(st), ua = rannyu(st);
     double sv, cv;
     qsincos_sreg(6.283185307179586 * u2, &sv, &cv);
-    const double rad = sigma * sqrt(-2.0 * sem_log(u1));
+    const double rad = jb.sigma * sqrt(-2.0 * sem_log(u1));
     sh.step[tid] = make_double2(rad * cv, rad * sv);
     sh.uacc[tid] = ua;
   }
-  st0 = (st0 * lcg_pow(3 * (uint64_t)nmv)) & ((1ULL << 48) - 1ULL);
-  typename Row::Z* mat = ainv + ((int64_t)w * 2 + sp) * mm * mm;
   Row r;
-  r.load(q, mat, mm, l, cg);
+  r.load(q, (const typename Row::Z*)jb.ainv + ((int64_t)w * 2 + sp) * jb.mm * jb.mm, jb.mm, l, cg);
   // tables of the thread's partner
   const int tp = tpair(sp, ptype(s, tid));
   const TabRef t2 = tabref<TK_U2>(s, tp), t3 = tabref<TK_U3>(s, tp);
-  double du_acc = 0.0, na = 0.0, pm = 1.0;
-  int pe = 0;
+  double du_acc = 0.0, pm = 1.0;
+  int pe = 0, na = 0;
   sem_sync<W>();
+  if (tid == 0) sh.rng = (st0 * lcg_pow(3 * nmv)) & ((1ULL << 48) - 1ULL);
   // (electron j has not moved before its own move: xs holds its position)
   for (int j = j0; j < j1; j++) {
     const int jj = j - p0, b = (j - j0) & 1;
@@ -290,7 +299,8 @@ __device__ __forceinline__ void sem_spin(const DevSys& s, Sh& sh, const double* 
     const double xn = xo.x + dx.x, yn = xo.y + dx.y;
     if (lane < Row::NCOL) {
       double sv, cv;
-      qsincos_sreg(gx * xn + gy * yn, &sv, &cv);
+      const double2 g = sh.g[lane];
+      qsincos_sreg(fma(g.x, xn, g.y * yn), &sv, &cv);
       sh.ap[wv][lane] = Col{(decltype(Col::x))cv, (decltype(Col::x))sv};
     }
     // the Jastrow change of partner tid: the u2 term and, with U3, the
@@ -345,7 +355,8 @@ __device__ __forceinline__ void sem_spin(const DevSys& s, Sh& sh, const double* 
       const double2 g = sh.gj[b];
       du -= 0.5 * ((gjx * gjx + gjy * gjy) - (g.x * g.x + g.y * g.y));
     }
-    if (ua < mod2 * sem_exp(-2.0 * du)) {
+    // (the same on every lane: a scalar branch)
+    if (__builtin_amdgcn_readfirstlane(ua < mod2 * sem_exp(-2.0 * du))) {
       r.update(sh.row[b], rr, mod2, l == jj, cg);
       if (tid == j) {
         wk.px = xn;
@@ -357,16 +368,18 @@ __device__ __forceinline__ void sem_spin(const DevSys& s, Sh& sh, const double* 
       }
       int e;
       pm = frexp(pm * mod2, &e);
-      pe += e;
+      pe += __builtin_amdgcn_readfirstlane(e);
       du_acc += du;
-      na += 1.0;
+      na++;
     }
     if (W == 1) sem_wave_sync();
   }
-  __asm__ volatile("" : "+v"(tid));
-  r.store(q, mat, mm, tid / Row::CG, tid % Row::CG);
-  wk.dlog += 0.5 * (sem_log(pm) + pe * 0.6931471805599453) - du_acc;
-  wk.nacc += na;
+  tid = sem_tid(wv);
+  r.store(q, (typename Row::Z*)jb.ainv + ((int64_t)w * 2 + sp) * jb.mm * jb.mm, jb.mm, tid / Row::CG, tid % Row::CG);
+  if (tid == 0) {
+    jb.dlogpsi[w] += 0.5 * fma(pe, 0.6931471805599453, sem_log(pm)) - du_acc;
+    jb.nacc[w] += na;
+  }
 }
 
 // The rows of a spin by kind: rows a spin needs, and f(Row) for the spin's
@@ -384,28 +397,31 @@ struct SemKind<2, MR, CG> {
   typedef CplxRow<float2, MR, CG> Row;
 };
 
-// Wavefronts per SIMD the compiler has to fit: the most at which the loop does
-// not spill (an FP64 row of 32 complex entries takes 128 registers of its own,
-// one of 16 half of that, the rest of a move some 60, 80 with u3).  A bound that
-// spills some 100 registers doubled the sweep's time.
+// Wavefronts per SIMD the compiler has to fit: the most at which no vector
+// register spills (an FP64 row of 32 complex entries takes 128 registers of its
+// own, one of 16 half of that, the rest of a move some 60, 80 with u3).  Spills
+// cost time (100 registers doubled the sweep's), and correctness: the compiler
+// places a spill at the start of the block where diverged lanes join again,
+// before it turns them on, so that lanes lose the value.  In the FP32 kernel of
+// two wavefronts the sums kept over the call went that way.
 template <int KIND, int W, bool U3>
 struct SemBound {
-  static constexpr int value = KIND == 1 ? (W == 2 ? 2 : W == 4 || U3 ? 3 : 4) : (W == 2 && U3 ? 3 : 4);
+  static constexpr int value = KIND == 1 ? (W == 2 ? 2 : U3 ? 3 : 4) : (W == 2 && U3 ? 3 : 4);
 };
 
-// The moves of walker w of a job by 64 W threads (tid), both spins in order.
+// The moves of walker w of a job by W wavefronts (wv), both spins in order.
 template <int KIND, int W, bool U3, class Sh>
-__device__ __forceinline__ void sem_walker(const SemJob& jb, Sh& sh, double* xs, int w, int tid) {
-  typedef typename SemKind<KIND, 16, 4>::Row::Z Z;
+__device__ __forceinline__ void sem_walker(const SemJob& jb, Sh& sh, double* xs, int w, int wv) {
+  int tid = sem_tid(wv);
   const DevSys& s = *jb.sys;
-  const int N = s.nptot;
+  const int N = __builtin_amdgcn_readfirstlane(s.nptot);
   double* xw = jb.x + (int64_t)w * 2 * N;
-  SemWalk wk{0.0, 0.0, 0.0, 0.0, jb.dlogpsi[w], jb.nacc[w]};
+  SemWalk wk{0.0, 0.0, 0.0, 0.0};
   if (tid < N) {
     wk.px = xs[2 * tid] = xw[2 * tid];
     wk.py = xs[2 * tid + 1] = xw[2 * tid + 1];
   }
-  uint64_t st = (uint64_t)jb.rng[w];
+  if (tid == 0) sh.rng = (uint64_t)jb.rng[w];
   sem_sync<W>();
   if (U3 && s.has_u3 && tid < N) {
     // G_p = sum_b xi(r_pb) (x_b - x_p), minimum image: the per-particle
@@ -425,7 +441,7 @@ __device__ __forceinline__ void sem_walker(const SemJob& jb, Sh& sh, double* xs,
     if (a >= e) continue;
     auto run = [&](auto mr, auto cg) {
       typedef typename SemKind<KIND, decltype(mr)::value, decltype(cg)::value>::Row Row;
-      sem_spin<Row, W, U3>(s, sh, xs, wk, w, tid, sp, a, e, jb.sigma, st, (Z*)jb.ainv, jb.mm);
+      sem_spin<Row, W, U3>(s, sh, xs, wk, w, wv, sp, a, e, jb);
     };
     typedef std::integral_constant<int, 2> C2;
     typedef std::integral_constant<int, 4> C4;
@@ -451,15 +467,12 @@ __device__ __forceinline__ void sem_walker(const SemJob& jb, Sh& sh, double* xs,
       else if constexpr (W == 4) run(R64{}, C4{});
     }
   }
+  tid = sem_tid(wv);
   if (tid < N) {
     xw[2 * tid] = wk.px;
     xw[2 * tid + 1] = wk.py;
   }
-  if (tid == 0) {
-    jb.rng[w] = (int64_t)st;
-    jb.dlogpsi[w] = wk.dlog;
-    jb.nacc[w] = wk.nacc;
-  }
+  if (tid == 0) jb.rng[w] = (int64_t)sh.rng;
 }
 
 // One launch moves the walkers of several jobs (contexts of different N, decks
@@ -481,15 +494,15 @@ __global__ __launch_bounds__(64 * W, (SemBound<KIND, W, U3>::value)) void k_sem_
   int k = 0;
   while (k + 1 < jobs.njobs && (int)blockIdx.x >= jobs.job[k + 1].w0) k++;
   const SemJob& jb = jobs.job[k];
-  const int b = blockIdx.x - jb.w0;
+  const int b = blockIdx.x - jb.w0, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if constexpr (PAIRS) {
     if (jb.narrow) {
-      const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = 2 * b + wv;
-      if (w < jb.nw) sem_walker<KIND, 1, U3>(jb, sh.two[wv], sr_lds + 2 * wv * jb.sys->nptot, w, threadIdx.x & 63);
+      const int w = 2 * b + wv;
+      if (w < jb.nw) sem_walker<KIND, 1, U3>(jb, sh.two[wv], sr_lds + 2 * wv * jb.sys->nptot, w, 0);
       return;
     }
   }
-  sem_walker<KIND, W, U3>(jb, sh.one, sr_lds, b, threadIdx.x);
+  sem_walker<KIND, W, U3>(jb, sh.one, sr_lds, b, wv);
 }
 
 int launch_sem_moves(const SemJobs& jobs, int nblocks, int kind, int waves, bool u3, int nmax, hipStream_t st) {
