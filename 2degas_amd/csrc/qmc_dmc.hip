@@ -23,49 +23,6 @@ __global__ void k_dmc_begin(int nw, double* __restrict__ wate) {
   if (w < nw) wate[w] = 1.0;
 }
 
-// Before a move: each walker's energy and age.
-__global__ void k_dmc_pre(int nw, int np_, int jetot, const double* __restrict__ props,
-                          const double* __restrict__ age, double* __restrict__ eprev,
-                          double* __restrict__ aprev) {
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= nw) return;
-  eprev[w] = props[(int64_t)w * np_ + jetot];
-  aprev[w] = age[w];
-}
-
-// After move + metropolis_test: the local energy metropolis_test leaves
-// (reptation.f:2630-2632, 2652-2653: the mean of the new and old energies
-// when accepted, the old one otherwise), the weight factor
-// peso = exp(-npnorm (elocal - etrial) delta) bounded at mmult
-// (reptation.f:897-903), wate *= peso, and averages(2) with weight wate
-// (reptation.f:4300-4305: blk += p_old wate, blk_norm += wate).  One
-// wavefront per walker, lanes over properties.
-__global__ __launch_bounds__(QMC_BLOCK) void k_dmc_weight(
-    int nw, int np_, int jetot, int npnorm, double delta, double etrial, double mage, double mmult,
-    const double* __restrict__ props, const double* __restrict__ age,
-    const double* __restrict__ eprev, const double* __restrict__ aprev, double* __restrict__ wate,
-    double* __restrict__ wsum, double* __restrict__ blk, int32_t* __restrict__ counts) {
-  const int w = blockIdx.x * (QMC_BLOCK / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (w >= nw) return;
-  const double* p = props + (int64_t)w * np_;
-  const double eold = eprev[w];
-  const double elocal = age[w] == 0.0 ? 0.5 * (p[jetot] + eold) : eold;
-  double peso = exp(-(double)npnorm * (elocal - etrial) * delta);
-  const bool bounded = peso > mmult;
-  if (bounded) peso = mmult;
-  const double wt = wate[w] * peso;
-  double* b = blk + (int64_t)w * np_;
-  for (int k = lane; k < np_; k += 64) b[k] += p[k] * wt;
-  if (lane == 0) {
-    wate[w] = wt;
-    wsum[w] += wt;
-    if (bounded) atomicAdd(&counts[0], 1);
-    // move counts a forced move when the age reached mage (reptation.f:4650-4653)
-    if (w == 0 && aprev[0] == mage) atomicAdd(&counts[3], 1);
-  }
-}
-
 // branch2 (reptation.f:2162-2271) over the nw ranks.  The sums of the
 // weights and of their fractional parts, which the reference forms in rank
 // order over the gathered values, and the comb run on one thread over LDS
@@ -311,20 +268,13 @@ extern "C" int qmc_dmc_sweep(qmc_ctx* c, const qmc_walkers* w, const qmc_dmc_sta
   const double var0 = 2.0 * s.hbs2m[0] * prm->delta;
   const double var1 = s.ntypes > 1 ? 2.0 * s.hbs2m[1] * prm->delta : 1.0;
   const int nw = w->nw, NP = c->info.n_props, jetot = c->info.jetot - 1;
-  // the moves add the weighted block sums here, not the plain ones
-  qmc_walkers wv = *w;
-  wv.blk = nullptr;
+  const DmcWeight dm{d->wate, d->wsum, d->counts, prm->etrial, prm->delta, (double)prm->mmult, jetot};
   const int wpb = QMC_BLOCK / 64;
   for (int k = 0; k < nsteps; k++) {
     hipLaunchKernelGGL(k_dmc_begin, dim3((nw + 255) / 256), dim3(256), 0, st, nw, d->wate);
     for (int m = 0; m < prm->mmstep; m++) {
-      hipLaunchKernelGGL(k_dmc_pre, dim3((nw + 255) / 256), dim3(256), 0, st, nw, NP, jetot, w->props, w->age,
-                         c->d_eprev, c->d_aprev);
-      rc = vmc_step(c, &wv, st, prm->delta, var0, var1, prm->mage, prm->bm_order, nullptr, nullptr);
+      rc = vmc_step(c, w, st, prm->delta, var0, var1, prm->mage, prm->bm_order, nullptr, nullptr, &dm);
       if (rc) return rc;
-      hipLaunchKernelGGL(k_dmc_weight, dim3((nw + wpb - 1) / wpb), dim3(QMC_BLOCK), 0, st, nw, NP, jetot,
-                         s.npnorm, prm->delta, prm->etrial, prm->mage, (double)prm->mmult, w->props, w->age,
-                         c->d_eprev, c->d_aprev, d->wate, d->wsum, w->blk, d->counts);
     }
     hipLaunchKernelGGL(k_dmc_branch, dim3(1), dim3(DMC_BRANCH_THREADS), dmc_branch_lds(nw), st, nw, d->wate,
                        d->rng2, d->src, d->counts);

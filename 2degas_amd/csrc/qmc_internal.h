@@ -83,8 +83,6 @@ struct qmc_ctx {
   int vmc_nw = 0;
   double *d_xn = nullptr, *d_gn = nullptr, *d_hn = nullptr, *d_pn = nullptr, *d_wold = nullptr;
   int32_t *d_stn = nullptr, *d_sticky = nullptr;
-  // DMC: each walker's energy and age before its latest move
-  double *d_eprev = nullptr, *d_aprev = nullptr;
   // the VMC step as a captured graph, and what it was captured with
   bool use_graph = true;
   hipGraphExec_t vmc_exec = nullptr;
@@ -129,10 +127,18 @@ void free_vmc_graph(qmc_ctx* c);
 // Workspace of the evaluation kernels for nw walkers (allocates when it grows).
 int ensure_ws(qmc_ctx* c, int nw);
 int ensure_vmc_scratch(qmc_ctx* c, int nw);
+// What a DMC move adds to the acceptance: each walker's weight and its sum
+// over moves, and the event counts.
+struct DmcWeight {
+  double *wate, *wsum;
+  int32_t* counts;
+  double etrial, delta, mmult;
+  int jetot;
+};
 // One VMC step for every walker of w (proposal, evaluation, acceptance;
-// block sums when w->blk is set), queued on st.
+// block sums when w->blk is set, weighted when dm is), queued on st.
 int vmc_step(qmc_ctx* c, const qmc_walkers* w, hipStream_t st, double delta, double var0, double var1,
-             double mage, int bm_order, double* tp, double* ta);
+             double mage, int bm_order, double* tp, double* ta, const DmcWeight* dm);
 void free_rmc(qmc_ctx* c);
 
 

@@ -1076,43 +1076,49 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
 // sum_j (A^-1 G^2 A)_jj = -sum_k |g_k|^2.  Those two kernels are not launched
 // (at N=26, 256 walkers 31 of an 82 us VMC step, at N=122 1.05 of a 1.9 ms
 // evaluation).
-__global__ __launch_bounds__(QMC_BLOCK) void k_final(DevSys s, WsLayout L, double* __restrict__ ws,
-                                                     double* __restrict__ props,
-                                                     double* __restrict__ gout,
-                                                     double* __restrict__ hout,
-                                                     double* __restrict__ grad2,
-                                                     int32_t* __restrict__ status, int nw,
-                                                     double delta) {
-  const int w = blockIdx.x * (QMC_BLOCK / 64) + (threadIdx.x >> 6);
+//
+// Bound by latency: one wavefront per block, so that a few hundred walkers
+// reach every CU, what it reads fetched before anything depends on it, and
+// sums of property slots formed in registers (with four walkers per block and
+// slots read back after their stores 6.8 us at N = 26, 256 walkers, now 4.9 us).
+__global__ __launch_bounds__(64) void k_final(DevSys s, WsLayout L, double* __restrict__ ws,
+                                              double* __restrict__ props,
+                                              double* __restrict__ gout,
+                                              double* __restrict__ hout,
+                                              double* __restrict__ grad2,
+                                              int32_t* __restrict__ status,
+                                              double delta) {
+  const int w = blockIdx.x;
   const int lane = threadIdx.x & 63;
-  if (w >= nw || (s.nact && w >= *s.nact)) return;
+  if (s.nact && w >= *s.nact) return;
   const int N = s.nptot;
-  double* wsw = ws + (int64_t)w * L.per_walker;
+  const double* __restrict__ wsw = ws + (int64_t)w * L.per_walker;
   const double* sc = wsw + L.off_sc;
   double ltf = sc[SC_LTF];
+  double h[2] = {sc[SC_H0], sc[SC_H1]};
+  const double pv[3] = {sc[SC_P0], sc[SC_P1], sc[SC_PT]};
+  const double g2in = grad2[w];
   bool sing = false, guard = false;
+  double hd[2] = {0.0, 0.0}, g2ph = 0.0;
   if (s.has_det) {
-    for (int sp = 0; sp < s.ntypes; sp++) {
-      if (pick2(s.np, sp) == 0) continue;
-      const double* dsc = wsw + pick2(L.off_det, sp);
+#pragma unroll
+    for (int sp = 0; sp < 2; sp++) {
+      if (sp >= s.ntypes || s.np[sp] == 0) continue;
+      const double* dsc = wsw + L.off_det[sp];
       ltf -= dsc[DS_LOGDET];
       if (dsc[DS_SING] != 0.0) sing = true;
+      if (s.plain) continue;
+      hd[0] += dsc[DS_H0] + dsc[DS_X0];
+      hd[1] += dsc[DS_H1] + dsc[DS_X1];
+      g2ph += dsc[DS_G2];
     }
     // underflow guard of slater_excitations (reptation.f:10087-10092)
     guard = !(exp(-ltf * 2.0) > 0.0);
   }
   const bool use_det = s.has_det && !guard && !sing;
-  double h[2] = {sc[SC_H0], sc[SC_H1]};
-  double g2ph = 0.0;
   if (use_det) {
-    for (int sp = 0; sp < s.ntypes; sp++) {
-      if (pick2(s.np, sp) == 0) continue;
-      const double* dsc = wsw + pick2(L.off_det, sp);
-      if (s.plain) continue;
-      h[0] += dsc[DS_H0] + dsc[DS_X0];
-      h[1] += dsc[DS_H1] + dsc[DS_X1];
-      g2ph += dsc[DS_G2];
-    }
+    h[0] += hd[0];
+    h[1] += hd[1];
   }
   double* gw = gout + (int64_t)w * 2 * N;
   double g2t[2] = {0.0, 0.0}, ggs = 0.0;
@@ -1181,18 +1187,21 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_final(DevSys s, WsLayout L, doubl
       p[s.jun[t]] = 1.0 / sqrt(g2t[t]);
     }
     if (s.ntypes == 1) hout[(int64_t)w * 2 + 1] = 0.0;
-    p[s.jkin0] = kin0 / s.npnorm;
     p[s.jgg] = (s.adrift == 0.0) ? 1.0 : ggs / s.npnorm;
     if (use_det) grad2[w] = g2ph;
-    const double g2v = grad2[w];
-    p[s.jefp] = (s.ntheta != 0) ? g2v / s.npnorm : 0.0;
     p[s.jltf] = ltf;
 #pragma unroll
     for (int t = 0; t < 2; t++)
-      if (t < s.ntypes && s.jpot[t] >= 0) p[s.jpot[t]] = (s.tailc[t] + sc[SC_P0 + t]) / s.np[t];
-    p[s.jpot0] = (s.tailc_tot + sc[SC_PT] + s.v0) / s.npnorm;
-    p[s.jetot] = p[s.jpot0] + p[s.jkin0] + p[s.jefp];
-    p[s.je2] = p[s.jetot] * p[s.jetot];
+      if (t < s.ntypes && s.jpot[t] >= 0) p[s.jpot[t]] = (s.tailc[t] + pv[t]) / s.np[t];
+    const double pkin = kin0 / s.npnorm;
+    const double pefp = (s.ntheta != 0) ? (use_det ? g2ph : g2in) / s.npnorm : 0.0;
+    const double ppot = (s.tailc_tot + pv[2] + s.v0) / s.npnorm;
+    const double ptot = ppot + pkin + pefp;
+    p[s.jkin0] = pkin;
+    p[s.jefp] = pefp;
+    p[s.jpot0] = ppot;
+    p[s.jetot] = ptot;
+    p[s.je2] = ptot * ptot;
     if (status) status[w] = (guard ? 1 : 0) | (sing ? 2 : 0);
   }
 }

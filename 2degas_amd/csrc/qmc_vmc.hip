@@ -12,23 +12,20 @@
 // move, proposal half (reptation.f:4630-4646): for every moving type,
 // particle and dimension chi = cos(pi u1) sqrt(-2 var log u2),
 // x_new = chi - var g_old + x_old, w = -sum chi^2 / var.
-// One wavefront per walker, lanes over coordinates.  The reference draws two
+// One block per walker, a thread per coordinate.  The reference draws two
 // uniforms per moved coordinate in coordinate order, so the coordinate with
 // ordinal o among the moved ones takes draws 2o+1 and 2o+2 of the walker's
-// stream: each lane jumps there with a^(2o+1).  The chi^2 terms go to LDS
-// and lane 0 adds them in the reference's order.
+// stream: each thread jumps there with a^(2o+1).  Bound by latency (a cosine, a
+// logarithm and the sum): with a wavefront per walker that walked over its
+// coordinates and one lane adding the chi^2 4.9 us at N = 26 and 7.9 us at
+// N = 74 (256 walkers), now 3.6 and 4.7.
 __global__ __launch_bounds__(QMC_BLOCK) void k_vmc_propose(
-    DevSys s, int nw, const double* __restrict__ x_old, const double* __restrict__ g_old,
+    DevSys s, const double* __restrict__ x_old, const double* __restrict__ g_old,
     double* __restrict__ x_new, int64_t* __restrict__ rng, double* __restrict__ wold,
     double var0, double var1, int bm_order) {
-  __shared__ double chi2[QMC_BLOCK / 64][2 * QMC_MAX_PARTICLES];
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int w = blockIdx.x * (QMC_BLOCK / 64) + wv;
-  if (w >= nw) return;  // no barrier below: each wavefront works alone
-  const int N = s.nptot, n2 = 2 * N;
-  const double* xo = x_old + (int64_t)w * n2;
-  const double* go = g_old + (int64_t)w * n2;
-  double* xn = x_new + (int64_t)w * n2;
+  __shared__ double red[2][QMC_BLOCK / 64];
+  const int e = threadIdx.x, w = blockIdx.x;
+  const int n2 = 2 * s.nptot;
   const uint64_t st0 = (uint64_t)rng[w];
   const double pi = 3.141592653589793;
   const uint64_t msk = (1ULL << 48) - 1ULL, a = 34522712143931ULL;
@@ -36,58 +33,99 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_vmc_propose(
   const bool mov0 = s.hbs2m[0] != 0.0, mov1 = two && s.hbs2m[1] != 0.0;
   const int m0 = mov0 ? 2 * s.np[0] : 0;  // moved coordinates of type 0
   const int nmov = m0 + (mov1 ? 2 * s.np[1] : 0);
-  double* c2 = chi2[wv];
-  for (int e = lane; e < n2; e += 64) {
-    const int t = two && e >= 2 * s.ipf[1] ? 1 : 0;
-    if (!(t ? mov1 : mov0)) {
-      xn[e] = xo[e];
-      continue;
+  double c2 = 0.0;
+  const int t = two && e >= 2 * s.ipf[1] ? 1 : 0;
+  if (e < n2) {
+    const double xo = x_old[(int64_t)w * n2 + e], go = g_old[(int64_t)w * n2 + e];
+    double xe = xo;
+    if (t ? mov1 : mov0) {
+      const int o = t ? m0 + e - 2 * s.ipf[1] : e - 2 * s.ipf[0];
+      const double var = t ? var1 : var0;
+      const uint64_t x1 = (lcg_pow10(2 * o + 1) * st0) & msk, x2 = (a * x1) & msk;
+      const double u1 = (double)x1 * 0x1p-48, u2 = (double)x2 * 0x1p-48;
+      const double ua = bm_order == 0 ? u1 : u2, ub = bm_order == 0 ? u2 : u1;
+      const double chi = cos(pi * ua) * sqrt(-2.0 * var * log(ub));
+      c2 = chi * chi;
+      xe = chi + (-var * go) + xo;
     }
-    const int o = t ? m0 + e - 2 * s.ipf[1] : e - 2 * s.ipf[0];
-    const double var = t ? var1 : var0;
-    const uint64_t x1 = (lcg_pow(2 * (uint64_t)o + 1) * st0) & msk, x2 = (a * x1) & msk;
-    const double u1 = (double)x1 * 0x1p-48, u2 = (double)x2 * 0x1p-48;
-    const double ua = bm_order == 0 ? u1 : u2, ub = bm_order == 0 ? u2 : u1;
-    const double chi = cos(pi * ua) * sqrt(-2.0 * var * log(ub));
-    c2[e] = chi * chi;
-    xn[e] = chi + (-var * go[e]) + xo[e];
+    x_new[(int64_t)w * n2 + e] = xe;
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if (lane == 0) {
-    double wo = 0.0;
-    for (int t = 0; t < s.ntypes; t++) {
-      if (!(t ? mov1 : mov0)) continue;
-      const double var = t == 0 ? var0 : var1;
-      const int e0 = 2 * pick2(s.ipf, t), e1 = e0 + 2 * pick2(s.np, t);
-      double wt = 0.0;
-      for (int e = e0; e < e1; e++) wt = wt - c2[e];
-      wo = wo + wt * (1.0 / var);
+  const double s0 = wave_sum(t ? 0.0 : c2), s1 = wave_sum(t ? c2 : 0.0);
+  if ((e & 63) == 0) {
+    red[0][e >> 6] = s0;
+    red[1][e >> 6] = s1;
+  }
+  __syncthreads();
+  if (e == 0) {
+    double w0 = 0.0, w1 = 0.0;
+    for (int v = 0; v < QMC_BLOCK / 64; v++) {
+      w0 -= red[0][v];
+      w1 -= red[1][v];
     }
+    double wo = 0.0;
+    if (mov0) wo = wo + w0 * (1.0 / var0);
+    if (mov1) wo = wo + w1 * (1.0 / var1);
     wold[w] = wo;
-    rng[w] = (int64_t)((lcg_pow(2 * (uint64_t)nmov) * st0) & msk);
+    rng[w] = (int64_t)((lcg_pow10(2 * nmov) * st0) & msk);
   }
 }
 
 // move, acceptance half (reptation.f:4648-4678) + metropolis_test
-// (reptation.f:2622-2659) + averages(2) (reptation.f:4300-4305).
-// One wavefront per walker.
+// (reptation.f:2622-2659) + averages(2) (reptation.f:4300-4305), and with DMC
+// the walker's weight: the local energy metropolis_test leaves
+// (reptation.f:2630-2632, 2652-2653: the mean of the new and old energies
+// when accepted, the old one otherwise), the factor
+// peso = exp(-npnorm (elocal - etrial) delta) bounded at mmult
+// (reptation.f:897-903), wate *= peso, and averages(2) with weight wate
+// (reptation.f:4300-4305: blk += p_old wate, blk_norm += wate).
+//
+// One block per walker.  The kernel is bound by latency: a few dependent
+// loads, the exponential, and the pass over the properties.  So every
+// wavefront forms the decision for itself from the same loads in the same
+// order, the properties, the block sums and the new configuration are fetched
+// before it, and one barrier stands between the last read and the first
+// write.  A wavefront per walker, walking over the properties 64 at a time
+// after the decision, took 11.0 us at N = 26 and 12.3 us at N = 74 (256 walkers;
+// now 4.8 and 4.6).  For 4096 walkers of N = 122 in DMC the bytes count, some
+// 0.4 GB of properties and sums: 86 us, where the weight's own kernel and pass
+// took 91 us after the acceptance.
+constexpr int VA_SLOTS = 4;  // properties per thread fetched ahead
+template <bool DMC>
 __global__ __launch_bounds__(QMC_BLOCK) void k_vmc_accept(
-    DevSys s, int nw, double var0, double var1, double mage, double* __restrict__ x_old,
+    DevSys s, double var0, double var1, double mage, double* __restrict__ x_old,
     double* __restrict__ g_old, double* __restrict__ h_old, double* __restrict__ p_old,
     double* __restrict__ age, const double* __restrict__ x_new, const double* __restrict__ g_new,
     const double* __restrict__ h_new, const double* __restrict__ p_new, int64_t* __restrict__ rng,
     const double* __restrict__ wold, const int32_t* __restrict__ status,
     int32_t* __restrict__ sticky, double* __restrict__ blk, double* __restrict__ trace_p,
-    double* __restrict__ trace_age, int jacc, int jltf) {
-  const int w = blockIdx.x * (QMC_BLOCK / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (w >= nw) return;
+    double* __restrict__ trace_age, int jacc, int jltf, DmcWeight dm) {
+  const int w = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int N = s.nptot, NP = s.n_props;
-  const double* xo = x_old + (int64_t)w * 2 * N;
+  double* xo = x_old + (int64_t)w * 2 * N;
   const double* xn = x_new + (int64_t)w * 2 * N;
   const double* gn = g_new + (int64_t)w * 2 * N;
+  double* po = p_old + (int64_t)w * NP;
+  const double* pn = p_new + (int64_t)w * NP;
+  double* b = blk ? blk + (int64_t)w * NP : nullptr;
+  double vn[VA_SLOTS], vo[VA_SLOTS], vb[VA_SLOTS];
+#pragma unroll
+  for (int u = 0; u < VA_SLOTS; u++) {
+    const int k = tid + u * QMC_BLOCK;
+    vn[u] = vo[u] = vb[u] = 0.0;
+    if (k < NP) {
+      vn[u] = pn[k];
+      vo[u] = po[k];
+      if (b) vb[u] = b[k];
+    }
+  }
+  double xk = 0.0, gk = 0.0, hk = 0.0;
+  if (tid < 2 * N) {
+    xk = xn[tid];
+    gk = gn[tid];
+  }
+  if (tid < 2) hk = h_new[(int64_t)w * 2 + tid];
+  const double age0 = age[w], ltf0 = po[jltf], ltf1 = pn[jltf], wo = wold[w];
+  uint64_t rs = (uint64_t)rng[w];
   double wt[2] = {0.0, 0.0};
   for (int ip = lane; ip < N; ip += 64) {
     const int t = ptype(s, ip);
@@ -101,58 +139,86 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_vmc_accept(
   }
   wt[0] = wave_sum(wt[0]);
   wt[1] = wave_sum(wt[1]);
-  double p = 0.0;
-  int acc = 0;
-  if (lane == 0) {
-    const double* po = p_old + (int64_t)w * NP;
-    const double* pn = p_new + (int64_t)w * NP;
-    if (age[w] == mage) {
-      p = 1.0;
-    } else {
-      double wnew = 0.0;
-      if (s.hbs2m[0] != 0.0) wnew = wnew + wt[0] * (1.0 / var0);
-      if (s.ntypes > 1 && s.hbs2m[1] != 0.0) wnew = wnew + wt[1] * (1.0 / var1);
-      p = (po[jltf] - pn[jltf]) * 2.0 + 0.5 * (wnew - wold[w]);
-      p = fmin(0.0, fmax(-50.0, p));
-      p = exp(p);
-    }
-    double u = 1.0;
-    if (p < 1.0) {
-      uint64_t st = (uint64_t)rng[w];
-      u = rannyu(st);
-      rng[w] = (int64_t)st;
-    }
-    acc = p >= u;
-    sticky[w] |= status[w];
+  double p;
+  if (age0 == mage) {
+    p = 1.0;
+  } else {
+    double wnew = 0.0;
+    if (s.hbs2m[0] != 0.0) wnew = wnew + wt[0] * (1.0 / var0);
+    if (s.ntypes > 1 && s.hbs2m[1] != 0.0) wnew = wnew + wt[1] * (1.0 / var1);
+    p = (ltf0 - ltf1) * 2.0 + 0.5 * (wnew - wo);
+    p = fmin(0.0, fmax(-50.0, p));
+    p = exp(p);
   }
-  acc = __shfl(acc, 0, 64);
-  p = __shfl(p, 0, 64);
+  double u = 1.0;
+  if (p < 1.0) u = rannyu(rs);
+  const bool acc = p >= u;
+  const double a = acc ? 0.0 : age0 + 1.0;
+  double wgt = 1.0, wsum0 = 0.0;
+  bool bounded = false;
+  if (DMC) {
+    const double eold = po[dm.jetot], enew = acc ? pn[dm.jetot] : eold;
+    const double elocal = a == 0.0 ? 0.5 * (enew + eold) : eold;
+    double peso = exp(-(double)s.npnorm * (elocal - dm.etrial) * dm.delta);
+    bounded = peso > dm.mmult;
+    if (bounded) peso = dm.mmult;
+    wgt = dm.wate[w] * peso;
+    wsum0 = dm.wsum[w];
+  }
+  __syncthreads();  // every wavefront has read what the stores below change
   // copy new into old where accepted, set p_old(jacc) = p and add p_old to
-  // the block sums; each lane owns its slots, so no lane reads another's
-  double* po = p_old + (int64_t)w * NP;
-  const double* pn = p_new + (int64_t)w * NP;
-  double* b = blk ? blk + (int64_t)w * NP : nullptr;
-  for (int k = lane; k < NP; k += 64) {
-    const double v = (k == jacc) ? p : (acc ? pn[k] : po[k]);
-    po[k] = v;
-    if (b) b[k] += v;
+  // the block sums
+#pragma unroll
+  for (int q = 0; q < VA_SLOTS; q++) {
+    const int k = tid + q * QMC_BLOCK;
+    if (k < NP) {
+      const double v = (k == jacc) ? p : (acc ? vn[q] : vo[q]);
+      if (acc || k == jacc) po[k] = v;
+      if (b) b[k] = DMC ? vb[q] + v * wgt : vb[q] + v;
+    }
+  }
+  for (int k0 = VA_SLOTS * QMC_BLOCK + tid; k0 < NP; k0 += VA_SLOTS * QMC_BLOCK) {
+    const double* ps = acc ? pn : po;
+#pragma unroll
+    for (int q = 0; q < VA_SLOTS; q++) {
+      const int k = k0 + q * QMC_BLOCK;
+      if (k < NP) {
+        vn[q] = k == jacc ? p : ps[k];
+        if (b) vb[q] = b[k];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < VA_SLOTS; q++) {
+      const int k = k0 + q * QMC_BLOCK;
+      if (k < NP) {
+        if (acc || k == jacc) po[k] = vn[q];
+        if (b) b[k] = DMC ? vb[q] + vn[q] * wgt : vb[q] + vn[q];
+      }
+    }
   }
   if (acc) {
-    double* xo2 = x_old + (int64_t)w * 2 * N;
-    double* go = g_old + (int64_t)w * 2 * N;
-    for (int k = lane; k < 2 * N; k += 64) {
-      xo2[k] = xn[k];
-      go[k] = gn[k];
+    if (tid < 2 * N) {
+      xo[tid] = xk;
+      g_old[(int64_t)w * 2 * N + tid] = gk;
     }
-    if (lane < 2) h_old[(int64_t)w * 2 + lane] = h_new[(int64_t)w * 2 + lane];
+    if (tid < 2) h_old[(int64_t)w * 2 + tid] = hk;
   }
-  if (lane == 0) {
-    const double a = acc ? 0.0 : age[w] + 1.0;
+  if (tid == 0) {
+    rng[w] = (int64_t)rs;
+    sticky[w] |= status[w];
     age[w] = a;
     if (trace_p) trace_p[w] = p;
     if (trace_age) trace_age[w] = a;
+    if (DMC) {
+      dm.wate[w] = wgt;
+      dm.wsum[w] = wsum0 + wgt;
+      if (bounded) atomicAdd(&dm.counts[0], 1);
+      // move counts a forced move when the age reached mage (reptation.f:4650-4653)
+      if (w == 0 && age0 == mage) atomicAdd(&dm.counts[3], 1);
+    }
   }
 }
+static_assert(2 * QMC_MAX_PARTICLES <= QMC_BLOCK, "one coordinate per thread");
 
 // read_conf's start: age 0 and p_old(jacc) = 1 after the evaluation.
 __global__ void k_vmc_start(int nw, int np_, int jacc, double* __restrict__ props,
@@ -173,11 +239,8 @@ void free_vmc(qmc_ctx* c) {
   (void)hipFree(c->d_wold);
   (void)hipFree(c->d_stn);
   (void)hipFree(c->d_sticky);
-  (void)hipFree(c->d_eprev);
-  (void)hipFree(c->d_aprev);
   c->d_xn = c->d_gn = c->d_hn = c->d_pn = c->d_wold = nullptr;
   c->d_stn = c->d_sticky = nullptr;
-  c->d_eprev = c->d_aprev = nullptr;
   c->vmc_nw = 0;
 }
 
@@ -193,8 +256,6 @@ int ensure_vmc_scratch(qmc_ctx* c, int nw) {
   HIPCHK(hipMalloc(&c->d_wold, sizeof(double) * nw));
   HIPCHK(hipMalloc(&c->d_stn, sizeof(int32_t) * nw));
   HIPCHK(hipMalloc(&c->d_sticky, sizeof(int32_t) * nw));
-  HIPCHK(hipMalloc(&c->d_eprev, sizeof(double) * nw));
-  HIPCHK(hipMalloc(&c->d_aprev, sizeof(double) * nw));
   HIPCHK(hipMemset(c->d_pn, 0, sizeof(double) * NP * nw));
   // a sweep may run without a start call (state loaded by the caller)
   HIPCHK(hipMemset(c->d_sticky, 0, sizeof(int32_t) * nw));
@@ -227,19 +288,18 @@ extern "C" int qmc_vmc_start(qmc_ctx* c, const qmc_walkers* w, void* stream) {
 
 // One VMC step for every walker: proposal, evaluation, acceptance.
 int vmc_step(qmc_ctx* c, const qmc_walkers* w, hipStream_t st, double delta, double var0, double var1,
-             double mage, int bm_order, double* tp, double* ta) {
+             double mage, int bm_order, double* tp, double* ta, const DmcWeight* dm) {
   const DevSys& s = c->s;
   const int nw = w->nw;
-  const int wpb = QMC_BLOCK / 64;
-  hipLaunchKernelGGL(k_vmc_propose, dim3((nw + wpb - 1) / wpb), dim3(QMC_BLOCK), 0, st, s, nw,
-                     w->x, w->g, c->d_xn, w->rng, c->d_wold, var0, var1, bm_order);
+  hipLaunchKernelGGL(k_vmc_propose, dim3(nw), dim3(QMC_BLOCK), 0, st, s, w->x, w->g, c->d_xn,
+                     w->rng, c->d_wold, var0, var1, bm_order);
   // the fixed-phase scratch is shared by proposals, as the COMMON is
   int rc = launch_eval(c, nw, c->d_xn, c->d_pn, c->d_gn, c->d_hn, w->grad2_ph, c->d_stn, st, delta);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_vmc_accept, dim3((nw + wpb - 1) / wpb), dim3(QMC_BLOCK), 0, st, s, nw,
+  hipLaunchKernelGGL(dm ? k_vmc_accept<true> : k_vmc_accept<false>, dim3(nw), dim3(QMC_BLOCK), 0, st, s,
                      var0, var1, mage, w->x, w->g, w->h, w->props, w->age, c->d_xn, c->d_gn,
                      c->d_hn, c->d_pn, w->rng, c->d_wold, c->d_stn, c->d_sticky, w->blk, tp, ta,
-                     c->info.jacc - 1, c->info.jltf - 1);
+                     c->info.jacc - 1, c->info.jltf - 1, dm ? *dm : DmcWeight{});
   return QMC_OK;
 }
 
@@ -277,7 +337,7 @@ extern "C" int qmc_vmc_sweep(qmc_ctx* c, const qmc_walkers* w, int nsteps, doubl
     for (int k = 0; k < nsteps; k++) {
       rc = vmc_step(c, w, st, delta, var0, var1, mage, bm_order,
                     trace_p ? trace_p + (int64_t)k * nw : nullptr,
-                    trace_age ? trace_age + (int64_t)k * nw : nullptr);
+                    trace_age ? trace_age + (int64_t)k * nw : nullptr, nullptr);
       if (rc) return rc;
     }
     HIPCHK(hipGetLastError());
@@ -302,7 +362,7 @@ extern "C" int qmc_vmc_sweep(qmc_ctx* c, const qmc_walkers* w, int nsteps, doubl
   if (!c->vmc_exec || key != c->vmc_key) {
     free_vmc_graph(c);
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    rc = vmc_step(c, w, c->stream, delta, var0, var1, mage, bm_order, nullptr, nullptr);
+    rc = vmc_step(c, w, c->stream, delta, var0, var1, mage, bm_order, nullptr, nullptr, nullptr);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc) {
