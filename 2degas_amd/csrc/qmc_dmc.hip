@@ -15,6 +15,8 @@
 // the properties; the age and sign live in separate arrays).
 #include "qmc_internal.h"
 
+#include <type_traits>
+
 #define DMC_WMULT 10.0  // branch2's bound of a weight (reptation.f:2167-2168)
 
 // Start of a step: every weight 1 (dmc, reptation.f:886-890).
@@ -23,16 +25,78 @@ __global__ void k_dmc_begin(int nw, double* __restrict__ wate) {
   if (w < nw) wate[w] = 1.0;
 }
 
-// branch2 (reptation.f:2162-2271) over the nw ranks.  The sums of the
-// weights and of their fractional parts, which the reference forms in rank
-// order over the gathered values, and the comb run on one thread over LDS
-// copies, in the reference's order of operations; the bound, the
-// normalization, the integer parts and the transfers (integer prefix sums)
-// are spread over the workgroup.  LDS: nw doubles (the weights, then their
-// fractional parts, then the prefix sums of the extra copies) and nw ints
-// (the multiplicities).  On return src[j] is the walker j takes its
-// configuration from.
+// branch2 (reptation.f:2162-2271) over the nw ranks.  What the reference forms
+// in rank order, one operation after the other, stays in that order on one
+// thread: the sum of the weights, the sum of their fractional parts and the
+// comb's running sum k.  Everything else is spread over the workgroup: the
+// bound, the normalization, the integer parts, the comb's draws and marks, the
+// transfers.  LDS: nw doubles (the weights, then their fractional parts,
+// then the prefix sums of the extra copies) and nw ints (the
+// multiplicities).  On return src[j] is the walker j takes its configuration
+// from.
+//
+// The comb (reptation.f:2196-2210) makes nint(k0) draws of rannyu2, one in each
+// unit of k.  The reference moves its walker pointer while k < r (then marks
+// the walker), then while k < 1, and subtracts 1 from k before each draw.  A
+// draw r is below 1, so that whether k has reached 1 does not depend on r:
+// walker j adds its fractional part, and 1 is taken off when k is then 1 or
+// more, which is what the fraction of k leaves (k < 2, the subtraction is
+// exact).  That chain, two operations per walker, is all that thread does; k0
+// is summed by a second wavefront meanwhile.  Thread c takes the walkers from
+// S c on: it gets k there, repeats their additions, counts the units that end
+// before them, jumps the stream to their draw and marks in parallel.  With the
+// draws, the comparisons with r and the marks on the one thread too, 4096
+// walkers took 242 us (now 72).
 #define DMC_BRANCH_THREADS 1024
+#define DMC_CHUNK 16
+
+// f(j, v[j]) for j = 0..nw-1 in order, two register chunks read in turn, each a
+// chunk's walk ahead of its use (the barriers keep the compiler from moving the
+// reads down to it).
+template <class F>
+__device__ __forceinline__ void dmc_in_order(const double* v, int nw, F&& f) {
+  constexpr int C = DMC_CHUNK;
+  const int n = nw / (2 * C) * (2 * C);
+  double a[C], b[C];
+  if (n > 0) {
+#pragma unroll
+    for (int u = 0; u < C; u++) a[u] = v[u];
+  }
+  for (int j = 0; j < n; j += 2 * C) {
+#pragma unroll
+    for (int u = 0; u < C; u++) b[u] = v[j + C + u];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < C; u++) f(j + u, a[u]);
+    const int jn = j + 2 * C < n ? j + 2 * C : j;
+#pragma unroll
+    for (int u = 0; u < C; u++) a[u] = v[jn + u];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < C; u++) f(j + C + u, b[u]);
+  }
+  for (int j = n; j < nw; j++) f(j, v[j]);
+}
+
+// Exclusive prefix sums over the workgroup of each thread's a and b; ta: the
+// total of a.
+__device__ __forceinline__ void dmc_scan(int tid, int* pa, int* pb, int& a, int& b, int& ta) {
+  const int a0 = a, b0 = b;
+  __syncthreads();
+  pa[tid] = a;
+  pb[tid] = b;
+  __syncthreads();
+  for (int o = 1; o < DMC_BRANCH_THREADS; o <<= 1) {
+    const int aa = tid >= o ? pa[tid - o] : 0, ab = tid >= o ? pb[tid - o] : 0;
+    __syncthreads();
+    pa[tid] += aa;
+    pb[tid] += ab;
+    __syncthreads();
+  }
+  a = pa[tid] - a0;
+  b = pb[tid] - b0;
+  ta = pa[DMC_BRANCH_THREADS - 1];
+}
 
 __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, double* __restrict__ wate,
                                                                    int64_t* __restrict__ rng2,
@@ -41,9 +105,19 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
   extern __shared__ __attribute__((aligned(16))) unsigned char dmc_lds[];
   double* sw = reinterpret_cast<double*>(dmc_lds);
   int* sm = reinterpret_cast<int*>(sw + nw);
-  __shared__ double sh_somma;
-  __shared__ int pe[DMC_BRANCH_THREADS], pr[DMC_BRANCH_THREADS];
+  // places used one after the other
+  __shared__ union {
+    struct {
+      double somma;
+      int odd;
+    };
+    double start[DMC_BRANCH_THREADS];
+    int scan[2][DMC_BRANCH_THREADS];
+  } sh;
+  __shared__ long sh_draws;
   const int tid = threadIdx.x;
+  const uint64_t st0 = (uint64_t)rng2[0];
+  if (tid == 0) sh.odd = 0;
   // weights above wmult are bounded (reptation.f:2176-2182)
   for (int i = tid; i < nw; i += DMC_BRANCH_THREADS) {
     double v = wate[i];
@@ -57,80 +131,132 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
   __syncthreads();
   if (tid == 0) {
     double somma = 0.0;
-#pragma unroll 8
-    for (int i = 0; i < nw; i++) somma = somma + sw[i];
-    sh_somma = somma;
+    dmc_in_order(sw, nw, [&](int, double v) { somma = somma + v; });
+    sh.somma = somma;
   }
   __syncthreads();
   // multiplicities: integer parts, and the fractional parts to comb
   // (reptation.f:2189-2195)
-  const double somma = sh_somma;
+  const double somma = sh.somma;
+  bool odd = false;
   for (int i = tid; i < nw; i += DMC_BRANCH_THREADS) {
     const double ww = ((double)nw * sw[i]) / somma;
     const int tm = (int)ww;
+    const double v = ww - (double)tm;
     sm[i] = tm;
-    sw[i] = ww - (double)tm;
+    sw[i] = v;
+    odd |= !(v >= 0.0 && v < 1.0);
   }
+  if (odd) sh.odd = 1;
   __syncthreads();
-  if (tid == 0) {
-    double k0 = 0.0;
-#pragma unroll 8
-    for (int i = 0; i < nw; i++) k0 = k0 + sw[i];
-    // The comb: nint(k0) draws of rannyu2, one in each unit of the running
-    // sum of the fractional parts (reptation.f:2196-2210).  The reference
-    // moves its walker pointer while k < r (then marks the walker), then
-    // while k < 1, and subtracts 1 from k before each draw; walked here in
-    // walker order, k gets the same additions and subtractions in the same
-    // order: after each walker's fractional part, the draws whose points
-    // that walker reaches are taken (marked, k reaches 1, k - 1 and the next
-    // draw), so the loads do not wait on the comparisons.
-    const long ndraw = lround(k0);
-    uint64_t st = (uint64_t)rng2[0];
-    long d = 0;
-    double k = 0.0, r = 0.0;
-    bool seek_r = false;
-    if (ndraw > 0) {
-      r = rannyu(st);
-      d = 1;
-      seek_r = true;  // k = 1 - 1 before the first draw
-    }
-    // eight fractional parts at a time into registers, the marks counted
-    // in registers and added to the multiplicities per chunk
-    for (int j0 = 0; j0 < nw && d > 0; j0 += 8) {
-      double v[8];
-      int mk[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        v[u] = j0 + u < nw ? sw[j0 + u] : 0.0;
-        mk[u] = 0;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        if (j0 + u < nw && d > 0) {
-          k = k + v[u];
-          for (;;) {
-            if (seek_r) {
-              if (k < r) break;
-              mk[u] += 1;
-              seek_r = false;
-            }
-            if (k < 1.0) break;
-            if (d >= ndraw) {
-              d = 0;
-              break;
-            }
-            k = k - 1.0;
-            r = rannyu(st);
-            d++;
-            seek_r = true;
+  // threads' walkers, in order
+  const int S = nw <= 4 * DMC_BRANCH_THREADS ? 4 : nw <= 8 * DMC_BRANCH_THREADS ? 8 : 16;
+  const int i0 = min(nw, tid * S), i1 = min(nw, i0 + S);
+  const bool any_odd = sh.odd;
+  __syncthreads();
+  if (any_odd) {
+    // fractional parts outside [0, 1) (weights below 0 or that are no
+    // numbers): the reference's walk as it is, on one thread
+    if (tid == 0) {
+      double k0 = 0.0, k = 0.0;
+      for (int i = 0; i < nw; i++) k0 = k0 + sw[i];
+      const long ndraw = lround(k0);
+      uint64_t st = st0;
+      long d = ndraw > 0 ? 1 : 0;
+      double r = d ? rannyu(st) : 0.0;
+      bool seek_r = true;  // k = 1 - 1 before the first draw
+      for (int j = 0; j < nw && d > 0; j++) {
+        k = k + sw[j];
+        for (;;) {
+          if (seek_r) {
+            if (k < r) break;
+            sm[j] += 1;
+            seek_r = false;
           }
+          if (k < 1.0) break;
+          if (d >= ndraw) {
+            d = 0;
+            break;
+          }
+          k = k - 1.0;
+          r = rannyu(st);
+          d++;
+          seek_r = true;
         }
       }
-#pragma unroll
-      for (int u = 0; u < 8; u++)
-        if (mk[u]) sm[j0 + u] += mk[u];
+      rng2[0] = (int64_t)st;
     }
-    rng2[0] = (int64_t)st;
+  } else {
+    // k at walker S c, c = 0, 1, ..: with its fractional part, before 1 is
+    // taken off
+    auto chain = [&](auto stride) {
+      constexpr int S = decltype(stride)::value;
+      double k = 0.0;
+      dmc_in_order(sw, nw, [&](int j, double v) {
+        const double t = k + v;
+        if (j % S == 0) sh.start[j / S] = t;
+        k = __builtin_amdgcn_fract(t);
+      });
+    };
+    if (tid == 0) {
+      if (S == 4) chain(std::integral_constant<int, 4>{});
+      else if (S == 8) chain(std::integral_constant<int, 8>{});
+      else chain(std::integral_constant<int, 16>{});
+    }
+    if (tid == 64) {
+      double k0 = 0.0;
+      dmc_in_order(sw, nw, [&](int, double v) { k0 = k0 + v; });
+      sh_draws = lround(k0);
+    }
+    __syncthreads();
+    const long ndraw = sh_draws;
+    // k after walker i0 - 1, and before 1 is taken off at walker i0
+    double kb = 0.0, t0 = 0.0;
+    if (i0 < i1) {
+      t0 = sh.start[tid];
+      if (i0 > 0) {
+        kb = __builtin_amdgcn_fract(sh.start[tid - 1]);
+        for (int i = i0 - S + 1; i < i0; i++) kb = __builtin_amdgcn_fract(kb + sw[i]);
+      }
+    }
+    int ends = 0, none = 0, units;
+    double t = t0;
+    for (int i = i0; i < i1; i++) {
+      if (i > i0) t = __builtin_amdgcn_fract(t) + sw[i];
+      ends += t >= 1.0 ? 1 : 0;
+    }
+    dmc_scan(tid, sh.scan[0], sh.scan[1], ends, none, units);
+    long d = 1 + ends;  // the draw walker i0 is combed with, if it is made
+    if (i0 < i1 && d <= ndraw) {
+      uint64_t st = (lcg_pow((uint32_t)d) * st0) & ((1ULL << 48) - 1ULL);
+      double r = (double)st * 0x1p-48;
+      // not marked by a walker before: k is still below it (the first draw's
+      // first walker has none before)
+      bool seek_r = i0 == 0 || kb < r;
+      t = t0;
+      for (int i = i0; i < i1; i++) {
+        if (i > i0) t = __builtin_amdgcn_fract(t) + sw[i];
+        int mk = 0;
+        if (seek_r && t >= r) {
+          mk = 1;
+          seek_r = false;
+        }
+        if (t >= 1.0) {
+          if (d < ndraw) {
+            r = rannyu(st);
+            seek_r = t - 1.0 < r;
+            if (!seek_r) mk++;
+          }
+          d++;
+        }
+        if (mk) sm[i] += mk;
+        if (d > ndraw) break;
+      }
+    }
+    if (tid == 0 && ndraw > 0) {
+      const long made = 1 + (units < ndraw - 1 ? (long)units : ndraw - 1);
+      rng2[0] = (int64_t)((lcg_pow((uint32_t)made) * st0) & ((1ULL << 48) - 1ULL));
+    }
   }
   __syncthreads();
   // The ranks left with no copy take the extra copies of the others: each
@@ -138,32 +264,19 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
   // none (reptation.f:2220-2258).  So receiver q (in walker order) takes
   // from the walker s whose extra copies, counted in walker order, cover q:
   // E(s) <= q < E(s+1), E the exclusive prefix sum of max(mult - 1, 0).
-  const int chunk = (nw + DMC_BRANCH_THREADS - 1) / DMC_BRANCH_THREADS;
-  const int i0 = min(nw, tid * chunk), i1 = min(nw, i0 + chunk);
-  int ne = 0, nr = 0;
+  int e = 0, q = 0, etot;
   for (int i = i0; i < i1; i++) {
-    ne += max(sm[i] - 1, 0);
-    nr += sm[i] == 0 ? 1 : 0;
+    e += max(sm[i] - 1, 0);
+    q += sm[i] == 0 ? 1 : 0;
   }
-  pe[tid] = ne;
-  pr[tid] = nr;
-  __syncthreads();
-  for (int o = 1; o < DMC_BRANCH_THREADS; o <<= 1) {
-    const int ae = tid >= o ? pe[tid - o] : 0, ar = tid >= o ? pr[tid - o] : 0;
-    __syncthreads();
-    pe[tid] += ae;
-    pr[tid] += ar;
-    __syncthreads();
-  }
+  dmc_scan(tid, sh.scan[0], sh.scan[1], e, q, etot);
   // exclusive prefix sums of the extras per walker, in the fractional parts'
   // place (no longer read); E(nw) is the total
   double* E = sw;
-  int e = pe[tid] - ne, q = pr[tid] - nr;
   for (int i = i0; i < i1; i++) {
     E[i] = (double)e;
     e += max(sm[i] - 1, 0);
   }
-  const int etot = pe[DMC_BRANCH_THREADS - 1];
   __syncthreads();
   for (int i = i0; i < i1; i++) {
     if (sm[i] >= 1) {

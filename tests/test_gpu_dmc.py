@@ -102,3 +102,32 @@ def test_sweep_step_equals_its_parts(oracle_mod):
     assert np.array_equal(a.age.cpu().numpy(), b.age.cpu().numpy())
     assert np.array_equal(a.rng.cpu().numpy(), b.rng.cpu().numpy())
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 17, 31, 33, 1025, 4096, 4097, 9000])
+@pytest.mark.parametrize("kind", ["spread", "equal", "halves", "rare", "negative"])
+def test_branch_sizes_match_oracle(oracle_mod, n, kind):
+    """Populations around the read-ahead chunks and the walkers per thread, with
+    weights whose fractional parts are spread, all zero, all halves, mostly
+    tiny, or below zero (the walk on one thread), against the oracle's walk in
+    rank order: the same origins, bounded weights and generator."""
+    import torch
+    hip, abi = pkg("hip"), pkg("abi")
+    r = np.random.default_rng(7 * n + len(kind))
+    w = {"spread": r.uniform(0.0, 3.0, n), "equal": np.ones(n), "halves": np.where(np.arange(n) % 2, 0.5, 1.5),
+         "rare": np.where(r.uniform(size=n) < 0.02, 12.0, 1e-3 * r.uniform(size=n)),
+         "negative": np.where(np.arange(n) % 7 == 3, -0.2, r.uniform(0.5, 1.5, n))}[kind]
+    limbs = [11, 22, 33, 2 * n + 1]
+    src, nmult, limbs2, _ = oracle_mod.branch2(w, limbs)
+    ctx = hip.Context(load_deck("n26g"), twist=(1, 1))
+    dev = torch.device("cuda:0")
+    wt = torch.tensor(w, dtype=torch.float64, device=dev)
+    rng2 = torch.tensor([abi.limbs_to_state(limbs)], dtype=torch.int64, device=dev)
+    got = torch.zeros(n, dtype=torch.int32, device=dev)
+    counts = torch.zeros(4, dtype=torch.int32, device=dev)
+    hip.dmc_branch(ctx, wt, rng2, got, counts)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), src)
+    assert int(counts[1].item()) == nmult
+    assert abi.state_to_limbs(int(rng2.item())) == limbs2
+    ctx.close()
