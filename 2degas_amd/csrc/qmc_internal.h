@@ -105,12 +105,10 @@ struct qmc_ctx {
 int launch_eval(qmc_ctx* c, int nw, const double* d_x, double* d_props, double* d_g, double* d_h,
                 double* d_g2, int32_t* d_status, hipStream_t st, double delta,
                 int precision = QMC_PREC_FP64, const int* nact = nullptr);
-// log|psi| alone of nw configurations (d_ltf[w] = ltf, d_status[w] bit 2 =
-// singular): the pair kernel's Jastrow pass and the determinant's pivots,
-// without F, the drift, the Laplacian or the potential.  d_props receives
-// nothing used; the matrix-core determinant path only.
-int launch_value(qmc_ctx* c, int nw, const double* d_x, double* d_ltf, int32_t* d_status, double* d_props,
-                 hipStream_t st, int precision);
+// log|det A| of both spins of nw walkers from the quasi-coordinates in the
+// workspace, by the determinants' pivots alone; the matrix-core determinant
+// path only.
+int launch_logdet(qmc_ctx* c, int nw, hipStream_t st);
 // The pair kernel (qmc_kernels.hip): its LDS for kc particles per phase chunk,
 // the doubles of its FP64 phase rows, and its launch.
 size_t pairs_lds(const DevSys& s, int kc, bool mix);

@@ -211,74 +211,259 @@ static int sem_check(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_state* d, i
 
 // With backflow every quasi-coordinate depends on every electron, so one
 // electron's move changes every column of both orbital matrices and no
-// low-rank update applies: each move evaluates the proposed configuration's
-// log|psi| (the pair kernel's Jastrow pass and quasi-coordinates, the
-// determinants' pivots: no F, drift, Laplacian or potential), accepted with
-// probability |psi'/psi|^2 = exp(-2 (ltf' - ltf)).  One wavefront per walker
-// copies the walker with electron j displaced (the same three draws per move
-// as the update path); after the evaluation one thread per walker takes the
-// decision and, when accepted, moves the electron and keeps the new ltf in
-// the walker's ltf slot.
-__global__ __launch_bounds__(256) void k_semf_propose(DevSys s, int nw, int j, double sigma,
-                                                      const double* __restrict__ x, double* __restrict__ xn,
-                                                      int64_t* __restrict__ rng, double* __restrict__ ua) {
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int w = blockIdx.x * 4 + wv;
-  if (w >= nw) return;
-  const int N = s.nptot;
-  const double* xw = x + (int64_t)w * 2 * N;
-  double* xo = xn + (int64_t)w * 2 * N;
-  for (int e = lane; e < 2 * N; e += 64)
-    if (e != 2 * j && e != 2 * j + 1) xo[e] = xw[e];
-  if (lane == 0) {
-    uint64_t st = (uint64_t)rng[w];
-    const double u1 = rannyu(st), u2 = rannyu(st), a = rannyu(st);
-    double sv, cv;
-    qsincos(6.283185307179586 * u2, &sv, &cv);
-    const double rad = sigma * sqrt(-2.0 * log(u1));
-    xo[2 * j] = xw[2 * j] + rad * cv;
-    xo[2 * j + 1] = xw[2 * j + 1] + rad * sv;
-    rng[w] = (int64_t)st;
-    ua[w] = a;
+// low-rank update applies: each move takes the determinants of the proposed
+// configuration anew (the pivots: no F, drift, Laplacian or potential) and is
+// accepted with probability |psi'/psi|^2 = exp(-2 (ltf' - ltf)).  What is a
+// sum over pairs changes by the pairs of the moved electron alone: the
+// quasi-coordinates q_p = x_p + sum_b eta(r_pb) (x_p - x_b), the three-body
+// vectors G_p and the Jastrow factor are formed at the start of a call
+// (k_semf_init) and then follow the moves.  The pair terms are those of the
+// evaluation in the call's precision (FP32 u2 and u3 tables in mixed
+// precision); their sums are FP64.
+//
+// So a move is two launches: k_semf_step takes the decision on the move before
+// and proposes the next, one block per walker with thread p taking partner p,
+// and the determinant kernel follows.  All pairs evaluated for each proposal,
+// with a copy of the walker, the evaluation's sum and the decision in kernels
+// of their own, made 41 us per move for 512 walkers of N = 58 (now 24).
+//
+// Per walker: the current q in qc, G in gc; the proposal's in the evaluation's
+// workspace, q where the determinants read it, G in the drift's place, and in
+// the scalars' place:
+enum { SF_U = 0, SF_UNEW = 1, SF_X = 2, SF_Y = 3, SF_UA = 4 };
+
+template <bool MIX>
+__device__ __forceinline__ double semf_spline(const DevSys& s, TabRef t, const PairGeo& p) {
+  if (MIX) {
+    const float4 c = tab_row(s.tab32, t, p.ind);
+    const float rm = (float)(p.rem * s.drti);
+    return (double)fmaf(rm, fmaf(rm, fmaf(rm, c.w, c.z), c.y), c.x);
+  }
+  const double4 c = tab_row(s.tab, t, p.ind);
+  const double rm = p.rem * s.drti;
+  return fma(rm, fma(rm, fma(rm, c.w, c.z), c.y), c.x);
+}
+
+// The terms of the pair (a, b) at separation p (u = x_a - x_b): u2 + (xi r)^2,
+// xi u and eta u.
+struct SemfPair {
+  double u, gx, gy, qx, qy;
+};
+template <bool MIX>
+__device__ __forceinline__ SemfPair semf_pair(const DevSys& s, TabRef t2, TabRef t3, TabRef tb, const PairGeo& p) {
+  SemfPair o{0.0, 0.0, 0.0, 0.0, 0.0};
+  if (t2.row0 >= 0) o.u = semf_spline<MIX>(s, t2, p);
+  if (t3.row0 >= 0) {
+    const double f = semf_spline<MIX>(s, t3, p), fr = f * p.r;
+    o.u += fr * fr;
+    o.gx = f * p.ux;
+    o.gy = f * p.uy;
+  }
+  if (tb.row0 >= 0) {
+    const double f = semf_spline<false>(s, tb, p);
+    o.qx = f * p.ux;
+    o.qy = f * p.uy;
+  }
+  return o;
+}
+
+// Sums over a block of up to two wavefronts of five values, on every thread.
+__device__ __forceinline__ void semf_sum(double (&v)[5], double (*red)[5], int tid) {
+#pragma unroll
+  for (int q = 0; q < 5; q++) v[q] = wave_sum(v[q]);
+  if ((tid & 63) == 0) {
+#pragma unroll
+    for (int q = 0; q < 5; q++) red[tid >> 6][q] = v[q];
+  }
+  __syncthreads();
+  if (blockDim.x > 64) {
+#pragma unroll
+    for (int q = 0; q < 5; q++) v[q] = red[0][q] + red[1][q];
   }
 }
 
-__global__ __launch_bounds__(256) void k_semf_accept(DevSys s, int nw, int j, int jltf, const double* __restrict__ xn,
-                                                     const double* __restrict__ ltfn, const int32_t* __restrict__ stn,
-                                                     const double* __restrict__ ua, double* __restrict__ x,
-                                                     double* __restrict__ props, double* __restrict__ dlogpsi,
-                                                     double* __restrict__ nacc) {
-  const int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= nw) return;
-  const int N = s.nptot, NP = s.n_props;
-  const double lo = props[(int64_t)w * NP + jltf], ln = ltfn[w];
-  // a singular proposal (status bit 2) has psi' = 0
-  if ((stn[w] & 2) != 0 || !(ua[w] < exp(-2.0 * (ln - lo)))) return;
-  x[(int64_t)w * 2 * N + 2 * j] = xn[(int64_t)w * 2 * N + 2 * j];
-  x[(int64_t)w * 2 * N + 2 * j + 1] = xn[(int64_t)w * 2 * N + 2 * j + 1];
-  props[(int64_t)w * NP + jltf] = ln;
-  dlogpsi[w] += lo - ln;
-  nacc[w] += 1.0;
+// q, G and U of the walker's configuration.  One block per walker, eight lanes
+// per particle, each summing over every eighth partner.
+template <bool MIX>
+__global__ __launch_bounds__(8 * QMC_MAX_PARTICLES) void k_semf_init(DevSys s, WsLayout L, double* __restrict__ ws,
+                                                                     const double* __restrict__ x,
+                                                                     double* __restrict__ qc,
+                                                                     double* __restrict__ gc) {
+  __shared__ __attribute__((aligned(16))) double xs[2 * QMC_MAX_PARTICLES];
+  __shared__ double red[8 * QMC_MAX_PARTICLES / 64];
+  const int w = blockIdx.x, tid = threadIdx.x, N = s.nptot;
+  const int64_t at = (int64_t)w * 2 * N;
+  for (int k = tid; k < 2 * N; k += blockDim.x) xs[k] = x[at + k];
+  __syncthreads();
+  const int a = tid >> 3;
+  const bool li = a < N;
+  double2 xp = make_double2(0.0, 0.0);
+  double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // U, G, q
+  if (li) {
+    const int ti = ptype(s, a);
+    xp = ld2(xs, a);
+    for (int b = tid & 7; b < N; b += 8) {
+      if (b == a) continue;
+      const int tp = tpair(ti, ptype(s, b));
+      const double2 xb = ld2(xs, b);
+      const SemfPair t = semf_pair<MIX>(s, tabref<TK_U2>(s, tp), tabref<TK_U3>(s, tp), tabref<TK_B>(s, tp),
+                                        pair_geo(s, xp.x, xp.y, xb.x, xb.y));
+      v[0] += t.u;
+      v[1] -= t.gx;
+      v[2] -= t.gy;
+      v[3] += t.qx;
+      v[4] += t.qy;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 5; q++) {
+    v[q] += dpp_f64<0xB1>(v[q]);
+    v[q] += dpp_f64<0x4E>(v[q]);
+    v[q] += dpp_f64<0x141>(v[q]);  // the quads of a group of eight, mirrored
+  }
+  double u = 0.0;
+  if (li && (tid & 7) == 0) {
+    *reinterpret_cast<double2*>(qc + at + 2 * a) = make_double2(xp.x + v[3], xp.y + v[4]);
+    *reinterpret_cast<double2*>(gc + at + 2 * a) = make_double2(v[1], v[2]);
+    u = 0.5 * (v[0] - (v[1] * v[1] + v[2] * v[2]));
+  }
+  u = wave_sum(u);
+  if ((tid & 63) == 0) red[tid >> 6] = u;
+  __syncthreads();
+  if (tid == 0) {
+    double t = 0.0;
+    for (int k = 0; k < (int)blockDim.x / 64; k++) t += red[k];
+    ws[(int64_t)w * L.per_walker + L.off_sc + SF_U] = t;
+  }
+}
+
+// Decision on the move of electron j - 1 (unless j is the call's first), then
+// the proposal of electron j's (unless j is the end): the same three draws per
+// move as the update path.
+template <bool MIX>
+__global__ __launch_bounds__(QMC_MAX_PARTICLES) void k_semf_step(
+    DevSys s, WsLayout L, double* __restrict__ ws, int j, int j0, int j1, double sigma, int jltf,
+    double* __restrict__ x, double* __restrict__ qc, double* __restrict__ gc, int64_t* __restrict__ rng,
+    double* __restrict__ props, double* __restrict__ dlogpsi, double* __restrict__ nacc) {
+  __shared__ double red[2][5];
+  const int w = blockIdx.x, tid = threadIdx.x, N = s.nptot;
+  const int64_t at = (int64_t)w * 2 * N;
+  double* wsw = ws + (int64_t)w * L.per_walker;
+  double* sc = wsw + L.off_sc;
+  const bool li = tid < N;
+  const int jp = j < j1 ? j : j - 1;  // the electron proposed (the last block only decides)
+  uint64_t st = (uint64_t)rng[w];
+  double2 xp = make_double2(0.0, 0.0), q = xp, g = xp, qn = xp, gn = xp;
+  if (li) {
+    xp = make_double2(x[at + 2 * tid], x[at + 2 * tid + 1]);
+    q = *reinterpret_cast<const double2*>(qc + at + 2 * tid);
+    g = *reinterpret_cast<const double2*>(gc + at + 2 * tid);
+    qn = make_double2(wsw[L.off_q + 2 * tid], wsw[L.off_q + 2 * tid + 1]);
+    gn = make_double2(wsw[L.off_gj + 2 * tid], wsw[L.off_gj + 2 * tid + 1]);
+  }
+  const double2 xj = make_double2(x[at + 2 * jp], x[at + 2 * jp + 1]);
+  double U = sc[SF_U];
+  if (j > j0) {
+    const double Un = sc[SF_UNEW], ua = sc[SF_UA], xn = sc[SF_X], yn = sc[SF_Y];
+    double* pl = props + (int64_t)w * s.n_props + jltf;
+    const double lo = *pl, dl = dlogpsi[w], na = nacc[w];
+    double ln = Un;
+    bool sing = false;  // a singular proposal has psi' = 0
+#pragma unroll
+    for (int sp = 0; sp < 2; sp++) {
+      if (sp >= s.ntypes || s.np[sp] == 0) continue;
+      const double* dsc = wsw + L.off_det[sp];
+      ln -= dsc[DS_LOGDET];
+      sing = sing || dsc[DS_SING] != 0.0;
+    }
+    const bool acc = !sing && ua < exp(-2.0 * (ln - lo));
+    __syncthreads();  // both wavefronts have read what is written below
+    if (acc) {
+      U = Un;
+      q = qn;
+      g = gn;
+      if (tid == j - 1) {
+        xp = make_double2(xn, yn);
+        x[at + 2 * tid] = xn;
+        x[at + 2 * tid + 1] = yn;
+      }
+      if (li) {
+        *reinterpret_cast<double2*>(qc + at + 2 * tid) = q;
+        *reinterpret_cast<double2*>(gc + at + 2 * tid) = g;
+      }
+      if (tid == 0) {
+        sc[SF_U] = U;
+        *pl = ln;
+        dlogpsi[w] = dl + (lo - ln);
+        nacc[w] = na + 1.0;
+      }
+    }
+  }
+  if (j >= j1) return;
+  const double u1 = rannyu(st), u2 = rannyu(st), ua = rannyu(st);
+  double sv, cv;
+  qsincos(6.283185307179586 * u2, &sv, &cv);
+  const double rad = sigma * sqrt(-2.0 * log(u1));
+  const double xn = xj.x + rad * cv, yn = xj.y + rad * sv;
+  // partner tid's terms at the new and the old position of j
+  double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // dU, then G and q of j at its new position
+  double2 dg = make_double2(0.0, 0.0), dq = dg;
+  if (li && tid != j) {
+    const int tp = tpair(ptype(s, j), ptype(s, tid));
+    const TabRef t2 = tabref<TK_U2>(s, tp), t3 = tabref<TK_U3>(s, tp), tb = tabref<TK_B>(s, tp);
+    const SemfPair a = semf_pair<MIX>(s, t2, t3, tb, pair_geo(s, xn, yn, xp.x, xp.y));
+    const SemfPair o = semf_pair<MIX>(s, t2, t3, tb, pair_geo(s, xj.x, xj.y, xp.x, xp.y));
+    dg = make_double2(a.gx - o.gx, a.gy - o.gy);
+    dq = make_double2(o.qx - a.qx, o.qy - a.qy);
+    // -1/2 (|G + dG|^2 - |G|^2) = -dG.G - 1/2 |dG|^2
+    v[0] = (a.u - o.u) - (g.x * dg.x + g.y * dg.y) - 0.5 * (dg.x * dg.x + dg.y * dg.y);
+    v[1] = -a.gx;
+    v[2] = -a.gy;
+    v[3] = a.qx;
+    v[4] = a.qy;
+  } else if (tid == j) {
+    v[0] = 0.5 * (g.x * g.x + g.y * g.y);
+  }
+  semf_sum(v, red, tid);
+  if (li) {
+    const bool me = tid == j;
+    wsw[L.off_q + 2 * tid] = me ? xn + v[3] : q.x + dq.x;
+    wsw[L.off_q + 2 * tid + 1] = me ? yn + v[4] : q.y + dq.y;
+    wsw[L.off_gj + 2 * tid] = me ? v[1] : g.x + dg.x;
+    wsw[L.off_gj + 2 * tid + 1] = me ? v[2] : g.y + dg.y;
+  }
+  if (tid == 0) {
+    sc[SF_UNEW] = U + v[0] - 0.5 * (v[1] * v[1] + v[2] * v[2]);
+    sc[SF_X] = xn;
+    sc[SF_Y] = yn;
+    sc[SF_UA] = ua;
+    rng[w] = (int64_t)st;
+  }
 }
 
 static int sem_moves_full(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_state* d, int j0, int j1, double sigma,
                           int precision, hipStream_t st) {
+  if (j0 >= j1) return QMC_OK;
   const int nw = w->nw;
+  const bool mix = precision == QMC_PREC_MIXED;
   int rc = ensure_vmc_scratch(c, nw);
   if (rc) return rc;
-  for (int j = j0; j < j1; j++) {
-    hipLaunchKernelGGL(k_semf_propose, dim3((nw + 3) / 4), dim3(256), 0, st, c->s, nw, j, sigma, w->x, c->d_xn,
-                       w->rng, c->d_wold);
-    // the proposal's ltf in d_hn (nw doubles of the proposal buffers)
-    rc = launch_value(c, nw, c->d_xn, c->d_hn, c->d_stn, c->d_pn, st, precision);
+  rc = ensure_ws(c, nw);
+  if (rc) return rc;
+  const dim3 block(c->s.nptot <= 64 ? 64 : QMC_MAX_PARTICLES);
+  hipLaunchKernelGGL(mix ? k_semf_init<true> : k_semf_init<false>, dim3(nw),
+                     dim3((8 * c->s.nptot + 63) / 64 * 64), 0, st, c->s, c->L, c->d_ws, w->x, c->d_gn, c->d_xn);
+  for (int j = j0; j <= j1; j++) {
+    hipLaunchKernelGGL(mix ? k_semf_step<true> : k_semf_step<false>, dim3(nw), block, 0, st, c->s, c->L, c->d_ws, j,
+                       j0, j1, sigma, c->info.jltf - 1, w->x, c->d_gn, c->d_xn, w->rng, w->props, d->dlogpsi,
+                       d->nacc);
+    if (j == j1) break;
+    rc = launch_logdet(c, nw, st);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_semf_accept, dim3((nw + 255) / 256), dim3(256), 0, st, c->s, nw, j, c->info.jltf - 1,
-                       c->d_xn, c->d_hn, c->d_stn, c->d_wold, w->x, w->props, d->dlogpsi, d->nacc);
   }
   HIPCHK(hipGetLastError());
   return QMC_OK;
 }
-
 
 // Kind of row and wavefronts per walker of a job's moves: real rows in FP64
 // where the orbitals are real (one wavefront up to 32 rows per spin, two above),

@@ -381,6 +381,52 @@ def test_backflow_moves_track_the_full_evaluation(name):
     assert lerr < 1e-9
 
 
+@pytest.mark.parametrize("nup,ndown,u3,twist,precision", [
+    (1, 1, True, (1, 1), 0), (5, 3, False, (2, 3), 0), (13, 13, True, (2, 3), 1), (33, 1, True, (1, 1), 0),
+    (32, 32, False, (1, 1), 1), (64, 0, True, (2, 3), 0), (61, 61, True, (1, 1), 0), (61, 61, True, (1, 1), 1)])
+def test_backflow_moves_over_sizes(tmp_path, nup, ndown, u3, twist, precision):
+    """Moves with backflow at the edges of the pair step's blocks (N up to and
+    above 64, one spin, one particle), real and twisted orbitals, with and
+    without u3, in both precisions: after two sweeps in uneven ranges the ltf
+    kept in the properties is that of a fresh evaluation of the positions in
+    the same precision, and a sweep in one range from the same start takes the
+    same decisions.  The kept sums follow up to 244 moves: some 1e3 additions
+    of rounding 1e-16 of values up to 1e3, amplified at most by the orbital
+    matrices' condition (1e4) in log|det|: 1e-9."""
+    import torch
+    hip, abi, dg, deck = pkg("hip"), pkg("abi"), pkg("deckgen"), pkg("deck")
+    dg.make_deck(str(tmp_path), "bf", nup, ndown, 5.0, 5, nshell_k=12, u3=u3, backflow="yk", jastrow="pade")
+    d = deck.read_deck(str(tmp_path))
+    N, nw = d.nptot, 6
+
+    def run(cuts):
+        ctx = hip.Context(d, twist=twist)
+        x = dg.lattice_configs(nw, N, d.el[0], 17)
+        wk = hip.Walkers(ctx, x, _states(nw, 900))
+        wk.start()
+        sm = hip.SingleMoves(wk, precision=precision)
+        sm.refresh()
+        for _ in range(2):
+            for a, b in zip(cuts[:-1], cuts[1:]):
+                sm.moves(a, b, 0.4)
+        torch.cuda.synchronize()
+        return ctx, wk, sm
+
+    ctx, wk, sm = run([0, 1, N // 3 + 1, N])
+    _, wk2, sm2 = run([0, N])
+    assert torch.equal(sm.nacc, sm2.nacc)
+    assert torch.equal(wk.rng, wk2.rng)
+    assert float((wk.x - wk2.x).abs().max()) == 0.0
+    props, g = torch.zeros_like(wk.props), torch.zeros_like(wk.x)
+    h = torch.zeros(nw, 2, dtype=torch.float64, device="cuda")
+    g2 = torch.zeros(nw, dtype=torch.float64, device="cuda")
+    ctx.eval_device(wk.x, props, g, h, g2, precision=precision)
+    torch.cuda.synchronize()
+    jltf = ctx.info["jltf"] - 1
+    assert 0 < float(sm.nacc.sum()) < 2 * N * nw
+    assert float((wk.props[:, jltf] - props[:, jltf]).abs().max()) < 1e-9
+
+
 def test_energy_with_backflow_agrees_with_all_electron_walk():
     """Statistical agreement on a backflow deck (n26g: u2 + u3 + the n26
     backflow, Gamma point, rs=1): the single-electron walk, every move
