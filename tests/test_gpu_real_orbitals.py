@@ -82,9 +82,12 @@ def test_list_forms_match_general_path(form, m, tmp_path, monkeypatch):
 
 
 def test_value_alone_equals_the_full_evaluation(tmp_path):
-    """log|psi| carried by moves with backflow (the value-only kernels) is the
-    full evaluation's, bit for bit, with real orbitals and tiles that differ
-    between the spins."""
+    """log|psi| carried by moves with backflow (the value-only determinants) is
+    the full evaluation's, with real orbitals and tiles that differ between the
+    spins.  The moves' quasi-coordinates and Jastrow sums follow the moved
+    electron's pairs, so the two agree to the rounding of some 1e3 additions of
+    1e-16 of values up to 1e3, times the orbital matrices' condition (1e4) in
+    log|det|: 1e-9."""
     print("\n[gpu] real orbitals, value-only moves 17+31", flush=True)
     import torch
     hip = pkg("hip")
@@ -99,7 +102,7 @@ def test_value_alone_equals_the_full_evaluation(tmp_path):
     kept = wk.props[:, ctx.info["jltf"] - 1].clone()
     wk.start()
     torch.cuda.synchronize()
-    assert torch.equal(kept, wk.props[:, ctx.info["jltf"] - 1])
+    assert float((kept - wk.props[:, ctx.info["jltf"] - 1]).abs().max()) < 1e-9
     assert sm.nacc.sum().item() > 0
     wk = sm = None
     ctx.close()
