@@ -24,6 +24,14 @@
 // double buffered.  Column tiles of R whose columns are all eliminated are
 // left out.
 //
+// The chain from block to block bounds the kernel (panel, pivot search, posted
+// rows, update), so U must not lengthen it: rows are taken from the registers
+// in index mode or, where the LDS allows, from a copy of the tiles stored while
+// the pivot steps run, which then also is the panel.  By a switch over the
+// registers, a dozen branches per row: N=122, 4096 walkers 471 us (now 440);
+// log|det| alone, N=58, 512 walkers 17.7 us (now 13.5); N=26, 256 walkers 9.9 us
+// (now 7.9), but 4096 walkers of N=26 33 us (now 34: the copy's LDS).
+//
 // Rows: the two rows of plane-wave pair n sit in one lane of a tile (rows
 // r and r + 4), so that one sin/cos gives R and both derivatives of both
 // rows.  A zero plane wave is the cos row of a pair of its own, whose sin row
@@ -34,12 +42,24 @@
 
 typedef double gr_d4 __attribute__((ext_vector_type(4)));
 
-template <int NT>
+// Whether a wavefront keeps a copy of its column tiles in LDS for the pivot
+// rows to be read from (as many stores as picking the four rows out of the
+// registers for one row tile, and none of them between a block's barrier and its
+// update); beyond, the LDS would bound the walkers per CU.
+template <int NT, int NP>
+constexpr bool gr_copies = NT == 1 || (NT == 2 && NP == 1);
+
+template <int NT, int NP>
 struct GrShared {
-  double q[2 * 64], g[2 * 32];
-  double panel[16 * NT * 4];      // the block's columns, row r at 4 r
+  static constexpr bool COPY = gr_copies<NT, NP>;
+  // a copied row's stride: rows 16 lanes read together fall on different banks
+  static constexpr int LDC = 18, PART = COPY ? 16 * NT * LDC : 8 * 16;
+  double q[2 * 16 * NT], g[2 * 8 * NT];
+  double panel[COPY ? 1 : 16 * NT * 4];  // the block's columns, row r at 4 r (else read from the copy)
   double Fl[2][16 * NT * 4];      // F' of the block, row r at 4 r
-  double u[NT][3][4 * 16];        // per wavefront: the block's pivot rows in its column tiles
+  // per wavefront: its column tiles, or the block's pivot rows in them and spare
+  // places
+  __attribute__((aligned(16))) double u[NT][NP * PART];
   double pinv[16 * NT], pabs[16 * NT];  // by pivot row
   int prow[2][4];
   int rank[16 * NT];              // step of pivot row r, -1: none
@@ -67,19 +87,27 @@ __device__ __forceinline__ void gr_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// f(integral_constant<i>) for the uniform run-time i in [0, 4 NT): a jump,
-// since registers cannot be indexed by a run-time value.
-template <int NT, class F>
-__device__ __forceinline__ void gr_switch(int i, F&& f) {
-#define GR_CASE(k)                                                     \
-  case k:                                                              \
-    if constexpr (k < 4 * NT) f(std::integral_constant<int, k>{});     \
-    break;
-  switch (i) {
-    GR_CASE(0) GR_CASE(1) GR_CASE(2) GR_CASE(3) GR_CASE(4) GR_CASE(5) GR_CASE(6) GR_CASE(7)
-    GR_CASE(8) GR_CASE(9) GR_CASE(10) GR_CASE(11) GR_CASE(12) GR_CASE(13) GR_CASE(14) GR_CASE(15)
+// Element i (uniform, run time) of a lane's 4 NT values of a part: register
+// index mode on a tuple of 8 or 16 values, where a switch is a dozen branches.
+typedef double gr_d8 __attribute__((ext_vector_type(8)));
+typedef double gr_d16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ double gr_pick4(const gr_d4& a, int i) {
+  const double x = i & 1 ? a[1] : a[0], y = i & 1 ? a[3] : a[2];
+  return i & 2 ? y : x;
+}
+template <int NT>
+__device__ __forceinline__ double gr_pick(const gr_d4 (&a)[NT], int i) {
+  if constexpr (NT == 1) {
+    return gr_pick4(a[0], i);
+  } else if constexpr (NT == 2) {
+    const gr_d8 v = __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    return v[i];
+  } else {
+    const gr_d8 v = __builtin_shufflevector(a[0], a[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    const gr_d8 w = __builtin_shufflevector(a[2], a[NT == 3 ? 2 : 3], 0, 1, 2, 3, 4, 5, 6, 7);
+    const gr_d16 x = __builtin_shufflevector(v, w, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+    return x[i];
   }
-#undef GR_CASE
 }
 
 // The pivot steps of columns k0..k0+nb-1 (panel in LDS) by one wavefront,
@@ -87,14 +115,15 @@ __device__ __forceinline__ void gr_switch(int i, F&& f) {
 // top 14 bits agree in the order of their index.  Every lane forms the
 // reciprocal of its own entry while the maximum is searched, so that the
 // chain waits for the longer of the two only.
-template <int NT>
-__device__ __forceinline__ void gr_pivots(GrShared<NT>& sh, int buf, int k0, int nb, int lane) {
+template <int NT, int NP>
+__device__ __forceinline__ void gr_pivots(GrShared<NT, NP>& sh, const double* panel, int buf, int k0, int nb,
+                                          int lane) {
   const bool in = NT == 4 || lane < 16 * NT;
   double P[4] = {0, 0, 0, 0}, Fp[4] = {0, 0, 0, 0};
   bool used = true;
   if (in) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) P[j] = sh.panel[4 * lane + j];
+    for (int j = 0; j < 4; j++) P[j] = panel[j];
     used = sh.used[lane] != 0;
   }
 #pragma unroll
@@ -122,6 +151,8 @@ __device__ __forceinline__ void gr_pivots(GrShared<NT>& sh, int buf, int k0, int
         sh.used[p] = 1;
         if (!(a > 0.0)) sh.sing = 1;
       }
+    } else if (lane == 0) {
+      sh.prow[buf][j] = 0;
     }
   }
   if (in) {
@@ -132,8 +163,8 @@ __device__ __forceinline__ void gr_pivots(GrShared<NT>& sh, int buf, int k0, int
 
 // Tables of the spin into LDS: quasi-coordinates (or positions) and pairs;
 // rows without an orbital are marked used.
-template <int NT>
-__device__ __forceinline__ void gr_setup(GrShared<NT>& sh, const double* __restrict__ q, const double* __restrict__ gp,
+template <int NT, int NP>
+__device__ __forceinline__ void gr_setup(GrShared<NT, NP>& sh, const double* __restrict__ q, const double* __restrict__ gp,
                                          int m, int nslot, int zero, int tid) {
   for (int e = tid; e < 2 * m; e += 64 * NT) sh.q[e] = q[e];
   for (int e = tid; e < 2 * nslot; e += 64 * NT) sh.g[e] = gp[e];
@@ -149,7 +180,7 @@ __device__ __forceinline__ void gr_setup(GrShared<NT>& sh, const double* __restr
 
 // The wavefront's column tile of R and, with NP = 3, of its two derivatives.
 template <int NT, int NP>
-__device__ __forceinline__ void gr_build(const GrShared<NT>& sh, gr_d4 (&acc)[NP][NT], int m, int nslot, int col,
+__device__ __forceinline__ void gr_build(const GrShared<NT, NP>& sh, gr_d4 (&acc)[NP][NT], int m, int nslot, int col,
                                          int lr) {
   const bool jn = col < m;
   const double qx = jn ? sh.q[2 * col] : 0.0, qy = jn ? sh.q[2 * col + 1] : 0.0;
@@ -181,52 +212,83 @@ __device__ __forceinline__ void gr_build(const GrShared<NT>& sh, gr_d4 (&acc)[NP
 // S R having row p_k equal to piv_k e_k; else R's eliminated column tiles are
 // left out.  Ends with a barrier.
 template <int NT, int NP, bool INPLACE>
-__device__ __forceinline__ void gr_eliminate(GrShared<NT>& sh, gr_d4 (&acc)[NP][NT], int m, int wave, int lane) {
+__device__ __forceinline__ void gr_eliminate(GrShared<NT, NP>& sh, gr_d4 (&acc)[NP][NT], int m, int wave, int lane) {
   // MFMA lane roles: accumulator rows lr + 4v, column lc; operand k index lr
   const int lr = lane >> 4, lc = lane & 15, ct = wave;
   // the block's columns from the accumulators of the wavefront that holds
   // them to LDS, and its pivot steps
-  auto panel = [&](int k0, int buf) {
-    const int j = lc - (k0 & 15);
-    if (j >= 0 && j < 4) {
+  double* ub = sh.u[wave];
+  constexpr bool COPY = GrShared<NT, NP>::COPY;
+  constexpr int LDC = GrShared<NT, NP>::LDC, PART = GrShared<NT, NP>::PART;
+  // the wavefront's tiles of parts t0..t1-1 to its copy
+  auto copy = [&](auto t0, auto t1) {
+#pragma unroll
+    for (int t = decltype(t0)::value; t < decltype(t1)::value; t++)
 #pragma unroll
       for (int T = 0; T < NT; T++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) sh.panel[4 * (16 * T + lr + 4 * v) + j] = acc[0][T][v];
+        for (int v = 0; v < 4; v++) ub[t * PART + (16 * T + lr + 4 * v) * LDC + lc] = acc[t][T][v];
+  };
+  typedef std::integral_constant<int, 0> C0;
+  typedef std::integral_constant<int, 1> C1;
+  typedef std::integral_constant<int, NP> CN;
+  auto panel = [&](int k0, int buf) {
+    const double* src;
+    if constexpr (COPY) {
+      copy(C0{}, C1{});
+      src = ub + lane * LDC + (k0 & 15);
+    } else {
+      const int j = lc - (k0 & 15);
+      if (j >= 0 && j < 4) {
+#pragma unroll
+        for (int T = 0; T < NT; T++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) sh.panel[4 * (16 * T + lr + 4 * v) + j] = acc[0][T][v];
+      }
+      src = sh.panel + 4 * lane;
     }
     gr_wave_sync();
     // every other wavefront waits for these steps: they issue first
     __builtin_amdgcn_s_setprio(1);
-    gr_pivots<NT>(sh, buf, k0, min(4, m - k0), lane);
+    gr_pivots(sh, src, buf, k0, min(4, m - k0), lane);
     __builtin_amdgcn_s_setprio(0);
+    if constexpr (COPY) copy(C1{}, CN{});
   };
   if (ct == 0) panel(0, 0);
+  else if constexpr (COPY) copy(C0{}, CN{});
   for (int k0 = 0; k0 < m; k0 += 4) {
     const int buf = (k0 >> 2) & 1, nb = min(4, m - k0);
     __syncthreads();
     const bool left = INPLACE || (k0 >> 4) <= ct;  // R's columns here are not all eliminated
-    double* ub = &sh.u[wave][0][0];
-    int pb[4] = {-1, -1, -1, -1};
+    int pb[4];
+    double uo[NP], fo[NT];
+    if constexpr (COPY) {
+      const int p = sh.prow[buf][lr];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      if (k < nb) {
-        const int p = pb[k] = __builtin_amdgcn_readfirstlane(sh.prow[buf][k]);
-        const bool me = lr == (p & 3);
-        gr_switch<NT>(p >> 2, [&](auto ic) {
-          constexpr int I = decltype(ic)::value;
-          if (me) {
-#pragma unroll
-            for (int t = 0; t < NP; t++) ub[t * 64 + k * 16 + lc] = acc[t][I >> 2][I & 3];
-          }
-        });
+      for (int t = 0; t < NP; t++) {
+        const double v = ub[t * PART + p * LDC + lc];
+        uo[t] = lr < nb ? v : 0.0;
       }
     }
-    gr_wave_sync();
-    double fo[NT], uo[NP];
+    if constexpr (!COPY || INPLACE) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) pb[k] = __builtin_amdgcn_readfirstlane(sh.prow[buf][k]);
+    }
+    if constexpr (!COPY) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        // the lanes that hold row p; the others' values go to their own places
+        // behind the block's rows
+        double* to = ub + (lr == (pb[k] & 3) ? k * 16 : (4 + lr) * 16) + lc;
+#pragma unroll
+        for (int t = 0; t < NP; t++) to[t * PART] = gr_pick<NT>(acc[t], pb[k] >> 2);
+      }
+      gr_wave_sync();
+#pragma unroll
+      for (int t = 0; t < NP; t++) uo[t] = lr < nb ? ub[t * PART + lane] : 0.0;
+    }
 #pragma unroll
     for (int T = 0; T < NT; T++) fo[T] = sh.Fl[buf][4 * (16 * T + lc) + lr];
-#pragma unroll
-    for (int t = 0; t < NP; t++) uo[t] = lr < nb ? ub[t * 64 + lane] : 0.0;
     if constexpr (INPLACE) {
       const int jj = lc - (k0 & 15);
       if ((k0 >> 4) == ct && jj >= 0 && jj < nb) {
@@ -246,7 +308,10 @@ __device__ __forceinline__ void gr_eliminate(GrShared<NT>& sh, gr_d4 (&acc)[NP][
     for (int t = 1; t < NP; t++)
 #pragma unroll
       for (int T = 0; T < NT; T++) acc[t][T] = gr_mfma(fo[T], uo[t], acc[t][T]);
-    if (k0 + 4 < m && ((k0 + 4) >> 4) == ct) panel(k0 + 4, buf ^ 1);
+    if (k0 + 4 < m) {
+      if (((k0 + 4) >> 4) == ct) panel(k0 + 4, buf ^ 1);
+      else if constexpr (COPY) copy(C0{}, CN{});
+    }
   }
   __syncthreads();
 }
@@ -255,7 +320,7 @@ template <int NT, bool VAL>
 __global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLayout L, double* __restrict__ ws,
                                                                   double* __restrict__ Fbuf, int sp0) {
   constexpr int NP = VAL ? 1 : 3;  // parts of the augmented matrix
-  __shared__ __attribute__((aligned(16))) GrShared<NT> sh;
+  __shared__ __attribute__((aligned(16))) GrShared<NT, NP> sh;
   const int w = blockIdx.x, sp = sp0 + blockIdx.y;
   if (s.nact && w >= *s.nact) return;
   const int m = pick2(s.np, sp);
@@ -316,7 +381,7 @@ __global__ __launch_bounds__(64 * NT, NT == 4 ? 3 : 4) void k_gjr(DevSys s, WsLa
 template <int NT>
 struct GrInverse {
   static constexpr int LD = 16 * NT + 1;
-  GrShared<NT> sh;
+  GrShared<NT, 1> sh;
   double X[16 * NT * LD];  // X(k, r) at k LD + r
   int pcol[16 * NT];       // pivot row of column c
 };
@@ -326,7 +391,7 @@ __global__ __launch_bounds__(64 * NT, 4) void k_gjr_inverse(DevSys s, int sp0, c
                                                             double2* __restrict__ ainv, int mm) {
   extern __shared__ __attribute__((aligned(16))) unsigned char gi_lds[];
   GrInverse<NT>& gi = *reinterpret_cast<GrInverse<NT>*>(gi_lds);
-  GrShared<NT>& sh = gi.sh;
+  GrShared<NT, 1>& sh = gi.sh;
   const int w = blockIdx.x, sp = sp0 + blockIdx.y;
   const int m = pick2(s.np, sp);
   if (m == 0) return;

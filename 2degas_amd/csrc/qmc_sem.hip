@@ -225,7 +225,7 @@ static int sem_check(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_state* d, i
 // and proposes the next, one block per walker with thread p taking partner p,
 // and the determinant kernel follows.  All pairs evaluated for each proposal,
 // with a copy of the walker, the evaluation's sum and the decision in kernels
-// of their own, made 41 us per move for 512 walkers of N = 58 (now 24).
+// of their own, made 41 us per move for 512 walkers of N = 58 (now 20).
 //
 // Per walker: the current q in qc, G in gc; the proposal's in the evaluation's
 // workspace, q where the determinants read it, G in the drift's place, and in
