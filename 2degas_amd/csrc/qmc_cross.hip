@@ -10,32 +10,80 @@
 // qa being the backflow Jacobian: 1 + Q_j on the particle's own block and
 // -(eta delta + eta' r u u) for a pair (reptation.f:10023-10058).
 //
-// One workgroup of 8 wavefronts per (walker, spin).  S_t is a 128 x 128
-// SYRK built from 16 x 16 tiles with v_mfma_f64_16x16x4f64: the 36 tiles of
-// the upper triangle go 9 to each pair of wavefronts, block rows g and 7-g
-// (8-g and g+1 tiles), split 5 + 4 between the pair.  V_t is staged in LDS 16
-// particles (32 columns) at a time, column-major so each MFMA operand is one
-// 8-byte LDS read per lane.  M is formed from F (L2) tile by tile when S_t is
+// One workgroup per (walker, spin).  S_t is a SYRK built from 16 x 16 tiles
+// with v_mfma_f64_16x16x4f64, the tiles of the upper triangle shared between the
+// wavefronts (XcShape).  V_t is staged in LDS 8 or 16 particles (KC columns) at
+// a time, column-major so each MFMA operand is one 8-byte LDS read per lane.  M is formed from F (L2) tile by tile when S_t is
 // complete, once for both particle types, so only the S accumulators stay in
 // registers through the chunks and F is read once per (walker, spin); it is
 // prefetched into L2 while the last chunk's products run.
+#include <type_traits>
+
 #include "qmc_dev.h"
 
 typedef double xc_d4 __attribute__((ext_vector_type(4)));
 
-// Tile i (0..8) of the group for block row g: row g then row 7-g.
-__host__ __device__ constexpr int xc_tj(int g, int i) { return i < 8 - g ? g : 7 - g; }
-__host__ __device__ constexpr int xc_tk(int g, int i) { return i < 8 - g ? g + i : (7 - g) + (i - (8 - g)); }
-// wavefront half h takes tiles [xc_i0(h), xc_i0(h) + xc_nt(h))
-__host__ __device__ constexpr int xc_i0(int h) { return h ? 5 : 0; }
-__host__ __device__ constexpr int xc_nt(int h) { return h ? 4 : 5; }
-__host__ __device__ constexpr bool xc_needs(int g, int h, int b) {
-  for (int q = 0; q < xc_nt(h); q++)
-    if (xc_tj(g, xc_i0(h) + q) == b || xc_tk(g, xc_i0(h) + q) == b) return true;
-  return false;
+// The kernel's shape for spins of up to 8 NB particles: NB 16-row tiles per
+// side of S, of which the upper triangle goes to W wavefronts, and chunks of
+// KC columns.  Padding to the full 128 rows made the tiles beyond the spin's the
+// larger part of the work (33 of 36 tiles at 13 particles per spin, 26 of 36 at
+// 29): N = 26, 4096 walkers 209 us (now 39), N = 58, 512 walkers 45 us (now 22),
+// N = 74, 256 walkers 36 us (now 27).  Wavefronts and chunk: enough threads to
+// form a chunk's entries in one or two turns, and LDS for as many blocks as the
+// registers allow. (N = 58 with chunks of 32 columns 32 us, with 8 wavefronts 28; N
+// = 26, 4096 walkers with 4 wavefronts 44, with one 45 us.)
+template <int NB>
+struct XcShape {
+  static constexpr int W = NB >= 6 ? 8 : NB == 4 ? 4 : 2, T = 64 * W;
+  static constexpr int KC = NB >= 6 ? 32 : 16;
+  static constexpr int JR = 8 * NB;        // particles (rows of 2)
+  static constexpr int RS = 16 * NB + 16;  // LDS row stride: the 16-lane groups of an operand read disjoint banks
+  static constexpr int NTILE = NB * (NB + 1) / 2;
+  static constexpr int TPW = (NTILE + W - 1) / W;  // most tiles per wavefront
+  static constexpr int EPT = (JR * (KC / 2) + T - 1) / T;  // entries of a chunk per thread
+  // tiles of wavefront w: the first NTILE % W take one more
+  __host__ __device__ static constexpr int nt(int w) { return NTILE / W + (w < NTILE % W ? 1 : 0); }
+  // tile q of wavefront w.  NB = 8: wavefronts g and g + 4 (one SIMD) share
+  // block rows g and 7 - g, 5 + 4 tiles; else the triangle row by row.
+  __host__ __device__ static constexpr int tile(int w, int q, bool col) {
+    if (NB == 8) {
+      const int g = w & 3, i = (w >> 2 ? 5 : 0) + q;
+      const int tj = i < 8 - g ? g : 7 - g;
+      return !col ? tj : i < 8 - g ? g + i : (7 - g) + (i - (8 - g));
+    }
+    int i = q;
+    for (int v = 0; v < w; v++) i += nt(v);
+    int tj = 0;
+    while (i >= NB - tj) i -= NB - tj++;
+    return col ? tj + i : tj;
+  }
+  __host__ __device__ static constexpr int tj(int w, int q) { return tile(w, q, false); }
+  __host__ __device__ static constexpr int tk(int w, int q) { return tile(w, q, true); }
+  __host__ __device__ static constexpr bool needs(int w, int b) {
+    for (int q = 0; q < nt(w); q++)
+      if (tj(w, q) == b || tk(w, q) == b) return true;
+    return false;
+  }
+};
+
+// f(integral_constant q) for q = 0..N-1.
+template <int N, class F>
+__device__ __forceinline__ void xc_each(F&& f) {
+  if constexpr (N > 0) {
+    xc_each<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
 }
 
-#define XC_TPW 5  // most tiles per wavefront
+// f(integral_constant NB) for the larger spin's size.
+template <class F>
+static auto with_cross_shape(const DevSys& s, F&& f) {
+  const int m = s.np[0] > s.np[1] ? s.np[0] : s.np[1];
+  if (m <= 16) return f(std::integral_constant<int, 2>{});
+  if (m <= 32) return f(std::integral_constant<int, 4>{});
+  if (m <= 48) return f(std::integral_constant<int, 6>{});
+  return f(std::integral_constant<int, 8>{});
+}
 
 // real part of the product of two elements of F (complex, or real orbitals')
 __device__ __forceinline__ double xc_re(zd a, zd b) { return a.x * b.x - a.y * b.y; }
@@ -48,12 +96,11 @@ __device__ __forceinline__ void xc_pin(xc_d4& a) { __asm__ volatile("" : "+v"(a)
 // The 2 x 2 diagonal blocks of S_t (rows and columns (j, a), (j, b); the
 // three distinct entries at index a + b), from the wavefronts that hold the
 // diagonal tiles: sd[(t * 64 + j) * 3 + a + b].
-template <int G, int H>
-__device__ __forceinline__ void xc_diag_blocks(const xc_d4 (&acc)[2][XC_TPW], double* __restrict__ sd, int lane) {
-#pragma unroll
-  for (int q = 0; q < xc_nt(H); q++) {
-    const int TJ = xc_tj(G, xc_i0(H) + q), TK = xc_tk(G, xc_i0(H) + q);
-    if (TJ != TK) continue;
+template <int NB, int V>
+__device__ __forceinline__ void xc_diag_blocks(const xc_d4 (&acc)[2][XcShape<NB>::TPW], double* __restrict__ sd, int lane) {
+  xc_each<XcShape<NB>::nt(V)>([&](auto qc) {
+    constexpr int q = decltype(qc)::value, TJ = XcShape<NB>::tj(V, q), TK = XcShape<NB>::tk(V, q);
+    if constexpr (TJ != TK) return;
     const int c = lane & 15;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
@@ -64,7 +111,7 @@ __device__ __forceinline__ void xc_diag_blocks(const xc_d4 (&acc)[2][XC_TPW], do
         sd[192 + e] = acc[1][q][v];
       }
     }
-  }
+  });
 }
 
 // Sums over the wavefront's tiles of M o (S_t - S_t's diagonal blocks), M
@@ -75,8 +122,8 @@ __device__ __forceinline__ void xc_diag_blocks(const xc_d4 (&acc)[2][XC_TPW], do
 // An element above the diagonal stands for its mirror image too, whose row is
 // its column.  The accumulator of v_mfma_f64_16x16x4f64 holds, in lane l and
 // register v, element (row l/16 + 4v, column l%16) of the 16 x 16 tile.
-template <int G, int H, typename Z>
-__device__ __forceinline__ void xc_contract(const xc_d4 (&acc)[2][XC_TPW], const double* __restrict__ sd,
+template <int NB, int V, typename Z>
+__device__ __forceinline__ void xc_contract(const xc_d4 (&acc)[2][XcShape<NB>::TPW], const double* __restrict__ sd,
                                             const Z* __restrict__ Fg, int m, int lane_in, int nT, double& t0,
                                             double& t1) {
   const int R = 2 * m;
@@ -86,9 +133,8 @@ __device__ __forceinline__ void xc_contract(const xc_d4 (&acc)[2][XC_TPW], const
   int lane = lane_in;
   __asm__ volatile("" : "+s"(Fq), "+v"(lane));
   t0 = t1 = 0.0;
-#pragma unroll
-  for (int q = 0; q < xc_nt(H); q++) {
-    const int TJ = xc_tj(G, xc_i0(H) + q), TK = xc_tk(G, xc_i0(H) + q);
+  xc_each<XcShape<NB>::nt(V)>([&](auto qc) {
+    constexpr int q = decltype(qc)::value, TJ = XcShape<NB>::tj(V, q), TK = XcShape<NB>::tk(V, q);
     if (TK < nT) {
       const int sc = 16 * TK + (lane & 15);
       const int ks = sc >> 1, bs = sc & 1;
@@ -115,17 +161,20 @@ __device__ __forceinline__ void xc_contract(const xc_d4 (&acc)[2][XC_TPW], const
     }
     // one tile's F values in flight at a time
     __asm__ volatile("" ::: "memory");
-  }
+  });
 }
 
-// Entry e (row j = e % 64, particle pc = e / 64) of the V chunk of
+// Entry e (row j = e % JR, particle pc = e / JR) of the V chunk of
 // particles c0..c0+cn-1: rows j beyond m and particles beyond cn are zero;
 // the 2 x 2 block of (j, ip) is symmetric.  Consecutive threads take
 // consecutive rows, so the column-major stores spread over the LDS banks.
+template <int NB>
 __device__ __forceinline__ void xc_entry(const DevSys& s, const double* __restrict__ Qd,
                                          const double* __restrict__ xs, double* __restrict__ Vt, TabRef tb,
                                          int e, int c0, int cn, int m, int p0) {
-  const int j = e & 63, pc = e >> 6;
+  typedef XcShape<NB> S;
+  const int j = e % S::JR, pc = e / S::JR;
+  if (S::JR * (S::KC / 2) % S::T != 0 && pc >= S::KC / 2) return;
   double v11 = 0, v12 = 0, v22 = 0;
   const int ip = c0 + pc;
   if (j < m && pc < cn) {
@@ -146,9 +195,9 @@ __device__ __forceinline__ void xc_entry(const DevSys& s, const double* __restri
     }
   }
   // rows 2j, 2j+1 of each of the two columns: one 16-byte store each
-  // (XC_RS is even, so both are 16-byte aligned)
-  *reinterpret_cast<double2*>(Vt + (2 * pc) * XC_RS + 2 * j) = make_double2(v11, v12);
-  *reinterpret_cast<double2*>(Vt + (2 * pc + 1) * XC_RS + 2 * j) = make_double2(v12, v22);
+  // (RS is even, so both are 16-byte aligned)
+  *reinterpret_cast<double2*>(Vt + (2 * pc) * S::RS + 2 * j) = make_double2(v11, v12);
+  *reinterpret_cast<double2*>(Vt + (2 * pc + 1) * S::RS + 2 * j) = make_double2(v12, v22);
 }
 
 // Destination of the L2 prefetch of F: one wavefront's 64 x 16 bytes, never read.
@@ -159,19 +208,21 @@ __shared__ __attribute__((aligned(16))) unsigned xc_sink[256];
 // double-buffered: while the matrix cores take this chunk's products the
 // vector units build the next chunk into the other buffer (two entries per
 // thread, placed between the MFMA steps), so a chunk costs one barrier.
-template <int G, int H, typename Z>
+template <int NB, int V, typename Z>
 __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ dsc, const double* __restrict__ Qd,
                                         const Z* __restrict__ Fg, const double* __restrict__ xs,
                                         double* __restrict__ Vt, double* red, int sp, int m, int p0, int tid) {
+  typedef XcShape<NB> S;
+  constexpr int XC_KC = S::KC, XC_RS = S::RS, XC_THREADS = S::T;
   const int lane = tid & 63;
   const int nT = (2 * m + 15) >> 4;
   // S_t accumulators of both particle types (zero for a type without
   // backflow to this spin), contracted with M in one pass over F at the end
-  xc_d4 acc[2][XC_TPW];
+  xc_d4 acc[2][S::TPW];
 #pragma unroll
   for (int t = 0; t < 2; t++)
 #pragma unroll
-    for (int q = 0; q < XC_TPW; q++) acc[t][q] = xc_d4{0.0, 0.0, 0.0, 0.0};
+    for (int q = 0; q < S::TPW; q++) acc[t][q] = xc_d4{0.0, 0.0, 0.0, 0.0};
   bool act[2];
 #pragma unroll
   for (int t = 0; t < 2; t++)
@@ -180,7 +231,7 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
   if (ft >= 0) {
     const int c0 = pick2(s.ipf, ft), cn = min(XC_KC / 2, pick2(s.np, ft));
     const TabRef tb = tabref<TK_B>(s, tpair(sp, ft));
-    for (int e = tid; e < 64 * (XC_KC / 2); e += XC_THREADS) xc_entry(s, Qd, xs, Vt, tb, e, c0, cn, m, p0);
+    for (int e = tid; e < S::JR * (XC_KC / 2); e += XC_THREADS) xc_entry<NB>(s, Qd, xs, Vt, tb, e, c0, cn, m, p0);
   }
   __syncthreads();
   int cur = 0;
@@ -207,27 +258,27 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
         if (2 * ks < cn) {
           // rows beyond 2m are zero in LDS, so tiles past the last block row
           // add zeros and need no branch here
-          double blk[8];
-#pragma unroll
-          for (int b = 0; b < 8; b++)
-            if (xc_needs(G, H, b)) blk[b] = base[ks * 4 * XC_RS + 16 * b];
-#pragma unroll
-          for (int q = 0; q < xc_nt(H); q++) {
-            const int TJ = xc_tj(G, xc_i0(H) + q), TK = xc_tk(G, xc_i0(H) + q);
+          double blk[NB];
+          xc_each<NB>([&](auto bc) {
+            constexpr int b = decltype(bc)::value;
+            if constexpr (XcShape<NB>::needs(V, b)) blk[b] = base[ks * 4 * XC_RS + 16 * b];
+          });
+          xc_each<XcShape<NB>::nt(V)>([&](auto qc) {
+            constexpr int q = decltype(qc)::value, TJ = XcShape<NB>::tj(V, q), TK = XcShape<NB>::tk(V, q);
             acc[t][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(blk[TJ], blk[TK], acc[t][q], 0, 0, 0);
-          }
+          });
 #pragma unroll
-          for (int q = 0; q < xc_nt(H); q++) xc_pin(acc[t][q]);
+          for (int q = 0; q < XcShape<NB>::nt(V); q++) xc_pin(acc[t][q]);
         }
-        if (nt >= 0 && (ks == 1 || ks == 5))
-          xc_entry(s, Qd, xs, Vn, ntb, tid + (ks == 5 ? XC_THREADS : 0), nc0, ncn, m, p0);
+        if (nt >= 0 && (ks == 1 || (S::EPT == 2 && ks == 1 + XC_KC / 8)))
+          xc_entry<NB>(s, Qd, xs, Vn, ntb, tid + (ks == 1 ? 0 : XC_THREADS), nc0, ncn, m, p0);
         // during the last chunk, F of this (walker, spin) is fetched into
         // the L2 cache (16 bytes a lane, into an LDS sink nothing reads), a
-        // quarter at every other step, so the contraction below reads it
+        // part at every other step, so the contraction below reads it
         // from there instead of waiting on HBM tile by tile
         if (nt < 0 && (ks & 1)) {
           const int nz = 2 * m * m * (int)sizeof(Z) / 16;
-          for (int i = tid + (ks >> 1) * XC_THREADS; i < nz; i += 4 * XC_THREADS)
+          for (int i = tid + (ks >> 1) * XC_THREADS; i < nz; i += XC_KC / 8 * XC_THREADS)
             __builtin_amdgcn_global_load_lds((const void*)((const double2*)Fg + i), (void __attribute__((address_space(3)))*)xc_sink,
                                              16, 0, 0);
         }
@@ -239,10 +290,10 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
     }
   }
   // the chunk buffers are free: the diagonal blocks go there
-  xc_diag_blocks<G, H>(acc, Vt, lane);
+  xc_diag_blocks<NB, V>(acc, Vt, lane);
   __syncthreads();
   double u0, u1;
-  xc_contract<G, H>(acc, Vt, Fg, m, lane, nT, u0, u1);
+  xc_contract<NB, V>(acc, Vt, Fg, m, lane, nT, u0, u1);
   u0 = block_sum<XC_THREADS>(u0, red);
   u1 = block_sum<XC_THREADS>(u1, red);
   if (tid == 0) {
@@ -251,22 +302,25 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
   }
 }
 
-// LDS: xs[2N], then two Vt[XC_KC][XC_RS] chunk buffers (column = (particle,
-// idim) of the chunk, row = (j, a)).
-template <typename Z>
-__device__ __forceinline__ void k_cross_body(const DevSys& s, const WsLayout& L, const double* __restrict__ x,
-                                             double* __restrict__ ws, const double* __restrict__ Fbuf) {
+// LDS: xs[2N], then two Vt[KC][RS] chunk buffers (column = (particle, idim) of
+// the chunk, row = (j, a)).  Z: zd (complex F: k_gjm, k_det) or double (k_gjr).
+template <typename Z, int NB>
+__global__ __launch_bounds__(XcShape<NB>::T, 4) void k_cross(DevSys s, WsLayout L, const double* __restrict__ x,
+                                                             double* __restrict__ ws,
+                                                             const double* __restrict__ Fbuf) {
+  constexpr int W = XcShape<NB>::W;
   extern __shared__ __attribute__((aligned(16))) double sm[];
-  __shared__ double red[XC_THREADS / 64];
-  // walkers and spins in the reverse of the order in which k_gjm wrote their
-  // F, so the first workgroups find theirs still in the memory-side cache
+  __shared__ double red[W];
+  // walkers and spins in the reverse of the order in which the determinant
+  // kernel wrote their F, so the first workgroups find theirs still in the
+  // memory-side cache
   const int w = gridDim.x - 1 - blockIdx.x, sp = gridDim.y - 1 - blockIdx.y;
   if (s.nact && w >= *s.nact) return;
   const int m = pick2(s.np, sp);
   if (m == 0) return;
   const int N = s.nptot, p0 = pick2(s.ipf, sp);
   const int tid = threadIdx.x;
-  const int w8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   double* wsw = ws + (int64_t)w * L.per_walker;
   double* dsc = wsw + pick2(L.off_det, sp);
   if (dsc[DS_SING] != 0.0) return;
@@ -275,30 +329,24 @@ __device__ __forceinline__ void k_cross_body(const DevSys& s, const WsLayout& L,
   double* xs = sm;
   double* Vt = sm + 2 * N;
   const double* xw = x + (int64_t)w * 2 * N;
-  for (int k = tid; k < 2 * N; k += XC_THREADS) xs[k] = xw[k];
+  for (int k = tid; k < 2 * N; k += 64 * W) xs[k] = xw[k];
   __syncthreads();
-  switch (w8) {
-    case 0: xc_body<0, 0>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
-    case 1: xc_body<1, 0>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
-    case 2: xc_body<2, 0>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
-    case 3: xc_body<3, 0>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
-    case 4: xc_body<0, 1>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
-    case 5: xc_body<1, 1>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
-    case 6: xc_body<2, 1>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
-    default: xc_body<3, 1>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid); break;
-  }
+#define XC_CASE(v)                                                                              \
+  case v:                                                                                       \
+    if constexpr (v < W) xc_body<NB, v>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid);           \
+    break;
+  switch (wv) { XC_CASE(0) XC_CASE(1) XC_CASE(2) XC_CASE(3) XC_CASE(4) XC_CASE(5) XC_CASE(6) XC_CASE(7) }
+#undef XC_CASE
 }
 
-// F complex (k_gjm, k_det)
-__global__ __launch_bounds__(XC_THREADS, 4) void k_cross(DevSys s, WsLayout L, const double* __restrict__ x,
-                                                         double* __restrict__ ws,
-                                                         const double* __restrict__ Fbuf) {
-  k_cross_body<zd>(s, L, x, ws, Fbuf);
-}
-
-// F real (k_gjr)
-__global__ __launch_bounds__(XC_THREADS, 4) void k_cross_real(DevSys s, WsLayout L, const double* __restrict__ x,
-                                                              double* __restrict__ ws,
-                                                              const double* __restrict__ Fbuf) {
-  k_cross_body<double>(s, L, x, ws, Fbuf);
+void launch_cross(const DevSys& s, const WsLayout& L, int nw, bool real, const double* x, double* ws,
+                  const double* F, hipStream_t st) {
+  with_cross_shape(s, [&](auto nb) {
+    constexpr int NB = decltype(nb)::value;
+    typedef XcShape<NB> S;
+    const size_t lds = sizeof(double) * (2 * s.nptot + 2 * S::KC * S::RS);
+    const dim3 grid(nw, s.ntypes);
+    if (real) hipLaunchKernelGGL((k_cross<double, NB>), grid, dim3(S::T), lds, st, s, L, x, ws, F);
+    else hipLaunchKernelGGL((k_cross<zd, NB>), grid, dim3(S::T), lds, st, s, L, x, ws, F);
+  });
 }

@@ -60,7 +60,7 @@ struct qmc_ctx {
   hipStream_t stream = nullptr;
   double delta = 0.0;  // current time step (COMMON delta) for the drift cutoff
   int kc = 16;
-  size_t lds_pairs = 0, lds_det = 0, lds_cross = 0;
+  size_t lds_pairs = 0, lds_det = 0;
   size_t lds_pairs_mix = 0;
   int kchunk_mix = 1;
   int tpp_det = 0;
@@ -109,6 +109,9 @@ int launch_eval(qmc_ctx* c, int nw, const double* d_x, double* d_props, double* 
 // workspace, by the determinants' pivots alone; the matrix-core determinant
 // path only.
 int launch_logdet(qmc_ctx* c, int nw, hipStream_t st);
+// The cross-term kernel of every spin on st (qmc_cross.hip); real: F of k_gjr.
+void launch_cross(const DevSys& s, const WsLayout& L, int nw, bool real, const double* x, double* ws,
+                  const double* F, hipStream_t st);
 // The pair kernel (qmc_kernels.hip): its LDS for kc particles per phase chunk,
 // the doubles of its FP64 phase rows, and its launch.
 size_t pairs_lds(const DevSys& s, int kc, bool mix);
