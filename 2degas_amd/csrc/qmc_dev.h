@@ -336,38 +336,6 @@ __device__ __forceinline__ PairGeo pair_geo(const DevSys& s, double xi, double y
 
 __device__ __forceinline__ int ptype(const DevSys& s, int i) { return i >= s.ipf[1] && s.ntypes > 1 ? 1 : 0; }
 
-// k_fgrad's schedule for one spin: nA = 32 steps of the spin's own block
-// (weight 3: both ends take drift terms) then nB = 64 steps across to the
-// other type (weight 2), split into four runs of equal weight, one per
-// wavefront.  A wavefront's LDS partial sums hold the backflow sums qb[5][64]
-// of the spin's particles, then zs[5][64] (drift and Laplacian terms of the
-// spin's particles) when its run has own-block steps and zo[5][64] (those of
-// the other type) when it has steps across.  Scalar functions of (nA, nB, w)
-// rather than a table, which a varying w would index in scratch memory.
-#define FG_NZ 5
-#define FG_NQ 5
-// first step of wavefront w's run (w = 4: the end)
-__host__ __device__ inline int fg_u(int nA, int nB, int w) {
-  if (w >= 4) return nA + nB;
-  const int C = 3 * nA + 2 * nB, T = (w * C) / 4;
-  const int u = T <= 3 * nA ? (T + 2) / 3 : nA + (T - 3 * nA + 1) / 2;
-  return u < nA + nB ? u : nA + nB;
-}
-__host__ __device__ inline bool fg_hasA(int nA, int nB, int w) {
-  return fg_u(nA, nB, w + 1) > fg_u(nA, nB, w) && fg_u(nA, nB, w) < nA;
-}
-__host__ __device__ inline bool fg_hasB(int nA, int nB, int w) {
-  return fg_u(nA, nB, w + 1) > fg_u(nA, nB, w) && fg_u(nA, nB, w + 1) > nA;
-}
-// start of wavefront w's partial sums (w = 4: their total), in doubles
-__host__ __device__ inline int fg_off(int nA, int nB, int w) {
-  int o = 0;
-  for (int v = 0; v < w; v++)
-    o += (fg_u(nA, nB, v + 1) > fg_u(nA, nB, v) ? FG_NQ * 64 : 0) + (fg_hasA(nA, nB, v) ? FG_NZ * 64 : 0) +
-         (fg_hasB(nA, nB, v) ? FG_NZ * 64 : 0);
-  return o;
-}
-
 // Maximum over the wavefront of a 32-bit key: DPP swaps inside quads, row
 // rotations by 4 and 8 inside each row of 16 lanes, then the four row maxima.
 // Every lane must be active.

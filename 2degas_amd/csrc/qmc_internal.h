@@ -74,7 +74,6 @@ struct qmc_ctx {
   bool sys_valid = false;
   bool gjm_part = false; // a spin below 49 particles: k_gjm_part, which skips the tiles beyond m
   size_t lds_gjm = 0;
-  size_t lds_fgrad = 0;
   // per-kernel event timing
   bool timing = false;
   std::vector<hipEvent_t> ev;  // TIMING_EVENTS events per recorded launch
@@ -109,6 +108,8 @@ int launch_eval(qmc_ctx* c, int nw, const double* d_x, double* d_props, double* 
 // workspace, by the determinants' pivots alone; the matrix-core determinant
 // path only.
 int launch_logdet(qmc_ctx* c, int nw, hipStream_t st);
+// Drift, backflow blocks and first-derivative Laplacian terms (qmc_fgrad.hip).
+void launch_fgrad(const DevSys& s, const WsLayout& L, int nw, const double* x, double* ws, hipStream_t st);
 // The cross-term kernel of every spin on st (qmc_cross.hip); real: F of k_gjr.
 void launch_cross(const DevSys& s, const WsLayout& L, int nw, bool real, const double* x, double* ws,
                   const double* F, hipStream_t st);

@@ -23,6 +23,7 @@
 #include <utility>
 
 #include "qmc_internal.h"
+#include "qmc_pairs.h"
 
 // k-vectors per thread and pass in k_pairs
 #define KMAXPT 4
@@ -34,21 +35,7 @@
 // the pair passes (NA x 6 x 2P doubles) and, afterwards, the phase steps (4N) and
 // phases of rho_k.
 //
-// The pair passes visit every unordered pair once, on a round-robin
-// schedule over blocks of P lanes, P = 16, 32 or 64 the power of two that
-// holds the larger type: the particles of type t sit in lanes 0..np_t-1 of a
-// block, and step d of block pair (I, J) pairs lane l of I with lane
-// (l + d) mod P of J, so within a step every lane has a distinct partner.
-// Within one type d runs over 1..P/2 (d = P/2 on the lower half of the lanes
-// only), across the two types over 0..P-1.  A wavefront takes 64 / P steps of
-// one block pair at a time, one per group of P lanes (P^2 / 32 wavefront
-// steps in all: with one group of 64 lanes for every size, N = 26 would take
-// 128 steps of 13 live lanes instead of 8), and the wavefront steps are split
-// into NW contiguous runs.  A pair's contribution to i stays in registers
-// until the wavefront's run leaves block I; its contribution to j is added to
-// the lane group's own partial sums in LDS (distinct j within a step, so no
-// two lanes touch one address), and the NA = NW 64 / P partial sums are added
-// in a fixed order afterwards: the result does not depend on scheduling.
+// The pair passes run on the schedule of qmc_pairs.h.
 //
 // What bounds it: a step is a chain of some 1500 cycles (geometry, table
 // loads, spline, LDS sums), so short runs count where few walkers are in
@@ -61,14 +48,6 @@
 // count depends on the deck alone, not on the batch, so that a walker's result
 // does not depend on the batch it is in.
 #define PP_NQ 6  // per-particle sums of a pass
-template <bool MIX, int P>
-struct PairShape {
-  static constexpr int NW = P == 16 || MIX ? 4 : 8;  // wavefronts
-  static constexpr int T = 64 * NW, SUB = 64 / P, NA = NW * SUB;
-  static constexpr int OWN = P / 2 / SUB, ACROSS = P / SUB;  // wavefront steps of a block pair
-  static constexpr int NS = 2 * P;  // particles a sum's row holds
-  static constexpr int PART = 6 * NS;  // doubles of one group's partial sums
-};
 
 // part[q * NS + p] += v for the lane group's partial sums
 template <int NS>
@@ -76,39 +55,6 @@ __device__ __forceinline__ void pp_add(double* part, int p, const double (&v)[PP
 #pragma unroll
   for (int q = 0; q < PP_NQ; q++)
     if (q < nq) part[q * NS + p] += v[q];
-}
-
-// The wavefront's run of pair steps: pair(T, i, j) for each of its lanes'
-// pairs, block(ti, tj) after each block pair's, end(ti) when the run leaves
-// block ti.
-template <bool MIX, int P, class Pair, class Block, class End>
-__device__ __forceinline__ void pair_run(const DevSys& s, int wv, int l, Pair&& pair, Block&& block, End&& end) {
-  using S = PairShape<MIX, P>;
-  const int lp = l & (P - 1), sub = l / P;
-  // schedule: both types present, or the one type t1
-  const bool two = s.ntypes > 1 && s.np[0] > 0 && s.np[1] > 0;
-  const int t1 = (s.ntypes > 1 && s.np[0] == 0) ? 1 : 0;
-  const int nU = two ? 2 * S::OWN + S::ACROSS : S::OWN;
-  const int u0 = wv * nU / S::NW, u1 = (wv + 1) * nU / S::NW;
-  // blocks (0, 0), (0, 1), (1, 1): type 0's own and across are one stretch of i
-  for (int blk = 0; blk < 3; blk++) {
-    if (!two && blk > 0) break;
-    const int ti = two ? (blk == 2 ? 1 : 0) : t1, tj = two ? (blk == 0 ? 0 : 1) : t1;
-    const int b0 = blk == 0 ? 0 : (blk == 1 ? S::OWN : S::OWN + S::ACROSS);
-    const int b1 = blk == 0 ? S::OWN : (blk == 1 ? S::OWN + S::ACROSS : 2 * S::OWN + S::ACROSS);
-    const int a = max(u0, b0), b = min(u1, b1);
-    if (a < b) {
-      const TpInfo* T = s.tpi + tpair(ti, tj);
-      const int ni = pick2(s.np, ti), nj = pick2(s.np, tj), i = pick2(s.ipf, ti) + lp;
-      for (int u = a; u < b; u++) {
-        const int d = (u - b0) * S::SUB + sub + (ti == tj ? 1 : 0);
-        const int jl = (lp + d) & (P - 1);
-        if (lp < ni && jl < nj && (ti != tj || d < P / 2 || lp < P / 2)) pair(T, i, pick2(s.ipf, tj) + jl);
-      }
-      block(ti, tj);
-    }
-    if (u0 < u1 && (blk == 2 || !two || (blk == 1 && u0 < b1))) end(ti);
-  }
 }
 
 // The NA partial sums of each of the nq per-particle sums, added in order
@@ -669,22 +615,6 @@ __global__ __launch_bounds__((PairShape<MIX, P>::T), MIX ? 5 : 6) void k_pairs(D
                                                               double* __restrict__ ws,
                                                               double* __restrict__ props) {
   k_pairs_body<MIX, P>(s, L, x, ws, props);
-}
-
-// Lanes per block of the pair schedule for a system.
-static int pair_lanes(const DevSys& s) {
-  const int m = s.np[0] > s.np[1] ? s.np[0] : s.np[1];
-  return m <= 16 ? 16 : m <= 32 ? 32 : 64;
-}
-
-// f(integral_constant P) for the system's lanes per block.
-template <class F>
-static auto with_lanes(const DevSys& s, F&& f) {
-  switch (pair_lanes(s)) {
-    case 16: return f(std::integral_constant<int, 16>{});
-    case 32: return f(std::integral_constant<int, 32>{});
-    default: return f(std::integral_constant<int, 64>{});
-  }
 }
 
 // LDS bytes of the pair kernels with kc particles per phase chunk (0: no
