@@ -72,8 +72,6 @@ struct qmc_ctx {
   // (FP64, FP32) and row class (16, 32, 64 rows)
   int sem_cg[2][3] = {{4, 2, 4}, {4, 2, 4}};
   bool sys_valid = false;
-  bool gjm_part = false; // a spin below 49 particles: k_gjm_part, which skips the tiles beyond m
-  size_t lds_gjm = 0;
   // per-kernel event timing
   bool timing = false;
   std::vector<hipEvent_t> ev;  // TIMING_EVENTS events per recorded launch
@@ -96,7 +94,7 @@ struct qmc_ctx {
   int32_t* d_rslot = nullptr;  // [nr] evaluation slot of each reptile, [mdelta] counts after it
 };
 
-// Queue one batched evaluation (k_pairs, k_gjm or k_gjm_part and k_fgrad, or
+// Queue one batched evaluation (k_pairs, then k_gjr or k_gjc and k_fgrad, or
 // k_det, then k_cross, k_final) on st.
 // delta is the time step the drift cutoff of kinetic uses (reptation.f:2755);
 // precision QMC_PREC_MIXED selects the mixed-precision pair kernel; nact (a
@@ -122,6 +120,8 @@ void launch_pairs(const DevSys& s, const WsLayout& L, int nw, bool mix, size_t l
 // The real-orbital determinant kernels of every spin (s.real_orb); value:
 // log|det A| alone.
 void launch_gjr(const DevSys& s, const WsLayout& L, int nw, bool value, double* ws, double* F, hipStream_t st);
+// The same for complex orbitals.
+void launch_gjc(const DevSys& s, const WsLayout& L, int nw, bool value, double* ws, double* F, hipStream_t st);
 // The FP64 inverses of single-electron moves at positions x (s.real_orb).
 void launch_gjr_inverse(const DevSys& s, int nw, const double* x, void* ainv, int mm, hipStream_t st);
 void free_vmc(qmc_ctx* c);
