@@ -18,7 +18,7 @@
 // inverse with two barriers and a copy of the matrix in LDS per block, then two
 // complex products, always on 64 rows, took 250 us for 4096 walkers of N=26 (now
 // 63), 267 us for 2048 of N=58 (now 130), 218 us for 1024 of N=74 (now 193), 191
-// us for 1024 of 61 polarized particles (now 185) and 16 us for one of N=26 (now
+// us for 1024 of 61 polarized particles (now 180) and 16 us for one of N=26 (now
 // 10).  Wavefronts per SIMD: what the accumulators allow without spills (48
 // registers per row tile); one part's operands are in registers at a time.
 #include "qmc_gj.h"
@@ -191,15 +191,25 @@ __global__ __launch_bounds__(64 * NT, VAL || NT == 1 ? 4 : 2) void k_gjc(DevSys 
     if constexpr (S::COPY) {
       p = sh.prow[buf][lr];
     } else {
+      int pb[4];
+#pragma unroll
+      for (int k = 0; k < 4; k++) pb[k] = __builtin_amdgcn_readfirstlane(sh.prow[buf][k]);
 #pragma unroll
       for (int k = 0; k < 4; k++) {
-        const int pk = __builtin_amdgcn_readfirstlane(sh.prow[buf][k]);
         // the lanes that hold row p; the others' values go to their own places
-        // behind the block's rows
-        double2* to = ub + (lr == (pk & 3) ? k * 16 : (4 + lr) * 16) + lc;
+        // behind the block's rows.  (Between the scheduling barriers the picks
+        // share one index mode instead of a switch for each.)
+        double2* to = ub + (lr == (pb[k] & 3) ? k * 16 : (4 + lr) * 16) + lc;
+        double2 row[NP];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < NP; t++)
-          to[t * PART] = make_double2(gr_pick<NT>(re[t], pk >> 2), gr_pick<NT>(im[t], pk >> 2));
+        for (int t = 0; t < NP; t++) {
+          row[t].x = gr_pick<NT>(re[t], pb[k] >> 2);
+          row[t].y = gr_pick<NT>(im[t], pb[k] >> 2);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < NP; t++) to[t * PART] = row[t];
       }
       gr_wave_sync();
     }

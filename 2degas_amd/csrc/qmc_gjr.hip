@@ -28,7 +28,7 @@
 // rows, update), so U must not lengthen it: rows are taken from the registers
 // in index mode or, where the LDS allows, from a copy of the tiles stored while
 // the pivot steps run, which then also is the panel.  By a switch over the
-// registers, a dozen branches per row: N=122, 4096 walkers 471 us (now 440);
+// registers, a dozen branches per row: N=122, 4096 walkers 471 us (now 436);
 // log|det| alone, N=58, 512 walkers 17.7 us (now 13.5); N=26, 256 walkers 9.9 us
 // (now 7.9), but 4096 walkers of N=26 33 us (now 34: the copy's LDS).
 //
@@ -231,10 +231,16 @@ __device__ __forceinline__ void gr_eliminate(GrShared<NT, NP>& sh, gr_d4 (&acc)[
 #pragma unroll
       for (int k = 0; k < 4; k++) {
         // the lanes that hold row p; the others' values go to their own places
-        // behind the block's rows
+        // behind the block's rows.  (Between the scheduling barriers the picks
+        // share one index mode instead of a switch for each.)
         double* to = ub + (lr == (pb[k] & 3) ? k * 16 : (4 + lr) * 16) + lc;
+        double row[NP];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t = 0; t < NP; t++) to[t * PART] = gr_pick<NT>(acc[t], pb[k] >> 2);
+        for (int t = 0; t < NP; t++) row[t] = gr_pick<NT>(acc[t], pb[k] >> 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < NP; t++) to[t * PART] = row[t];
       }
       gr_wave_sync();
 #pragma unroll
