@@ -303,7 +303,7 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
 }
 
 // LDS: xs[2N], then two Vt[KC][RS] chunk buffers (column = (particle, idim) of
-// the chunk, row = (j, a)).  Z: zd (complex F: k_gjm, k_det) or double (k_gjr).
+// the chunk, row = (j, a)).  Z: zd (complex F: k_gjc, k_det) or double (k_gjr).
 template <typename Z, int NB>
 __global__ __launch_bounds__(XcShape<NB>::T, 4) void k_cross(DevSys s, WsLayout L, const double* __restrict__ x,
                                                              double* __restrict__ ws,

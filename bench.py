@@ -33,16 +33,23 @@ KERNELS = ["pairs", "det", "fgrad", "cross", "final"]
 
 
 def gj_path():
-    """The library's determinant path: k_gjm unless QMC_NO_GJ is set."""
+    """The library's determinant path: the matrix-core kernels unless QMC_NO_GJ is set."""
     return os.environ.get("QMC_NO_GJ") is None
 
 
-def kernel_flops(nup, ndown, nk_ewald):
+def real_orbitals(gvec, counts):
+    """Whether the occupied plane waves of every spin come with their
+    opposites (the library then works on their cosines and sines)."""
+    return all({tuple(g) for g in gvec[:m].tolist()} == {tuple(-g + 0.0) for g in gvec[:m]} for m in counts if m > 0)
+
+
+def kernel_flops(nup, ndown, nk_ewald, real):
     """Algorithmic flops per walker of each kernel (pairs, determinant,
-    drift/diagonal terms, cross, final).  The determinant is k_gjm (matrix
-    cores; k_fgrad then does the diagonal terms) unless QMC_NO_GJ selects
-    k_det, which does both; the determinant's count is the Gauss-Jordan
-    solve's, whichever kernel runs it.  The cross term is counted as the
+    drift/diagonal terms, cross, final).  The determinant is k_gjr for real
+    orbitals and k_gjc for complex ones (matrix cores; k_fgrad then does the
+    diagonal terms) unless QMC_NO_GJ selects k_det, which does both.  Counted:
+    the elimination of the m x 3m augmented matrix, 5 m^3, four times that
+    complex; k_det's LU and products 24 m^3.  The cross term is counted as the
     work of its formulation: per spin the symmetric product S = V V^T of
     the 2m x 2N backflow Jacobian, 2m (2m+1) 2N flops, and the contraction
     with M, 2 (2m)^2.  (The per-evaluation formula qmc_flops_per_eval counts
@@ -52,7 +59,7 @@ def kernel_flops(nup, ndown, nk_ewald):
     n = nup + ndown
     pairs = 160.0 * n * (n - 1) / 2 + 5.0 * n * nk_ewald + 20.0 * nk_ewald
     gj = gj_path()
-    det = sum(24.0 * m ** 3 + (0.0 if gj else 37.0 * m * m) for m in (nup, ndown))
+    det = sum(((5.0 if real else 20.0) if gj else 24.0) * m ** 3 + (0.0 if gj else 37.0 * m * m) for m in (nup, ndown))
     fgrad = sum(37.0 * m * m for m in (nup, ndown)) if gj else 0.0
     cross = sum(2.0 * m * (2 * m + 1) * 2.0 * n + 2.0 * (2 * m) ** 2 for m in (nup, ndown) if m > 0)
     return [pairs, det, fgrad, cross, 0.0]
@@ -229,11 +236,11 @@ def main():
     guard = int((st.cpu().numpy() & 1).sum())
     ref64 = {"props": props.cpu().numpy(), "g": g.cpu().numpy()}
     mixed = bench_mixed(args, ctx, xt, props, g, h, g2, st, stream, ref64, value)
-    kf = kernel_flops(args.nup, args.ndown, info["nk_ewald"])
+    real = real_orbitals(hip.twist_gvec(d.kvec, d.el, d.ntheta, 1, 1), (args.nup, args.ndown))
+    kf = kernel_flops(args.nup, args.ndown, info["nk_ewald"], real)
     names = KERNELS
     gj = gj_path()
-    part = any(0 < m <= 48 for m in (args.nup, args.ndown))
-    det_kernel = ("k_gjm_part" if part else "k_gjm") if gj else "k_det"
+    det_kernel = ("k_gjr" if real else "k_gjc") if gj else "k_det"
     kname = {"pairs": "k_pairs", "det": det_kernel, "fgrad": "k_fgrad",
              "cross": "k_cross", "final": "k_final"}
     dom = int(np.argmax(ms_k))

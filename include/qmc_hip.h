@@ -388,9 +388,10 @@ int qmc_dmc_branch(qmc_ctx* ctx, int nw, double* d_wate, int64_t* d_rng2, int32_
  * electron changes one column of its spin's matrix A(k, j) = exp(i g_k . r_j)
  * and the inverse is updated (the two- and three-body Jastrow factors are
  * both supported).  With backflow every quasi-coordinate moves with the
- * electron, no low-rank update applies, and each move evaluates the
- * proposed configuration's log|psi| (Jastrow sums, quasi-coordinates and
- * the determinants' pivots): there ainv is not used (may be NULL),
+ * electron, no low-rank update applies, and each move takes the proposed
+ * configuration's determinants anew (their pivots), the Jastrow sums and
+ * quasi-coordinates following the moved electron's pairs: there ainv is not
+ * used (may be NULL),
  * qmc_sem_refresh does nothing, and the walkers' ltf slot of props must
  * hold the current value (qmc_vmc_start) and is kept current.
  *
@@ -427,8 +428,8 @@ int qmc_sem_moves(qmc_ctx* ctx, const qmc_walkers* w, const qmc_sem_state* d, in
 
 /*
  * qmc_sem_moves for up to 16 jobs (contexts of any N, decks and walker sets
- * on one device, none with backflow) in one launch per spin: spin 0's moves
- * of every job, then spin 1's.  Each job's results are those of its own
+ * on one device, none with backflow) in one launch per kind of inverse row
+ * (real, complex) and walker width.  Each job's results are those of its own
  * qmc_sem_moves call with the same range, bit for bit.  No counterpart in
  * the reference (one system per run); for services that run many small
  * jobs at once.
@@ -448,6 +449,7 @@ int qmc_sem_moves_packed(const qmc_sem_job* jobs, int njobs, int precision, void
  * counterpart in the reference): threads per row of the inverse (4, or 2
  * for the 32- and 64-row classes; a row class holds spins of up to 16, 32
  * or 64 particles) at a precision.  Defaults: 2 for 32 rows, 4 otherwise.
+ * It applies to complex rows; FP64 inverses of real orbitals have one shape.
  * The walk depends on it only through the order of the Jastrow sums
  * (rounding); an autotuner times the shapes (SingleMoves.tune_tile in the
  * Python binding) and sets the faster.
@@ -460,7 +462,7 @@ int qmc_sem_set_tile(qmc_ctx* ctx, int precision, int rows, int threads_per_row)
  * which has no timers).  qmc_timing(ctx, 1) resets and enables,
  * qmc_timing(ctx, 0) disables.  qmc_timing_read waits for the recorded work
  * and returns the mean milliseconds per launch of the kernels in the order
- * pairs, determinant (k_gjm, k_gjm_part or k_det), drift and diagonal terms
+ * pairs, determinant (k_gjr, k_gjc or k_det), drift and diagonal terms
  * (k_fgrad; 0 when k_det does them), cross term, final (ms[5]) and the
  * launches counted.
  */
