@@ -228,12 +228,20 @@ __device__ __forceinline__ TabRef tabref(const DevSys& s, int tp) {
   return TabRef{pick3(s.trow[KIND], tp), pick3(s.tng[KIND], tp)};
 }
 
-// Row of a table at grid index ind >= 0 (rows beyond the last one: the last).
+// Row 0..ng of a table for grid index ind.  Indices beyond the last row take the
+// last one, and so do negative ones: a distance is not negative, but what the
+// conversion of one that is no number gives is not defined, and whatever it is
+// must not leave the table.  (As unsigned numbers the negative indices are the
+// largest: one minimum, no instruction more than the upper end alone.)
+__host__ __device__ inline unsigned tab_index(int ind, int ng) {
+  return (unsigned)ind < (unsigned)ng ? (unsigned)ind : (unsigned)ng;
+}
+
 // The byte offset is 32 bits from a uniform base, so that a lane's address is
 // two integer instructions (and the load's own base), not a 64-bit sum.
 template <typename V>
 __device__ __forceinline__ V tab_row(const V* tab, TabRef t, int ind) {
-  const unsigned i = (unsigned)(ind < t.ng ? ind : t.ng) * (unsigned)sizeof(V);
+  const unsigned i = tab_index(ind, t.ng) * (unsigned)sizeof(V);
   return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(tab + t.row0) + i);
 }
 
