@@ -300,12 +300,12 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
           pp_add<S::NS>(part, j, ja, PP_NQ);
         },
         [&](int ti, int tj) {
-          const double h0 = (ti == 0 ? hb : 0.0) + (tj == 0 ? hb : 0.0);
-          acc_h0 += h0;
-          acc_h1 += 2.0 * hb - h0;
-          const double v0 = (ti == 0 ? vb : 0.0) + (tj == 0 ? vb : 0.0);
-          acc_v0 += v0;
-          acc_v1 += 2.0 * vb - v0;
+          // (selected, not subtracted: what is infinite or no number in one
+          // type's pairs stays out of the other's sums)
+          acc_h0 += (ti == 0 ? hb : 0.0) + (tj == 0 ? hb : 0.0);
+          acc_h1 += (ti == 0 ? 0.0 : hb) + (tj == 0 ? 0.0 : hb);
+          acc_v0 += (ti == 0 ? vb : 0.0) + (tj == 0 ? vb : 0.0);
+          acc_v1 += (ti == 0 ? 0.0 : vb) + (tj == 0 ? 0.0 : vb);
           hb = vb = 0.0;
         },
         [&](int ti) {
@@ -368,9 +368,8 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
           hb += h3;
         },
         [&](int ti, int tj) {
-          const double h0 = (ti == 0 ? hb : 0.0) + (tj == 0 ? hb : 0.0);
-          acc_h0 += h0;
-          acc_h1 += 2.0 * hb - h0;
+          acc_h0 += (ti == 0 ? hb : 0.0) + (tj == 0 ? hb : 0.0);
+          acc_h1 += (ti == 0 ? 0.0 : hb) + (tj == 0 ? 0.0 : hb);
           hb = 0.0;
         },
         [&](int ti) {
