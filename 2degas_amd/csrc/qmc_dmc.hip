@@ -98,6 +98,19 @@ __device__ __forceinline__ void dmc_scan(int tid, int* pa, int* pb, int& a, int&
   ta = pa[DMC_BRANCH_THREADS - 1];
 }
 
+struct DmcBranchShared {
+  // places used one after the other
+  union {
+    struct {
+      double somma;
+      int odd;
+    };
+    double start[DMC_BRANCH_THREADS];
+    int scan[2][DMC_BRANCH_THREADS];
+  };
+  long draws;
+};
+
 __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, double* __restrict__ wate,
                                                                    int64_t* __restrict__ rng2,
                                                                    int32_t* __restrict__ src,
@@ -105,16 +118,7 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
   extern __shared__ __attribute__((aligned(16))) unsigned char dmc_lds[];
   double* sw = reinterpret_cast<double*>(dmc_lds);
   int* sm = reinterpret_cast<int*>(sw + nw);
-  // places used one after the other
-  __shared__ union {
-    struct {
-      double somma;
-      int odd;
-    };
-    double start[DMC_BRANCH_THREADS];
-    int scan[2][DMC_BRANCH_THREADS];
-  } sh;
-  __shared__ long sh_draws;
+  __shared__ DmcBranchShared sh;
   const int tid = threadIdx.x;
   const uint64_t st0 = (uint64_t)rng2[0];
   if (tid == 0) sh.odd = 0;
@@ -206,10 +210,10 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
     if (tid == 64) {
       double k0 = 0.0;
       dmc_in_order(sw, nw, [&](int, double v) { k0 = k0 + v; });
-      sh_draws = lround(k0);
+      sh.draws = lround(k0);
     }
     __syncthreads();
-    const long ndraw = sh_draws;
+    const long ndraw = sh.draws;
     // k after walker i0 - 1, and before 1 is taken off at walker i0
     double kb = 0.0, t0 = 0.0;
     if (i0 < i1) {
@@ -328,12 +332,13 @@ static int check_dmc(qmc_ctx* c, int nw, const qmc_dmc_state* d) {
   return QMC_OK;
 }
 
-// The branching's LDS holds 12 bytes per walker: the populations the LDS of
-// a workgroup can take (13000 walkers at 160 KB).
+// The branching's LDS holds 12 bytes per walker beside the kernel's own 8.2 KB
+// (16-byte steps): the populations that the LDS of a workgroup can take, 12969
+// walkers at 160 KB.
 static int dmc_branch_check(qmc_ctx* c, int nw) {
   int lds_max = 0;
   HIPCHK(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
-  const size_t need = dmc_branch_lds(nw) + 64;
+  const size_t need = ((sizeof(DmcBranchShared) + 15) & ~(size_t)15) + dmc_branch_lds(nw);
   if (need > (size_t)lds_max) return arg_fail("DMC population above what the branching's LDS holds", QMC_ERR_LIMIT);
   if (need > 65536)
     HIPCHK(hipFuncSetAttribute((const void*)k_dmc_branch, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -391,6 +396,8 @@ extern "C" int qmc_dmc_sweep(qmc_ctx* c, const qmc_walkers* w, const qmc_dmc_sta
     }
     hipLaunchKernelGGL(k_dmc_branch, dim3(1), dim3(DMC_BRANCH_THREADS), dmc_branch_lds(nw), st, nw, d->wate,
                        d->rng2, d->src, d->counts);
+    // without this branching's sources no walker is copied
+    HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_dmc_copy, dim3((nw + wpb - 1) / wpb), dim3(QMC_BLOCK), 0, st, nw, s.nptot, NP, d->src,
                        w->x, w->g, w->h, w->props);
   }

@@ -1,0 +1,113 @@
+"""Host code of the library under failures that a GPU does not show on demand:
+limits, refused launches and allocations.  Each scenario runs in a process of
+its own against a stand-in of the HIP runtime (hip_stub.cpp) that logs the
+launches and keeps device memory on the host; no GPU takes part."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "2degas_amd", "lib2degas_hip.so")
+HIP_INCLUDE = "/opt/rocm/include"
+
+PRELUDE = r"""
+import ctypes, importlib, os, sys
+import numpy as np
+sys.modules["torch"] = None  # the binding imports it only to share its runtime
+stub = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+stub.stub_log.restype = ctypes.c_char_p
+sys.path.insert(0, sys.argv[2])
+hip, abi, deck = (importlib.import_module("2degas_amd." + m) for m in ("hip", "abi", "deck"))
+L = hip.lib()
+
+def load(name):
+    return deck.read_deck(os.path.join(sys.argv[2], "tests", "golden", "decks", name))
+
+def log(kind=None):
+    lines = [ln.split(" ", 1) for ln in stub.stub_log().decode().splitlines()]
+    return [b for a, b in lines if kind is None or a == kind]
+
+def fail(name, n=1):
+    stub.stub_fail(name.encode(), n)
+
+def buffers(ctx, nw):
+    # host arrays in the places of device buffers
+    n, np_ = ctx.deck.nptot, ctx.info["n_props"]
+    w, keep = abi.QmcWalkers(), {}
+    w.nw = nw
+    for k, sh in dict(x=(nw, n, 2), g=(nw, n, 2), h=(nw, 2), props=(nw, np_), grad2_ph=nw, age=nw, blk=(nw, np_)).items():
+        keep[k] = np.zeros(sh)
+        setattr(w, k, keep[k].ctypes.data)
+    keep["rng"] = np.ones(nw, np.int64)
+    w.rng = keep["rng"].ctypes.data
+    return w, keep
+
+def dmc_state(nw):
+    d = abi.QmcDmcState()
+    keep = dict(wate=np.ones(nw), wsum=np.zeros(nw), src=np.zeros(nw, np.int32), rng2=np.ones(1, np.int64),
+                counts=np.zeros(4, np.int32))
+    for k, a in keep.items():
+        setattr(d, k, a.ctypes.data)
+    return d, keep
+"""
+
+
+@pytest.fixture(scope="module")
+def run_host(tmp_path_factory):
+    if not os.path.exists(LIB) or not os.path.isdir(HIP_INCLUDE) or not shutil.which("g++"):
+        pytest.skip("needs the built library, the HIP headers and g++")
+    so = str(tmp_path_factory.mktemp("stub") / "libhip_stub.so")
+    subprocess.run(["g++", "-O1", "-fPIC", "-shared", "-std=c++17", "-I" + HIP_INCLUDE,
+                    os.path.join(ROOT, "tests", "hip_stub.cpp"), "-o", so], check=True)
+
+    def run(body):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body, so, ROOT], stdout=subprocess.PIPE,
+                           stderr=subprocess.STDOUT, timeout=120)
+        assert r.returncode == 0, r.stdout.decode()
+    return run
+
+
+def test_dmc_population_limit(run_host):
+    """The branching's LDS, its own beside the walkers', decides which
+    populations are taken: a larger one is refused before anything is launched,
+    by the branching alone and by a sweep."""
+    run_host(r"""
+ctx = hip.Context(load("n26g"), twist=(1, 1))
+fits = (163840 - 8208) // 12
+for nw, ok in ((fits, True), (fits + 1, False), (13500, False), (13648, False)):
+    d, keep = dmc_state(nw)
+    stub.stub_clear()
+    rc = L.qmc_dmc_branch(ctx.h, nw, d.wate, d.rng2, d.src, d.counts, None)
+    assert rc == (0 if ok else abi.QMC_ERR_LIMIT), (nw, rc)
+    assert len(log("launch")) == (1 if ok else 0), log()
+w, keep = buffers(ctx, 13500)
+d, keep2 = dmc_state(13500)
+p = abi.QmcDmcParams()
+p.delta, p.mage, p.mmstep, p.mmult = 0.01, 1e30, 1, 10
+stub.stub_clear()
+rc = L.qmc_dmc_sweep(ctx.h, ctypes.byref(w), ctypes.byref(d), 1, ctypes.byref(p), None)
+assert rc == abi.QMC_ERR_LIMIT, rc
+assert not log("launch"), log("launch")
+""")
+
+
+def test_dmc_copies_follow_a_branching(run_host):
+    """No walker is copied by the sources of an earlier branching when this
+    one's launch fails."""
+    run_host(r"""
+ctx = hip.Context(load("n26g"), twist=(1, 1))
+w, keep = buffers(ctx, 16)
+d, keep2 = dmc_state(16)
+p = abi.QmcDmcParams()
+p.delta, p.mage, p.mmstep, p.mmult = 0.01, 1e30, 1, 10
+sweep = lambda n: L.qmc_dmc_sweep(ctx.h, ctypes.byref(w), ctypes.byref(d), n, ctypes.byref(p), None)
+assert sweep(1) == 0
+assert [sum(k in n for n in log("launch")) for k in ("k_dmc_branch", "k_dmc_copy")] == [1, 1]
+stub.stub_clear()
+fail("launch:k_dmc_branch", 2)
+assert sweep(3) == abi.QMC_ERR_HIP
+assert [sum(k in n for n in log("launch")) for k in ("k_dmc_branch", "k_dmc_copy")] == [1, 1]
+""")
