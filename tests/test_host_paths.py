@@ -111,3 +111,40 @@ fail("launch:k_dmc_branch", 2)
 assert sweep(3) == abi.QMC_ERR_HIP
 assert [sum(k in n for n in log("launch")) for k in ("k_dmc_branch", "k_dmc_copy")] == [1, 1]
 """)
+
+
+def test_host_evaluation_without_pinned_memory(run_host):
+    """A host-pointer call goes through the copies when no pinned memory can be
+    had, and through the pinned buffer once it can."""
+    run_host(r"""
+ctx = hip.Context(load("n26"), twist=(1, 1))
+x = np.zeros((2, 26, 2))
+fail("hipHostMalloc", 1)
+stub.stub_clear()
+ctx.eval(x)
+assert len(log("copy")) == 8 and not any("k_stage" in k for k in log("launch")), log()
+stub.stub_clear()
+ctx.eval(x)
+assert not log("copy") and sum("k_stage" in k for k in log("launch")) == 2, log()
+""")
+
+
+def test_host_evaluation_that_fails_after_staging(run_host):
+    """An evaluation that is refused after its inputs were staged returns the
+    error, leaves the caller's arrays as they are, and the next call works."""
+    run_host(r"""
+ctx = hip.Context(load("n26"), twist=(1, 1))
+x = np.zeros((2, 26, 2))
+ctx.eval(x)
+fail("launch:k_final", 1)
+g2 = np.full(2, 3.5)
+try:
+    ctx.eval(x, grad2_in=g2)
+    raise SystemExit("no error")
+except hip.QmcError as e:
+    assert e.code == abi.QMC_ERR_HIP
+assert (g2 == 3.5).all()
+stub.stub_clear()
+ctx.eval(x)
+assert sum("k_stage" in k for k in log("launch")) == 2
+""")
