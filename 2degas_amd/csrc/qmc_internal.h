@@ -12,6 +12,7 @@
 extern thread_local std::string g_last_error;
 
 inline int hip_fail(hipError_t e, const char* what) {
+  (void)hipGetLastError();  // reported here: not the next call's
   char buf[256];
   snprintf(buf, sizeof buf, "%s: %s", what, hipGetErrorString(e));
   g_last_error = buf;

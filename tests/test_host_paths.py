@@ -148,3 +148,39 @@ stub.stub_clear()
 ctx.eval(x)
 assert sum("k_stage" in k for k in log("launch")) == 2
 """)
+
+
+def test_set_twist_that_fails_changes_nothing(run_host):
+    """A list that cannot be stored, on the device or on the host, leaves the
+    context with the one it had (its orbitals read that, not freed memory), and
+    the error it returned is not reported again by the next call."""
+    run_host(r"""
+import resource
+ctx = hip.Context(load("n26g"), twist=(1, 1))
+old, x = ctx.gvec.copy(), np.zeros((1, 26, 2))
+real = lambda: any("k_gjr" in k for k in log("launch"))
+other = old.copy()
+other[5] = 1.25 * other[5]  # its opposite is another wave: complex orbitals
+for name in ("hipMalloc", "hipMemcpy"):
+    stub.stub_clear()
+    fail(name, 1)
+    assert L.qmc_set_twist(ctx.h, abi.dptr(other), len(other)) == abi.QMC_ERR_HIP
+    given = log("malloc")
+    assert sorted(log("free")) == sorted(given), log()  # what was allocated, and nothing else
+    ctx.eval(x)
+    assert real()
+soft, hard = resource.getrlimit(resource.RLIMIT_AS)
+resource.setrlimit(resource.RLIMIT_AS, (8 << 30, hard))
+stub.stub_clear()
+assert L.qmc_set_twist(ctx.h, abi.dptr(other), 1 << 29) == abi.QMC_ERR_HIP
+resource.setrlimit(resource.RLIMIT_AS, (soft, hard))
+assert not log("free")
+ctx.eval(x)
+assert real()
+stub.stub_clear()
+ctx.set_twist(other)
+assert len(log("free")) == 1
+stub.stub_clear()
+ctx.eval(x)
+assert not real()
+""")
