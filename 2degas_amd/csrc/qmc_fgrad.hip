@@ -97,7 +97,7 @@ __global__ __launch_bounds__((PairShape<false, P>::T), 4) void k_fgrad(DevSys s,
   // ALL: every determinant couples to every type
   auto run = [&](auto allc) {
     constexpr bool ALL = decltype(allc)::value;
-    pair_run<false, P>(
+    pair_run<S, P>(
         s, wv, l,
         [&](const TpInfo* T, int i, int j) {
           const TabRef tb{T->row[TK_B], T->ng[TK_B]};
@@ -248,7 +248,7 @@ void launch_fgrad(const DevSys& s, const WsLayout& L, int nw, const double* x, d
       constexpr bool R = decltype(real)::value, O = decltype(one)::value;
       hipLaunchKernelGGL((k_fgrad<R, O, P>), dim3(nw), dim3(T), (FgShape<R, O, P>::lds(s.nptot)), st, s, L, x, ws);
     };
-    const bool one = s.ntypes == 1 || s.np[0] == 0 || s.np[1] == 0;
+    const bool one = pair_one(s);
     if (s.real_orb && one) go(std::true_type{}, std::true_type{});
     else if (s.real_orb) go(std::true_type{}, std::false_type{});
     else if (one) go(std::false_type{}, std::true_type{});

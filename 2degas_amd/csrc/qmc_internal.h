@@ -113,9 +113,9 @@ void launch_fgrad(const DevSys& s, const WsLayout& L, int nw, const double* x, d
 void launch_cross(const DevSys& s, const WsLayout& L, int nw, bool real, const double* x, double* ws,
                   const double* F, hipStream_t st);
 // The pair kernel (qmc_kernels.hip): its LDS for kc particles per phase chunk,
-// the doubles of its FP64 phase rows, and its launch.
+// the FP64 chunk for a system, and its launch.
 size_t pairs_lds(const DevSys& s, int kc, bool mix);
-size_t rho_doubles(const DevSys& s, int kc);
+int pairs_chunk(const DevSys& s);
 void launch_pairs(const DevSys& s, const WsLayout& L, int nw, bool mix, size_t lds, const double* x, double* ws,
                   double* props, hipStream_t st);
 // The real-orbital determinant kernels of every spin (s.real_orb); value:

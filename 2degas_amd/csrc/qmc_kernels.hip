@@ -34,21 +34,23 @@
 // ---------------------------------------------------------------------------
 // k_pairs
 // LDS: xs[2N], Gs[2N], red[8 NW], then a region shared by the partial sums of
-// the pair passes (NA x 6 x 2P doubles) and, afterwards, the phase steps (4N) and
+// the pair passes (NA x 6 x NS doubles) and, afterwards, the phase steps (4N) and
 // phases of rho_k.
 //
 // The pair passes run on the schedule of qmc_pairs.h.
 //
 // What bounds it: a step is a chain of some 1500 cycles (geometry, table
 // loads, spline, LDS sums), so short runs count where few walkers are in
-// flight, and occupancy where many are.  Measured, 8 wavefronts against 4:
-// N=74, 256 walkers 42 us (75 before the blocks of P lanes, with 4); N=58, 256
-// walkers 26 against 31 us, 8192 walkers 326 against 260; N=122, 4096 walkers
-// 500 against 528.  16 wavefronts: 701 us there.  The mixed kernel's FP32
-// phases need more registers, and 4 wavefronts are the better count at both
-// ends (N=122 413 against 554 us, N=58 at 8192 walkers 276 against 445).  The
-// count depends on the deck alone, not on the batch, so that a walker's result
-// does not depend on the batch it is in.
+// flight, and occupancy where many are.  8 wavefronts against 4 (200 shells of
+// k-vectors): N=58, 1 walker 26 against 38 us, 256 walkers 30 against 40, 1024
+// walkers 70 against 66, 8192 walkers 428 against 391; N=122, 4096 walkers 500
+// against 528 (16 wavefronts: 701).  The count depends on the deck alone, not on
+// the batch, so that a walker's result does not depend on the batch it is in;
+// between the two ends it favours the small batch, which a served job's steps
+// and a reptation move evaluate and where the kernel is the longest of the call
+// (10 of 73 us at N=58, 256 walkers, against 37 of 876 at 8192).  The mixed
+// kernel's FP32 phases need more registers, and 4 wavefronts are the better count
+// at both ends (N=122 413 against 554 us, N=58 at 8192 walkers 276 against 445).
 #define PP_NQ 6  // per-particle sums of a pass
 
 // part[q * NS + p] += v for the lane group's partial sums
@@ -61,9 +63,8 @@ __device__ __forceinline__ void pp_add(double* part, int p, const double (&v)[PP
 
 // The NA partial sums of each of the nq per-particle sums, added in order
 // into the first one.
-template <bool MIX, int P>
+template <class S>
 __device__ __forceinline__ void pp_reduce(double* parts, int nq, int tid) {
-  using S = PairShape<MIX, P>;
   __syncthreads();
   for (int e = tid; e < nq * S::NS; e += S::T) {
     double v = parts[e];
@@ -106,23 +107,25 @@ __device__ __forceinline__ void kspace_terms(const DevSys& s, int k, double c0, 
 // A task is one 16 x 16 tile of (a, b) of one type, 4 accumulators on one
 // wavefront; the phases of kchunk particles of each type at a time go to LDS
 // (row = particle: C_a, S_a, C_b, S_b), an operand being one 8-byte read a
-// lane.  On vector units, one product per k-vector, the same sums read three
+// lane.  A type without particles has no rows and no tasks (it had: k_pairs of 61
+// polarized particles, 4096 walkers, 225 us, now 200).  On vector units, one product per k-vector, the same sums read three
 // 16-byte phases from LDS for each pair of k-vectors and particle and took
 // twice as many operations (both signs of ky separately).
 #define KRUN2 5  // phases of one particle from one sin/cos and the step's products
 typedef double pk_d4 __attribute__((ext_vector_type(4)));
 
-template <int P>
+template <class S>
 __device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restrict__ xs, double* __restrict__ ks,
                                           double* __restrict__ ph, double* __restrict__ pw, int tid) {
-  using S = PairShape<false, P>;
   const int N = s.nptot, lane = tid & 63, lr = lane >> 4, lc = lane & 15;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int na = s.nkax, nb = s.nkby, ta = (na + 15) >> 4, tb = (nb + 15) >> 4;
   const int ox = 16 * ta, oy = 32 * ta, ld = 32 * (ta + tb) + 16;
-  const int nt = s.ntypes > 1 ? 2 : 1, ntask = ta * tb * nt;
+  // the types that have particles: both, or t1 alone
+  constexpr int nt = S::ONE ? 1 : 2;
+  const int t1 = S::ONE && s.ntypes > 1 && s.np[0] == 0 ? 1 : 0, ntask = ta * tb * nt;
   const int kc = (s.kchunk + 3) & ~3;  // rows per type and chunk
-  const int nmax = max(s.np[0], nt > 1 ? s.np[1] : 0);
+  const int nmax = S::ONE ? pick2(s.np, t1) : max(s.np[0], s.np[1]);
   // items of a phase row: runs of KRUN2 phases; the thread's first item
   const int gx = (na + KRUN2 - 1) / KRUN2, ng = gx + (nb + KRUN2 - 1) / KRUN2;
   const int row_0 = tid / ng, g_0 = tid - row_0 * ng, row_d = S::T / ng, g_d = S::T - row_d * ng;
@@ -137,7 +140,8 @@ __device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restr
   for (int t0 = 0; t0 < ntask; t0 += S::NW) {
     const int task = t0 + wv;
     const bool on = task < ntask;
-    const int type = on ? task / (ta * tb) : 0, tile = on ? task % (ta * tb) : 0;
+    const int row_t = on && nt > 1 ? task / (ta * tb) : 0, tile = on ? task - row_t * ta * tb : 0;
+    const int type = S::ONE ? t1 : row_t;
     const int ra = 16 * (tile / tb), rb = 16 * (tile % tb);
     pk_d4 cc{0, 0, 0, 0}, cs{0, 0, 0, 0}, sc{0, 0, 0, 0}, ss{0, 0, 0, 0};
     for (int c0 = 0; c0 < nmax; c0 += kc) {
@@ -150,7 +154,7 @@ __device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restr
           row++;
           if (row >= nt * kc) break;
         }
-        const int t = row >= kc ? 1 : 0, c = c0 + row - t * kc;
+        const int r1 = nt > 1 && row >= kc ? 1 : 0, t = S::ONE ? t1 : r1, c = c0 + row - r1 * kc;
         const int np_t = pick2(s.np, t);
         if (c >= ((np_t + 3) & ~3)) continue;
         const bool isx = g < gx, live = c < np_t;
@@ -188,7 +192,7 @@ __device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restr
       __syncthreads();
       if (on) {
         const int cn = min(kc, pick2(s.np, type) - c0);
-        const double* base = ph + (type * kc + lr) * ld + lc;
+        const double* base = ph + (row_t * kc + lr) * ld + lc;
         for (int k = 0; k < cn; k += 4) {
           const double* row = base + k * ld;
           const double ca = row[ra], sa = row[ox + ra], cb = row[oy + rb], sb = row[oy + 16 * tb + rb];
@@ -226,12 +230,12 @@ __device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restr
 // over each chunk of particles in FP32, the chunk sums added in FP64; the
 // pair geometry, the backflow coordinates, every accumulator and the k-space
 // sum stay FP64.
-template <bool MIX, int P>
+template <bool MIX, int P, bool ONE>
 __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
                                              const double* __restrict__ x,
                                              double* __restrict__ ws,
                                              double* __restrict__ props) {
-  using S = PairShape<MIX, P>;
+  using S = PairShape<MIX, P, ONE>;
   extern __shared__ __attribute__((aligned(16))) double sm[];
   const int w = blockIdx.x;
   if (s.nact && w >= *s.nact) return;
@@ -255,7 +259,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   {
     double ia[PP_NQ] = {0, 0, 0, 0, 0, 0};  // gx, gy, Gx, Gy, qx, qy of particle i
     double hb = 0.0, vb = 0.0;              // the block pair's Laplacian and potential
-    pair_run<MIX, P>(
+    pair_run<S, P>(
         s, wv, l,
         [&](const TpInfo* T, int i, int j) {
           const TabRef tu2{T->row[TK_U2], T->ng[TK_U2]}, tu3{T->row[TK_U3], T->ng[TK_U3]},
@@ -314,7 +318,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
           for (int q = 0; q < PP_NQ; q++) ia[q] = 0.0;
         });
   }
-  pp_reduce<MIX, P>(parts, PP_NQ, tid);
+  pp_reduce<S>(parts, PP_NQ, tid);
   // Gs for pass 2, q out, g kept
   double gpx = 0.0, gpy = 0.0;  // gradient of particle tid (N <= 128)
   if (tid < N) {
@@ -342,7 +346,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
     __syncthreads();
     double ia[PP_NQ] = {0, 0, 0, 0, 0, 0};  // g3x, g3y, e11, e12, e22 of particle i
     double hb = 0.0;
-    pair_run<MIX, P>(
+    pair_run<S, P>(
         s, wv, l,
         [&](const TpInfo* T, int i, int j) {
           const TabRef tu3{T->row[TK_U3], T->ng[TK_U3]};
@@ -377,7 +381,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
 #pragma unroll
           for (int q = 0; q < PP_NQ; q++) ia[q] = 0.0;
         });
-    pp_reduce<MIX, P>(parts, 5, tid);
+    pp_reduce<S>(parts, 5, tid);
     if (tid < N) {
       double v[5];
 #pragma unroll
@@ -407,10 +411,17 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   double* pw = props + (int64_t)w * s.n_props;
   if (!MIX && s.nrhok && s.nkax > 0) {
     __syncthreads();  // Gs and the partial sums have been read
-    rho_tiles<P>(s, xs, parts, parts + 4 * N, pw, tid);
+    rho_tiles<S>(s, xs, parts, parts + 4 * N, pw, tid);
     __syncthreads();  // rho_k of this walker is in memory
-    const double* r0 = s.irhok[0] ? pw + s.jrhok + (s.irhok[0] - 1) * 2 * s.nk : nullptr;
-    const double* r1 = s.ntypes > 1 && s.irhok[1] ? pw + s.jrhok + (s.irhok[1] - 1) * 2 * s.nk : nullptr;
+    double* r0 = s.irhok[0] ? pw + s.jrhok + (s.irhok[0] - 1) * 2 * s.nk : nullptr;
+    double* r1 = s.ntypes > 1 && s.irhok[1] ? pw + s.jrhok + (s.irhok[1] - 1) * 2 * s.nk : nullptr;
+    if constexpr (S::ONE) {
+      // rho_k of a type without particles
+      double*& none = s.np[0] == 0 ? r0 : r1;
+      if (none)
+        for (int k = tid; k < 2 * s.nk; k += S::T) none[k] = 0.0;
+      none = nullptr;
+    }
     for (int k = tid; k < s.nk; k += S::T)
       kspace_terms(s, k, r0 ? r0[2 * k] : 0.0, r0 ? r0[2 * k + 1] : 0.0, r1 ? r1[2 * k] : 0.0,
                    r1 ? r1[2 * k + 1] : 0.0, pk0, pk1, pkt);
@@ -611,11 +622,24 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
 
 // (6 and 5 wavefronts per SIMD fit without spilling vector registers: the pair
 // sums leave for LDS before the phases, whose loops need the registers)
-template <bool MIX, int P>
-__global__ __launch_bounds__((PairShape<MIX, P>::T), MIX ? 5 : 6) void k_pairs(DevSys s, WsLayout L, const double* __restrict__ x,
-                                                              double* __restrict__ ws,
-                                                              double* __restrict__ props) {
-  k_pairs_body<MIX, P>(s, L, x, ws, props);
+template <bool MIX, int P, bool ONE>
+__global__ __launch_bounds__((PairShape<MIX, P, ONE>::T), MIX ? 5 : 6) void k_pairs(DevSys s, WsLayout L,
+                                                                                   const double* __restrict__ x,
+                                                                                   double* __restrict__ ws,
+                                                                                   double* __restrict__ props) {
+  k_pairs_body<MIX, P, ONE>(s, L, x, ws, props);
+}
+
+// f(integral_constant P, bool_constant ONE) for the system's pair kernel.
+template <class F>
+static auto with_pairs(const DevSys& s, F&& f) {
+  return with_lanes(s, [&](auto p) { return pair_one(s) ? f(p, std::true_type{}) : f(p, std::false_type{}); });
+}
+
+// Doubles of the FP64 phase rows of kc particles of each type that has any.
+static size_t rho_doubles(const DevSys& s, int kc) {
+  const size_t ld = 32 * (size_t)((s.nkax + 15) / 16 + (s.nkby + 15) / 16) + 16;
+  return (pair_one(s) ? 1 : 2) * (size_t)((kc + 3) & ~3) * ld;
 }
 
 // LDS bytes of the pair kernels with kc particles per phase chunk (0: no
@@ -623,8 +647,8 @@ __global__ __launch_bounds__((PairShape<MIX, P>::T), MIX ? 5 : 6) void k_pairs(D
 size_t pairs_lds(const DevSys& s, int kc, bool mix) {
   const size_t N = s.nptot;
   auto sums = [&](auto m) {
-    return with_lanes(s, [&](auto p) {
-      using S = PairShape<decltype(m)::value, decltype(p)::value>;
+    return with_pairs(s, [&](auto p, auto one) {
+      using S = PairShape<decltype(m)::value, decltype(p)::value, decltype(one)::value>;
       return std::pair<size_t, size_t>(8 * S::NW, (size_t)S::NA * S::PART);
     });
   };
@@ -638,21 +662,35 @@ size_t pairs_lds(const DevSys& s, int kc, bool mix) {
   return sizeof(double) * (4 * N + red) + region;
 }
 
-// Doubles of the FP64 phase rows of kc particles of each type.
-size_t rho_doubles(const DevSys& s, int kc) {
-  const size_t ld = 32 * (size_t)((s.nkax + 15) / 16 + (s.nkby + 15) / 16) + 16;
-  return (s.ntypes > 1 ? 2 : 1) * (size_t)((kc + 3) & ~3) * ld;
+// Particles of each type per FP64 phase chunk: at most 32, and as many as fit
+// where two types' partial sums do.  (A CU holds as many blocks with that LDS as
+// the registers allow.  One type's sums are half of that: rows that fit there,
+// 16 at N = 61 and 900 k-vectors, take 204 us for 4096 walkers, 32 rows 199 and
+// all 64, with two blocks per CU, 235.)  As many chunks as that takes, of equal
+// size.
+int pairs_chunk(const DevSys& s) {
+  const size_t room = with_lanes(s, [&](auto p) {
+    using S = PairShape<false, decltype(p)::value>;
+    return sizeof(double) * ((size_t)S::NA * S::PART - 4 * s.nptot);
+  });
+  int kc = 32;
+  while (kc > 4 && sizeof(double) * rho_doubles(s, kc) > room) kc -= 4;
+  const int most = std::max(s.np[0], s.np[1]), n = (most + kc - 1) / kc;
+  return std::max(4, ((most + n - 1) / n + 3) & ~3);
 }
 
 // Queue the pair kernel of nw walkers on st.
 void launch_pairs(const DevSys& s, const WsLayout& L, int nw, bool mix, size_t lds, const double* x, double* ws,
                   double* props, hipStream_t st) {
-  with_lanes(s, [&](auto p) {
+  with_pairs(s, [&](auto p, auto one) {
     constexpr int P = decltype(p)::value;
-    if (mix)
-      hipLaunchKernelGGL((k_pairs<true, P>), dim3(nw), dim3(PairShape<true, P>::T), lds, st, s, L, x, ws, props);
-    else
-      hipLaunchKernelGGL((k_pairs<false, P>), dim3(nw), dim3(PairShape<false, P>::T), lds, st, s, L, x, ws, props);
+    constexpr bool O = decltype(one)::value;
+    auto go = [&](auto m) {
+      constexpr bool M = decltype(m)::value;
+      hipLaunchKernelGGL((k_pairs<M, P, O>), dim3(nw), dim3(PairShape<M, P, O>::T), lds, st, s, L, x, ws, props);
+    };
+    if (mix) go(std::true_type{});
+    else go(std::false_type{});
   });
 }
 

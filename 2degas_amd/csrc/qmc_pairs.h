@@ -20,21 +20,22 @@
 // the lane group's own partial sums in LDS (distinct j within a step, so no
 // two lanes touch one address), and the NA = NW 64 / P partial sums are added
 // in a fixed order afterwards: the result does not depend on scheduling.
-template <bool MIX, int P>
+// ONE: particles of one type alone, whose sums take half the LDS.
+template <bool MIX, int P, bool ONE_ = false>
 struct PairShape {
+  static constexpr bool ONE = ONE_;
   static constexpr int NW = P == 16 || MIX ? 4 : 8;  // wavefronts
   static constexpr int T = 64 * NW, SUB = 64 / P, NA = NW * SUB;
   static constexpr int OWN = P / 2 / SUB, ACROSS = P / SUB;  // wavefront steps of a block pair
-  static constexpr int NS = 2 * P;  // particles a sum's row holds
+  static constexpr int NS = ONE ? P : 2 * P;  // particles a sum's row holds
   static constexpr int PART = 6 * NS;  // doubles of one group's partial sums (k_pairs)
 };
 
 // The wavefront's run of pair steps: pair(T, i, j) for each of its lanes'
 // pairs, block(ti, tj) after each block pair's, end(ti) when the run leaves
 // block ti.
-template <bool MIX, int P, class Pair, class Block, class End>
+template <class S, int P, class Pair, class Block, class End>
 __device__ __forceinline__ void pair_run(const DevSys& s, int wv, int l, Pair&& pair, Block&& block, End&& end) {
-  using S = PairShape<MIX, P>;
   const int lp = l & (P - 1), sub = l / P;
   // schedule: both types present, or the one type t1
   const bool two = s.ntypes > 1 && s.np[0] > 0 && s.np[1] > 0;
@@ -67,6 +68,9 @@ static inline int pair_lanes(const DevSys& s) {
   const int m = s.np[0] > s.np[1] ? s.np[0] : s.np[1];
   return m <= 16 ? 16 : m <= 32 ? 32 : 64;
 }
+
+// Whether all particles are of one type.
+static inline bool pair_one(const DevSys& s) { return s.ntypes == 1 || s.np[0] == 0 || s.np[1] == 0; }
 
 // f(integral_constant P) for the system's lanes per block.
 template <class F>

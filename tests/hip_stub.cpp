@@ -3,8 +3,9 @@
 // host code run without a GPU, and calls fail where a test asks for it.
 //   stub_fail(name, n)    from now on the n-th call of that name fails (0: none);
 //                         "launch:<part of a kernel's name>" for launches
-//   stub_log(), stub_clear()   one line per launch ("launch <kernel>"),
-//                         asynchronous copy, allocation and release
+//   stub_log(), stub_clear()   one line per launch ("launch <kernel>", and "lds
+//                         <bytes> <kernel>"), asynchronous copy, allocation
+//                         and release
 #define __HIP_PLATFORM_AMD__
 #include <hip/hip_runtime_api.h>
 
@@ -66,7 +67,7 @@ STUB hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, 
   *st = g_call.st;
   return hipSuccess;
 }
-STUB hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_t) {
+STUB hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t lds, hipStream_t) {
   const std::string& k = g_kernels[f];
   for (auto& e : g_fail)
     if (e.first.compare(0, 7, "launch:") == 0 && k.find(e.first.substr(7)) != std::string::npos &&
@@ -75,6 +76,7 @@ STUB hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipSt
       return hipErrorLaunchFailure;
     }
   note("launch", k);
+  note("lds", std::to_string(lds) + " " + k);
   return hipSuccess;
 }
 STUB hipError_t hipGetLastError() {

@@ -184,3 +184,18 @@ stub.stub_clear()
 ctx.eval(x)
 assert not real()
 """)
+
+
+def test_an_empty_type_takes_no_lds(run_host):
+    """The pair kernel's sums and phase rows are those of the types that have
+    particles: 61 of one type take less than 61 + 61."""
+    run_host(r"""
+lds = {}
+for name in ("g61p", "g122"):
+    d = load(name)
+    ctx = hip.Context(d, twist=(1, 1))
+    stub.stub_clear()
+    ctx.eval(np.zeros((1, d.nptot, 2)))
+    lds[name], = [int(e.split()[0]) for e in log("lds") if "k_pairs" in e]
+assert lds["g61p"] < 0.85 * lds["g122"], lds
+""")
