@@ -472,14 +472,16 @@ int qmc_timing_read(qmc_ctx* ctx, double* ms, int* nlaunch);
 /*
  * Autotuner of the pair kernels' phase chunk (no counterpart in the
  * reference): times full evaluations of nw synthetic configurations
- * (uniform in the box) on `stream` for the size-based default chunk and
- * chunks of 1, 2, 4, ... 32 particles (those whose LDS fits in 64 KB), for
+ * (uniform in the box) on `stream` for the current chunk and chunks of 1, 2,
+ * 4, ... 32 particles (FP64: 4, 8, ... 32 of each type, rows come in fours;
+ * up to the particles there are and those whose LDS fits in 64 KB), for
  * the FP64 and the mixed-precision
  * pair kernel, and keeps the fastest for the context.  kchunk_out[2] and
  * ms_out[2] (optional) receive the chosen chunks and their ms per
  * evaluation.  Different chunks add the rho_k phases in a different order
- * (rounding only).  Decks whose k-vectors do not factor into distinct
- * components have nothing to tune (kchunk_out 1).
+ * (rounding only).  A precision for which the deck's k-vectors do not factor
+ * into few distinct components has nothing to tune (its one form is timed;
+ * without either factored form nothing is, and kchunk_out is 1).
  */
 int qmc_autotune(qmc_ctx* ctx, int nw, int32_t* kchunk_out, double* ms_out, void* stream);
 

@@ -146,3 +146,17 @@ STUB hipError_t hipStreamDestroy(hipStream_t s) {
   return hipSuccess;
 }
 STUB hipError_t hipStreamSynchronize(hipStream_t) { return done("hipStreamSynchronize"); }
+STUB hipError_t hipEventCreate(hipEvent_t* e) {
+  *e = (hipEvent_t)calloc(1, 8);
+  return hipSuccess;
+}
+STUB hipError_t hipEventDestroy(hipEvent_t e) {
+  free(e);
+  return hipSuccess;
+}
+STUB hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+STUB hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+STUB hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+  *ms = 3.0f;
+  return hipSuccess;
+}
