@@ -107,6 +107,7 @@ class Context:
 
     def __init__(self, deck, twist=(1, 1), gvec=None, device=0):
         self.deck = deck
+        self.tiles = {}  # (precision, rows): threads per row set for single-electron moves
         s, keep = deck.pack()
         h = C.c_void_p()
         rc = lib().qmc_ctx_create(C.byref(s), device, C.byref(h))
@@ -341,6 +342,26 @@ def backflow_zero(deck):
     return True
 
 
+def real_orbitals(gvec, counts):
+    """True when every spin's plane waves (the first of gvec) come with their
+    opposites, as the library finds it: its FP64 single-electron moves then keep
+    real rows, which have one tile."""
+    for m in counts:
+        if m > len(gvec):
+            return False
+        open_, zero = [], 0
+        for gx, gy in np.asarray(gvec, dtype=np.float64)[:m]:
+            if gx == 0.0 and gy == 0.0:
+                zero += 1
+            elif (-gx, -gy) in open_:
+                open_.remove((-gx, -gy))
+            else:
+                open_.append((gx, gy))
+        if open_ or zero > 1:
+            return False
+    return True
+
+
 class SingleMoves:
     """Single-electron moves over a Walkers set (qmc_sem_state): the inverse
     Slater matrices ([nw][2][mm][mm] complex, float64 or, with
@@ -422,6 +443,7 @@ class SingleMoves:
         rc = lib().qmc_sem_set_tile(self.wk.ctx.h, self.precision, int(rows), int(threads_per_row))
         if rc:
             raise QmcError(rc, "qmc_sem_set_tile")
+        self.wk.ctx.tiles[self.precision, int(rows)] = int(threads_per_row)
 
     def tune_tile(self, sigma, sweeps=3):
         """Autotune the move kernel's tile: for the row classes of this
@@ -429,7 +451,10 @@ class SingleMoves:
         4 threads per row on a copy of the walkers (the walkers themselves
         do not move) and keep the faster.  Returns {threads: ms per sweep}
         and the choice (None when every spin is in the 16-row class, which
-        has one shape)."""
+        has one shape).  FP64 inverses of real orbitals have one shape too,
+        whatever the tile: it is timed once, both entries hold its time, and
+        the tile in force, which other orbitals would use, stays and is
+        returned."""
         import torch
         d = self.wk.ctx.deck
         rows = sorted({16 if m <= 16 else 32 if m <= 32 else 64 for m in d.np[:d.ntypes] if m > 0} - {16})
@@ -439,10 +464,8 @@ class SingleMoves:
         wk.start()
         sm = SingleMoves(wk, precision=self.precision)
         ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
-        times = {}
-        for cg in (2, 4):
-            for r in rows:
-                sm.set_tile(r, cg)
+
+        def time_sweeps():
             sm.refresh()
             sm.sweep(sigma)
             torch.cuda.synchronize()
@@ -451,7 +474,16 @@ class SingleMoves:
                 sm.sweep(sigma)
             ev[1].record()
             torch.cuda.synchronize()
-            times[cg] = ev[0].elapsed_time(ev[1]) / sweeps
+            return ev[0].elapsed_time(ev[1]) / sweeps
+
+        if self.precision == abi.QMC_PREC_FP64 and real_orbitals(self.wk.ctx.gvec, d.np[:d.ntypes]):
+            ms = time_sweeps()
+            return {2: ms, 4: ms}, self.wk.ctx.tiles.get((self.precision, rows[-1]), 2 if rows[-1] == 32 else 4)
+        times = {}
+        for cg in (2, 4):
+            for r in rows:
+                sm.set_tile(r, cg)
+            times[cg] = time_sweeps()
         best = min(times, key=times.get)
         for r in rows:
             self.set_tile(r, best)

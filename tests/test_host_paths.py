@@ -224,3 +224,36 @@ else:
 assert nmix == 4 * 6, nmix  # 26 particles: the default, 1, 2, 4, 8, 16
 assert (ms > 0).all()
 """)
+
+
+def test_binding_knows_real_orbitals(run_host):
+    """real_orbitals says what the library does with a list: which determinant
+    kernel an evaluation launches."""
+    run_host(r"""
+d = load("n26g")
+ctx = hip.Context(d, twist=(1, 1))
+base, x = ctx.gvec.copy(), np.zeros((1, 26, 2))
+neg0 = base.copy()
+neg0[neg0 == 0.0] = -0.0
+shuffled = base.copy()
+shuffled[:13] = base[np.random.default_rng(3).permutation(13)]
+lone = base.copy()
+lone[12] = base[20]
+two_zeros = base.copy()
+two_zeros[1:3] = 0.0
+twice = base.copy()
+twice[3:5] = base[1:3]
+twisted = base + 0.1
+seen = set()
+for name, g in dict(base=base, neg0=neg0, shuffled=shuffled, lone=lone, two_zeros=two_zeros, twice=twice,
+                    twisted=twisted).items():
+    ctx.set_twist(g)
+    stub.stub_clear()
+    ctx.eval(x)
+    real = any("k_gjr" in k for k in log("launch"))
+    assert real != any("k_gjc" in k for k in log("launch"))
+    assert hip.real_orbitals(ctx.gvec, d.np[:d.ntypes]) == real, name
+    seen.add(real)
+assert seen == {True, False}
+assert not hip.real_orbitals(base[:12], [13, 13])
+""")
