@@ -545,11 +545,20 @@ static int sem_moves_jobs(const qmc_sem_job* jobs, int njobs, int precision, hip
   return QMC_OK;
 }
 
+// The orbitals that a call's kernels read are there.
+static int sem_orbitals(const qmc_ctx* c) {
+  for (int sp = 0; sp < c->s.ntypes; sp++)
+    if (c->s.np[sp] > c->s.ng) return arg_fail("fewer g-vectors than particles of a spin", QMC_ERR_NOTWIST);
+  return QMC_OK;
+}
+
 extern "C" int qmc_sem_refresh(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_state* d, int precision,
                                void* stream) {
   int rc = sem_check(c, w, d, precision);
   if (rc) return rc;
   if (w->nw == 0 || !c->b_zero) return QMC_OK;  // backflow: no inverse is carried
+  rc = sem_orbitals(c);
+  if (rc) return rc;
   HIPCHK(hipSetDevice(c->device));
   const int mm = sem_mm(c);
   if (c->s.real_orb && precision == QMC_PREC_FP64) {
@@ -573,6 +582,8 @@ extern "C" int qmc_sem_moves(qmc_ctx* c, const qmc_walkers* w, const qmc_sem_sta
   if (j0 < 0 || j1 > c->s.nptot || j0 > j1) return arg_fail("electron range out of bounds");
   if (!(sigma > 0.0)) return arg_fail("sigma must be positive");
   if (w->nw == 0 || j0 == j1) return QMC_OK;
+  rc = sem_orbitals(c);
+  if (rc) return rc;
   HIPCHK(hipSetDevice(c->device));
   if (!c->b_zero) return sem_moves_full(c, w, d, j0, j1, sigma, precision, (hipStream_t)stream);
   const qmc_sem_job one = {c, w, d, j0, j1, sigma};
@@ -591,6 +602,8 @@ extern "C" int qmc_sem_moves_packed(const qmc_sem_job* jobs, int njobs, int prec
     if (jb.ctx->device != jobs[0].ctx->device) return arg_fail("packed jobs must share one device");
     if (jb.j0 < 0 || jb.j1 > jb.ctx->s.nptot || jb.j0 > jb.j1) return arg_fail("electron range out of bounds");
     if (!(jb.sigma > 0.0)) return arg_fail("sigma must be positive");
+    rc = jb.w->nw > 0 && jb.j0 < jb.j1 ? sem_orbitals(jb.ctx) : QMC_OK;
+    if (rc) return rc;
   }
   HIPCHK(hipSetDevice(jobs[0].ctx->device));
   return sem_moves_jobs(jobs, njobs, precision, st);

@@ -257,3 +257,41 @@ for name, g in dict(base=base, neg0=neg0, shuffled=shuffled, lone=lone, two_zero
 assert seen == {True, False}
 assert not hip.real_orbitals(base[:12], [13, 13])
 """)
+
+
+@pytest.mark.parametrize("name", ["c26", "n26g"])
+def test_moves_need_the_orbitals(run_host, name):
+    """Single-electron moves of a context whose list holds fewer waves than a spin
+    has particles (or none yet) are refused, with and without backflow, before
+    anything is launched: not read beyond the list."""
+    run_host("name = %r" % name + r"""
+ctx = hip.Context(load(name), twist=(1, 1))
+w, keep = buffers(ctx, 4)
+s = abi.QmcSemState()
+keep2 = [np.zeros(4 * 2 * 13 * 13 * 2), np.zeros(4), np.zeros(4)]
+s.ainv, s.dlogpsi, s.nacc = (a.ctypes.data for a in keep2)
+job = (abi.QmcSemJob * 1)()
+job[0].ctx, job[0].w, job[0].d = ctx.h.value, ctypes.addressof(w), ctypes.addressof(s)
+job[0].j0, job[0].j1, job[0].sigma = 0, 26, 0.5
+refresh = lambda p: L.qmc_sem_refresh(ctx.h, ctypes.byref(w), ctypes.byref(s), p, None)
+moves = lambda p: L.qmc_sem_moves(ctx.h, ctypes.byref(w), ctypes.byref(s), 0, 26, 0.5, p, None)
+packed = lambda p: L.qmc_sem_moves_packed(job, 1, p, None)
+full = ctx.gvec.copy()
+for waves in (0, 5, 12):
+    ctx.set_twist(full[:waves])
+    for call in (refresh, moves, packed):
+        for prec in (0, 1):
+            stub.stub_clear()
+            # (with backflow a refresh does nothing, and jobs are not packed)
+            want = abi.QMC_ERR_NOTWIST
+            if name == "n26g":
+                want = {refresh: abi.QMC_OK, packed: abi.QMC_ERR_ARG}.get(call, want)
+            assert call(prec) == want, (waves, prec)
+            assert not log("launch"), log()
+    # nothing to move, nothing to read
+    w.nw = 0
+    assert refresh(0) == 0 and moves(0) == 0
+    w.nw = 4
+ctx.set_twist(full[:13])
+assert refresh(0) == 0 and moves(0) == 0 and log("launch")
+""")
