@@ -203,11 +203,11 @@ __device__ __forceinline__ void xc_entry(const DevSys& s, const double* __restri
 // Destination of the L2 prefetch of F: one wavefront's 64 x 16 bytes, never read.
 __shared__ __attribute__((aligned(16))) unsigned xc_sink[256];
 
-// Per-wavefront body for tile group (G, H).  The V chunks (16 particles of
-// one type at a time, over the types with backflow to this spin) are
-// double-buffered: while the matrix cores take this chunk's products the
-// vector units build the next chunk into the other buffer (two entries per
-// thread, placed between the MFMA steps), so a chunk costs one barrier.
+// Body of wavefront V.  The V_t chunks (KC / 2 particles of one type at a time,
+// over the types with backflow to this spin) are double-buffered: while the
+// matrix cores take this chunk's products the vector units build the next chunk
+// into the other buffer (EPT entries per thread, one or two, placed between the
+// MFMA steps), so a chunk costs one barrier.
 template <int NB, int V, typename Z>
 __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ dsc, const double* __restrict__ Qd,
                                         const Z* __restrict__ Fg, const double* __restrict__ xs,

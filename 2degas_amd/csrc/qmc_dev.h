@@ -366,8 +366,6 @@ __device__ __forceinline__ double gj_readlane(double v, int l) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Block-wide sum of a double over QMC_BLOCK threads; red must hold
-// QMC_BLOCK/64 doubles.  All threads get the result.
 // v of the lane a DPP control names (every lane of the row active).
 template <int CTRL>
 __device__ __forceinline__ double dpp_f64(double v) {
@@ -387,7 +385,8 @@ __device__ __forceinline__ double wave_sum(double v) {
   v += dpp_f64<0x128>(v);
   return (gj_readlane(v, 0) + gj_readlane(v, 16)) + (gj_readlane(v, 32) + gj_readlane(v, 48));
 }
-// Sum over a workgroup of NT threads (red holds NT / 64 doubles).
+// Sum over a workgroup of NT threads (red holds NT / 64 doubles); all threads
+// get the result.
 template <int NT = QMC_BLOCK>
 __device__ __forceinline__ double block_sum(double v, double* red) {
   v = wave_sum(v);

@@ -9,7 +9,7 @@
 // imaginary accumulators (a complex product is four real MFMAs); blocks of 4
 // columns, one barrier each; row p_k of the two right parts ends as piv_k
 // F_b(k, .).  Pivot choice is zgefa's (largest |re|+|im| among the rows not yet
-// used, reptation.f:9286-9298; rows whose magnitudes agree to 13 bits may be
+// used, reptation.f:9286-9298; rows whose magnitudes agree to 14 bits may be
 // taken in another order, which changes rounding only).
 //
 // What bounds it: at 64 particles the matrix cores (2700 products per walker) and

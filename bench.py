@@ -444,7 +444,7 @@ def bench_dmc(args, hip, deck, dg):
     """DMC steps/s (a move of every walker, its weight, the weighted block
     sums, the branching and the copies: qmc_dmc_sweep with mmstep 1) on the
     N=122 workload with 4096 walkers and on the plain N=26 one with 256,
-    and the time of the branching alone (one thread over the walkers)."""
+    and the time of the branching alone (one block over the walkers)."""
     import numpy as np
     import torch
     abi = importlib.import_module("2degas_amd.abi")
@@ -636,7 +636,7 @@ def bench_sem(args, hip, deck, dg):
         ctx.close()
     # packing: 16 small jobs (N 26, 42, 58, 74, four each; 256 walkers; u2
     # only, zero backflow), one sweep each as separate calls on one stream
-    # against one packed call per spin and row class
+    # against one packed call
     jobs = []
     for k in range(16):
         nu = (13, 21, 29, 37)[k % 4]

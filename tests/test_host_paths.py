@@ -202,9 +202,9 @@ assert lds["g61p"] < 0.85 * lds["g122"], lds
 
 
 @pytest.mark.parametrize("grid", [True, False])
-def test_autotune_times_each_form_once(run_host, grid):
+def test_autotune_times_the_forms_there_are(run_host, grid):
     """FP64 phase rows come in fours of one type's particles: the autotuner times
-    every such chunk once and names the one it keeps; a k list off the grid (a
+    every such chunk, no form under two names, each in two rounds, and names the one it keeps; a k list off the grid (a
     k-vector five times over) has one FP64 form."""
     run_host("grid = %r" % grid + r"""
 d = load("n26g")
@@ -217,11 +217,11 @@ stub.stub_clear()
 assert L.qmc_autotune(ctx.h, 8, abi.iptr(kc), abi.dptr(ms), None) == 0
 n64, nmix = (sum("k_pairsILb%d" % b in k for k in log("launch")) for b in (0, 1))
 if grid:
-    assert n64 == 4 * 3, n64  # 13 particles of a type: 16, 4, 8
+    assert n64 == 2 * 4 * 3, n64  # 13 particles of a type: 16, 4, 8
     assert kc[0] == 16
 else:
-    assert n64 == 4 and kc[0] == 1, (n64, kc)
-assert nmix == 4 * 6, nmix  # 26 particles: the default, 1, 2, 4, 8, 16
+    assert n64 == 2 * 4 and kc[0] == 1, (n64, kc)
+assert nmix == 2 * 4 * 6, nmix  # 26 particles: the default, 1, 2, 4, 8, 16
 assert (ms > 0).all()
 """)
 
