@@ -233,7 +233,7 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
     const TabRef tb = tabref<TK_B>(s, tpair(sp, ft));
     for (int e = tid; e < S::JR * (XC_KC / 2); e += XC_THREADS) xc_entry<NB>(s, Qd, xs, Vt, tb, e, c0, cn, m, p0);
   }
-  __syncthreads();
+  block_sync();
   int cur = 0;
 #pragma unroll
   for (int t = 0; t < 2; t++) {
@@ -285,13 +285,13 @@ __device__ __forceinline__ void xc_body(const DevSys& s, double* __restrict__ ds
         // the next step's operands are read after this step's MFMAs issue
         __asm__ volatile("" ::: "memory");
       }
-      __syncthreads();
+      block_sync();
       cur ^= 1;
     }
   }
   // the chunk buffers are free: the diagonal blocks go there
   xc_diag_blocks<NB, V>(acc, Vt, lane);
-  __syncthreads();
+  block_sync();
   double u0, u1;
   xc_contract<NB, V>(acc, Vt, Fg, m, lane, nT, u0, u1);
   u0 = block_sum<XC_THREADS>(u0, red);
@@ -330,7 +330,7 @@ __global__ __launch_bounds__(XcShape<NB>::T, 4) void k_cross(DevSys s, WsLayout 
   double* Vt = sm + 2 * N;
   const double* xw = x + (int64_t)w * 2 * N;
   for (int k = tid; k < 2 * N; k += 64 * W) xs[k] = xw[k];
-  __syncthreads();
+  block_sync();
 #define XC_CASE(v)                                                                              \
   case v:                                                                                       \
     if constexpr (v < W) xc_body<NB, v>(s, dsc, Qd, Fg, xs, Vt, red, sp, m, p0, tid);           \

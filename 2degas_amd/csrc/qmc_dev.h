@@ -211,6 +211,20 @@ __device__ __forceinline__ uint64_t lcg_pow10(uint32_t n) {
   return p;
 }
 
+// Barrier of the workgroup.  The wait for the wavefront's own LDS operations
+// (lgkmcnt 0, the other counters at their largest) is written out: the one that
+// __syncthreads() stands for is dropped by the compiler (ROCm 7.2) at a barrier
+// that heads a loop when nothing is outstanding on the way into the loop,
+// whatever its back edge brings, and other wavefronts then read LDS that this
+// one's writes have not reached (one of some 3e7 inverses of 29 orbitals came
+// out wrong).
+__device__ __forceinline__ void block_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 enum { TK_U2 = 0, TK_U3 = 1, TK_B = 2, TK_V = 3 };
 
 // Element i of a 2- or 3-entry member array without a dynamic index (a
@@ -391,9 +405,9 @@ template <int NT = QMC_BLOCK>
 __device__ __forceinline__ double block_sum(double v, double* red) {
   v = wave_sum(v);
   int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  __syncthreads();
+  block_sync();
   if (l == 0) red[w] = v;
-  __syncthreads();
+  block_sync();
   double t = 0.0;
 #pragma unroll
   for (int k = 0; k < NT / 64; k++) t += red[k];

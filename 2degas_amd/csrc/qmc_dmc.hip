@@ -82,16 +82,16 @@ __device__ __forceinline__ void dmc_in_order(const double* v, int nw, F&& f) {
 // total of a.
 __device__ __forceinline__ void dmc_scan(int tid, int* pa, int* pb, int& a, int& b, int& ta) {
   const int a0 = a, b0 = b;
-  __syncthreads();
+  block_sync();
   pa[tid] = a;
   pb[tid] = b;
-  __syncthreads();
+  block_sync();
   for (int o = 1; o < DMC_BRANCH_THREADS; o <<= 1) {
     const int aa = tid >= o ? pa[tid - o] : 0, ab = tid >= o ? pb[tid - o] : 0;
-    __syncthreads();
+    block_sync();
     pa[tid] += aa;
     pb[tid] += ab;
-    __syncthreads();
+    block_sync();
   }
   a = pa[tid] - a0;
   b = pb[tid] - b0;
@@ -132,13 +132,13 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
     }
     sw[i] = v;
   }
-  __syncthreads();
+  block_sync();
   if (tid == 0) {
     double somma = 0.0;
     dmc_in_order(sw, nw, [&](int, double v) { somma = somma + v; });
     sh.somma = somma;
   }
-  __syncthreads();
+  block_sync();
   // multiplicities: integer parts, and the fractional parts to comb
   // (reptation.f:2189-2195)
   const double somma = sh.somma;
@@ -152,12 +152,12 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
     odd |= !(v >= 0.0 && v < 1.0);
   }
   if (odd) sh.odd = 1;
-  __syncthreads();
+  block_sync();
   // threads' walkers, in order
   const int S = nw <= 4 * DMC_BRANCH_THREADS ? 4 : nw <= 8 * DMC_BRANCH_THREADS ? 8 : 16;
   const int i0 = min(nw, tid * S), i1 = min(nw, i0 + S);
   const bool any_odd = sh.odd;
-  __syncthreads();
+  block_sync();
   if (any_odd) {
     // fractional parts outside [0, 1) (weights below 0 or that are no
     // numbers): the reference's walk as it is, on one thread
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
       dmc_in_order(sw, nw, [&](int, double v) { k0 = k0 + v; });
       sh.draws = lround(k0);
     }
-    __syncthreads();
+    block_sync();
     const long ndraw = sh.draws;
     // k after walker i0 - 1, and before 1 is taken off at walker i0
     double kb = 0.0, t0 = 0.0;
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
       rng2[0] = (int64_t)((lcg_pow((uint32_t)made) * st0) & ((1ULL << 48) - 1ULL));
     }
   }
-  __syncthreads();
+  block_sync();
   // The ranks left with no copy take the extra copies of the others: each
   // transfer from the lowest rank with more than one to the lowest rank with
   // none (reptation.f:2220-2258).  So receiver q (in walker order) takes
@@ -281,7 +281,7 @@ __global__ __launch_bounds__(DMC_BRANCH_THREADS) void k_dmc_branch(int nw, doubl
     E[i] = (double)e;
     e += max(sm[i] - 1, 0);
   }
-  __syncthreads();
+  block_sync();
   for (int i = i0; i < i1; i++) {
     if (sm[i] >= 1) {
       src[i] = i;

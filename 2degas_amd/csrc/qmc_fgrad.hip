@@ -87,7 +87,7 @@ __global__ __launch_bounds__((PairShape<false, P>::T), 4) void k_fgrad(DevSys s,
     }
   }
   for (int k = tid; k < S::NA * G::PART; k += S::T) parts[k] = 0.0;
-  __syncthreads();
+  block_sync();
   bool all = true;
 #pragma unroll
   for (int e = 0; e < 4; e++)
@@ -165,7 +165,7 @@ __global__ __launch_bounds__((PairShape<false, P>::T), 4) void k_fgrad(DevSys s,
   };
   if (all) run(std::true_type{});
   else run(std::false_type{});
-  __syncthreads();
+  block_sync();
   // the groups' partial sums in order, then each particle's own block
   double g2 = 0.0;
   for (int e = tid; e < NQ * NS; e += S::T) {
@@ -174,7 +174,7 @@ __global__ __launch_bounds__((PairShape<false, P>::T), 4) void k_fgrad(DevSys s,
     for (int a = 1; a < S::NA; a++) v += parts[a * G::PART + e];
     parts[e] = v;
   }
-  __syncthreads();
+  block_sync();
   if (tid < N) {
     const int p = tid, t = ptype(s, p);
     double v[NQ];
@@ -222,7 +222,7 @@ __global__ __launch_bounds__((PairShape<false, P>::T), 4) void k_fgrad(DevSys s,
       for (int q = 0; q < 3; q++) red[wv][q] = v[q];
     }
   }
-  __syncthreads();
+  block_sync();
   if (tid == 0) {
     double v[3] = {0.0, 0.0, 0.0};
 #pragma unroll

@@ -119,7 +119,7 @@ __global__ __launch_bounds__(64 * NT, VAL || NT == 1 ? 4 : 2) void k_gjc(DevSys 
     sh.rank[r] = -1;
   }
   if (tid == 0) sh.sing = 0;
-  __syncthreads();
+  block_sync();
   gr_d4 re[NP][NT], im[NP][NT];
   {
     const bool jn = col < m;
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(64 * NT, VAL || NT == 1 ? 4 : 2) void k_gjc(DevSys 
   else if constexpr (S::COPY) copy(C0{}, CN{});
   for (int k0 = 0; k0 < m; k0 += 4) {
     const int buf = (k0 >> 2) & 1, nb = min(4, m - k0);
-    __syncthreads();
+    block_sync();
     int p = 0;
     if constexpr (S::COPY) {
       p = sh.prow[buf][lr];
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(64 * NT, VAL || NT == 1 ? 4 : 2) void k_gjc(DevSys 
       else if constexpr (S::COPY) copy(C0{}, CN{});
     }
   }
-  __syncthreads();
+  block_sync();
   double* dsc = ws + (int64_t)w * L.per_walker + pick2(L.off_det, sp);
   if constexpr (!VAL) {
     // F_b(k, j): row p_k of part b over piv_k; the diagonal also goes to the

@@ -128,7 +128,7 @@ __device__ __forceinline__ void gr_setup(GrShared<NT, NP>& sh, const double* __r
     sh.rank[r] = -1;
   }
   if (tid == 0) sh.sing = 0;
-  __syncthreads();
+  block_sync();
 }
 
 // The wavefront's column tile of R and, with NP = 3, of its two derivatives.
@@ -211,7 +211,7 @@ __device__ __forceinline__ void gr_eliminate(GrShared<NT, NP>& sh, gr_d4 (&acc)[
   else if constexpr (COPY) copy(C0{}, CN{});
   for (int k0 = 0; k0 < m; k0 += 4) {
     const int buf = (k0 >> 2) & 1, nb = min(4, m - k0);
-    __syncthreads();
+    block_sync();
     const bool left = INPLACE || (k0 >> 4) <= ct;  // R's columns here are not all eliminated
     int pb[4];
     double uo[NP], fo[NT];
@@ -272,7 +272,7 @@ __device__ __forceinline__ void gr_eliminate(GrShared<NT, NP>& sh, gr_d4 (&acc)[
       else if constexpr (COPY) copy(C0{}, CN{});
     }
   }
-  __syncthreads();
+  block_sync();
 }
 
 template <int NT, bool VAL>
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(64 * NT, 4) void k_gjr_inverse(DevSys s, int sp0, c
   gr_eliminate<NT, 1, true>(sh, acc, m, wave, lane);
   for (int r = tid; r < 16 * NT; r += 64 * NT)
     if (sh.rank[r] >= 0) gi.pcol[sh.rank[r]] = r;
-  __syncthreads();
+  block_sync();
   if (col < m) {
     const int pc = gi.pcol[col];
 #pragma unroll
@@ -376,7 +376,7 @@ __global__ __launch_bounds__(64 * NT, 4) void k_gjr_inverse(DevSys s, int sp0, c
         if (k >= 0) gi.X[k * GrInverse<NT>::LD + pc] = acc[0][T][v] * sh.pinv[r];
       }
   }
-  __syncthreads();
+  block_sync();
   double2* out = ainv + ((int64_t)w * 2 + sp) * mm * mm;
   const int2* kpm = sp ? s.kpm[1] : s.kpm[0];
   for (int e = tid; e < m * nslot; e += 64 * NT) {

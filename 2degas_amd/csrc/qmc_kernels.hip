@@ -65,14 +65,14 @@ __device__ __forceinline__ void pp_add(double* part, int p, const double (&v)[PP
 // into the first one.
 template <class S>
 __device__ __forceinline__ void pp_reduce(double* parts, int nq, int tid) {
-  __syncthreads();
+  block_sync();
   for (int e = tid; e < nq * S::NS; e += S::T) {
     double v = parts[e];
 #pragma unroll
     for (int a = 1; a < S::NA; a++) v += parts[a * S::PART + e];
     parts[e] = v;
   }
-  __syncthreads();
+  block_sync();
 }
 
 // Ewald sums over the k-vectors that carry coefficients, from the rho_k of a
@@ -145,7 +145,7 @@ __device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restr
     const int ra = 16 * (tile / tb), rb = 16 * (tile % tb);
     pk_d4 cc{0, 0, 0, 0}, cs{0, 0, 0, 0}, sc{0, 0, 0, 0}, ss{0, 0, 0, 0};
     for (int c0 = 0; c0 < nmax; c0 += kc) {
-      __syncthreads();
+      block_sync();
       // rows: type t's particles c0..c0+kc-1 (zero beyond its count, up to a
       // multiple of 4)
       for (int row = row_0, g = g_0; row < nt * kc; row += row_d, g += g_d) {
@@ -189,7 +189,7 @@ __device__ __forceinline__ void rho_tiles(const DevSys& s, const double* __restr
           }
         }
       }
-      __syncthreads();
+      block_sync();
       if (on) {
         const int cn = min(kc, pick2(s.np, type) - c0);
         const double* base = ph + (row_t * kc + lr) * ld + lc;
@@ -251,7 +251,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   const int lp = l & (P - 1);
   for (int k = tid; k < 2 * N; k += S::T) xs[k] = xw[k];
   for (int k = tid; k < S::NA * S::PART; k += S::T) parts[k] = 0.0;
-  __syncthreads();
+  block_sync();
   double* wsw = ws + (int64_t)w * L.per_walker;
   double acc_ltf = 0.0, acc_h0 = 0.0, acc_h1 = 0.0, acc_v0 = 0.0, acc_v1 = 0.0;
 
@@ -334,7 +334,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
     wsw[L.off_q + 2 * p + 1] = xs[2 * p + 1] + v[5];
     acc_ltf -= 0.5 * (v[2] * v[2] + v[3] * v[3]);
   }
-  __syncthreads();
+  block_sync();
 
   // pass 2: three-body contraction (dotg, reptation.f:2928-2979), written per
   // particle i as g_i += sum_k M_ik (G_i - G_k),
@@ -343,7 +343,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   // even in the pair, M dG is odd
   if (s.has_u3) {
     for (int k = tid; k < S::NA * S::PART; k += S::T) parts[k] = 0.0;
-    __syncthreads();
+    block_sync();
     double ia[PP_NQ] = {0, 0, 0, 0, 0, 0};  // g3x, g3y, e11, e12, e22 of particle i
     double hb = 0.0;
     pair_run<S, P>(
@@ -410,9 +410,9 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
   double pk0 = 0.0, pk1 = 0.0, pkt = 0.0;
   double* pw = props + (int64_t)w * s.n_props;
   if (!MIX && s.nrhok && s.nkax > 0) {
-    __syncthreads();  // Gs and the partial sums have been read
+    block_sync();  // Gs and the partial sums have been read
     rho_tiles<S>(s, xs, parts, parts + 4 * N, pw, tid);
-    __syncthreads();  // rho_k of this walker is in memory
+    block_sync();  // rho_k of this walker is in memory
     double* r0 = s.irhok[0] ? pw + s.jrhok + (s.irhok[0] - 1) * 2 * s.nk : nullptr;
     double* r1 = s.ntypes > 1 && s.irhok[1] ? pw + s.jrhok + (s.irhok[1] - 1) * 2 * s.nk : nullptr;
     if constexpr (S::ONE) {
@@ -470,7 +470,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
         const int nv = s.nkxv + s.nkyv;
         for (int c0 = 0; c0 < N; c0 += s.kchunk) {
           const int cn = min(s.kchunk, N - c0);
-          __syncthreads();
+          block_sync();
           if (s.kprog) {
             // runs of KRUN phases: the first directly, the rest by products
             // with e^{i dk x} (at most KRUN - 1 roundings from a direct value)
@@ -506,7 +506,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
               ph[e] = float2{(float)cv, (float)sv};
             }
           }
-          __syncthreads();
+          block_sync();
           // particles of type 0 come first: [0, split) of the chunk, each
           // type a loop of its own
           const int split = s.ntypes > 1 ? min(max(s.ipf[1] - c0, 0), cn) : cn;
@@ -587,7 +587,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
       for (int q = 0; q < 3; q++) red[8 * wv + 5 + q] = v[q];
     }
   }
-  __syncthreads();
+  block_sync();
   if (wv != 0) return;
   // lane q adds sum q of the wavefronts
   double mine = 0.0;
@@ -736,7 +736,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
     A[i * m + k] = z;
     Ag[k * m + i] = z;
   }
-  __syncthreads();
+  block_sync();
 
   // 2. LU with partial pivoting, LINPACK zgefa semantics: pivot = first row
   // of maximal |re|+|im|; rows are swapped only right of the pivot column.
@@ -761,9 +761,9 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
         if (v == 0.0) s_sing = 1;
       }
     }
-    __syncthreads();
+    block_sync();
     if (s_pmax == 0.0) {  // column already triangular (zgefa info = k)
-      __syncthreads();
+      block_sync();
       continue;
     }
     const int l = s_l;
@@ -788,19 +788,19 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
         }
       }
     }
-    __syncthreads();
+    block_sync();
     for (int e = tid; e < nr * nr; e += QMC_BLOCK) {
       const int jj = e / nr, ii = e - jj * nr;
       const int i = k + 1 + ii, j = k + 1 + jj;
       A[j * m + i] = zfma(A[j * m + k], A[k * m + i], A[j * m + i]);
     }
-    __syncthreads();
+    block_sync();
   }
   if (tid == 0) {
     s_piv[m - 1] = m - 1;
     if (cabs1(A[(m - 1) * m + (m - 1)]) == 0.0) s_sing = 1;
   }
-  __syncthreads();
+  block_sync();
   // log|det| = sum log|U_kk| (zgedi det + log, reptation.f:10063, 9412-9430)
   {
     double v = 0.0;
@@ -823,7 +823,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
       else if (e < k) colk[e] = A[k * m + e];
       else colk[e] = A[k * m + k];
     }
-    __syncthreads();
+    block_sync();
     const zd tk = zrcp(colk[k]);
     const int ncol = m - k - 1;
     for (int e = tid; e < (k + 1) * (ncol + 1); e += QMC_BLOCK) {
@@ -837,7 +837,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
         A[j * m + i] = zfma(rowk[j], ci, base);
       }
     }
-    __syncthreads();
+    block_sync();
   }
   // 3b. inverse(U) * inverse(L), right to left, with the column swaps
   zd* work = (zd*)U;
@@ -845,7 +845,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
   for (int k = m - 2; k >= 0; k--) {
     for (int i = tid; i < m; i += QMC_BLOCK)
       if (i > k) work[i] = A[k * m + i];
-    __syncthreads();
+    block_sync();
     {
       const int g = tid >> 6, i = tid & 63;
       zd acc = zmk(0.0, 0.0);
@@ -853,14 +853,14 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
         for (int j = k + 1 + g; j < m; j += 4) acc = zfma(work[j], A[j * m + i], acc);
       if (i < m) part[g * m + i] = acc;
     }
-    __syncthreads();
+    block_sync();
     if (tid < m) {
       const int i = tid;
       zd v = (i <= k) ? A[k * m + i] : zmk(0.0, 0.0);
       for (int g = 0; g < 4; g++) v = zadd(v, part[g * m + i]);
       A[k * m + i] = v;
     }
-    __syncthreads();
+    block_sync();
     const int l = s_piv[k];
     if (l != k) {
       for (int i = tid; i < m; i += QMC_BLOCK) {
@@ -869,7 +869,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
         A[l * m + i] = a;
       }
     }
-    __syncthreads();
+    block_sync();
   }
 
   // 4. F_b = A^-1 diag(i g^b) A (zv, reptation.f:10182-10194), 4x4 tiles;
@@ -886,7 +886,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
     for (int k0 = 0; k0 < m; k0 += kc) {
       const int kn = min(kc, m - k0);
       for (int e = tid; e < kn * m; e += QMC_BLOCK) Ac[e] = Ag[k0 * m + e];
-      __syncthreads();
+      block_sync();
       if (l0 < m && j0 < m) {
         for (int kk = 0; kk < kn; kk++) {
           const int k = k0 + kk;
@@ -908,7 +908,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
             }
         }
       }
-      __syncthreads();
+      block_sync();
     }
     // F = i Q; store and keep the diagonal
     double* dl = U;  // d[j][b] complex: 4 doubles per j
@@ -936,7 +936,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_det(DevSys s, WsLayout L,
   double* xs = U + 4 * m;
   const double* xw = x + (int64_t)w * 2 * N;
   for (int k = tid; k < 2 * N; k += QMC_BLOCK) xs[k] = xw[k];
-  __syncthreads();
+  block_sync();
 
   // 5. drift and the first-derivative Laplacian terms for every particle
   // (reptation.f:10195-10240; the second-derivative ones are k_cross's), with the backflow Jacobian qa and the

@@ -59,7 +59,7 @@ __global__ __launch_bounds__(RMC_SLOT_THREADS) void k_rmc_begin(RmcK k, const in
   __shared__ int cnt[RMC_MAX_MDELTA + 2], base[RMC_MAX_MDELTA + 2], fill[RMC_MAX_MDELTA + 2];
   const int tid = threadIdx.x;
   for (int b = tid; b < RMC_MAX_MDELTA + 2; b += RMC_SLOT_THREADS) cnt[b] = base[b] = fill[b] = 0;
-  __syncthreads();
+  block_sync();
   for (int r = tid; r < k.nr; r += RMC_SLOT_THREADS) {
     uint64_t st = (uint64_t)rng[r];
     const double u1 = rannyu(st);
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(RMC_SLOT_THREADS) void k_rmc_begin(RmcK k, const in
     mv[3 * r + 2] = idir == 1 ? ends[2 * r + 1] : ends[2 * r];
     atomicAdd(&cnt[nd], 1);
   }
-  __syncthreads();
+  block_sync();
   if (tid == 0) {
     int acc = 0;
     for (int b = k.mdelta; b >= 1; b--) {
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(RMC_SLOT_THREADS) void k_rmc_begin(RmcK k, const in
       nact[b - 1] = acc;  // reptiles with ndelta >= b
     }
   }
-  __syncthreads();
+  block_sync();
   for (int r = tid; r < k.nr; r += RMC_SLOT_THREADS) {
     const int b = mv[3 * r + 1];
     slot[r] = base[b] + atomicAdd(&fill[b], 1);
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_rmc_propose(
       for (int q = 0; q < 6; q++) red[q][e >> 6] = v[q];
     }
   }
-  __syncthreads();
+  block_sync();
   if (e < 3) {
     double v[2] = {0.0, 0.0};
 #pragma unroll
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_rmc_step(
     xq[tid] = acc ? x1 : x0;
     gq[tid] = acc ? g1 : g0;
   }
-  __syncthreads();  // every wavefront has read the stream
+  block_sync();  // every wavefront has read the stream
   if (tid == 0) {
     rng[r] = (int64_t)st;
     const double wg = k.delta * k.npnorm * (kinj + kinr);
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_rmc_finish(
     age = rage[r];
     st = (uint64_t)rng[r];
   }
-  __syncthreads();
+  block_sync();
   if (tid == 0) {
     const double m = k.mezzo, h = k.half, o = k.one, on = k.one_nds;
     double wn = (-l4[0] * (1 + 2 * m) - l4[1] * (1 - 2 * m) + l4[2] * (1 + 2 * m) + l4[3] * (1 - 2 * m));
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_rmc_finish(
       tr[3] = age;
     }
   }
-  __syncthreads();
+  block_sync();
   const int acc = s_acc;
 #pragma unroll
   for (int q = 0; q < RS_SLOTS; q++) {
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(64) void k_rmc_links(RmcK k, const double* __restri
       p = fmin(0.0, fmax(-50.0, p));
       pq[k.jacc] = exp(p);
     }
-    __syncthreads();
+    block_sync();
   }
   if (lane == 0) {
     ends[2 * r] = 0;

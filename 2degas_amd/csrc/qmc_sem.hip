@@ -100,7 +100,7 @@ __global__ __launch_bounds__(MR* CG) void k_sem_inverse(DevSys s, int sp, const 
         cbest[wv] = mag;
         cidx[wv] = idx;
       }
-      __syncthreads();
+      block_sync();
       double bm = cbest[0];
       int p = cidx[0];
 #pragma unroll
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(MR* CG) void k_sem_inverse(DevSys s, int sp, const 
         if (cg == 0) rk[p] = c;
       }
       if (tid == 0) pr[c] = p;
-      __syncthreads();
+      block_sync();
 #pragma unroll
       for (int ii = 0; ii < EPT; ii++) {
         const int k = cg + CG * ii;
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(MR* CG) void k_sem_inverse(DevSys s, int sp, const 
       }
     }
   }
-  __syncthreads();
+  block_sync();
   if (l < m) {
     Z* out = ainv + ((int64_t)w * 2 + sp) * mm * mm + (int64_t)rk[l] * mm;
 #pragma unroll
@@ -275,7 +275,7 @@ __device__ __forceinline__ void semf_sum(double (&v)[5], double (*red)[5], int t
 #pragma unroll
     for (int q = 0; q < 5; q++) red[tid >> 6][q] = v[q];
   }
-  __syncthreads();
+  block_sync();
   if (blockDim.x > 64) {
 #pragma unroll
     for (int q = 0; q < 5; q++) v[q] = red[0][q] + red[1][q];
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(8 * QMC_MAX_PARTICLES) void k_semf_init(DevSys s, W
   const int w = blockIdx.x, tid = threadIdx.x, N = s.nptot;
   const int64_t at = (int64_t)w * 2 * N;
   for (int k = tid; k < 2 * N; k += blockDim.x) xs[k] = x[at + k];
-  __syncthreads();
+  block_sync();
   const int a = tid >> 3;
   const bool li = a < N;
   double2 xp = make_double2(0.0, 0.0);
@@ -329,7 +329,7 @@ __global__ __launch_bounds__(8 * QMC_MAX_PARTICLES) void k_semf_init(DevSys s, W
   }
   u = wave_sum(u);
   if ((tid & 63) == 0) red[tid >> 6] = u;
-  __syncthreads();
+  block_sync();
   if (tid == 0) {
     double t = 0.0;
     for (int k = 0; k < (int)blockDim.x / 64; k++) t += red[k];
@@ -377,7 +377,7 @@ __global__ __launch_bounds__(QMC_MAX_PARTICLES) void k_semf_step(
       sing = sing || dsc[DS_SING] != 0.0;
     }
     const bool acc = !sing && ua < exp(-2.0 * (ln - lo));
-    __syncthreads();  // both wavefronts have read what is written below
+    block_sync();  // both wavefronts have read what is written below
     if (acc) {
       U = Un;
       q = qn;

@@ -243,7 +243,7 @@ struct SemWalk {
 
 template <int W>
 __device__ __forceinline__ void sem_sync() {
-  if (W > 1) __syncthreads();
+  if (W > 1) block_sync();
   else sem_wave_sync();
 }
 

@@ -55,7 +55,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_vmc_propose(
     red[0][e >> 6] = s0;
     red[1][e >> 6] = s1;
   }
-  __syncthreads();
+  block_sync();
   if (e == 0) {
     double w0 = 0.0, w1 = 0.0;
     for (int v = 0; v < QMC_BLOCK / 64; v++) {
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(QMC_BLOCK) void k_vmc_accept(
     wgt = dm.wate[w] * peso;
     wsum0 = dm.wsum[w];
   }
-  __syncthreads();  // every wavefront has read what the stores below change
+  block_sync();  // every wavefront has read what the stores below change
   // copy new into old where accepted, set p_old(jacc) = p and add p_old to
   // the block sums
 #pragma unroll
