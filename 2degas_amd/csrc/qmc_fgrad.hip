@@ -99,10 +99,10 @@ __global__ __launch_bounds__((PairShape<false, P>::T), 4) void k_fgrad(DevSys s,
     constexpr bool ALL = decltype(allc)::value;
     pair_run<S, P>(
         s, wv, l,
-        [&](const TpInfo* T, int i, int j) {
+        [&](TpPtr T, int tp, int i, int j) {
           const TabRef tb{T->row[TK_B], T->ng[TK_B]};
           if (tb.row0 < 0) return;
-          const int tp = (int)(T - s.tpi), ti = tp == 2, tj = tp >= 1;
+          const int ti = tp == 2, tj = tp >= 1;
           const double2 xi2 = ld2(xs, i), xj2 = ld2(xs, j);
           const PairGeo p = pair_geo(s, xi2.x, xi2.y, xj2.x, xj2.y);
           double eta, deta, ddeta;

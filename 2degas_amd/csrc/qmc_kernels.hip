@@ -261,7 +261,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
     double hb = 0.0, vb = 0.0;              // the block pair's Laplacian and potential
     pair_run<S, P>(
         s, wv, l,
-        [&](const TpInfo* T, int i, int j) {
+        [&](TpPtr T, int, int i, int j) {
           const TabRef tu2{T->row[TK_U2], T->ng[TK_U2]}, tu3{T->row[TK_U3], T->ng[TK_U3]},
               tb{T->row[TK_B], T->ng[TK_B]}, tv{T->row[TK_V], T->ng[TK_V]};
           const double2 xi2 = ld2(xs, i), xj2 = ld2(xs, j);
@@ -348,7 +348,7 @@ __device__ __forceinline__ void k_pairs_body(const DevSys& s, const WsLayout& L,
     double hb = 0.0;
     pair_run<S, P>(
         s, wv, l,
-        [&](const TpInfo* T, int i, int j) {
+        [&](TpPtr T, int, int i, int j) {
           const TabRef tu3{T->row[TK_U3], T->ng[TK_U3]};
           if (tu3.row0 < 0) return;
           const double2 xi2 = ld2(xs, i), xj2 = ld2(xs, j);
